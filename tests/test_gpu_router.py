@@ -50,6 +50,15 @@ def test_router_topk(gpu, dtype, T, H, E, K):
     assert torch.equal(scores != 0, torch.zeros_like(scores, dtype=torch.bool).scatter_(1, idx, topw != 0))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H,E,K", [(500, 16, 16, 16), (500, 16, 64, 8), (95, 1040, 64, 9), (161, 528, 256, 16), (64, 96, 129, 3),
+                                     (31, 2880, 128, 1)])
+def test_router_topk_lane_groups(gpu, dtype, T, H, E, K):
+    """One, two, four and eight blocks of 32 experts (8 to 32 lanes per token, 4 or 8 logits each), more picks than lanes
+    per token, contractions shorter than a step per wave and with every kind of remainder."""
+    test_router_topk(gpu, dtype, T, H, E, K)
+
+
 def test_router_ties_pick_lower_expert(gpu):
     from yamoe_amd import _cabi
     # identical weight rows give identical logits: the pick order must be by expert id

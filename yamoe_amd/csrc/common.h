@@ -135,6 +135,14 @@ __device__ inline void copy16_to_lds(const void *uniform_base, uint32_t lane_byt
                : "memory", "m0");
 }
 
+// the same from a full address per lane
+__device__ inline void copy16_to_lds(const char *lane_addr, uint32_t lds_base) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(lane_addr), "s"(__builtin_amdgcn_readfirstlane(lds_base))
+               : "memory", "m0");
+}
+
 // ---- schedule: device-built work lists shared by the expert GEMM kernels ---------------------
 // Layout of the schedule region (int32 words):
 //   [0] n_row_tiles   number of (expert, row-block) entries for the MFMA kernels

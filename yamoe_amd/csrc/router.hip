@@ -4,13 +4,15 @@
 //
 // A workgroup takes 32 tokens.  logits[32, E] = x[32, H] * W[E, H]^T: both operands are k-contiguous in memory,
 // which is exactly the register layout of the 32x32x16 MFMA operands (lane l holds 8 consecutive k of row l % 32,
-// starting at 8 * (l / 32)), so fragments go from global memory straight into registers, no LDS.  (fp32: a lane's
+// starting at 8 * (l / 32)), so a fragment is one 16-byte read.  (fp32: a lane's
 // 16 bytes are 4 consecutive k starting at 4 * (l / 32), fed to four v_mfma_f32_32x32x2_f32, whose two lane halves are
-// the two k of an instruction: any pairing of k values is fine as long as both operands use the same.)  The four waves
-// split the contraction, their partial tiles meet in LDS, the bias is added and the logits are rounded to the
-// activation dtype as the reference's linear does.  Then one thread per token picks the top-k (ties: lowest expert
-// id first) and the softmax of the k picked values is computed in fp32, rounded once, and scattered into the dense
+// the two k of an instruction: any pairing of k values is fine as long as both operands use the same.)  Four waves
+// split the contraction of a block of 32 experts, their partial tiles meet in LDS, the bias is added and the logits are
+// rounded to the activation dtype as the reference's linear does.  Then the lanes of a token pick the top-k together (ties: lowest
+// expert id first) and the softmax of the k picked values is computed in fp32, rounded once, and written into the dense
 // [T, E] score row (zero elsewhere).
+#include <type_traits>
+
 #include "common.h"
 
 namespace yamoe {
@@ -39,102 +41,201 @@ template <> struct RouterMma<float> {
   }
 };
 
-// NB = number of 32-expert column blocks (E <= 32 * NB)
-template <typename T, int NB>
-__global__ __launch_bounds__(kRouterThreads) void router_topk_kernel(const T *__restrict__ x, const T *__restrict__ w,
+// NB = number of 32-expert column blocks (E <= 32 * NB), WB = how many of them a wave computes.  A workgroup has
+// 4 * NB / WB waves: in every chunk of the contraction (128 bytes of a row, four steps) wave w takes step w % 4 of the
+// blocks starting at (w / 4) * WB, so every logit is summed in the same order whatever NB is.
+//
+// What bounds it is getting the operands in: a workgroup reads its 32 token rows and all E weight rows, 32 * (1 + NB) * 128
+// bytes per chunk against a handful of MFMAs.  The chunks come in by asynchronous copies of whole 128-byte pieces, eight
+// rows per instruction, into a ring of S stages (S - 1 chunks on their way while one is used).  Fragments fetched
+// straight from global memory touch 32 cache lines per instruction for 32 bytes of each, which the L1's tag rate holds at
+// 30 us for one token and 58 us for 8192 on a [128, 2880] router (17.7 and 20.1 us this way).
+//
+// The pick is made by the lanes of the token together: L = 8 * NB / WB lanes hold 32 * NB / L consecutive logits each in
+// registers, and every round is a maximum over the lane's own values followed by log2(L) exchanges.  (One thread per
+// token walking its row in LDS, the picks in scratch memory, took 90 of the kernel's 103 us at 1536 tokens of 2048 values,
+// 64 experts, top-8, which takes 13.3 us now.)
+template <int NB> struct RouterRing {
+  static constexpr int kRows = kRouterTokens + 32 * NB;
+  static constexpr int kStage = kRows * 128;
+  static constexpr int S = NB <= 2 ? 8 : NB <= 4 ? 6 : 4;  // 64, 96, 120, 144 KB
+  static constexpr int kLd = 32 * NB + 1;                  // padded row of the logits tile, which takes the ring's place
+  static constexpr int kBytes = S * kStage;
+  static_assert(kRouterTokens * kLd * 4 <= kBytes, "the logits tile fits the ring");
+};
+
+// a logit as an unsigned number in the same order (equal floats give equal numbers: -0 becomes +0 first); 0 is below all
+__device__ inline uint32_t router_order(float v) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, v + 0.0f);
+  return (b & 0x80000000u) ? max(~b, 1u) : (b | 0x80000000u);  // (the lowest is a NaN's: it stays above the 0 of "taken")
+}
+__device__ inline float router_unorder(uint32_t o) {
+  return __builtin_bit_cast(float, (o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
+}
+
+template <typename T, int NB, int WB>
+__global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(const T *__restrict__ x, const T *__restrict__ w,
                                                                      const T *__restrict__ bias, int Tn, int H, int E, int K,
                                                                      long long *__restrict__ indices, T *__restrict__ scores,
                                                                      T *__restrict__ topk_weights, T *__restrict__ logits_out) {
-  constexpr int kLd = 32 * NB + 1;  // padded row of the logits tile
-  __shared__ float tile[kRouterTokens * kLd];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int kThreads = kRouterThreads * NB / WB, kWaves = kThreads / kWave;
+  typedef RouterRing<NB> R;
+  constexpr int kLd = R::kLd, S = R::S;
+  extern __shared__ __attribute__((aligned(16))) char ring[];
+  float *tile = (float *)ring;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kq = wave & 3, nb0 = (wave >> 2) * WB;
   const int rl = lane & 31, g = lane >> 5;
   const int t0 = blockIdx.x * kRouterTokens;
 
-  for (int i = tid; i < kRouterTokens * kLd; i += kRouterThreads) tile[i] = 0.0f;
-  __syncthreads();
-
-  f32x16 acc[NB];
+  f32x16 acc[WB];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
+  for (int nb = 0; nb < WB; ++nb)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[nb][v] = 0.0f;
 
-  // rows past the end re-read the last valid one; their results are never used
-  constexpr int V = 16 / (int)sizeof(T);  // elements of a lane's 16 bytes; a step of the contraction is 2 * V of them
-  const T *xa = x + (long long)min(t0 + rl, Tn - 1) * H + g * V;
-  const T *wb[NB];
+  // Copies: copy q of a chunk brings rows 8 q + lane / 8 of the stage (32 token rows, then the weight rows), 16 bytes per
+  // lane; position lane % 8 of row r holds piece pos ^ ((r >> 1) & 7), so that 32 lanes reading one piece of 32 rows touch
+  // every bank.  Wave w issues copies w, w + kWaves, ...  Rows past the end re-read the last valid one, pieces past the
+  // end of a row its first; their products are never used.
+  constexpr int kCopies = R::kRows / 8, kPerWave = (kCopies + kWaves - 1) / kWaves;
+  constexpr int kFewer = kPerWave * kWaves - kCopies;  // the last kFewer waves issue one copy less
+  const bool fewer = wave >= kWaves - kFewer;
+  const int row_bytes = H * (int)sizeof(T);
+  const char *src[kPerWave];
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) wb[nb] = w + (long long)min(nb * 32 + rl, E - 1) * H + g * V;
-
-  const int n_steps = H / (2 * V);
-  for (int s = wave; s < n_steps; s += 4) {
-    u32x4 fa = *(const u32x4 *)(xa + s * 2 * V);
-    u32x4 fb[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) fb[nb] = *(const u32x4 *)(wb[nb] + s * 2 * V);
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) RouterMma<T>::run(fa, fb[nb], acc[nb]);
+  for (int i = 0; i < kPerWave; ++i) {
+    const int row = 8 * (wave + i * kWaves) + (lane >> 3);
+    src[i] = row < kRouterTokens ? (const char *)x + (long long)min(t0 + row, Tn - 1) * row_bytes
+                                 : (const char *)w + (long long)min(row - kRouterTokens, E - 1) * row_bytes;
   }
-  // acc[nb][v]: token 8 * (v / 4) + 4 * g + v % 4, expert nb * 32 + rl; the four waves add up in LDS, one after another
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)ring);
+  auto issue = [&](int chunk, int stage) {
+#pragma unroll
+    for (int i = 0; i < kPerWave; ++i) {
+      if (i == kPerWave - 1 && fewer) break;
+      const int row = 8 * (wave + i * kWaves) + (lane >> 3);
+      int at = chunk * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+      if (at >= row_bytes) at = 0;
+      copy16_to_lds(src[i] + at, lds0 + (uint32_t)(stage * R::kStage + 8 * (wave + i * kWaves) * 128));
+    }
+  };
+  // every copy but those of the youngest `chunks` has landed
+  auto wait_but = [&](auto chunks) {
+    constexpr int C = decltype(chunks)::value;
+    if (kFewer > 0 && fewer) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C * (kPerWave - 1)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C * kPerWave) : "memory");
+  };
+  const int n_steps = row_bytes / 32, n_chunks = (n_steps + 3) / 4;
+  const int rd = rl * 128 + (((2 * kq + g) ^ ((rl >> 1) & 7)) << 4);
+  auto use = [&](int chunk, int stage) {
+    if (4 * chunk + kq < n_steps) {
+      const char *st = ring + stage * R::kStage + rd;
+      const u32x4 fa = *(const u32x4 *)st;
+#pragma unroll
+      for (int nb = 0; nb < WB; ++nb) RouterMma<T>::run(fa, *(const u32x4 *)(st + (1 + nb0 + nb) * 4096), acc[nb]);
+    }
+  };
+#pragma unroll
+  for (int c = 0; c < S - 1; ++c)
+    if (c < n_chunks) issue(c, c);
+  int c = 0, stage = 0;
+  for (; c + S - 1 < n_chunks; ++c) {
+    wait_but(std::integral_constant<int, S - 2>());
+    __syncthreads();  // chunk c is there for every wave, and nobody reads the stage of chunk c - 1 any more
+    const int free_stage = stage == 0 ? S - 1 : stage - 1;
+    issue(c + S - 1, free_stage);
+    use(c, stage);
+    stage = stage == S - 1 ? 0 : stage + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  for (; c < n_chunks; ++c) {
+    use(c, stage);
+    stage = stage == S - 1 ? 0 : stage + 1;
+  }
+  __syncthreads();  // the ring is dead: the logits tile takes its place
+  // acc[nb][v]: token 8 * (v / 4) + 4 * g + v % 4, expert (nb0 + nb) * 32 + rl; the four waves of a block add up in LDS,
+  // one after another
   for (int turn = 0; turn < 4; ++turn) {
-    if (wave == turn) {
+    if (kq == turn) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
+      for (int nb = 0; nb < WB; ++nb)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) tile[(8 * (v >> 2) + 4 * g + (v & 3)) * kLd + nb * 32 + rl] += acc[nb][v];
+        for (int v = 0; v < 16; ++v) {
+          float *at = tile + (8 * (v >> 2) + 4 * g + (v & 3)) * kLd + (nb0 + nb) * 32 + rl;
+          *at = turn == 0 ? acc[nb][v] : *at + acc[nb][v];
+        }
     }
     __syncthreads();
   }
-  // bias, rounding to the activation dtype (the value the reference's top-k sees)
-  for (int i = tid; i < kRouterTokens * 32 * NB; i += kRouterThreads) {
-    int r = i / (32 * NB), e = i - r * (32 * NB);
+
+  // The L lanes of token r take its logits M * sub .. M * sub + M - 1: bias, rounding to the activation dtype (the value
+  // the reference's top-k sees), and the sortable form; experts past the end are 0, below every logit.
+  constexpr int L = kThreads / kRouterTokens, M = 32 * NB / L;
+  const int r = tid / L, sub = tid % L;
+  const long long t = t0 + r;
+  uint32_t key[M];
+  float prob[M];
+#pragma unroll
+  for (int j = 0; j < M; ++j) {
+    const int e = sub * M + j;
+    key[j] = 0u;
+    prob[j] = 0.0f;
     if (e < E) {
-      float v = tile[r * kLd + e] + (bias != nullptr ? ElemTraits<T>::to_f32(bias[e]) : 0.0f);
-      T q = ElemTraits<T>::from_f32(v);
-      tile[r * kLd + e] = ElemTraits<T>::to_f32(q);
-      if (logits_out != nullptr && t0 + r < Tn) logits_out[(long long)(t0 + r) * E + e] = q;
+      const T q = ElemTraits<T>::from_f32(tile[r * kLd + e] + (bias != nullptr ? ElemTraits<T>::to_f32(bias[e]) : 0.0f));
+      key[j] = router_order(ElemTraits<T>::to_f32(q));
+      if (logits_out != nullptr && t < Tn) logits_out[t * E + e] = q;
     }
   }
-  __syncthreads();
-  // dense score rows start at zero
-  for (int i = tid; i < kRouterTokens * E; i += kRouterThreads) {
-    int r = i / E, e = i - r * E;
-    if (t0 + r < Tn) scores[(long long)(t0 + r) * E + e] = ElemTraits<T>::from_f32(0.0f);
+  float first = 0.0f, sum = 0.0f;
+  float mine[kRouterMaxK / 8] = {};  // lane `sub` keeps the weights of picks sub and (8 lanes per token) sub + 8
+  for (int k = 0; k < K; ++k) {
+    uint32_t best = 0u;
+    int at = 0;
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+      if (key[j] > best) { best = key[j]; at = sub * M + j; }
+#pragma unroll
+    for (int d = 1; d < L; d <<= 1) {
+      const uint32_t other = (uint32_t)__shfl_xor((int)best, d);
+      const int other_at = __shfl_xor(at, d);
+      // ties: the lower expert id (the lower lane holds the lower ids)
+      if (other > best || (other == best && other_at < at)) { best = other; at = other_at; }
+    }
+    const float v = router_unorder(best);
+    if (k == 0) first = v;
+    const float p = expf(v - first);
+    sum += p;
+#pragma unroll
+    for (int j = 0; j < M; ++j)
+      if (at == sub * M + j) { key[j] = 0u; prob[j] = p; }
+#pragma unroll
+    for (int i = 0; i < kRouterMaxK / 8; ++i)
+      if (k == sub + i * L) mine[i] = p;
+    if (sub == 0 && t < Tn) indices[t * K + k] = at;
   }
-  __syncthreads();
-  if (tid < kRouterTokens && t0 + tid < Tn) {
-    float *row = tile + tid * kLd;
-    const long long t = t0 + tid;
-    int pick[kRouterMaxK];
-    float val[kRouterMaxK];
-    for (int k = 0; k < K; ++k) {
-      int best = -1;
-      float bv = 0.0f;
-      for (int e = 0; e < E; ++e) {
-        float v = row[e];
-        bool taken = false;
-        for (int j = 0; j < k; ++j) taken |= pick[j] == e;
-        if (!taken && (best < 0 || v > bv)) { best = e; bv = v; }
-      }
-      pick[k] = best;
-      val[k] = bv;
-    }
-    float sum = 0.0f, p[kRouterMaxK];
-    for (int k = 0; k < K; ++k) { p[k] = expf(val[k] - val[0]); sum += p[k]; }
-    for (int k = 0; k < K; ++k) {
-      T q = ElemTraits<T>::from_f32(p[k] / sum);
-      indices[t * K + k] = pick[k];
-      scores[t * E + pick[k]] = q;
-      if (topk_weights != nullptr) topk_weights[t * K + k] = q;
-    }
+  if (t >= Tn) return;
+#pragma unroll
+  for (int j = 0; j < M; ++j) {
+    const int e = sub * M + j;
+    if (e < E) scores[t * E + e] = ElemTraits<T>::from_f32(prob[j] == 0.0f ? 0.0f : prob[j] / sum);
+  }
+  if (topk_weights != nullptr) {
+#pragma unroll
+    for (int i = 0; i < kRouterMaxK / 8; ++i)
+      if (sub + i * L < K) topk_weights[t * K + sub + i * L] = ElemTraits<T>::from_f32(mine[i] / sum);
   }
 }
 
-template <typename T, int NB>
+template <typename T, int NB, int WB>
 static int launch_router(const void *x, const void *w, const void *bias, int Tn, int H, int E, int K, long long *indices,
                          void *scores, void *topk_weights, void *logits, hipStream_t stream) {
-  hipLaunchKernelGGL((router_topk_kernel<T, NB>), dim3(ceil_div(Tn, kRouterTokens)), dim3(kRouterThreads), 0, stream,
+  auto kernel = router_topk_kernel<T, NB, WB>;
+  static DeviceFlags attr_done;  // one per kernel instantiation
+  if (int rc = ensure_dynamic_lds((const void *)kernel, RouterRing<NB>::kBytes, attr_done, "router_topk_kernel")) return rc;
+  hipLaunchKernelGGL(kernel, dim3(ceil_div(Tn, kRouterTokens)), dim3(kRouterThreads * NB / WB), RouterRing<NB>::kBytes, stream,
                      (const T *)x, (const T *)w, (const T *)bias, Tn, H, E, K, indices, (T *)scores, (T *)topk_weights,
                      (T *)logits);
   return check_launch("router_topk_kernel");
@@ -144,10 +245,10 @@ template <typename T>
 static int router_dispatch(const void *x, const void *w, const void *bias, int Tn, int H, int E, int K, long long *indices,
                            void *scores, void *topk_weights, void *logits, hipStream_t stream) {
   int nb = ceil_div(E, 32);
-  if (nb <= 1) return launch_router<T, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  if (nb <= 2) return launch_router<T, 2>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  if (nb <= 4) return launch_router<T, 4>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  return launch_router<T, 8>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  if (nb <= 1) return launch_router<T, 1, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  if (nb <= 2) return launch_router<T, 2, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  if (nb <= 4) return launch_router<T, 4, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  return launch_router<T, 8, 2>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
 }
 
 // ---- gradient of the step, first part: from the gradient of the dense scores to the gradient of the logits --------
