@@ -77,20 +77,19 @@ int stream_gate_up(const void *, const int *, const void *, const void *, void *
 template <typename T>
 int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
 
-template <typename T>
+template <typename T, bool RAGGED>
 int gemm_async_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
                        int, int, int, int, hipStream_t);
-template <typename T>
+template <typename T, bool RAGGED>
 int gemm_async_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, int,
                     hipStream_t);
-template <typename T>
+template <typename T, bool RAGGED>
 int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
                      const void *, float *, hipStream_t);
 template <typename T>
 int gemm_async_wgrad(const void *, const int *, int, int, const void *, void *, void *, const int *, const int *, int, int,
                      int, int, hipStream_t);
 bool wgrad_writes_bias(int Md, int Nd);
-bool gemm_async_supported(int Kd, int Nd, int lda, int ldb, long long a_span_bytes);
 bool gemm_f32_supported(int Kd, int Nd, int lda, int ldb, long long a_span_bytes);
 int gemm_f32_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
                      int, int, hipStream_t);
@@ -114,37 +113,44 @@ template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
 template <typename T> struct HasStreamPath { static constexpr bool value = sizeof(T) == 2; };
 
-// The MFMA tile kernels for the two forward products: the asynchronous-copy pipeline when the dtype
-// and shape allow it, the register-staged kernel otherwise.
-template <typename T>
+static int gathered_span_ok(const char *who, long long span_bytes) {
+  if (span_bytes < (1ll << 32)) return 0;
+  set_error("%s: gathered rows span 4 GiB or more", who);
+  return YAMOE_E_ARG;
+}
+
+// The MFMA tile kernels for the two forward products: 16-bit data on the asynchronous-copy pipeline (contractions that are
+// not multiples of 64 in instantiations of their own), fp32 on its own when the shape allows it and on the
+// register-staged kernel otherwise.
 // `small_rows`: experts with at most this many kept rows are on the schedule's streaming list, not tiled (0 when
 // unknown); it only tightens the grid.
 // sorted_idx == nullptr: x holds one row per sorted row, in order (the callers permute a hidden_states tensor of 4 GiB or
 // more first: the kernels address gathered rows with 32-bit byte offsets from the start of the tensor).
+template <typename T>
 static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
                          const void *sched, int N, int K, int E, int H, int I, int small_rows, hipStream_t stream) {
+  // the gathered source rows span the whole hidden_states tensor: N / K tokens of H elements
   const long long span = sorted_idx != nullptr ? (long long)(N / K) * H * (long long)sizeof(T) : 0;
+  if (int rc = gathered_span_ok("tiles_gate_up", span)) return rc;
   if constexpr (sizeof(T) == 2) {
-    // the gathered source rows span the whole hidden_states tensor: N / K tokens of H elements
-    if (gemm_async_supported(H, 2 * I, H, 2 * I, span))
-      return gemm_async_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, stream);
+    auto run = H % 64 ? gemm_async_gate_up<T, true> : gemm_async_gate_up<T, false>;
+    return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, stream);
   } else {
     if (gemm_f32_supported(H, 2 * I, H, 2 * I, span))
       return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
+    return gemm_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
   }
-  if (span >= (1ll << 32)) { set_error("tiles_gate_up: gathered rows span 4 GiB or more"); return YAMOE_E_ARG; }
-  return gemm_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
 }
 template <typename T>
 static int tiles_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E,
                       int H, int I, int small_rows, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
-    if (gemm_async_supported(I, H, I, H, 0))
-      return gemm_async_down<T>(act, w, bias, y, sched, N, E, H, I, small_rows, stream);
+    auto run = I % 64 ? gemm_async_down<T, true> : gemm_async_down<T, false>;
+    return run(act, w, bias, y, sched, N, E, H, I, small_rows, stream);
   } else {
     if (gemm_f32_supported(I, H, I, H, 0)) return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
+    return gemm_down<T>(act, w, bias, y, sched, N, E, H, I, stream);
   }
-  return gemm_down<T>(act, w, bias, y, sched, N, E, H, I, stream);
 }
 
 // g_rows == nullptr: g holds one row per sorted row; otherwise row p of the product reads g[g_rows[p] / g_div]
@@ -154,12 +160,14 @@ template <typename T>
 static int tiles_dgrad(const void *g, const int *g_rows, int g_div, long long g_span_bytes, const void *w, void *out,
                        const void *sched, int N, int E, int Kd, int Nd, const void *dot_with, float *dot_part,
                        hipStream_t stream) {
+  if (g_rows != nullptr)
+    if (int rc = gathered_span_ok("tiles_dgrad", g_span_bytes)) return rc;
   if constexpr (sizeof(T) == 2) {
-    if (gemm_async_supported(Kd, Nd, Kd, Kd, g_rows ? g_span_bytes : 0))
-      return gemm_async_dgrad<T>(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
+    auto run = Kd % 64 ? gemm_async_dgrad<T, true> : gemm_async_dgrad<T, false>;
+    return run(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
+  } else {
+    return gemm_dgrad<T>(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
   }
-  if (g_rows != nullptr && g_span_bytes >= (1ll << 32)) { set_error("tiles_dgrad: gathered rows span 4 GiB or more"); return YAMOE_E_ARG; }
-  return gemm_dgrad<T>(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
 }
 
 // True when the weight-gradient kernel for this dtype and shape can gather the rows of its left operand by token

@@ -1,0 +1,488 @@
+// Grouped weight gradients for 16-bit data on gfx950, on the asynchronous-copy pipeline of gemm_async_tile.h.
+#include "gemm_async_tile.h"
+
+namespace yamoe {
+
+namespace async {
+
+constexpr int kBN = 256;
+
+// ---- weight gradients: dW[e] = L[rows of e]^T * R[rows of e] -----------------------------------------------
+// (csrc/experts_backward.cu:198, 311).  The contraction runs over the expert's kept rows, so both operands are
+// [k][m] / [k][n] in memory: both stay that way in LDS (single-slab buffers of 32 k-rows) and both are read with
+// the LDS transpose read.  The last slab of an expert is usually partial: the copies of its missing rows read
+// whatever follows in memory (the caller keeps that readable) and the wave that issued them overwrites them with
+// zeros in LDS before anybody reads the slab.
+struct WgradArgs {
+  const void *A;  // [N, Md] rows in expert order; with a_rows: [*, Md], sorted row p is row a_rows[p] / a_div of it
+  const void *B;  // [N, Nd]
+  void *C;        // [E, Md, Nd]
+  const int *counts, *offsets;
+  const int *a_rows;
+  FastDiv a_div;
+  int a_rows_max;  // largest value a_rows may hold
+  int capacity, E, Md, Nd, n_m_tiles, n_n_tiles;
+  // optional: [E, Nd] column sums of the expert's rows of B (the bias gradient that goes with this weight gradient,
+  // csrc/experts_backward.cu:277, 308); needs Md % 128 != 0 (see wgrad_writes_bias)
+  void *bias_grad;
+};
+
+template <bool P1_, bool P2_, bool NEXT_, bool ZERO_, int VM_> struct WStepCfg {
+  static constexpr bool P1 = P1_, P2 = P2_, NEXT = NEXT_, ZERO = ZERO_;
+  static constexpr int VM = VM_;
+};
+
+// 128 x 256 tiles with a three-slab ring (72 KB of LDS, at most 256 registers per lane), so that two workgroups
+// share a CU: an expert's contraction is short (its kept rows), a tile spends a third of its time filling the ring
+// and storing its result, and with a second workgroup on the same SIMDs the matrix pipe works through that.
+constexpr int kSmallBM = 128, kSmallStages = 3;
+constexpr int kSmallAStage = kBK * kSmallBM * 2, kSmallBStage = kBK * kBN * 2;  // 8 KB + 16 KB per slab
+constexpr int kSmallBRing = kSmallStages * kSmallAStage;
+constexpr int kSmallRing = kSmallStages * (kSmallAStage + kSmallBStage);
+constexpr int kSmallStaging = kSmallBM * (kBN * 2 + 16);
+constexpr int kSmallLds = kSmallRing > kSmallStaging ? kSmallRing : kSmallStaging;
+
+// bias_tile: this is the last row tile of the gradient and has room below its rows_m valid rows.  Column rows_m of the
+// left operand's LDS tile then holds 1 for every valid k (planted after each slab's copies have landed), so that row
+// rows_m of the product is 1^T . R, the column sums of the expert's rows of R: the bias gradient, taken by the same
+// MFMAs in fp32 instead of by a launch of its own over the same rows (17.5 + 37 us at the GPT-OSS-20B shape).
+template <typename T, int NMI, bool GATHER>
+__device__ inline void run_wgrad_tile_small(const WgradArgs &args, const int tid, const int expert, const int m0,
+                                            const int n0, const int rows_m, const long long first, const int rows,
+                                            const bool bias_tile) {
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  constexpr int NACC = NMI > 0 ? NMI : 1;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
+
+  f32x16 acc[NACC][4];
+#pragma unroll
+  for (int mi = 0; mi < NACC; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0.0f;
+
+  const int n_slabs = (rows + kBK - 1) / kBK;
+  const long long lda_bytes = (long long)args.Md * (long long)sizeof(T), ldb_bytes = (long long)args.Nd * (long long)sizeof(T);
+
+  // A copies: piece i (0..1) = k rows 4*(2*wave + i) + (lane >> 4) of the slab, 256 bytes each; LDS position lane & 15
+  // holds piece pos ^ ((k & 3) << 2).  B copies as in the large kernel: piece i (0..3) = k rows 8*wave + 2*i + (lane >> 5).
+  uint32_t a_off[2], b_off[4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    int k = 4 * (2 * wave + i) + (lane >> 4);
+    int piece = (lane & 15) ^ ((k & 3) << 2);
+    int ca = m0 + piece * 8;
+    if (ca >= args.Md) ca = m0;
+    a_off[i] = (uint32_t)((GATHER ? 0ll : k * lda_bytes) + (long long)(ca - m0) * (long long)sizeof(T));
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int k = 8 * wave + 2 * i + (lane >> 5);
+    int piece = (lane & 31) ^ ((k & 3) << 2);
+    int cb = n0 + piece * 8;
+    if (cb >= args.Nd) cb = n0;
+    b_off[i] = (uint32_t)(k * ldb_bytes + (long long)(cb - n0) * (long long)sizeof(T));
+  }
+  const char *a_base = (const char *)((const T *)args.A + (GATHER ? 0ll : first * args.Md) + m0);
+  const char *b_base = (const char *)((const T *)args.B + first * args.Nd + n0);
+  // Gathered A rows: the four k rows of piece i of a slab are rows a_rows[first + 32*slab + 4*(2*wave + i) + 0..3]
+  // / a_div of A.  The positions are the same for the whole wave, so the look-ups are scalar loads (rows_of), issued
+  // at the start of the half slab whose last slot issues the copy; there the lane picks its row and turns it into a
+  // byte offset (row_bytes).  Positions past the expert's rows (up to 31 past the end of the list: the caller keeps
+  // that readable) hold somebody else's row or anything at all: the value is clamped to the list's range, and what the
+  // copy fetches is zeroed in LDS before use.  The list is read through the constant address space, which makes the loads scalar whatever the
+  // compiler can prove about the memory in between (the list was written by an earlier launch).
+  typedef const __attribute__((address_space(4))) int *ConstInts;
+  ConstInts a_rows = GATHER ? (ConstInts)(uintptr_t)(args.a_rows + first) : (ConstInts)0;
+  auto rows_of = [&](int slab, int i, int (&ix)[4]) {
+    if constexpr (GATHER) {
+      const int k0 = slab * kBK + 4 * (2 * wave + i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ix[j] = a_rows[k0 + j];
+    }
+  };
+  auto row_bytes = [&](int (&ix)[4]) -> uint32_t {
+    if constexpr (!GATHER) return 0u;
+    // the four values pass through an empty statement: the loads stay where rows_of put them, all four of them, and
+    // what follows is three selects rather than loads under branches
+    int r0 = ix[0], r1 = ix[1], r2 = ix[2], r3 = ix[3];
+    asm volatile("" : "+s"(r0), "+s"(r1), "+s"(r2), "+s"(r3));
+    const bool odd = (lane & 16) != 0, high = (lane & 32) != 0;
+    const int lo = odd ? r1 : r0, hi = odd ? r3 : r2;
+    const uint32_t r = min((uint32_t)(high ? hi : lo), (uint32_t)args.a_rows_max);
+    return (uint32_t)fast_div((int)r, args.a_div) * (uint32_t)lda_bytes;
+  };
+  auto copy_a = [&](int slab, int i, uint32_t row) {
+    copy16_to_lds(a_base + (GATHER ? 0ll : (long long)slab * kBK * lda_bytes), a_off[i] + row,
+                  lds0 + (uint32_t)(slab % kSmallStages) * kSmallAStage + (uint32_t)(4 * (2 * wave + i)) * 256u);
+  };
+  auto copy_a_now = [&](int slab, int i) {  // look-up and copy in one go: outside the pipelined loop
+    int ix[4] = {0, 0, 0, 0};
+    rows_of(slab, i, ix);
+    copy_a(slab, i, row_bytes(ix));
+  };
+  auto copy_b = [&](int slab, int i) {
+    copy16_to_lds(b_base + (long long)slab * kBK * ldb_bytes, b_off[i],
+                  lds0 + kSmallBRing + (uint32_t)(slab % kSmallStages) * kSmallBStage + (uint32_t)(8 * wave + 2 * i) * 512u);
+  };
+  auto copy_slab = [&](int slab) {
+    copy_a_now(slab, 0); copy_b(slab, 0); copy_b(slab, 1); copy_a_now(slab, 1); copy_b(slab, 2); copy_b(slab, 3);
+  };
+  auto zero_tail = [&](int slab) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      int k = 4 * (2 * wave + i) + (lane >> 4);
+      if (slab * kBK + k >= rows)
+        *(u32x4 *)(lds + (slab % kSmallStages) * kSmallAStage + 4 * (2 * wave + i) * 256 + lane * 16) = (u32x4){0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      int k = 8 * wave + 2 * i + (lane >> 5);
+      if (slab * kBK + k >= rows)
+        *(u32x4 *)(lds + kSmallBRing + (slab % kSmallStages) * kSmallBStage + (8 * wave + 2 * i) * 512 + lane * 16) = (u32x4){0, 0, 0, 0};
+    }
+  };
+
+  // the ones column of slab `slab` (whose copies by this wave have landed): this wave's 8 k rows; lane l and the seven
+  // lanes l + 8 j write the same value to the same place (a branch on the lane number here would be the loop's only
+  // divergent one)
+  const int ones_k = 8 * wave + (lane & 7);
+  char *const ones_at = lds + ones_k * 256 + (((rows_m >> 3) ^ ((ones_k & 3) << 2)) << 4) + (rows_m & 7) * 2;
+  auto plant_ones = [&](int slab) {
+    if (bias_tile)
+      *(T *)(ones_at + (slab % kSmallStages) * kSmallAStage) = ElemTraits<T>::from_f32(slab * kBK + ones_k < rows ? 1.0f : 0.0f);
+  };
+
+  const int g = lane >> 5, rl = lane & 31, j4 = (lane & 15) >> 2, q4 = lane & 3;
+  int a_rd[NACC], b_rd[4];
+#pragma unroll
+  for (int mi = 0; mi < NACC; ++mi) {
+    int col = (mi * 2 + wm) * 32 + 16 * ((lane >> 4) & 1) + 4 * q4;
+    a_rd[mi] = (g * 8 + j4) * 256 + ((((col >> 3) ^ (j4 << 2))) << 4) + (col & 7) * 2;
+  }
+#pragma unroll
+  for (int ni = 0; ni < 4; ++ni) {
+    int col = wn * 128 + ni * 32 + 16 * ((lane >> 4) & 1) + 4 * q4;
+    b_rd[ni] = (g * 8 + j4) * 512 + ((((col >> 3) ^ (j4 << 2))) << 4) + (col & 7) * 2;
+  }
+  u32x4 fa0[NACC], fa1[NACC], fb0[4], fb1[4];
+  constexpr int kFrags = NMI > 0 ? 4 + NMI : 0;
+  // fragment order B0, A0, B1, B2, B3, A1
+  auto read_frag = [&](int s, int ks, int f, u32x4 (&fa)[NACC], u32x4 (&fb)[4]) {
+    const bool is_a = f == 1 || f >= 5;
+    const int idx = is_a ? (f == 1 ? 0 : f - 4) : (f == 0 ? 0 : f - 1);
+    const char *sp = is_a ? lds + (s % kSmallStages) * kSmallAStage + a_rd[idx] + ks * 4096
+                          : lds + kSmallBRing + (s % kSmallStages) * kSmallBStage + b_rd[idx] + ks * 8192;
+    u32x2 lo = lds_read_tr16(sp);
+    u32x2 hi = lds_read_tr16(sp + (is_a ? 1024 : 2048));
+    u32x4 v = (u32x4){lo[0], lo[1], hi[0], hi[1]};
+    if (is_a) fa[idx] = v; else fb[idx] = v;
+  };
+  auto read_frags = [&](int s, int ks, u32x4 (&fa)[NACC], u32x4 (&fb)[4]) {
+#pragma unroll
+    for (int f = 0; f < kFrags; ++f) read_frag(s, ks, f, fa, fb);
+  };
+
+  // pipeline: slab t+3 goes into the buffer slab t leaves at its mid-slab barrier: first half of its copies
+  // (A piece 0, B pieces 0-1) in the second k-step of slab t, second half in the first k-step of slab t+1; "slab
+  // s+1 has landed" = at most 6 younger copies in flight
+  constexpr int kMma = 4 * NMI;
+  constexpr int kSlots = kMma > 2 ? kMma - 2 : 1;
+  if (n_slabs > 0) {
+#pragma unroll
+    for (int s = 0; s < kSmallStages; ++s)
+      if (s < n_slabs) copy_slab(s);
+    if (n_slabs >= 6) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");  // slab 0 is enough to start with
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    plant_ones(0);
+#pragma unroll
+    for (int s = 0; s < kSmallStages; ++s)
+      if (n_slabs < 6 && s < n_slabs && (s + 1) * kBK > rows) zero_tail(s);
+    __syncthreads();
+    read_frags(0, 0, fa0, fb0);
+  }
+  // In the pipelined loop the ring stage of every slab is a compile-time constant (the loop is unrolled by the ring
+  // depth), so that an operand read is one ds_read with an immediate offset from a per-lane base and a copy's LDS
+  // address one scalar add: with the stage computed per slab (a division by 3, then one vector add per read) the
+  // loop carried 3.4 vector instructions per MFMA, 30 of them in a block ahead of each slab's first MFMA.
+  const char *pa[NACC], *pb[4];
+#pragma unroll
+  for (int mi = 0; mi < NACC; ++mi) pa[mi] = lds + a_rd[mi];
+#pragma unroll
+  for (int ni = 0; ni < 4; ++ni) pb[ni] = lds + kSmallBRing + b_rd[ni];
+  const uint32_t lds_a_wave = lds0 + (uint32_t)(8 * wave) * 256u, lds_b_wave = lds0 + kSmallBRing + (uint32_t)(8 * wave) * 512u;
+  auto read_frag_c = [&](auto stage, int ks, int f, u32x4 (&fa)[NACC], u32x4 (&fb)[4]) {
+    constexpr int ST = decltype(stage)::value;
+    const bool is_a = f == 1 || f >= 5;
+    const int idx = is_a ? (f == 1 ? 0 : f - 4) : (f == 0 ? 0 : f - 1);
+    const char *sp = is_a ? pa[idx] + ST * kSmallAStage + ks * 4096 : pb[idx] + ST * kSmallBStage + ks * 8192;
+    u32x2 lo = lds_read_tr16(sp);
+    u32x2 hi = lds_read_tr16(sp + (is_a ? 1024 : 2048));
+    u32x4 v = (u32x4){lo[0], lo[1], hi[0], hi[1]};
+    if (is_a) fa[idx] = v; else fb[idx] = v;
+  };
+  auto copy_a_c = [&](auto stage, int slab, int i, uint32_t row) {
+    constexpr int ST = decltype(stage)::value;
+    copy16_to_lds(a_base + (GATHER ? 0ll : (long long)slab * kBK * lda_bytes), a_off[i] + row,
+                  lds_a_wave + (uint32_t)(ST * kSmallAStage + 4 * i * 256));
+  };
+
+  auto copy_b_c = [&](auto stage, int slab, int i) {
+    constexpr int ST = decltype(stage)::value;
+    copy16_to_lds(b_base + (long long)slab * kBK * ldb_bytes, b_off[i], lds_b_wave + (uint32_t)(ST * kSmallBStage + 2 * i * 512));
+  };
+  // slab s sits in ring stage ST
+  auto slab_step = [&](int s, auto cfg, auto stage) {
+    typedef decltype(cfg) C;
+    constexpr int ST = decltype(stage)::value;
+    typedef std::integral_constant<int, (ST + 1) % kSmallStages> Next;   // slab s + 1
+    typedef std::integral_constant<int, (ST + 2) % kSmallStages> Next2;  // slab s + 2; slab s + 3 takes stage ST again
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      constexpr int kC = C::P1 ? 3 : 0, kItems = kC + kFrags;
+      int ix[4] = {0, 0, 0, 0};  // gathered rows: the four rows of the A piece copied in this half slab
+#pragma unroll
+      for (int j = 0; j < (kMma > 0 ? kMma : 1); ++j) {
+        if (j < kMma) Mma<T>::run(fb0[j & 3], fa0[j >> 2], acc[j >> 2][j & 3]);
+        if (j < kSlots) {
+#pragma unroll
+          for (int i = j * kItems / kSlots; i < (j + 1) * kItems / kSlots; ++i) {
+            if (i < kC) {
+              if (i == 0) { if constexpr (GATHER) rows_of(s + 2, 1, ix); else copy_a_c(Next2(), s + 2, 1, 0u); }
+              else copy_b_c(Next2(), s + 2, 1 + i);
+            }
+            else read_frag_c(stage, 1, i - kC, fa1, fb1);
+          }
+          if (GATHER && kC > 0 && j == kSlots - 1) copy_a_c(Next2(), s + 2, 1, row_bytes(ix));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (C::VM == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if constexpr (C::VM == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (C::NEXT) plant_ones(s + 1);
+    if constexpr (C::ZERO) zero_tail(s + 1);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      constexpr int kC = C::P2 ? 3 : 0, kItems = kC + (C::NEXT ? kFrags : 0);
+      int ix[4] = {0, 0, 0, 0};  // gathered rows: the four rows of the A piece copied in this half slab
+#pragma unroll
+      for (int j = 0; j < (kMma > 0 ? kMma : 1); ++j) {
+        if (j < kMma) Mma<T>::run(fb1[j & 3], fa1[j >> 2], acc[j >> 2][j & 3]);
+        if (j < kSlots) {
+#pragma unroll
+          for (int i = j * kItems / kSlots; i < (j + 1) * kItems / kSlots; ++i) {
+            if (i < kC) {
+              if (i == 0) { if constexpr (GATHER) rows_of(s + 3, 0, ix); else copy_a_c(stage, s + 3, 0, 0u); }
+              else copy_b_c(stage, s + 3, i - 1);
+            }
+            else read_frag_c(Next(), 0, i - kC, fa0, fb0);
+          }
+          if (GATHER && kC > 0 && j == kSlots - 1) copy_a_c(stage, s + 3, 0, row_bytes(ix));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  // the same step with the ring stage taken from the slab number at run time: for the slabs the unrolled loop leaves
+  // over and for the last three (the stage they start in depends on the slab count)
+  auto slab_step_rt = [&](int s, auto cfg) {
+    typedef decltype(cfg) C;
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      constexpr int kC = C::P1 ? 3 : 0, kItems = kC + kFrags;
+      int ix[4] = {0, 0, 0, 0};  // gathered rows: the four rows of the A piece copied in this half slab
+#pragma unroll
+      for (int j = 0; j < (kMma > 0 ? kMma : 1); ++j) {
+        if (j < kMma) Mma<T>::run(fb0[j & 3], fa0[j >> 2], acc[j >> 2][j & 3]);
+        if (j < kSlots) {
+#pragma unroll
+          for (int i = j * kItems / kSlots; i < (j + 1) * kItems / kSlots; ++i) {
+            if (i < kC) {
+              if (i == 0) { if constexpr (GATHER) rows_of(s + 2, 1, ix); else copy_a(s + 2, 1, 0u); }
+              else copy_b(s + 2, 1 + i);
+            }
+            else read_frag(s, 1, i - kC, fa1, fb1);
+          }
+          if (GATHER && kC > 0 && j == kSlots - 1) copy_a(s + 2, 1, row_bytes(ix));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (C::VM == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    else if constexpr (C::VM == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (C::NEXT) plant_ones(s + 1);
+    if constexpr (C::ZERO) zero_tail(s + 1);
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      constexpr int kC = C::P2 ? 3 : 0, kItems = kC + (C::NEXT ? kFrags : 0);
+      int ix[4] = {0, 0, 0, 0};  // gathered rows: the four rows of the A piece copied in this half slab
+#pragma unroll
+      for (int j = 0; j < (kMma > 0 ? kMma : 1); ++j) {
+        if (j < kMma) Mma<T>::run(fb1[j & 3], fa1[j >> 2], acc[j >> 2][j & 3]);
+        if (j < kSlots) {
+#pragma unroll
+          for (int i = j * kItems / kSlots; i < (j + 1) * kItems / kSlots; ++i) {
+            if (i < kC) {
+              if (i == 0) { if constexpr (GATHER) rows_of(s + 3, 0, ix); else copy_a(s + 3, 0, 0u); }
+              else copy_b(s + 3, i - 1);
+            }
+            else read_frag(s + 1, 0, i - kC, fa0, fb0);
+          }
+          if (GATHER && kC > 0 && j == kSlots - 1) copy_a(s + 3, 0, row_bytes(ix));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  if (n_slabs >= 6) {
+    typedef std::integral_constant<int, 0> S0;
+    typedef std::integral_constant<int, 1> S1;
+    typedef std::integral_constant<int, 2> S2;
+    typedef WStepCfg<true, true, true, false, 6> Steady;
+    slab_step(0, WStepCfg<false, true, true, false, 6>(), S0());
+    int s = 1;
+    for (; s + 5 < n_slabs; s += 3) {  // steady state, three slabs per round: stages 1, 2, 0
+      slab_step(s, Steady(), S1());
+      slab_step(s + 1, Steady(), S2());
+      slab_step(s + 2, Steady(), S0());
+    }
+    for (; s + 3 < n_slabs; ++s) slab_step_rt(s, Steady());  // at most two
+    // the last three slabs (s = n_slabs - 3): no new copies; the last slab's missing rows are zeroed
+    slab_step_rt(s, WStepCfg<true, false, true, false, 6>());
+    slab_step_rt(s + 1, WStepCfg<false, false, true, true, 0>());
+    slab_step_rt(s + 2, WStepCfg<false, false, false, false, -1>());
+  } else {
+    for (int s = 0; s < n_slabs; ++s) {
+      if (kFrags > 0) read_frags(s, 1, fa1, fb1);
+#pragma unroll
+      for (int j = 0; j < kMma; ++j) Mma<T>::run(fb0[j & 3], fa0[j >> 2], acc[j >> 2][j & 3]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      if (s + 1 < n_slabs) plant_ones(s + 1);
+      if (s + 1 < n_slabs && (s + 2) * kBK > rows) zero_tail(s + 1);
+      __syncthreads();
+      if (s + kSmallStages < n_slabs) copy_slab(s + kSmallStages);
+      if (s + 1 < n_slabs) read_frags(s + 1, 0, fa0, fb0);
+#pragma unroll
+      for (int j = 0; j < kMma; ++j) Mma<T>::run(fb1[j & 3], fa1[j >> 2], acc[j >> 2][j & 3]);
+    }
+  }
+
+  // epilogue: stage the tile in LDS, store whole row segments
+  constexpr int stride = kBN * 2 + 16;
+  // (operands exchanged in the MFMAs, as in the forward kernel) acc[mi][ni][v]: tile row (mi*2+wm)*32 + lane%32,
+  // tile column wn*128 + ni*32 + 8*(v/4) + 4*(lane/32) + v%4
+  __syncthreads();
+  {
+    char *lp = lds + (wm * 32 + rl) * stride + (wn * 128 + 4 * g) * 2;
+#pragma unroll
+    for (int ni = 0; ni < 4; ++ni)
+#pragma unroll
+      for (int mi = 0; mi < NMI; ++mi)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x16 &a = acc[mi][ni];
+          u32x2 v = {pack2<T>(a[4 * q], a[4 * q + 1]), pack2<T>(a[4 * q + 2], a[4 * q + 3])};
+          *(u32x2 *)(lp + mi * 64 * stride + (ni * 32 + 8 * q) * 2) = v;
+        }
+  }
+  __syncthreads();
+  {
+    constexpr int chunks = kBN >> 3, rows_per_pass = kThreads / chunks;
+    const int c = tid % chunks;
+    if (n0 + c * 8 < args.Nd) {
+      T *p = (T *)args.C + ((long long)expert * args.Md + m0) * args.Nd + n0 + c * 8;
+      for (int r = tid / chunks; r < rows_m; r += rows_per_pass) {
+        // streaming stores: 1.6 GB of gradients per backward pass that nobody reads back soon would otherwise push the
+        // operand tiles out of L2
+        __builtin_nontemporal_store(*(const u32x4 *)(lds + r * stride + c * 16), (u32x4 *)(p + (long long)r * args.Nd));
+      }
+      // the row below the valid ones: the column sums
+      if (bias_tile && tid < chunks)
+        *(u32x4 *)((T *)args.bias_grad + (long long)expert * args.Nd + n0 + c * 8) = *(const u32x4 *)(lds + rows_m * stride + c * 16);
+    }
+  }
+}
+
+template <typename T, bool GATHER>
+__global__ __launch_bounds__(kThreads, 2) void wgrad_small_kernel(const WgradArgs args) {
+  const int tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1;
+  const int per_expert = args.n_m_tiles * args.n_n_tiles;
+  const int total = args.E * per_expert;
+  const int total8 = (total + kXcds - 1) / kXcds * kXcds;
+  const int b = blockIdx.x;
+  if (b >= total8) return;
+  const int L = (b % kXcds) * (total8 / kXcds) + b / kXcds;
+  if (L >= total) return;
+  const int expert = L / per_expert, r = L - expert * per_expert;
+  const int n0 = (r / args.n_m_tiles) * kBN, m0 = (r % args.n_m_tiles) * kSmallBM;
+  const int rows_m = min(kSmallBM, args.Md - m0);
+  // (the same for every lane; said explicitly, so that the operand addresses built from them stay in scalar registers)
+  int rows = min(__builtin_amdgcn_readfirstlane(args.counts[expert]), args.capacity);
+  if (rows < 0) rows = 0;
+  const long long first = __builtin_amdgcn_readfirstlane(args.offsets[expert]);
+  const bool bias_tile = args.bias_grad != nullptr && rows_m < kSmallBM;  // (the last row tile; see wgrad_writes_bias)
+  const int n_blocks32 = (rows_m + (bias_tile ? 1 : 0) + 31) >> 5;
+  const int n_mi = (n_blocks32 - wm + 1) >> 1;
+  switch (n_mi) {
+    case 2: run_wgrad_tile_small<T, 2, GATHER>(args, tid, expert, m0, n0, rows_m, first, rows, bias_tile); break;
+    case 1: run_wgrad_tile_small<T, 1, GATHER>(args, tid, expert, m0, n0, rows_m, first, rows, bias_tile); break;
+    default: run_wgrad_tile_small<T, 0, GATHER>(args, tid, expert, m0, n0, rows_m, first, rows, bias_tile); break;
+  }
+}
+
+}  // namespace async
+
+// dW[E, Md, Nd] = per expert L^T R over its kept rows.  Both operand buffers must stay readable for 32 rows past
+// their last row (the copies of a partial last slab run over; what they fetch is zeroed before use).
+bool wgrad_async_supported(int Md, int Nd) { return Md % 8 == 0 && Nd % 8 == 0; }
+// True when gemm_async_wgrad can leave the bias gradient (the column sums of the right operand's rows per expert) next
+// to the weight gradient: its last 128-row tile of the Md output rows must have a spare row.
+bool wgrad_writes_bias(int Md, int Nd) { return wgrad_async_supported(Md, Nd) && Md % async::kSmallBM != 0; }
+
+namespace async {
+template <typename T, bool GATHER> static int launch_wgrad(const WgradArgs &a, hipStream_t stream) {
+  auto kernel = wgrad_small_kernel<T, GATHER>;
+  static DeviceFlags attr_done;  // one per kernel instantiation
+  if (int rc = ensure_dynamic_lds((const void *)kernel, kSmallLds, attr_done, "wgrad_small_kernel")) return rc;
+  long long total = (long long)a.E * a.n_m_tiles * a.n_n_tiles;
+  if (total <= 0) return 0;
+  total = (total + kXcds - 1) / kXcds * kXcds;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(kThreads), kSmallLds, stream, a);
+  return check_launch("wgrad_small_kernel");
+}
+}  // namespace async
+
+// With l_rows the left operand is not in expert order: sorted row p is row l_rows[p] / l_div of L (rows of a
+// [n_rows / l_div, Md] tensor gathered by token, which must span less than 4 GiB); l_rows holds n_rows values below
+// n_rows and must stay readable for 32 values more, and L needs no readable rows past its end.
+template <typename T>
+int gemm_async_wgrad(const void *L, const int *l_rows, int l_div, int n_rows, const void *R, void *dW, void *d_bias,
+                     const int *counts, const int *offsets, int capacity, int E, int Md, int Nd, hipStream_t stream) {
+  if (d_bias != nullptr && !wgrad_writes_bias(Md, Nd)) {
+    set_error("gemm_async_wgrad: no spare row for the bias gradient at Md = %d", Md);
+    return YAMOE_E_ARG;
+  }
+  async::WgradArgs a = {};
+  a.A = L; a.B = R; a.C = dW; a.counts = counts; a.offsets = offsets; a.capacity = capacity; a.bias_grad = d_bias;
+  a.a_rows = l_rows; a.a_div = make_fast_div(l_rows != nullptr ? l_div : 1); a.a_rows_max = n_rows > 0 ? n_rows - 1 : 0;
+  a.E = E; a.Md = Md; a.Nd = Nd;
+  a.n_m_tiles = ceil_div(Md, async::kSmallBM);
+  a.n_n_tiles = ceil_div(Nd, async::kBN);
+  if (l_rows != nullptr) return async::launch_wgrad<T, true>(a, stream);
+  return async::launch_wgrad<T, false>(a, stream);
+}
+
+#define YAMOE_INSTANTIATE_WGRAD(T)                                                                                   \
+  template int gemm_async_wgrad<T>(const void *, const int *, int, int, const void *, void *, void *, const int *,     \
+                                   const int *, int, int, int, int, hipStream_t);
+YAMOE_INSTANTIATE_WGRAD(bf16_t)
+YAMOE_INSTANTIATE_WGRAD(f16_t)
+
+}  // namespace yamoe
