@@ -57,14 +57,6 @@ int launch_combine_backward(const void *, const void *, const int *, const int *
 template <typename T>
 int launch_expert_colsum(const void *, const int *, const int *, int, void *, int, int, hipStream_t);
 template <typename T>
-int gemm_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
-                 int, int, hipStream_t);
-template <typename T>
-int gemm_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
-template <typename T>
-int gemm_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int, const void *,
-               float *, hipStream_t);
-template <typename T>
 int gemm_wgrad(const void *, const void *, void *, const int *, const int *, int, int, int, int, hipStream_t);
 template <typename T>
 int glu_backward_rows(const void *, const void *, const float *, const float *, int, const int *, const int *, void *,
@@ -77,23 +69,24 @@ int stream_gate_up(const void *, const int *, const void *, const void *, void *
 template <typename T>
 int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
 
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
                        int, int, int, int, hipStream_t);
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, int,
                     hipStream_t);
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
                      const void *, float *, hipStream_t);
 template <typename T>
 int gemm_async_wgrad(const void *, const int *, int, int, const void *, void *, void *, const int *, const int *, int, int,
                      int, int, hipStream_t);
 bool wgrad_writes_bias(int Md, int Nd);
-bool gemm_f32_supported(int Kd, int Nd, int lda, int ldb, long long a_span_bytes);
 int gemm_f32_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
                      int, int, hipStream_t);
 int gemm_f32_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
+int gemm_f32_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int, hipStream_t);
+int gemm_f32_wgrad(const void *, const void *, void *, const int *, const int *, int, int, int, int, hipStream_t);
 bool wgrad_async_supported(int Md, int Nd);
 
 template <typename T>
@@ -113,6 +106,11 @@ template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
 template <typename T> struct HasStreamPath { static constexpr bool value = sizeof(T) == 2; };
 
+static bool takes_small_tiles(int N, int E, int Nd) {
+  const char *e = getenv("YT");
+  return e && e[0] == '1';
+}
+
 static int gathered_span_ok(const char *who, long long span_bytes) {
   if (span_bytes < (1ll << 32)) return 0;
   set_error("%s: gathered rows span 4 GiB or more", who);
@@ -120,8 +118,7 @@ static int gathered_span_ok(const char *who, long long span_bytes) {
 }
 
 // The MFMA tile kernels for the two forward products: 16-bit data on the asynchronous-copy pipeline (contractions that are
-// not multiples of 64 in instantiations of their own), fp32 on its own when the shape allows it and on the
-// register-staged kernel otherwise.
+// not multiples of 64 in instantiations of their own), fp32 on its own.
 // `small_rows`: experts with at most this many kept rows are on the schedule's streaming list, not tiled (0 when
 // unknown); it only tightens the grid.
 // sorted_idx == nullptr: x holds one row per sorted row, in order (the callers permute a hidden_states tensor of 4 GiB or
@@ -133,23 +130,22 @@ static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, co
   const long long span = sorted_idx != nullptr ? (long long)(N / K) * H * (long long)sizeof(T) : 0;
   if (int rc = gathered_span_ok("tiles_gate_up", span)) return rc;
   if constexpr (sizeof(T) == 2) {
-    auto run = H % 64 ? gemm_async_gate_up<T, true> : gemm_async_gate_up<T, false>;
+    auto run = H % 64 ? gemm_async_gate_up<T, 256, true> : gemm_async_gate_up<T, 256, false>;
+    if (takes_small_tiles(N, E, 2 * I)) run = H % 64 ? gemm_async_gate_up<T, 128, true> : gemm_async_gate_up<T, 128, false>;
     return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, stream);
   } else {
-    if (gemm_f32_supported(H, 2 * I, H, 2 * I, span))
-      return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
-    return gemm_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
+    return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
   }
 }
 template <typename T>
 static int tiles_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E,
                       int H, int I, int small_rows, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
-    auto run = I % 64 ? gemm_async_down<T, true> : gemm_async_down<T, false>;
+    auto run = I % 64 ? gemm_async_down<T, 256, true> : gemm_async_down<T, 256, false>;
+    if (takes_small_tiles(N, E, H)) run = I % 64 ? gemm_async_down<T, 128, true> : gemm_async_down<T, 128, false>;
     return run(act, w, bias, y, sched, N, E, H, I, small_rows, stream);
   } else {
-    if (gemm_f32_supported(I, H, I, H, 0)) return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
-    return gemm_down<T>(act, w, bias, y, sched, N, E, H, I, stream);
+    return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
   }
 }
 
@@ -163,10 +159,11 @@ static int tiles_dgrad(const void *g, const int *g_rows, int g_div, long long g_
   if (g_rows != nullptr)
     if (int rc = gathered_span_ok("tiles_dgrad", g_span_bytes)) return rc;
   if constexpr (sizeof(T) == 2) {
-    auto run = Kd % 64 ? gemm_async_dgrad<T, true> : gemm_async_dgrad<T, false>;
+    auto run = Kd % 64 ? gemm_async_dgrad<T, 256, true> : gemm_async_dgrad<T, 256, false>;
+    if (takes_small_tiles(N, E, Nd)) run = Kd % 64 ? gemm_async_dgrad<T, 128, true> : gemm_async_dgrad<T, 128, false>;
     return run(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
   } else {
-    return gemm_dgrad<T>(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, dot_with, dot_part, stream);
+    return gemm_f32_dgrad(g, g_rows, g_div, w, out, sched, N, E, Kd, Nd, stream);  // (no row dots: n_part is 0)
   }
 }
 
@@ -194,7 +191,8 @@ static int tiles_wgrad(const void *L, const int *l_rows, int l_div, int n_rows, 
       return gemm_async_wgrad<T>(L, l_rows, l_div, n_rows, R, dW, d_bias, counts, offsets, capacity, E, Md, Nd, stream);
   }
   if (l_rows != nullptr || d_bias != nullptr) { set_error("tiles_wgrad: this kernel takes its rows in expert order and sums no bias"); return YAMOE_E_ARG; }
-  return gemm_wgrad<T>(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
+  if constexpr (sizeof(T) == 4) return gemm_f32_wgrad(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
+  else return gemm_wgrad<T>(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
 }
 
 __global__ void fill_zero_kernel(uint32_t *p, long long n_words) {
@@ -311,7 +309,7 @@ static size_t carve_backward(const yamoe_problem *p, void *ws, BackwardBuffers *
   b->row_dot = (float *)c.take(N * (es == 8 ? sizeof(double) : sizeof(float)));
   // 16-bit data: partial row dots of the down projection's input gradient with the activations, two per 256-column
   // tile of I, written by that GEMM from its fp32 accumulators
-  b->n_part = es == 2 ? 2 * ceil_div(p->I, kColTile) : 0;
+  b->n_part = es == 2 ? 2 * ceil_div(p->I, takes_small_tiles(p->T * p->K, p->E, p->I) ? 128 : kColTile) : 0;
   b->dot_part = b->n_part ? (float *)c.take(N * (size_t)b->n_part * sizeof(float)) : nullptr;
   // the weight-gradient kernel's copies of an expert's last, partial slab of rows run up to 32 rows past the
   // end of its operand buffers; every operand is followed by another buffer of this workspace, and this pad
@@ -812,9 +810,12 @@ static int router_backward_impl(const void *d_scores, const long long *indices, 
   YAMOE_TRY(yamoe_build_schedule(b.counts, b.offsets, Tn, 1, Tn, stream_rows, b.schedule, b.schedule_bytes, (void *)stream));
   // d_hidden [T, H] = d_logits [T, E] . weight [E, H]: the down-projection launchers compute rows[., Kd] x w[Kd, Nd]
   YAMOE_TRY(down_both<T>(b.d_logits, weight, nullptr, d_hidden, b.schedule, Tn, 1, /*H=*/H, /*I=*/E, stream));
-  // d_weight [E, H] = d_logits^T . hidden, contraction over the T rows (the register-staged kernel: it reads nothing
-  // past the end of the caller's tensors)
-  YAMOE_TRY(gemm_wgrad<T>(b.d_logits, hidden, d_weight, b.counts, b.offsets, Tn, 1, /*Md=*/E, /*Nd=*/H, stream));
+  // d_weight [E, H] = d_logits^T . hidden, contraction over the T rows (kernels that read nothing past the end of the
+  // caller's tensors: the register-staged one for 16-bit data)
+  if constexpr (sizeof(T) == 4)
+    YAMOE_TRY(gemm_f32_wgrad(b.d_logits, hidden, d_weight, b.counts, b.offsets, Tn, 1, /*Md=*/E, /*Nd=*/H, stream));
+  else
+    YAMOE_TRY(gemm_wgrad<T>(b.d_logits, hidden, d_weight, b.counts, b.offsets, Tn, 1, /*Md=*/E, /*Nd=*/H, stream));
   if (d_bias != nullptr) YAMOE_TRY(launch_expert_colsum<T>(b.d_logits, b.counts, b.offsets, Tn, d_bias, 1, E, stream));
   return 0;
 }

@@ -597,15 +597,9 @@ int gemm_wgrad(const void *L, const void *R, void *dW, const int *counts, const 
   return launch_gemm<T, OP_TRANSPOSED, OP_TRANSPOSED, EPI_STORE, PROB_WGRAD, false>(a, E * a.n_row_tiles_wgrad, stream);
 }
 
-template int gemm_gate_up<float>(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
-                                 int, int, int, hipStream_t);
-template int gemm_down<float>(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
-template int gemm_dgrad<float>(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
-                               const void *, float *, hipStream_t);
 #define YAMOE_INSTANTIATE_WGRAD(T)                                                                                  \
   template int gemm_wgrad<T>(const void *, const void *, void *, const int *, const int *, int, int, int, int,      \
                              hipStream_t);
-YAMOE_INSTANTIATE_WGRAD(float)
 YAMOE_INSTANTIATE_WGRAD(bf16_t)
 YAMOE_INSTANTIATE_WGRAD(f16_t)
 

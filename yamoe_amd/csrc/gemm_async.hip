@@ -1,19 +1,15 @@
 // Grouped expert GEMMs for 16-bit data on gfx950: the products over the rows of the schedule's tiles (the forward's two
-// and the two input gradients) on 256 x 256 tiles.  This file holds the instantiations for contractions of whole slab
-// pairs, gemm_async_ragged.hip the others (it includes this one; they are two files so that they compile side by side).
+// and the two input gradients).  This file holds the instantiations for 256 x 256 tiles and contractions of whole slab
+// pairs; gemm_async_ragged.hip (other contractions) and gemm_async_small.hip (128 x 128 tiles) include it, so that the
+// three compile side by side.
 #include "gemm_async_tile.h"
-
-#ifndef YAMOE_RAGGED
-#define YAMOE_RAGGED false
-#endif
 
 namespace yamoe {
 
-typedef async::Tile<256, 256> BigTile;
-static_assert(BigTile::BM == kRowTile && BigTile::BN == kColTile, "tiles of the schedule must match the GEMM tile");
+static_assert(async::Tile<256, 256>::BM == kRowTile && async::Tile<256, 256>::BN == kColTile,
+              "tiles of the schedule must match the GEMM tile");
 
-#if !YAMOE_RAGGED_TU
-#ifdef YAMOE_TILE_STAMPS
+#if defined(YAMOE_TILE_STAMPS) && !defined(YAMOE_INSTANTIATE_ROWS)
 // Where the next launches of gemm_async_kernel leave their per-tile clock stamps (device memory, 8 words per tile, room
 // for `tiles` tiles; nullptr switches them off).  Exported by the diagnostic build only.
 extern "C" void yamoe_debug_tile_stamps(void *buffer, int32_t tiles) {
@@ -21,9 +17,8 @@ extern "C" void yamoe_debug_tile_stamps(void *buffer, int32_t tiles) {
   async::g_tile_stamps_cap = buffer ? tiles : 0;
 }
 #endif
-#endif
 
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
                        const void *sched, int N, int K, int E, int H, int I, int small_rows, hipStream_t stream) {
   async::Args a = {};
@@ -31,29 +26,29 @@ int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, cons
   a.a_rows = sorted_idx; a.a_div = make_fast_div(K); a.sched = (const int *)sched;
   a.Kd = H; a.Nd = 2 * I; a.lda = H; a.ldb = 2 * I; a.ldc = I;
   a.b_expert_stride = (long long)H * 2 * I;
-  a.n_col_tiles = ceil_div(2 * I, kColTile);
+  a.n_col_tiles = ceil_div(2 * I, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  return async::launch<T, BigTile, async::EPI_GLU, true, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
+  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_GLU, true, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
 }
 
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
                     int I, int small_rows, hipStream_t stream) {
   async::Args a = {};
   a.A = act; a.B = w; a.bias = bias; a.C = y; a.sched = (const int *)sched;
   a.Kd = I; a.Nd = H; a.lda = I; a.ldb = H; a.ldc = H;
   a.b_expert_stride = (long long)I * H;
-  a.n_col_tiles = ceil_div(H, kColTile);
+  a.n_col_tiles = ceil_div(H, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  return async::launch<T, BigTile, async::EPI_STORE, false, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
+  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
 }
 
 // C[rows, Nd] = A[rows, Kd] * W[e]^T with W[e] stored [Nd, Kd]: the input gradients of both projections
 // (csrc/experts_backward.cu:279-282, 309-311), without materialising a transposed weight.
 // With g_rows the source row of sorted row p is g_rows[p] / g_div (rows of a [T, Kd] tensor gathered by token).
-template <typename T, bool RAGGED>
+template <typename T, int TILE, bool RAGGED>
 int gemm_async_dgrad(const void *g, const int *g_rows, int g_div, const void *w, void *out, const void *sched, int N,
                      int E, int Kd, int Nd, const void *dot_with, float *dot_part, hipStream_t stream) {
   async::Args a = {};
@@ -62,21 +57,25 @@ int gemm_async_dgrad(const void *g, const int *g_rows, int g_div, const void *w,
   a.a_rows = g_rows; a.a_div = make_fast_div(g_rows != nullptr ? g_div : 1);
   a.Kd = Kd; a.Nd = Nd; a.lda = Kd; a.ldb = Kd; a.ldc = Nd;
   a.b_expert_stride = (long long)Nd * Kd;
-  a.n_col_tiles = ceil_div(Nd, kColTile);
+  a.n_col_tiles = ceil_div(Nd, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  if (g_rows != nullptr) return async::launch<T, BigTile, async::EPI_STORE, true, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
-  return async::launch<T, BigTile, async::EPI_STORE, false, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
+  if (g_rows != nullptr) return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, true, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
+  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
 }
 
-#define YAMOE_INSTANTIATE_ASYNC(T)                                                                               \
-  template int gemm_async_gate_up<T, YAMOE_RAGGED>(const void *, const int *, const void *, const void *, void *, void *,      \
-                                     const void *, int, int, int, int, int, int, hipStream_t);                   \
-  template int gemm_async_down<T, YAMOE_RAGGED>(const void *, const void *, const void *, void *, const void *, int, int, int, \
-                                  int, int, hipStream_t);                                                             \
-  template int gemm_async_dgrad<T, YAMOE_RAGGED>(const void *, const int *, int, const void *, void *, const void *, int, int, int,  \
-                                   int, const void *, float *, hipStream_t);
-YAMOE_INSTANTIATE_ASYNC(bf16_t)
-YAMOE_INSTANTIATE_ASYNC(f16_t)
+#define YAMOE_INSTANTIATE_ASYNC(T, TILE, RAGGED)                                                                        \
+  template int gemm_async_gate_up<T, TILE, RAGGED>(const void *, const int *, const void *, const void *, void *,       \
+                                                   void *, const void *, int, int, int, int, int, int, hipStream_t);    \
+  template int gemm_async_down<T, TILE, RAGGED>(const void *, const void *, const void *, void *, const void *, int,    \
+                                                int, int, int, int, hipStream_t);                                       \
+  template int gemm_async_dgrad<T, TILE, RAGGED>(const void *, const int *, int, const void *, void *, const void *,    \
+                                                 int, int, int, int, const void *, float *, hipStream_t);
+#ifndef YAMOE_INSTANTIATE_ROWS
+#define YAMOE_INSTANTIATE_ROWS            \
+  YAMOE_INSTANTIATE_ASYNC(bf16_t, 256, false) \
+  YAMOE_INSTANTIATE_ASYNC(f16_t, 256, false)
+#endif
+YAMOE_INSTANTIATE_ROWS
 
 }  // namespace yamoe

@@ -76,6 +76,8 @@ template <int BM_, int BN_> struct Tile {
   // copies per wave (1 KB each): an A pair, a slab of B, a pair of [n][k] B; a B copy covers kBRows k rows
   static constexpr int kACopies = BM / 32, kBRows = 512 / BN, kBCopies = 8 / kBRows, kBPairCopies = BN / 32;
   static constexpr int kMi = BM / 64, kNi = BN / 64;           // 32-row and 32-column blocks of a wave
+  static constexpr int kParts = kRowTile / BM;                 // tiles that a row tile of the schedule is cut into
+  static constexpr int kPerSimd = BM * BN <= 128 * 128 ? 2 : 1;  // workgroups per CU that registers and LDS are kept small for
 };
 
 enum { EPI_STORE = 0, EPI_GLU = 1 };
@@ -638,7 +640,7 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
 }
 
 template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED>
-__global__ __launch_bounds__(kThreads) void gemm_async_kernel(const Args args) {
+__global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const Args args) {
   constexpr int kBN = S::BN;
 
   // Workgroup b runs on XCD b % 8 and takes tile b / 8 of that XCD's share of the tile list.  The shares have
@@ -651,7 +653,7 @@ __global__ __launch_bounds__(kThreads) void gemm_async_kernel(const Args args) {
 #endif
   int L;
   {
-    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds, slots = gridDim.x / kXcds;
+    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds / S::kParts, slots = gridDim.x / kXcds / S::kParts;
     const int first = sched_cut(args.sched, xcd, args.n_col_tiles);
     const int count = sched_cut(args.sched, xcd + 1, args.n_col_tiles) - first;
     if (i < count) {
@@ -710,6 +712,18 @@ __global__ __launch_bounds__(kThreads) void gemm_async_kernel(const Args args) {
     ti.expert = __builtin_amdgcn_readfirstlane(te[0]);
     ti.row0 = __builtin_amdgcn_readfirstlane(te[1]);
     ti.rows_valid = __builtin_amdgcn_readfirstlane(te[2]);
+    if constexpr (S::kParts == 2) {
+      // The row tile's two halves are neighbours in the grid, on one XCD.  More than 128 rows are cut into two parts of
+      // whole 32-row blocks as equal as they get; up to 128 rows are one part, and the other workgroup has nothing to do.
+      const int first_rows = ti.rows_valid > S::BM ? ((ti.rows_valid + 63) >> 6) * 32 : ti.rows_valid;
+      if ((blockIdx.x / kXcds) & 1) {
+        ti.row0 += first_rows;
+        ti.rows_valid -= first_rows;
+        if (ti.rows_valid <= 0) return;
+      } else {
+        ti.rows_valid = first_rows;
+      }
+    }
     ti.n0 = col_tile * kBN;
 #ifdef YAMOE_TILE_STAMPS
     ti.slot = L; ti.t_entry = t_entry;
@@ -777,21 +791,26 @@ __global__ __launch_bounds__(kThreads) void gemm_async_kernel(const Args args) {
   const int n_ni = (n_blocks32_n - wn + 1) >> 1;
 #define YAMOE_RUN(NMI_, NNI_) run_tile<T, S, EPI, NMI_, BNK, RAGGED, NNI_>(args, ti, tid, a_base, a_off, b_base, b_off, b_slab_bytes)
 #define YAMOE_RUN6(NNI_) run_tile<T, S, EPI, 3, BNK, RAGGED, NNI_, 6>(args, ti, tid, a_base, a_off, b_base, b_off, b_slab_bytes)
-  // six row blocks (161..192 rows, what an expert with a few rows more than two full tiles is cut into): both wave
-  // rows have three, and only six of the eight blocks are copied
-  const bool six = n_blocks32 == 6;
-  if (n_ni <= 2 && n_mi >= 3) {
-    if (n_ni <= 1) { if (n_mi == 4) YAMOE_RUN(4, 1); else if (six) YAMOE_RUN6(1); else YAMOE_RUN(3, 1); }
-    else { if (n_mi == 4) YAMOE_RUN(4, 2); else if (six) YAMOE_RUN6(2); else YAMOE_RUN(3, 2); }
-    return;
-  }
-  if (six) { YAMOE_RUN6(4); return; }
-  switch (n_mi) {
-    case 4: YAMOE_RUN(4, 4); break;
-    case 3: YAMOE_RUN(3, 4); break;
-    case 2: YAMOE_RUN(2, 4); break;
-    case 1: YAMOE_RUN(1, 4); break;
-    default: YAMOE_RUN(0, 4); break;
+  if constexpr (S::kMi == 4) {
+    // six row blocks (161..192 rows, what an expert with a few rows more than two full tiles is cut into): both wave
+    // rows have three, and only six of the eight blocks are copied
+    const bool six = n_blocks32 == 6;
+    if (n_ni <= 2 && n_mi >= 3) {
+      if (n_ni <= 1) { if (n_mi == 4) YAMOE_RUN(4, 1); else if (six) YAMOE_RUN6(1); else YAMOE_RUN(3, 1); }
+      else { if (n_mi == 4) YAMOE_RUN(4, 2); else if (six) YAMOE_RUN6(2); else YAMOE_RUN(3, 2); }
+      return;
+    }
+    if (six) { YAMOE_RUN6(4); return; }
+    switch (n_mi) {
+      case 4: YAMOE_RUN(4, 4); break;
+      case 3: YAMOE_RUN(3, 4); break;
+      case 2: YAMOE_RUN(2, 4); break;
+      case 1: YAMOE_RUN(1, 4); break;
+      default: YAMOE_RUN(0, 4); break;
+    }
+  } else {
+    if (n_ni <= 1) { if (n_mi == 2) YAMOE_RUN(2, 1); else if (n_mi == 1) YAMOE_RUN(1, 1); else YAMOE_RUN(0, 1); }
+    else { if (n_mi == 2) YAMOE_RUN(2, 2); else if (n_mi == 1) YAMOE_RUN(1, 2); else YAMOE_RUN(0, 2); }
   }
 #undef YAMOE_RUN
 #undef YAMOE_RUN6
@@ -810,7 +829,7 @@ static int launch(const Args &args, int max_row_tiles, hipStream_t stream) {
   if (int rc = ensure_dynamic_lds((const void *)kernel, lds_bytes, attr_done, "gemm_async_kernel")) return rc;
   long long total = (long long)max_row_tiles * args.n_col_tiles;
   if (total <= 0) return 0;
-  total = (total + kXcds - 1) / kXcds * kXcds;
+  total = (total + kXcds - 1) / kXcds * kXcds * S::kParts;
 #ifdef YAMOE_TILE_STAMPS
   Args stamped = args;
   stamped.stamps = g_tile_stamps;
