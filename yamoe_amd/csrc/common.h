@@ -150,18 +150,21 @@ __device__ inline void copy16_to_lds(const char *lane_addr, uint32_t lds_base) {
 //   [2] n_active      experts with at least one kept row
 //   [3] n_kept        total kept rows
 //   [4] weight_total  sum of the experts' cost weights (sched_group_weight)
+//   [5] n_half_tiles  number of 128-row tiles when the same experts' rows are cut into full tiles and a remainder
 //   [8 + 4x ...)      x = 0..8: where the tile list is cut so that each of the 8 XCDs gets the same share of
 //                     the cost: {first row tile of the expert the cut falls in, f, 0, row tiles of that
 //                     expert}, f = the cut's position inside that expert's tiles in 1/65536ths; in a GEMM
 //                     with n column tiles the cut is at flat tile index
 //                     first * n + ((f * n) >> 16) * row_tiles, i.e. on a column-tile boundary of that expert
 //   [48 ...)          row tiles: 8 words each  {expert, first sorted row, valid rows,
-//                       index of the expert's first row tile, number of row tiles of the expert, 0,0,0}
+//                       index of the expert's first row tile, number of row tiles of the expert,
+//                       multiplier and shift that divide by that number, 128-row tiles of the experts before this one}
 //   then              small experts: 4 words each {expert, first sorted row, valid rows, 0}
 constexpr int kRowTile = 256;  // rows of one MFMA row tile
 constexpr int kColTile = 256;  // columns of one MFMA tile
 constexpr int kSchedHeader = 48;
 constexpr int kSchedCuts = 8;  // word offset of the XCD cut table
+constexpr int kSchedHalfTiles = 5;
 constexpr int kXcds = 8;
 
 // Relative cost of one row tile in the MFMA kernels: a fixed part (prologue, epilogue, copies of the weight

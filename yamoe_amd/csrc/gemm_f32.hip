@@ -14,6 +14,12 @@
 //  * Operands go global -> LDS with asynchronous 16-byte copies (no staging registers), two stages of 32 KB, one
 //    workgroup barrier per slab of 32 (16 000 clocks of matrix work): while a workgroup waits at its barrier or
 //    runs its epilogue, the other workgroup on the CU keeps the matrix pipe busy.
+//  * The workgroups are resident, two per CU, and go through the tiles that have rows; the next tile is looked up and its
+//    first slab requested before the epilogue of the one before.
+//  README workload, gate_up and down product: 2328 + 1342 us with a workgroup per half row tile, 2100 + 1160 now, 130 and 117
+//  TFLOP/s of the 154 that a register-only loop of the instruction reaches on random data; of the difference, 5 % is LDS
+//  reads and barriers (a loop of these alone runs at 148), the rest the turn from tile to tile (20 us for the two tiles of a
+//  CU, most of it the stores) and the last, partly filled round.
 //  * An operand that is [row][k] in memory (activations, [n][k] weights of the input gradients) keeps that layout in LDS
 //    (128-byte rows, 16-byte pieces XOR-swizzled with the row number on the global side of the copy); a lane's 16-byte
 //    read holds four contraction steps.
@@ -26,6 +32,8 @@
 //    overwrite what they copied of the left operand there with zeros before the barrier.
 //
 // Requirements: leading dimensions and, for row products, the contraction length multiples of 4 elements.
+#include <type_traits>
+
 #include "common.h"
 
 namespace yamoe {
@@ -39,6 +47,8 @@ constexpr int kBStage = kBK * kBN * 4;
 constexpr int kStage = kAStage + kBStage;
 constexpr int kStages = 2;
 constexpr int kLds = kStages * kStage;  // 64 KB: two workgroups per CU
+
+constexpr int kWorkgroups = 2 * 256;    // two on each of the 256 CUs, each going through its share of the tiles
 
 static_assert(kRowTile == 2 * kBM, "an expert has at most twice as many tiles here as row tiles in the schedule");
 
@@ -63,57 +73,22 @@ struct Args {
   long long b_expert_stride;
 };
 
+// One output tile: what it is (the same for every lane) and where this lane's copies come from
+struct Tile {
+  int expert, row0, rows_valid, n0, k_len;  // rows of the tile: sorted rows, or (WGRAD) rows of the gradient
+  const char *a_base, *b_base;
+  uint32_t a_off[4], b_off[4];
+};
+
 template <int EPI, int MODE, bool GATHER>
 __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr bool A_ROWS = MODE != WGRAD, B_ROWS = MODE == ROWS_NK;  // operands that are [row][k]
+  constexpr int kStores = MODE == ROWS_NK ? 64 : 32;  // stores of a whole tile per wave (a wait can count 63 at most)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave >> 1, wn = wave & 1;
   const int rl = lane & 31, g = lane >> 5;
-
-  // ---- which tile.  Workgroup ids are dealt round-robin over the XCDs, so id b takes logical tile
-  // (b % 8) * per_xcd + b / 8.  Row products run expert-major, then column tile, then the expert's tiles of rows, so the
-  // tiles in flight on one XCD share weight columns through its L2; weight gradients run column by column of one expert's
-  // output tiles.
-  int expert, n0, k_len;
-  int row0, rows_valid;  // rows of the output tile: sorted rows, or (WGRAD) rows of the gradient
-  long long k_first = 0;
-  {
-    const int n_rows = MODE == WGRAD ? args.E * args.n_m_tiles : 2 * args.sched[0];
-    const int total = n_rows * args.n_col_tiles;
-    const int total8 = (total + kXcds - 1) / kXcds * kXcds;
-    const int b = blockIdx.x;
-    if (b >= total8) return;
-    const int L = (b % kXcds) * (total8 / kXcds) + b / kXcds;
-    if (L >= total) return;
-    if constexpr (MODE == WGRAD) {
-      const int per_expert = args.n_m_tiles * args.n_col_tiles;
-      expert = L / per_expert;
-      const int local = L - expert * per_expert, col_tile = local / args.n_m_tiles;
-      row0 = (local - col_tile * args.n_m_tiles) * kBM;
-      rows_valid = min(kBM, args.Md - row0);
-      n0 = col_tile * kBN;
-      k_len = max(min(__builtin_amdgcn_readfirstlane(args.counts[expert]), args.capacity), 0);
-      k_first = __builtin_amdgcn_readfirstlane(args.offsets[expert]);
-    } else {
-      const int *tiles = args.sched + kSchedHeader;
-      const int t0 = (L / args.n_col_tiles) >> 1;
-      const int gfirst = tiles[8 * t0 + 3], gcount = tiles[8 * t0 + 4];
-      const int local = L - 2 * gfirst * args.n_col_tiles;
-      const int col_tile = local / (2 * gcount);
-      const int part = local - col_tile * 2 * gcount;  // the expert's tile of rows
-      const int *last = tiles + 8 * (gfirst + gcount - 1);
-      expert = tiles[8 * gfirst];
-      row0 = tiles[8 * gfirst + 1] + part * kBM;
-      rows_valid = min(last[1] + last[2] - row0, kBM);
-      n0 = col_tile * kBN;
-      k_len = args.Kd;
-      if (rows_valid <= 0) return;  // (the expert has fewer tiles of 128 than twice its row tiles)
-    }
-  }
-  const int cols_valid = min(kBN, args.Nd - n0);
-  const int n_slabs = (k_len + kBK - 1) / kBK;
 
   // ---- copies.  A [row][k] operand: copy i (0..3) fetches rows 32*i + 8*wave + (lane >> 3), 16 bytes of each; LDS position
   // lane & 7 of the row holds piece pos ^ ((row >> 1) & 7).  A [k][column] operand: copy i fetches k rows
@@ -122,70 +97,117 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
   // (a gathering instantiation without a row list reads its rows in order: see gemm_async_tile.h)
   const bool gathers = GATHER && args.a_rows != nullptr;
   const int piece = (lane & 7) ^ ((4 * wave + (lane >> 4)) & 7);  // (the same for all four copies)
-  uint32_t a_off[4], b_off[4];
-  auto column_off = [&](int i, int valid, int ld) {
-    const int k = 8 * wave + 2 * i + (lane >> 5);
-    const int col = (lane & 31) * 4;
-    return (uint32_t)(((long long)k * ld + (col >= valid ? 0 : col)) * 4);
-  };
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = 32 * i + 8 * wave + (lane >> 3);
-    if constexpr (A_ROWS) {
-      const int r = min(row, rows_valid - 1);
-      long long src = r;
-      if (gathers) src = args.a_rows[row0 + r] / args.a_div;
-      a_off[i] = (uint32_t)((src * args.lda + piece * 4) * 4);
-    } else {
-      a_off[i] = column_off(i, rows_valid, args.lda);
-    }
-    if constexpr (B_ROWS) b_off[i] = (uint32_t)(((long long)min(row, cols_valid - 1) * args.ldb + piece * 4) * 4);
-    else b_off[i] = column_off(i, cols_valid, args.ldb);
-  }
-  const char *a_base = A_ROWS ? (const char *)(args.A + (gathers ? 0ll : (long long)row0 * args.lda))
-                              : (const char *)(args.A + k_first * args.lda + row0);
-  const char *b_base = MODE == ROWS_KN   ? (const char *)(args.B + (long long)expert * args.b_expert_stride + n0)
-                       : MODE == ROWS_NK ? (const char *)(args.B + (long long)expert * args.b_expert_stride + (long long)n0 * args.ldb)
-                                         : (const char *)(args.B + k_first * args.ldb + n0);
   const long long a_slab_bytes = A_ROWS ? kBK * 4 : (long long)kBK * args.lda * 4;
   const long long b_slab_bytes = B_ROWS ? kBK * 4 : (long long)kBK * args.ldb * 4;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)lds);
-  auto issue = [&](int slab) {
-    const uint32_t st = lds0 + (uint32_t)(slab & (kStages - 1)) * kStage;
-    const char *ab = a_base + (long long)slab * a_slab_bytes;
-    const char *bb = b_base + (long long)slab * b_slab_bytes;
-    const int left = k_len - slab * kBK;  // (below 32 in a last slab that the contraction does not fill)
+
+  // ---- the tiles: tile L of the launch.  Row products run expert-major, then column tile, then the expert's 128-row
+  // tiles; weight gradients expert-major, then column by column of the expert's output tiles.
+  const int total = (MODE == WGRAD ? args.E * args.n_m_tiles : args.sched[kSchedHalfTiles]) * args.n_col_tiles;
+  // Workgroups go through the tiles in rounds of kWorkgroups.  Where the last round has tiles for at most half of the CUs,
+  // they are dealt out in halves of 64 rows (both wave rows stay busy): item i of the launch is tile i up to there.  (The
+  // down product of the README workload has 3.05 rounds: 2 % of the whole forward.)
+  constexpr bool SPLITS = MODE != WGRAD;
+  const int whole_rounds = total / kWorkgroups * kWorkgroups;
+  const bool splits = SPLITS && 4 * (total - whole_rounds) <= kWorkgroups;
+  const int items = splits ? 2 * total - whole_rounds : total;
+  auto set_tile = [&](int item, Tile &t) {
+    const bool half = splits && item >= whole_rounds;
+    const int L = half ? whole_rounds + ((item - whole_rounds) >> 1) : item;
+    long long k_first = 0;
+    if constexpr (MODE == WGRAD) {
+      const int per_expert = args.n_m_tiles * args.n_col_tiles;
+      t.expert = L / per_expert;
+      const int local = L - t.expert * per_expert, col_tile = local / args.n_m_tiles;
+      t.row0 = (local - col_tile * args.n_m_tiles) * kBM;
+      t.rows_valid = min(kBM, args.Md - t.row0);
+      t.n0 = col_tile * kBN;
+      t.k_len = max(min(__builtin_amdgcn_readfirstlane(args.counts[t.expert]), args.capacity), 0);
+      k_first = __builtin_amdgcn_readfirstlane(args.offsets[t.expert]);
+    } else {
+      // the last row tile of the schedule whose expert starts at or before tile L
+      const int *tiles = args.sched + kSchedHeader;
+      const int n_tiles = args.sched[0];
+      int found = -1;
+      for (int base = 0; base < n_tiles; base += kWave) {
+        const bool before = base + lane < n_tiles && tiles[8 * (base + lane) + 7] * args.n_col_tiles <= L;
+        const int n = __popcll(__ballot(before));
+        found += n;
+        if (n < kWave) break;
+      }
+      const int *te = tiles + 8 * __builtin_amdgcn_readfirstlane(found);  // the expert's last row tile
+      const int *first = tiles + 8 * __builtin_amdgcn_readfirstlane(te[3]);
+      const int row_first = __builtin_amdgcn_readfirstlane(first[1]);
+      const int rows = __builtin_amdgcn_readfirstlane(te[1] + te[2]) - row_first;
+      const int parts = (rows + kBM - 1) / kBM;
+      const int local = L - __builtin_amdgcn_readfirstlane(te[7]) * args.n_col_tiles;
+      const int col_tile = (int)((uint32_t)local / (uint32_t)parts);
+      const int part = local - col_tile * parts;
+      t.expert = __builtin_amdgcn_readfirstlane(te[0]);
+      t.row0 = row_first + part * kBM;
+      t.rows_valid = min(rows - part * kBM, kBM);
+      if (half) {
+        // (a half without rows is gone through like the others and stores nothing: its first row only has to exist)
+        const bool second = ((item - whole_rounds) & 1) != 0;
+        t.rows_valid = second ? t.rows_valid - 64 : min(t.rows_valid, 64);
+        if (second && t.rows_valid > 0) t.row0 += 64;
+      }
+      t.n0 = col_tile * kBN;
+      t.k_len = args.Kd;
+    }
+    const int cols_valid = min(kBN, args.Nd - t.n0);
+    auto column_off = [&](int i, int valid, int ld) {
+      const int k = 8 * wave + 2 * i + (lane >> 5);
+      const int col = (lane & 31) * 4;
+      return (uint32_t)(((long long)k * ld + (col >= valid ? 0 : col)) * 4);
+    };
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int k = 8 * wave + 2 * i + (lane >> 5);
-      const int past = max(k - (left - 1), 0);  // k rows past the end re-read the last one, pieces past it the row's first
-      const uint32_t a_adj = A_ROWS ? (piece * 4 >= left ? piece * 16u : 0u) : (uint32_t)past * (uint32_t)args.lda * 4u;
-      const uint32_t b_adj = B_ROWS ? (piece * 4 >= left ? piece * 16u : 0u) : (uint32_t)past * (uint32_t)args.ldb * 4u;
-      copy16_to_lds(ab, a_off[i] - a_adj, st + (uint32_t)(A_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512));
-      copy16_to_lds(bb, b_off[i] - b_adj, st + kAStage + (uint32_t)(B_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512));
+      const int row = 32 * i + 8 * wave + (lane >> 3);
+      if constexpr (A_ROWS) {
+        const int r = max(min(row, t.rows_valid - 1), 0);
+        long long src = r;
+        if (gathers) src = args.a_rows[t.row0 + r] / args.a_div;
+        t.a_off[i] = (uint32_t)((src * args.lda + piece * 4) * 4);
+      } else {
+        t.a_off[i] = column_off(i, t.rows_valid, args.lda);
+      }
+      if constexpr (B_ROWS) t.b_off[i] = (uint32_t)(((long long)min(row, cols_valid - 1) * args.ldb + piece * 4) * 4);
+      else t.b_off[i] = column_off(i, cols_valid, args.ldb);
+    }
+    t.a_base = A_ROWS ? (const char *)(args.A + (gathers ? 0ll : (long long)t.row0 * args.lda))
+                      : (const char *)(args.A + k_first * args.lda + t.row0);
+    t.b_base = MODE == ROWS_KN   ? (const char *)(args.B + (long long)t.expert * args.b_expert_stride + t.n0)
+               : MODE == ROWS_NK ? (const char *)(args.B + (long long)t.expert * args.b_expert_stride + (long long)t.n0 * args.ldb)
+                                 : (const char *)(args.B + k_first * args.ldb + t.n0);
+  };
+  auto issue = [&](const Tile &t, int slab, int stage) {
+    const uint32_t st = lds0 + (uint32_t)(stage & (kStages - 1)) * kStage;
+    const char *ab = t.a_base + (long long)slab * a_slab_bytes;
+    const char *bb = t.b_base + (long long)slab * b_slab_bytes;
+    const int left = t.k_len - slab * kBK;  // (below 32 in a last slab that the contraction does not fill)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t a_adj = 0, b_adj = 0;
+      if (left < kBK) {  // k rows past the end re-read the last one, pieces past it the row's first
+        const int past = max(8 * wave + 2 * i + (lane >> 5) - (left - 1), 0);
+        a_adj = A_ROWS ? (piece * 4 >= left ? piece * 16u : 0u) : (uint32_t)past * (uint32_t)args.lda * 4u;
+        b_adj = B_ROWS ? (piece * 4 >= left ? piece * 16u : 0u) : (uint32_t)past * (uint32_t)args.ldb * 4u;
+      }
+      copy16_to_lds(ab, t.a_off[i] - a_adj, st + (uint32_t)(A_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512));
+      copy16_to_lds(bb, t.b_off[i] - b_adj, st + kAStage + (uint32_t)(B_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512));
     }
   };
   // what this wave copied of the last slab's left operand past the end of the contraction
-  auto zero_tail = [&](int slab) {
-    const int left = k_len - slab * kBK;
-    char *st = lds + (slab & (kStages - 1)) * kStage + lane * 16;
+  auto zero_tail = [&](const Tile &t, int slab, int stage) {
+    const int left = t.k_len - slab * kBK;
+    char *st = lds + (stage & (kStages - 1)) * kStage + lane * 16;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const bool past = A_ROWS ? piece * 4 >= left : 8 * wave + 2 * i + (lane >> 5) >= left;
       if (past) *(u32x4 *)(st + (A_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512)) = (u32x4){0, 0, 0, 0};
     }
   };
-
-  // ---- accumulators: acc[a][b][v], instruction row i = 8*(v/4) + 4*g + v%4 and column rl, is
-  //   row (a*2+wm)*32 + i of the tile, or (WGRAD, "even" and "odd" rows) wm*64 + 2*i + a
-  //   column wn*64 + 2*rl + b, or (ROWS_NK) (b*2+wn)*32 + rl
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
 
   // [row][k] operand of block x in k-step ks (8 contraction steps): row (x*2+w)*32 + rl, piece 2*ks + g; the four values of
   // the piece feed four instructions, in which the lanes of half g hold k = 8*ks + 4*g + q.  (Rows 64 apart share
@@ -197,102 +219,195 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
     a_rd[ks] = A_ROWS ? (wm * 32 + rl) * 128 + p : g * 4 * 512 + (wm * 64 + 2 * rl) * 4 + ks * 8 * 512;
     b_rd[ks] = B_ROWS ? (wn * 32 + rl) * 128 + p : g * 4 * 512 + (wn * 64 + 2 * rl) * 4 + ks * 8 * 512;
   }
-  // blocks of this wave that hold anything: rows of a row product by 32-row blocks, everything else by the wave's 64
-  const int blocks = (rows_valid + 31) >> 5;
-  const bool active_n = B_ROWS ? wn * 32 < cols_valid : wn * 64 < cols_valid;
-  const int n_a = !active_n ? 0 : A_ROWS ? (blocks - wm + 1) >> 1 : (wm * 64 < rows_valid ? 2 : 0);
+  // accumulators: acc[a][b][v], instruction row i = 8*(v/4) + 4*g + v%4 and column rl, is
+  //   row (a*2+wm)*32 + i of the tile, or (WGRAD, "even" and "odd" rows) wm*64 + 2*i + a
+  //   column wn*64 + 2*rl + b, or (ROWS_NK) (b*2+wn)*32 + rl
+  f32x16 acc[2][2];
 
-  if (n_slabs > 0) issue(0);
-  for (int s = 0; s < n_slabs; ++s) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (s == n_slabs - 1 && (k_len & (kBK - 1)) != 0) zero_tail(s);
-    __syncthreads();  // slab s has landed for every wave, and nobody reads the other stage any more
-    if (s + 1 < n_slabs) issue(s + 1);
-    const char *sa = lds + (s & (kStages - 1)) * kStage;
-    const char *sb = sa + kAStage;
-    if (n_a > 0) {
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        f32x4 fa[2], fb[2];
+  // A slab is four k-steps of 4 * NA * 2 MFMAs (1024 clocks for NA = 2).  The operands of a k-step are read from LDS while
+  // the MFMAs of the one before run, in a fixed order (left to itself the compiler reads each value right before its use).
+  // The wait for the next slab and the barrier stand before the last k-step, whose operands are in registers by then: the
+  // copies and the first reads of the next slab are issued under its MFMAs.  (Slab 0's copies are on their way already,
+  // into stage `stage`; slab s sits in stage + s.  `stores`: behind them, this wave has exactly
+  // kStores stores of the previous tile in flight, which nothing waits for here.)
+  auto contract = [&](const Tile &t, int stage, bool stores, auto na) {
+    constexpr int NA = decltype(na)::value;
+    const int n_slabs = (t.k_len + kBK - 1) / kBK;
+    float va[2][4][2], vb[2][4][2];  // [set][q][block]
+    auto read = [&](int s, int ks, float (&ra)[4][2], float (&rb)[4][2]) {
+      if constexpr (NA > 0) {
+        const char *sa = lds + ((stage + s) & (kStages - 1)) * kStage;
+        const char *sb = sa + kAStage;
         if constexpr (A_ROWS) {
-          fa[0] = *(const f32x4 *)(sa + a_rd[ks]);
-          fa[1] = *(const f32x4 *)(sa + a_rd[ks] + 64 * 128);
+#pragma unroll
+          for (int x = 0; x < NA; ++x) {
+            const f32x4 v = *(const f32x4 *)(sa + a_rd[ks] + x * 64 * 128);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) ra[q][x] = v[q];
+          }
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x2 v = *(const f32x2 *)(sa + a_rd[ks] + q * 512);
+            ra[q][0] = v[0];
+            ra[q][1] = v[1];
+          }
         }
         if constexpr (B_ROWS) {
-          fb[0] = *(const f32x4 *)(sb + b_rd[ks]);
-          fb[1] = *(const f32x4 *)(sb + b_rd[ks] + 64 * 128);
-        }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float va[2], vb[2];
-          if constexpr (A_ROWS) {
-            va[0] = fa[0][q]; va[1] = fa[1][q];
-          } else {
-            const f32x2 t = *(const f32x2 *)(sa + a_rd[ks] + q * 512);
-            va[0] = t[0]; va[1] = t[1];
+          for (int x = 0; x < 2; ++x) {
+            const f32x4 v = *(const f32x4 *)(sb + b_rd[ks] + x * 64 * 128);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rb[q][x] = v[q];
           }
-          if constexpr (B_ROWS) {
-            vb[0] = fb[0][q]; vb[1] = fb[1][q];
-          } else {
-            const f32x2 t = *(const f32x2 *)(sb + b_rd[ks] + q * 512);
-            vb[0] = t[0]; vb[1] = t[1];
-          }
-          acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[0], vb[0], acc[0][0], 0, 0, 0);
-          acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[0], vb[1], acc[0][1], 0, 0, 0);
-          if (n_a > 1) {
-            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[1], vb[0], acc[1][0], 0, 0, 0);
-            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[1], vb[1], acc[1][1], 0, 0, 0);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const f32x2 v = *(const f32x2 *)(sb + b_rd[ks] + q * 512);
+            rb[q][0] = v[0];
+            rb[q][1] = v[1];
           }
         }
       }
+    };
+    auto multiply = [&](const float (&ra)[4][2], const float (&rb)[4][2]) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[q][a], rb[q][b], acc[a][b], 0, 0, 0);
+    };
+    // slab s is there for every wave, and nobody reads the other stage any more (the reads of a wave are complete when it
+    // gets here: its next MFMAs need them)
+    auto arrive = [&](int s) {
+      // (slab 0 was requested ahead of the previous tile's stores, and vector memory operations complete in order)
+      if (s == 0 && stores) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kStores < 64 ? kStores : 0) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+      if (s == n_slabs - 1 && (t.k_len & (kBK - 1)) != 0) zero_tail(t, s, stage + s);
+      __syncthreads();
+      if (s + 1 < n_slabs) issue(t, s + 1, stage + s + 1);
+    };
+    if (n_slabs > 0) {
+      arrive(0);
+      read(0, 0, va[0], vb[0]);
     }
-  }
+    for (int s = 0; s < n_slabs; ++s) {
+#pragma unroll
+      for (int ks = 0; ks < 3; ++ks) {
+        __builtin_amdgcn_sched_barrier(0);
+        read(s, ks + 1, va[(ks + 1) & 1], vb[(ks + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(va[ks & 1], vb[ks & 1]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (s + 1 < n_slabs) {
+        arrive(s + 1);
+        read(s + 1, 0, va[0], vb[0]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(va[1], vb[1]);
+    }
+  };
 
-  // ---- epilogue: straight from the accumulators; a half wave covers 256 (128 for act and ROWS_NK) contiguous bytes of a row
-  if (n_a == 0) return;
-  const int col = n0 + (B_ROWS ? wn * 32 + rl : wn * 64 + 2 * rl);  // (GLU: even, the gate column of pair col / 2)
-  float b0 = 0.0f, b1 = 0.0f;
-  if (MODE == ROWS_KN && args.bias != nullptr && col < args.Nd) {
-    const float *bp = args.bias + (long long)expert * args.Nd + col;
-    b0 = bp[0];
-    b1 = bp[1];
-  }
-  float *C = args.C + (MODE == WGRAD ? (long long)expert * args.Md * args.Nd : 0ll);
+  // ---- workgroup b takes tiles b, b + gridDim.x, ...  The next tile is looked up and its first slab requested before the
+  // epilogue of the current one.
+  // The places in a round of a CU's two, workgroups b and b + 256, are b and 511 - b: in the order of the tiles a full tile
+  // and an expert's remainder often alternate, and a CU should get one of each (2 % of the step of a layer of 16 experts
+  // with 187 rows).
+  int L = blockIdx.x < kWorkgroups / 2 ? blockIdx.x : kWorkgroups / 2 + kWorkgroups - 1 - blockIdx.x, stage = 0;
+  bool stores = false;
+  if (L >= items) return;
+  Tile t;
+  set_tile(L, t);
+  if (t.k_len > 0) issue(t, 0, stage);
+  for (;;) {
 #pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    if (a < n_a) {
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[a][b][v] = 0.0f;
+    // blocks of this wave that hold anything: rows of a row product by 32-row blocks, everything else by the wave's 64
+    // (every wave of the workgroup goes through the same copies, waits and barriers, whatever it multiplies)
+    const int cols_valid = min(kBN, args.Nd - t.n0);
+    const bool active_n = B_ROWS ? wn * 32 < cols_valid : wn * 64 < cols_valid;
+    const int n_a = !active_n || t.rows_valid <= 0 ? 0 : A_ROWS ? (((t.rows_valid + 31) >> 5) - wm + 1) >> 1 : (wm * 64 < t.rows_valid ? 2 : 0);
+    if (n_a == 2) contract(t, stage, stores, std::integral_constant<int, 2>());
+    else if (n_a == 1) contract(t, stage, stores, std::integral_constant<int, 1>());
+    else contract(t, stage, stores, std::integral_constant<int, 0>());
+
+    // (the stage after the last slab's has been free since the barrier in front of that slab)
+    stage += (t.k_len + kBK - 1) / kBK;
+    const int row0 = t.row0, rows_valid = t.rows_valid, expert = t.expert;
+    const bool whole = rows_valid == kBM && cols_valid == kBN;
+    const int col = t.n0 + (B_ROWS ? wn * 32 + rl : wn * 64 + 2 * rl);  // (GLU: even, the gate column of pair col / 2)
+    L += kWorkgroups;
+    if (L < items) {
+      set_tile(L, t);
+      if (t.k_len > 0) issue(t, 0, stage);
+    }
+
+    // epilogue: straight from the accumulators; a half wave covers 256 (128 for act and ROWS_NK) contiguous bytes of a row
+    if (n_a > 0) {
+      float b0 = 0.0f, b1 = 0.0f;
+      if (MODE == ROWS_KN && args.bias != nullptr && col < args.Nd) {
+        const float *bp = args.bias + (long long)expert * args.Nd + col;
+        b0 = bp[0];
+        b1 = bp[1];
+      }
+      float *C = args.C + (MODE == WGRAD ? (long long)expert * args.Md * args.Nd : 0ll);
+      auto store = [&](int a, int v, long long orow) {
+        if constexpr (MODE == ROWS_NK) {
+          C[orow * args.ldc + col] = acc[a][0][v];
+          C[orow * args.ldc + col + 64] = acc[a][1][v];
+        } else {
+          const float x0 = acc[a][0][v] + b0, x1 = acc[a][1][v] + b1;
+          if constexpr (EPI == EPI_STORE) {
+            *(f32x2 *)(C + orow * args.ldc + col) = (f32x2){x0, x1};
+          } else {
+            C[orow * args.ldc + (col >> 1)] = glu_forward(x0, x1);
+            if (args.C2 != nullptr) *(f32x2 *)(args.C2 + orow * args.Nd + col) = (f32x2){x0, x1};
+          }
+        }
+      };
+      auto row_of = [&](int a, int v) {
         const int i = 8 * (v >> 2) + 4 * g + (v & 3);
-        const int r = A_ROWS ? (a * 2 + wm) * 32 + i : wm * 64 + 2 * i + a;
-        if (r < rows_valid) {
-          const long long orow = row0 + r;
-          if constexpr (MODE == ROWS_NK) {
-            if (col < args.Nd) C[orow * args.ldc + col] = acc[a][0][v];
-            if (col + 64 < args.Nd) C[orow * args.ldc + col + 64] = acc[a][1][v];
-          } else if (col < args.Nd) {
-            const float x0 = acc[a][0][v] + b0, x1 = acc[a][1][v] + b1;
-            if constexpr (EPI == EPI_STORE) {
-              *(f32x2 *)(C + orow * args.ldc + col) = (f32x2){x0, x1};
-            } else {
-              C[orow * args.ldc + (col >> 1)] = glu_forward(x0, x1);
-              if (args.C2 != nullptr) *(f32x2 *)(args.C2 + orow * args.Nd + col) = (f32x2){x0, x1};
+        return A_ROWS ? (a * 2 + wm) * 32 + i : wm * 64 + 2 * i + a;
+      };
+      if (whole) {  // (kStores stores, one or two per register)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) store(a, v, row0 + row_of(a, v));
+      } else {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int r = row_of(a, v);
+            if (a < n_a && r < rows_valid && col < args.Nd) {
+              if constexpr (MODE == ROWS_NK) {
+                C[(long long)(row0 + r) * args.ldc + col] = acc[a][0][v];
+                if (col + 64 < args.Nd) C[(long long)(row0 + r) * args.ldc + col + 64] = acc[a][1][v];
+              } else {
+                store(a, v, row0 + r);
+              }
             }
           }
-        }
       }
     }
+    stores = whole && kStores < 64 && (EPI != EPI_GLU || args.C2 == nullptr);
+    if (L >= items) return;
   }
 }
 
 template <int EPI, int MODE, bool GATHER>
-static int launch(const Args &args, long long tiles, hipStream_t stream) {
+static int launch(const Args &args, hipStream_t stream) {
   auto kernel = gemm_f32_kernel<EPI, MODE, GATHER>;
   static DeviceFlags attr_done;  // one per kernel instantiation
   if (int rc = ensure_dynamic_lds((const void *)kernel, kLds, attr_done, "gemm_f32_kernel")) return rc;
-  if (tiles <= 0) return 0;
-  tiles = (tiles + kXcds - 1) / kXcds * kXcds;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles), dim3(kThreads), kLds, stream, args);
+  hipLaunchKernelGGL(kernel, dim3(kWorkgroups), dim3(kThreads), kLds, stream, args);
   return check_launch("gemm_f32_kernel");
 }
 
@@ -306,7 +421,7 @@ int gemm_f32_gate_up(const void *x, const int *sorted_idx, const void *w, const 
   a.Kd = H; a.Nd = 2 * I; a.lda = H; a.ldb = 2 * I; a.ldc = I;
   a.b_expert_stride = (long long)H * 2 * I;
   a.n_col_tiles = ceil_div(2 * I, f32::kBN);
-  return f32::launch<f32::EPI_GLU, f32::ROWS_KN, true>(a, 2ll * sched_max_row_tiles(N, E) * a.n_col_tiles, stream);
+  return f32::launch<f32::EPI_GLU, f32::ROWS_KN, true>(a, stream);
 }
 
 int gemm_f32_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
@@ -317,7 +432,7 @@ int gemm_f32_down(const void *act, const void *w, const void *bias, void *y, con
   a.Kd = I; a.Nd = H; a.lda = I; a.ldb = H; a.ldc = H;
   a.b_expert_stride = (long long)I * H;
   a.n_col_tiles = ceil_div(H, f32::kBN);
-  return f32::launch<f32::EPI_STORE, f32::ROWS_KN, false>(a, 2ll * sched_max_row_tiles(N, E) * a.n_col_tiles, stream);
+  return f32::launch<f32::EPI_STORE, f32::ROWS_KN, false>(a, stream);
 }
 
 // out[p, :] = g[row p, :] . W[e]^T with W[e] stored [Nd, Kd]; with g_rows the source row of p is g_rows[p] / g_div
@@ -329,9 +444,8 @@ int gemm_f32_dgrad(const void *g, const int *g_rows, int g_div, const void *w, v
   a.Kd = Kd; a.Nd = Nd; a.lda = Kd; a.ldb = Kd; a.ldc = Nd;
   a.b_expert_stride = (long long)Nd * Kd;
   a.n_col_tiles = ceil_div(Nd, f32::kBN);
-  const long long tiles = 2ll * sched_max_row_tiles(N, E) * a.n_col_tiles;
-  if (g_rows != nullptr) return f32::launch<f32::EPI_STORE, f32::ROWS_NK, true>(a, tiles, stream);
-  return f32::launch<f32::EPI_STORE, f32::ROWS_NK, false>(a, tiles, stream);
+  if (g_rows != nullptr) return f32::launch<f32::EPI_STORE, f32::ROWS_NK, true>(a, stream);
+  return f32::launch<f32::EPI_STORE, f32::ROWS_NK, false>(a, stream);
 }
 
 // dW[e] = L[rows of e]^T . R[rows of e], rows in expert order; an expert without rows gets zeros
@@ -343,7 +457,7 @@ int gemm_f32_wgrad(const void *L, const void *R, void *dW, const int *counts, co
   a.Nd = Nd; a.lda = Md; a.ldb = Nd; a.ldc = Nd;
   a.n_col_tiles = ceil_div(Nd, f32::kBN);
   a.n_m_tiles = ceil_div(Md, f32::kBM);
-  return f32::launch<f32::EPI_STORE, f32::WGRAD, false>(a, (long long)E * a.n_m_tiles * a.n_col_tiles, stream);
+  return f32::launch<f32::EPI_STORE, f32::WGRAD, false>(a, stream);
 }
 
 }  // namespace yamoe

@@ -148,7 +148,7 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
                                            int stream_max_rows, int *sched, const int lane) {
   int *row_tiles = sched + kSchedHeader;
   int *small = row_tiles + 8 * sched_max_row_tiles(N, E);
-  int n_tiles = 0, n_small = 0, n_active = 0, n_kept = 0;
+  int n_tiles = 0, n_small = 0, n_active = 0, n_kept = 0, n_half = 0;
   // Experts of 17 to 32 rows stream only when every expert streams: next to experts that need the tile kernels anyway
   // they are better off as tiles (two half-filled launches one after the other are slower than one: 0.35 against
   // 0.31 ms for 32 experts of about 32 rows, where 0.27 against 0.31 ms is gained when all of them have at most 32).
@@ -172,9 +172,11 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     // entries on the streaming list: one, or with `everything` one per chunk of kStreamMaxRows rows
     int is_small = everything ? ceil_div(kept, kStreamMaxRows) : (kept > 0 && kept <= stream_max_rows);
     int tiles = (kept > 0 && !is_small) ? ceil_div(kept, kRowTile) : 0;
-    int tot_small, tot_tiles, tot_active, tot_kept;
+    int tot_small, tot_tiles, tot_active, tot_kept, tot_half;
     int pos_small = wave_exclusive_scan(is_small, lane, tot_small);
     int pos_tiles = wave_exclusive_scan(tiles, lane, tot_tiles);
+    const int halves = tiles > 0 ? ceil_div(kept, kRowTile / 2) : 0;
+    const int pos_half = n_half + wave_exclusive_scan(halves, lane, tot_half);
     wave_exclusive_scan(kept > 0 ? 1 : 0, lane, tot_active);
     wave_exclusive_scan(kept, lane, tot_kept);
     for (int c = 0; c < is_small; ++c) {
@@ -190,9 +192,9 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     for (int t = 0; t < tiles; ++t) {
       int *w = row_tiles + 8 * (gfirst + t);
       w[0] = e; w[1] = first + t * per_tile; w[2] = min(per_tile, kept - t * per_tile); w[3] = gfirst; w[4] = tiles;
-      w[5] = (int)by_tiles.mul; w[6] = (int)by_tiles.shift; w[7] = 0;
+      w[5] = (int)by_tiles.mul; w[6] = (int)by_tiles.shift; w[7] = pos_half;
     }
-    n_small += tot_small; n_tiles += tot_tiles; n_active += tot_active; n_kept += tot_kept;
+    n_small += tot_small; n_tiles += tot_tiles; n_active += tot_active; n_kept += tot_kept; n_half += tot_half;
   }
   // Second pass: cut the tile list into 8 shares of equal cost.  Groups (experts with row tiles) are weighed
   // by the sum of their tiles' weights; cut x falls into the group that contains x/8 of the total.
@@ -225,7 +227,7 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   }
   if (lane == 0) {
     sched[0] = n_tiles; sched[1] = n_small; sched[2] = n_active; sched[3] = n_kept;
-    sched[4] = w_total; sched[5] = 0; sched[6] = 0; sched[7] = 0;
+    sched[4] = w_total; sched[kSchedHalfTiles] = n_half; sched[6] = 0; sched[7] = 0;
     int *c = sched + kSchedCuts + 4 * kXcds;  // the end of the list
     c[0] = n_tiles; c[1] = 0; c[2] = 0; c[3] = 0;
     if (w_total == 0)
