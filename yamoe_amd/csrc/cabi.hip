@@ -552,6 +552,18 @@ static int down_both(const void *act, const void *w, const void *bias, void *y, 
   if constexpr (HasStreamPath<T>::value) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, stream));
   return 0;
 }
+// The same for E groups of `rows` rows each (the work list of yamoe_build_schedule for them is made here, with counts and
+// offsets): whether they stream or are tiles is known on the host, so only one of the two kernels is launched (the other
+// would find an empty list for 4 us).
+template <typename T>
+static int down_regular(const void *act, const void *w, const void *bias, void *y, int *counts, int *offsets, void *sched,
+                        size_t sched_bytes, int E, int rows, int H, int I, hipStream_t stream) {
+  const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
+  YAMOE_TRY(regular_schedule(counts, offsets, E, rows, stream_rows, sched, sched_bytes, stream));
+  if constexpr (HasStreamPath<T>::value)
+    if (rows <= stream_rows) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream);
+  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, stream);
+}
 
 extern "C" int yamoe_gate_up(const void *x, const int32_t *sorted_idx, const void *gate_up_proj,
                              const void *gate_up_proj_bias, void *act, void *pre_act, const void *schedule, int32_t N,
@@ -859,11 +871,8 @@ static int batch_mm_impl(const void *x, const void *w, void *out, int E, int C, 
   int *offsets = (int *)c.take(((size_t)E + 1) * 4);
   size_t sched_bytes = yamoe_schedule_bytes(E * C, E);
   void *sched = c.take(sched_bytes);
-  YAMOE_TRY(yamoe_regular_groups(counts, offsets, E, C, (void *)stream));
-  const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
-  YAMOE_TRY(yamoe_build_schedule(counts, offsets, E * C, E, C, stream_rows, sched, sched_bytes, (void *)stream));
   // the down-projection launchers compute rows[.,Kd] x w[e][Kd,Nd] with no bias: exactly this product
-  return down_both<T>(x, w, nullptr, out, sched, E * C, E, /*H=*/Nd, /*I=*/Kd, stream);
+  return down_regular<T>(x, w, nullptr, out, counts, offsets, sched, sched_bytes, E, C, /*H=*/Nd, /*I=*/Kd, stream);
 }
 
 extern "C" int yamoe_batch_mm(const void *x, const void *weights, void *output, int32_t E, int32_t C, int32_t Kd,

@@ -226,6 +226,9 @@ int route_and_schedule(const void *router_indices, int32_t idx_i64, int32_t N, i
                        void *workspace, size_t workspace_bytes, int32_t stream_max_rows, void *schedule,
                        size_t schedule_bytes, void *stream);
 
+int regular_schedule(int *counts, int *offsets, int E, int rows, int stream_max_rows, void *schedule, size_t schedule_bytes,
+                     hipStream_t stream);
+
 // error reporting for the C ABI
 void set_error(const char *fmt, ...);
 int check_launch(const char *what);

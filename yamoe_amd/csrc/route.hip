@@ -241,6 +241,14 @@ __global__ __launch_bounds__(kWave) void build_schedule_kernel(const int *counts
   build_schedule_wave(counts, offsets, N, E, capacity, stream_max_rows, sched, threadIdx.x);
 }
 
+// counts[e] = rows, offsets[e] = e * rows and their work lists in one launch (a lane reads back only what it wrote itself)
+__global__ __launch_bounds__(kWave) void regular_schedule_kernel(int *counts, int *offsets, int E, int rows, int stream_max_rows,
+                                                                 int *sched) {
+  for (int e = threadIdx.x; e < E; e += kWave) { counts[e] = rows; offsets[e] = e * rows; }
+  if (threadIdx.x == 0) offsets[E] = E * rows;
+  build_schedule_wave(counts, offsets, E * rows, E, rows, stream_max_rows, sched, threadIdx.x);
+}
+
 // ---- single-block form: everything in one launch -------------------------------------------------
 // Dynamic LDS: hist[kRouteWaves][buckets] + total[buckets] + offsets[buckets+1] + scratch + the N keys as 16-bit
 // values.  The kernel runs once per forward on a cold instruction cache, so its loops stay rolled (straight-line
@@ -616,6 +624,17 @@ extern "C" int yamoe_route(const void *router_indices, int32_t idx_i64, int32_t 
                            size_t workspace_bytes, void *stream_) {
   return route_and_schedule(router_indices, idx_i64, N, E, capacity, sorted_expert, sorted_idx, counts, offsets, inv_pos,
                             workspace, workspace_bytes, 0, nullptr, 0, stream_);
+}
+
+int yamoe::regular_schedule(int *counts, int *offsets, int E, int rows, int stream_max_rows, void *schedule,
+                            size_t schedule_bytes, hipStream_t stream) {
+  if (schedule_bytes < yamoe_schedule_bytes(E * rows, E)) {
+    set_error("regular_schedule: schedule region too small");
+    return YAMOE_E_WORKSPACE;
+  }
+  hipLaunchKernelGGL(regular_schedule_kernel, dim3(1), dim3(kWave), 0, stream, counts, offsets, E, rows, stream_max_rows,
+                     (int *)schedule);
+  return check_launch("regular_schedule_kernel");
 }
 
 extern "C" size_t yamoe_schedule_bytes(int32_t N, int32_t E) {

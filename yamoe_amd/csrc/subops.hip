@@ -16,6 +16,8 @@ constexpr int kSortThreads = 1024;
 constexpr int kSortWaves = kSortThreads / kWave;
 constexpr int kSortSeg = 1024;  // elements per wave segment
 constexpr int kRadix = 256;
+constexpr int kScatterWaves = 16 * 256;    // waves that keep HBM busy in the scatter
+constexpr int kScatterOneBlock = 16384;    // slots that one workgroup indexes in one launch
 
 template <typename K>
 __device__ inline unsigned digit_of(K key, int shift, int bits, bool flip_sign) {
@@ -58,19 +60,10 @@ __global__ __launch_bounds__(kRadix) void sort_scan_kernel(int *seg_counts, int 
   }
 }
 
+// Places keys b .. e-1, one wave, in order: `cursor` (LDS, of this wave alone) holds where each digit's next key goes.
 template <typename K>
-__global__ __launch_bounds__(kSortThreads) void sort_place_kernel(const K *keys, const K *vals, bool iota_vals, int n,
-                                                                  int shift, int bits, bool flip_sign,
-                                                                  const int *seg_cursors, K *keys_out, K *vals_out) {
-  __shared__ int cursor_all[kSortWaves * kRadix];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int i = tid; i < kSortWaves * kRadix; i += kSortThreads)
-    cursor_all[i] = seg_cursors[(size_t)blockIdx.x * kSortWaves * kRadix + i];
-  __syncthreads();
-  int *cursor = cursor_all + wave * kRadix;
-  long long seg = (long long)blockIdx.x * kSortWaves + wave;
-  long long b = seg * kSortSeg, e = b + kSortSeg;
-  if (e > n) e = n;
+__device__ inline void sort_place_segment(const K *keys, const K *vals, bool iota_vals, long long b, long long e, int lane, int shift,
+                                          int bits, bool flip_sign, int *cursor, K *keys_out, K *vals_out) {
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   for (long long base = b; base < e; base += kWave) {
     long long i = base + lane;
@@ -98,6 +91,66 @@ __global__ __launch_bounds__(kSortThreads) void sort_place_kernel(const K *keys,
     // stores above); lanes address the cursor by key, so the compiler cannot carry its values across steps
     __builtin_amdgcn_wave_barrier();
   }
+}
+
+template <typename K>
+__global__ __launch_bounds__(kSortThreads) void sort_place_kernel(const K *keys, const K *vals, bool iota_vals, int n,
+                                                                  int shift, int bits, bool flip_sign,
+                                                                  const int *seg_cursors, K *keys_out, K *vals_out) {
+  __shared__ int cursor_all[kSortWaves * kRadix];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < kSortWaves * kRadix; i += kSortThreads)
+    cursor_all[i] = seg_cursors[(size_t)blockIdx.x * kSortWaves * kRadix + i];
+  __syncthreads();
+  int *cursor = cursor_all + wave * kRadix;
+  long long seg = (long long)blockIdx.x * kSortWaves + wave;
+  long long b = seg * kSortSeg, e = b + kSortSeg;
+  if (e > n) e = n;
+  sort_place_segment(keys, vals, iota_vals, b, e, lane, shift, bits, flip_sign, cursor, keys_out, vals_out);
+}
+
+// One pass over at most kSortWaves * kSortSeg keys, by one workgroup: each wave takes an equal contiguous segment, counts
+// its digits in LDS, the counts become cursors, and the wave places its keys.  Three launches in one; each launch of the
+// chain costs 4 us or more, whatever it does (4096 int32 keys of 4 bits: 25.0 us in three, 6.8 us in one).
+template <typename K>
+__global__ __launch_bounds__(kSortThreads) void sort_block_kernel(const K *keys, const K *vals, bool iota_vals, int n, int shift,
+                                                                  int bits, bool flip_sign, K *keys_out, K *vals_out) {
+  __shared__ int hist[kSortWaves * kRadix];
+  __shared__ int group_total[kRadix / kWave];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < kSortWaves * kRadix; i += kSortThreads) hist[i] = 0;
+  __syncthreads();
+  const int seg = ceil_div(ceil_div(n, kSortWaves), kWave) * kWave;
+  const int b = min(wave * seg, n), e = min(b + seg, n);
+  int *cursor = hist + wave * kRadix;
+  for (int i = b + lane; i < e; i += kWave) atomicAdd(&cursor[digit_of(keys[i], shift, bits, flip_sign)], 1);
+  __syncthreads();
+  // thread d: keys of digit d in the waves before each one, then in all smaller digits
+  int total = 0, before = 0;
+  if (tid < kRadix) {
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) {
+      const int c = hist[w * kRadix + tid];
+      hist[w * kRadix + tid] = total;
+      total += c;
+    }
+    int up = total;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const int v = __shfl_up(up, d);
+      if (lane >= d) up += v;
+    }
+    if (lane == kWave - 1) group_total[wave] = up;
+    before = up - total;
+  }
+  __syncthreads();
+  if (tid < kRadix) {
+    for (int g = 0; g < wave; ++g) before += group_total[g];
+#pragma unroll
+    for (int w = 0; w < kSortWaves; ++w) hist[w * kRadix + tid] += before;
+  }
+  __syncthreads();
+  sort_place_segment(keys, vals, iota_vals, b, e, lane, shift, bits, flip_sign, cursor, keys_out, vals_out);
 }
 
 template <typename K>
@@ -132,6 +185,14 @@ static int sort_impl(const void *x, int n, int end_bit, void *x_out, void *iota_
     K *dst_k = to_out ? (K *)x_out : tmp_k, *dst_v = to_out ? (K *)iota_out : tmp_v;
     int shift = 8 * p, bits = end_bit - shift < 8 ? end_bit - shift : 8;
     bool flip = (end_bit == width) && (p == passes - 1);
+    if (n_blocks == 1) {
+      hipLaunchKernelGGL(sort_block_kernel<K>, dim3(1), dim3(kSortThreads), 0, stream, src_k, src_v, p == 0, n, shift, bits, flip,
+                         dst_k, dst_v);
+      if (int rc = check_launch("sort_block_kernel")) return rc;
+      src_k = dst_k;
+      src_v = dst_v;
+      continue;
+    }
     hipLaunchKernelGGL(sort_hist_kernel<K>, dim3(n_blocks), dim3(kSortThreads), 0, stream, src_k, n, shift, bits, flip,
                        seg_counts);
     hipLaunchKernelGGL(sort_scan_kernel, dim3(1), dim3(kRadix), 0, stream, seg_counts, n_seg);
@@ -211,47 +272,106 @@ __global__ __launch_bounds__(256) void padded_gather_kernel(const T *x, const in
 }
 
 // ---- padded scatter (csrc/scatter.cu:66-147): y[tok,:] += src[e,i,:] * w[start_e+i] -----------------------
-// Done without atomics: pass 1 records, for every flat slot, which padded row (if any) feeds it; pass 2
-// owns one output row per wave and adds that token's rows in slot order.
-__global__ void scatter_index_kernel(const int *idx, const int *bins, int *slot_row, int S, int E, int C) {
-  int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= S) return;
-  // expert of sorted position p: first e with bins[e] > p
-  int lo = 0, hi = E;
-  while (lo < hi) {
-    int mid = (lo + hi) >> 1;
-    if (bins[mid] > p) hi = mid; else lo = mid + 1;
+// Done without atomics: pass 1 records, for every flat slot, which padded row (if any) feeds it; in pass 2 one to four
+// waves own an output row and add that token's rows in slot order.
+// slots[flat] = {padded row, sorted position} of every flat slot, {-1, -1} for slots without a row.  With few slots one
+// workgroup clears and fills them in one launch; `clear` is false where scatter_clear_kernel has run before.
+__global__ __launch_bounds__(1024) void scatter_index_kernel(const int *idx, const int *bins, int2 *slots, int S, int E, int C,
+                                                             bool clear) {
+  if (clear) {  // (a grid of one workgroup)
+    for (int p = threadIdx.x; p < S; p += blockDim.x) slots[p] = make_int2(-1, -1);
+    __syncthreads();
   }
-  if (lo >= E) return;
-  int start = lo == 0 ? 0 : bins[lo - 1];
-  int i = p - start;
-  int flat = idx[p];
-  if (i < C && flat >= 0 && flat < S) slot_row[flat] = lo * C + i;
+  const long long step = (long long)gridDim.x * blockDim.x;
+  for (long long at = (long long)blockIdx.x * blockDim.x + threadIdx.x; at < S; at += step) {
+    const int p = (int)at;
+    // expert of sorted position p: first e with bins[e] > p
+    int lo = 0, hi = E;
+    while (lo < hi) {
+      int mid = (lo + hi) >> 1;
+      if (bins[mid] > p) hi = mid; else lo = mid + 1;
+    }
+    if (lo >= E) continue;
+    int start = lo == 0 ? 0 : bins[lo - 1];
+    int i = p - start;
+    int flat = idx[p];
+    if (i < C && flat >= 0 && flat < S) slots[flat] = make_int2(lo * C + i, p);
+  }
 }
-template <typename T>
-__global__ __launch_bounds__(256) void padded_scatter_kernel(const T *src, const int *slot_row, const int *idx_unused,
-                                                             const int *bins, const T *weights, T *y, int Tn, int H, int C,
-                                                             int top_k, int E) {
+// KS > 0: 16-byte chunks, all rows of a token (at most KS slots, the same for all lanes of the wave) requested together;
+// 0: any number of slots, any width or alignment.  Both add the rows to y in slot order.  HBM-bound; one element per lane
+// with the row number looked up and divided for each took 37.6 us for 2048 tokens x 2 x 1024 fp16, this takes 5.5.
+template <typename T, int KS>
+__global__ __launch_bounds__(256) void padded_scatter_kernel(const T *__restrict__ src, const int2 *__restrict__ slots,
+                                                             const T *__restrict__ weights, T *__restrict__ y, int Tn, int H,
+                                                             int top_k, int split) {
+  typedef typename ElemTraits<T>::acc_t acc_t;
   const int lane = threadIdx.x & 63;
-  for (int t = blockIdx.x * 4 + (threadIdx.x >> 6); t < Tn; t += gridDim.x * 4) {
-    for (int c = lane; c < H; c += 64) {
-      typedef typename ElemTraits<T>::acc_t acc_t;
-      acc_t acc = ElemTraits<T>::to_acc(y[(long long)t * H + c]);
-      for (int k = 0; k < top_k; ++k) {
-        int row = slot_row[t * top_k + k];
-        if (row < 0) continue;
-        int e = row / C, i = row - e * C;
-        int start = e == 0 ? 0 : bins[e - 1];
-        acc_t w = weights ? ElemTraits<T>::to_acc(weights[start + i]) : (acc_t)1;
-        acc += w * ElemTraits<T>::to_acc(src[(long long)row * H + c]);
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int part = wave % split;
+  for (int t = wave / split; t < Tn; t += gridDim.x * 4 / split) {
+    if constexpr (KS > 0) {
+      constexpr int V = ElemTraits<T>::kVec;
+      int row[KS];
+      acc_t w[KS];
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const int2 at = k < top_k ? slots[t * top_k + k] : make_int2(-1, -1);
+        row[k] = at.x;
+        w[k] = at.x >= 0 && weights != nullptr ? ElemTraits<T>::to_acc(weights[at.y]) : (acc_t)1;
       }
-      y[(long long)t * H + c] = ElemTraits<T>::from_acc(acc);
+      u32x4 *dst = (u32x4 *)(y + (long long)t * H);
+      for (int c = part * kWave + lane; c < H / V; c += kWave * split) {
+        u32x4 raw[KS], o = dst[c];
+#pragma unroll
+        for (int k = 0; k < KS; ++k) raw[k] = ((const u32x4 *)(src + (long long)max(row[k], 0) * H))[c];
+        T *ov = (T *)&o;
+        acc_t acc[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[j] = ElemTraits<T>::to_acc(ov[j]);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) {
+          if (row[k] < 0) continue;
+          const T *v = (const T *)&raw[k];
+#pragma unroll
+          for (int j = 0; j < V; ++j) acc[j] += w[k] * ElemTraits<T>::to_acc(v[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < V; ++j) ov[j] = ElemTraits<T>::from_acc(acc[j]);
+        dst[c] = o;
+      }
+    } else {
+      for (int c = part * kWave + lane; c < H; c += kWave * split) {
+        acc_t acc = ElemTraits<T>::to_acc(y[(long long)t * H + c]);
+        for (int k = 0; k < top_k; ++k) {
+          const int2 at = slots[t * top_k + k];
+          if (at.x < 0) continue;
+          acc_t w = weights != nullptr ? ElemTraits<T>::to_acc(weights[at.y]) : (acc_t)1;
+          acc += w * ElemTraits<T>::to_acc(src[(long long)at.x * H + c]);
+        }
+        y[(long long)t * H + c] = ElemTraits<T>::from_acc(acc);
+      }
     }
   }
 }
-__global__ void fill_i32_kernel(int *p, int n, int v) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = v;
+template <typename T>
+static void launch_padded_scatter(const void *src, const int2 *slots, const void *weights, void *y, int Tn, int H, int top_k,
+                                  hipStream_t stream) {
+  const int split = Tn >= kScatterWaves ? 1 : 2 * Tn >= kScatterWaves ? 2 : 4;
+  const int blocks = min(ceil_div(Tn, 4 / split), 65536);
+  const bool chunks = H % ElemTraits<T>::kVec == 0 && ((uintptr_t)src | (uintptr_t)y) % 16 == 0 && top_k <= 8;
+#define YAMOE_SCATTER(KS)                                                                                             \
+  hipLaunchKernelGGL((padded_scatter_kernel<T, KS>), dim3(blocks), dim3(256), 0, stream, (const T *)src, slots,       \
+                     (const T *)weights, (T *)y, Tn, H, top_k, split)
+  if (!chunks) YAMOE_SCATTER(0);
+  else if (top_k > 4) YAMOE_SCATTER(8);
+  else if (top_k > 2) YAMOE_SCATTER(4);
+  else YAMOE_SCATTER(2);
+#undef YAMOE_SCATTER
+}
+__global__ void scatter_clear_kernel(int2 *slots, int S) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < S) slots[i] = make_int2(-1, -1);
 }
 
 // ---- index_select_out (csrc/index_select.cu:7-51): out[i] = in[idx[i]] ------------------------------------
@@ -330,7 +450,7 @@ extern "C" int yamoe_padded_gather(const void *x, const int32_t *indices, const 
   return check_launch("padded_gather_kernel");
 }
 
-extern "C" size_t yamoe_padded_scatter_workspace_bytes(int32_t S) { return align_up((size_t)(S > 0 ? S : 1) * 4, 256); }
+extern "C" size_t yamoe_padded_scatter_workspace_bytes(int32_t S) { return align_up((size_t)(S > 0 ? S : 1) * 8, 256); }
 
 extern "C" int yamoe_padded_scatter(const void *src, const int32_t *indices, const int32_t *bins, const void *weights,
                                     void *y, int32_t T_, int32_t H, int32_t E, int32_t C, int32_t top_k, int32_t dtype,
@@ -343,12 +463,12 @@ extern "C" int yamoe_padded_scatter(const void *src, const int32_t *indices, con
     return YAMOE_E_ARG;
   }
   hipStream_t st = (hipStream_t)stream;
-  int *slot_row = (int *)workspace;
-  hipLaunchKernelGGL(fill_i32_kernel, dim3(ceil_div(S, 256)), dim3(256), 0, st, slot_row, S, -1);
-  hipLaunchKernelGGL(scatter_index_kernel, dim3(ceil_div(S, 256)), dim3(256), 0, st, indices, bins, slot_row, S, E, C);
-  int blocks = (T_ + 3) / 4 < 65536 ? (T_ + 3) / 4 : 65536;
-  YAMOE_DISPATCH(dtype, hipLaunchKernelGGL(padded_scatter_kernel<T>, dim3(blocks), dim3(256), 0, st, (const T *)src, slot_row,
-                                           indices, bins, (const T *)weights, (T *)y, T_, H, C, top_k, E));
+  int2 *slots = (int2 *)workspace;
+  const bool one = S <= kScatterOneBlock;
+  if (!one) hipLaunchKernelGGL(scatter_clear_kernel, dim3(ceil_div(S, 256)), dim3(256), 0, st, slots, S);
+  hipLaunchKernelGGL(scatter_index_kernel, dim3(one ? 1 : ceil_div(S, 256)), dim3(one ? 1024 : 256), 0, st, indices, bins, slots,
+                     S, E, C, one);
+  YAMOE_DISPATCH(dtype, launch_padded_scatter<T>(src, slots, weights, y, T_, H, top_k, st));
   return check_launch("padded_scatter_kernel");
 }
 
