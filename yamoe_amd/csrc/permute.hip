@@ -9,11 +9,9 @@
 
 namespace yamoe {
 
-#ifndef YAMOE_COMBINE_SPLIT_T
-#define YAMOE_COMBINE_SPLIT_T 1024
-#endif
 constexpr int kRowThreads = 256;
 constexpr int kRowWaves = kRowThreads / kWave;
+constexpr int kCombineWaves = 16 * 256;  // waves that keep HBM busy in the combine
 
 // x_perm[p,:] = x[sorted_idx[p] / K,:]   (csrc/gather.cu:6-66 without the padding rows)
 template <typename T>
@@ -52,44 +50,42 @@ __device__ inline float slot_weight(const T *rw, const void *idx, int t, int k, 
 }
 
 // out[t,:] = sum_k w(t,k) * y_perm[inv_pos[t*K+k],:]
-// `split` waves per token (1, or the 4 of a workgroup when there are few tokens: a lone wave goes through a 2880-wide
-// row in six dependent rounds of loads).  The K (position, weight) pairs of the token are fetched once (up to
-// kMaxSlots of them sit in registers), then every lane streams its 16-byte chunks of the K rows.
-constexpr int kMaxSlots = 8;
-
-template <typename T, bool I64>
+// HBM-bound, so what counts is how many rows are on the way.  `split` waves share a token (1, 2 or the 4 of a workgroup, so
+// that a few tokens still fill the chip).  KS: the slots of a token, rounded up to 1, 2, 4 or 8 (0: any number, or rows
+// that are not whole 16-byte chunks).  The token is the same for all lanes of a wave and said to be, so the (position,
+// weight) pairs come through scalar loads and the rows of a chunk are requested together before the first of them is
+// added (a dropped slot requests row 0 and adds nothing); with a test in front of each row's load the wave waited for
+// one row after the other: us before -> now, 1536 tokens x 8 x 2048 bf16: 24.4 -> 13.4 (4.2 TB/s); 2003 x 4 x 2880:
+// 15.4 -> 11.9; 4096 x 4 x 2880: 26.2 -> 23.4 (5 TB/s); 1 x 4 x 2880: 5.3 -> 4.5, a launch's own cost.
+template <typename T, bool I64, int KS>
 __global__ __launch_bounds__(kRowThreads) void combine_kernel(
     const T *__restrict__ y_perm, const int *__restrict__ inv_pos, const void *__restrict__ idx,
     const T *__restrict__ rw, int rw_cols, T *__restrict__ out, int Tn, int K, int E, int H, int split) {
   const int lane = threadIdx.x & (kWave - 1);
-  const int wave = blockIdx.x * kRowWaves + threadIdx.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * kRowWaves + threadIdx.x / kWave);
   const int n_waves = gridDim.x * kRowWaves;
   constexpr int V = ElemTraits<T>::kVec;
-  const bool vec_ok = (H % V) == 0;
   const int part = wave % split, stride = kWave * split;
   for (int t = wave / split; t < Tn; t += n_waves / split) {
     T *dst = out + (size_t)t * H;
-    if (vec_ok && K <= kMaxSlots) {
-      int pos[kMaxSlots];
-      float w[kMaxSlots];
+    if constexpr (KS > 0) {
+      int pos[KS];
+      float w[KS];
 #pragma unroll
-      for (int k = 0; k < kMaxSlots; ++k) {
-        pos[k] = -1;
-        w[k] = 0.0f;
-        if (k < K) {
-          pos[k] = inv_pos[(size_t)t * K + k];
-          if (pos[k] >= 0) w[k] = slot_weight<T, I64>(rw, idx, t, k, K, E, rw_cols);
-        }
-      }
+      for (int k = 0; k < KS; ++k) pos[k] = k < K ? inv_pos[(size_t)t * K + k] : -1;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) w[k] = pos[k] >= 0 ? slot_weight<T, I64>(rw, idx, t, k, K, E, rw_cols) : 0.0f;
       for (int c = part * kWave + lane; c < H / V; c += stride) {
+        u32x4 raw[KS];
+#pragma unroll
+        for (int k = 0; k < KS; ++k) raw[k] = ((const u32x4 *)(y_perm + (size_t)max(pos[k], 0) * H))[c];
         float acc[V];
 #pragma unroll
         for (int j = 0; j < V; ++j) acc[j] = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kMaxSlots; ++k) {
+        for (int k = 0; k < KS; ++k) {
           if (pos[k] < 0) continue;
-          u32x4 raw = ((const u32x4 *)(y_perm + (size_t)pos[k] * H))[c];
-          const T *v = (const T *)&raw;
+          const T *v = (const T *)&raw[k];
 #pragma unroll
           for (int j = 0; j < V; ++j) acc[j] += w[k] * ElemTraits<T>::to_f32(v[j]);
         }
@@ -359,14 +355,22 @@ int launch_combine(const void *y_perm, const int *inv_pos, const void *idx, int 
                    const void *rw, int rw_cols, void *out, int Tn, int K, int E, int H,
                    hipStream_t stream) {
   if (Tn == 0) return 0;
-  const int split = Tn <= YAMOE_COMBINE_SPLIT_T ? kRowWaves : 1;  // (the grid is a whole number of groups of `split` waves)
-  int blocks = min(ceil_div(Tn * split, kRowWaves), 256 * 16);
-  if (idx_i64)
-    hipLaunchKernelGGL((combine_kernel<T, true>), dim3(blocks), dim3(kRowThreads), 0, stream,
-                       (const T *)y_perm, inv_pos, idx, (const T *)rw, rw_cols, (T *)out, Tn, K, E, H, split);
-  else
-    hipLaunchKernelGGL((combine_kernel<T, false>), dim3(blocks), dim3(kRowThreads), 0, stream,
-                       (const T *)y_perm, inv_pos, idx, (const T *)rw, rw_cols, (T *)out, Tn, K, E, H, split);
+  // 16 waves per CU, or as many as four per token give (the grid is a whole number of groups of `split` waves)
+  const int split = Tn >= kCombineWaves ? 1 : 2 * Tn >= kCombineWaves ? 2 : kRowWaves;
+  const int blocks = min(ceil_div(Tn * split, kRowWaves), 256 * 16);
+  const bool chunks = H % ElemTraits<T>::kVec == 0;
+#define YAMOE_COMBINE(I64, KS)                                                                                        \
+  hipLaunchKernelGGL((combine_kernel<T, I64, KS>), dim3(blocks), dim3(kRowThreads), 0, stream, (const T *)y_perm, inv_pos, \
+                     idx, (const T *)rw, rw_cols, (T *)out, Tn, K, E, H, split)
+#define YAMOE_COMBINE_SLOTS(I64)                \
+  if (!chunks || K > 8) YAMOE_COMBINE(I64, 0);  \
+  else if (K > 4) YAMOE_COMBINE(I64, 8);        \
+  else if (K > 2) YAMOE_COMBINE(I64, 4);        \
+  else if (K > 1) YAMOE_COMBINE(I64, 2);        \
+  else YAMOE_COMBINE(I64, 1);
+  if (idx_i64) { YAMOE_COMBINE_SLOTS(true) } else { YAMOE_COMBINE_SLOTS(false) }
+#undef YAMOE_COMBINE_SLOTS
+#undef YAMOE_COMBINE
   return check_launch("combine_kernel");
 }
 
