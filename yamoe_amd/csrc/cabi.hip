@@ -106,9 +106,18 @@ template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
 template <typename T> struct HasStreamPath { static constexpr bool value = sizeof(T) == 2; };
 
+// Whether a product of N rows over E experts with Nd columns runs on 128 x 128 tiles (two workgroups per CU) instead of
+// 256 x 256 (one).  The small tiles read twice the operand bytes per flop, so they pay only where the large ones leave CUs
+// idle: while the whole product is little more than one small tile per CU.  An expert's last tile is half full on average,
+// and an expert has a tile at least, hence the estimate; its rows are not known on the host.
+// Each side measured over 104 layers (16 to 64 experts, widths 304 to 2880, 300 to 8192 tokens), the four products of a
+// training step, large / small in us: 312 small tiles, 250 rows per expert, 1024 x 1024: down 24.8 / 17.0, its input
+// gradient 31.9 / 17.8; 316, 2048 x 512: 49.4 / 33.0; 256, 19 rows, 2048 x 1024: 32.0 / 24.9; but 368, 38 rows, 720 x 2880:
+// 14.8 / 20.4; 376, 125 rows, 1024 x 1024: 22.6 / 27.9; 384, 125 rows, 2048 x 1024: 21.6 / 27.8.  Where nearly every
+// expert is one tile the weights are the bound and the line lies lower (320 of 37 rows, 1024 x 608: 21.1 / 26.6).
 static bool takes_small_tiles(int N, int E, int Nd) {
-  const char *e = getenv("YT");
-  return e && e[0] == '1';
+  const long long cols = ceil_div(Nd, 128), rows = ((long long)N + 64ll * E) / 128;
+  return rows <= E ? E * cols <= 256 : rows * cols <= 320;
 }
 
 static int gathered_span_ok(const char *who, long long span_bytes) {
@@ -817,11 +826,9 @@ static int router_backward_impl(const void *d_scores, const long long *indices, 
   RouterBackwardBuffers b;
   carve_router_backward(Tn, E, ElemTraits<T>::kDtype, ws, &b);
   YAMOE_TRY(launch_router_backward_logits<T>(d_scores, indices, scores, Tn, E, K, b.d_logits, stream));
-  YAMOE_TRY(yamoe_regular_groups(b.counts, b.offsets, 1, Tn, (void *)stream));
-  const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
-  YAMOE_TRY(yamoe_build_schedule(b.counts, b.offsets, Tn, 1, Tn, stream_rows, b.schedule, b.schedule_bytes, (void *)stream));
   // d_hidden [T, H] = d_logits [T, E] . weight [E, H]: the down-projection launchers compute rows[., Kd] x w[Kd, Nd]
-  YAMOE_TRY(down_both<T>(b.d_logits, weight, nullptr, d_hidden, b.schedule, Tn, 1, /*H=*/H, /*I=*/E, stream));
+  YAMOE_TRY(down_regular<T>(b.d_logits, weight, nullptr, d_hidden, b.counts, b.offsets, b.schedule, b.schedule_bytes, 1, Tn,
+                            /*H=*/H, /*I=*/E, stream));
   // d_weight [E, H] = d_logits^T . hidden, contraction over the T rows (kernels that read nothing past the end of the
   // caller's tensors: the register-staged one for 16-bit data)
   if constexpr (sizeof(T) == 4)
