@@ -20,6 +20,7 @@ struct WgradArgs {
   const int *counts, *offsets;
   const int *a_rows;
   FastDiv a_div;
+  FastDiv band_div;  // division by kWgradBand * n_n_tiles
   int a_rows_max;  // largest value a_rows may hold
   int capacity, E, Md, Nd, n_m_tiles, n_n_tiles;
   // optional: [E, Nd] column sums of the expert's rows of B (the bias gradient that goes with this weight gradient,
@@ -37,6 +38,10 @@ template <bool P1_, bool P2_, bool NEXT_, bool ZERO_, int VM_> struct WStepCfg {
 // and storing its result, and with a second workgroup on the same SIMDs the matrix pipe works through that.
 constexpr int kSmallBM = 128, kSmallStages = 3;
 constexpr int kSmallAStage = kBK * kSmallBM * 2, kSmallBStage = kBK * kBN * 2;  // 8 KB + 16 KB per slab
+// From four slabs on (97 rows) a tile goes through the pipelined loop, which starts once one slab is there; shorter ones
+// wait for everything they contract.  (With the line at six slabs, forward + backward of 32 experts of 128 rows, 2048 x 2048,
+// took 882 us against 848; of 125 rows, 2880 x 2880, 1383 against 1334.)
+constexpr int kSmallPipelined = kSmallStages + 1;
 constexpr int kSmallBRing = kSmallStages * kSmallAStage;
 constexpr int kSmallRing = kSmallStages * (kSmallAStage + kSmallBStage);
 constexpr int kSmallStaging = kSmallBM * (kBN * 2 + 16);
@@ -196,12 +201,12 @@ __device__ inline void run_wgrad_tile_small(const WgradArgs &args, const int tid
 #pragma unroll
     for (int s = 0; s < kSmallStages; ++s)
       if (s < n_slabs) copy_slab(s);
-    if (n_slabs >= 6) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");  // slab 0 is enough to start with
+    if (n_slabs >= kSmallPipelined) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");  // slab 0 is enough to start with
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     plant_ones(0);
 #pragma unroll
     for (int s = 0; s < kSmallStages; ++s)
-      if (n_slabs < 6 && s < n_slabs && (s + 1) * kBK > rows) zero_tail(s);
+      if (n_slabs < kSmallPipelined && s < n_slabs && (s + 1) * kBK > rows) zero_tail(s);
     __syncthreads();
     read_frags(0, 0, fa0, fb0);
   }
@@ -341,7 +346,7 @@ __device__ inline void run_wgrad_tile_small(const WgradArgs &args, const int tid
       }
     }
   };
-  if (n_slabs >= 6) {
+  if (n_slabs >= kSmallPipelined) {
     typedef std::integral_constant<int, 0> S0;
     typedef std::integral_constant<int, 1> S1;
     typedef std::integral_constant<int, 2> S2;
@@ -410,6 +415,15 @@ __device__ inline void run_wgrad_tile_small(const WgradArgs &args, const int tid
   }
 }
 
+// An expert's output tiles are taken in bands of this many row tiles, each band column by column.  An XCD has 64 tiles in
+// flight, and they write their gradients as they finish: in a band those are 4 row tiles of 16 neighbouring columns, whole
+// 8 KB stretches of a gradient's rows, and 4 + 16 operand tiles shared in the L2.  Column by column over the whole expert
+// they were 16 to 23 row tiles of 3 or 4 columns, and the writes (1.1 GB a step) went out as 2 KB pieces one row apart.
+// Forward + backward, whole columns / bands of 2 / 3 / 4 / 6 / rows of all columns, us: 1536 x 8 tokens on 64 experts,
+// 2048 x 2048: 2022 / 1940 / 1937 / 1953 / 1948 / 1941; 1000 x 4 on 32, 2880 x 2880: 1452 / 1389 / 1388 / 1383 / 1386 / 1400;
+// 4096 x 4 on 32, 2880 x 2880: 3319 / 3294 / 3303 / 3286 / 3281 / 3307.  Experts with few row tiles (1024 x 1024) don't care.
+constexpr int kWgradBand = 4;
+
 template <typename T, bool GATHER>
 __global__ __launch_bounds__(kThreads, 2) void wgrad_small_kernel(const WgradArgs args) {
   const int tid = threadIdx.x, wave = tid >> 6, wm = wave >> 1;
@@ -421,7 +435,10 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_small_kernel(const WgradArg
   const int L = (b % kXcds) * (total8 / kXcds) + b / kXcds;
   if (L >= total) return;
   const int expert = L / per_expert, r = L - expert * per_expert;
-  const int n0 = (r / args.n_m_tiles) * kBN, m0 = (r % args.n_m_tiles) * kSmallBM;
+  const int band = fast_div(r, args.band_div), in_band = r - band * kWgradBand * args.n_n_tiles;
+  const int band_rows = min(kWgradBand, args.n_m_tiles - band * kWgradBand);
+  const int col_tile = in_band / band_rows;
+  const int n0 = col_tile * kBN, m0 = (band * kWgradBand + in_band - col_tile * band_rows) * kSmallBM;
   const int rows_m = min(kSmallBM, args.Md - m0);
   // (the same for every lane; said explicitly, so that the operand addresses built from them stay in scalar registers)
   int rows = min(__builtin_amdgcn_readfirstlane(args.counts[expert]), args.capacity);
@@ -475,6 +492,7 @@ int gemm_async_wgrad(const void *L, const int *l_rows, int l_div, int n_rows, co
   a.E = E; a.Md = Md; a.Nd = Nd;
   a.n_m_tiles = ceil_div(Md, async::kSmallBM);
   a.n_n_tiles = ceil_div(Nd, async::kBN);
+  a.band_div = make_fast_div(async::kWgradBand * a.n_n_tiles);
   if (l_rows != nullptr) return async::launch_wgrad<T, true>(a, stream);
   return async::launch_wgrad<T, false>(a, stream);
 }
