@@ -227,3 +227,25 @@ def test_router_backward(gpu, dtype, T, H, E, K):
     z_x, z_w, z_b = _cabi.router_backward(g0.to(gpu), idx, scores, x.to(gpu), w.to(gpu), K)
     torch.cuda.synchronize()
     assert float(z_x.abs().max()) == 0 and float(z_w.abs().max()) == 0 and float(z_b.abs().max()) == 0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,H,E,K", [(1, 8, 8, 1), (31, 40, 72, 20), (33, 1032, 64, 16), (513, 72, 200, 17), (1040, 96, 128, 4)])
+def test_router_backward_edges(gpu, dtype, T, H, E, K):
+    """Tokens around a slab of 32 and around the 16 slabs that the waves of a workgroup share, experts and columns that end
+    inside a tile, more picks than lanes per token.  The scores come from the oracle (the forward picks at most 16)."""
+    from yamoe_amd import _cabi
+    print("router backward edges", dtype, T, H, E, K, flush=True)
+    x, w, b = draw(T, H, E, dtype, 5 * T + E)
+    idx = torch.topk(x.float() @ w.float().T + b.float(), K, dim=1).indices
+    leaves = [t.float().requires_grad_(True) for t in (x, w, b)]
+    _, want_scores, _ = O.router(*leaves, K, compute_dtype=torch.float32, picks=idx)
+    g = torch.randn(T, E, generator=torch.Generator().manual_seed(T)).to(dtype)
+    want = torch.autograd.grad(want_scores, leaves, g.float())
+    got = _cabi.router_backward(g.to(gpu), idx.to(gpu), want_scores.detach().to(dtype).to(gpu), x.to(gpu), w.to(gpu), K)
+    torch.cuda.synchronize()
+    for name, a, ref in zip(("d_hidden", "d_weight", "d_bias"), got, want):
+        if K > 1:   # (one pick: its score is 1 whatever the logits are, every gradient is zero)
+            assert report("router backward " + name, a.cpu().double(), ref.double(), 2e-2) < 2e-2, name
+        else:
+            assert float(a.abs().max()) == 0, name

@@ -57,8 +57,6 @@ int launch_combine_backward(const void *, const void *, const int *, const int *
 template <typename T>
 int launch_expert_colsum(const void *, const int *, const int *, int, void *, int, int, hipStream_t);
 template <typename T>
-int gemm_wgrad(const void *, const void *, void *, const int *, const int *, int, int, int, int, hipStream_t);
-template <typename T>
 int glu_backward_rows(const void *, const void *, const float *, const float *, int, const int *, const int *, void *,
                       float *, int, int, hipStream_t);
 template <typename T>
@@ -91,6 +89,8 @@ bool wgrad_async_supported(int Md, int Nd);
 
 template <typename T>
 int launch_router_backward_logits(const void *, const long long *, const void *, int, int, int, void *, hipStream_t);
+template <typename T>
+int launch_router_weight_grad(const void *, const void *, int, int, int, void *, void *, hipStream_t);
 
 // the plain-FMA path (plain.hip): double precision, and sizes that are not whole 16-byte chunks
 template <typename T>
@@ -196,12 +196,11 @@ template <typename T>
 static int tiles_wgrad(const void *L, const int *l_rows, int l_div, int n_rows, const void *R, void *dW, void *d_bias,
                        const int *counts, const int *offsets, int capacity, int E, int Md, int Nd, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
-    if (wgrad_async_supported(Md, Nd))
-      return gemm_async_wgrad<T>(L, l_rows, l_div, n_rows, R, dW, d_bias, counts, offsets, capacity, E, Md, Nd, stream);
+    return gemm_async_wgrad<T>(L, l_rows, l_div, n_rows, R, dW, d_bias, counts, offsets, capacity, E, Md, Nd, stream);
+  } else {
+    if (l_rows != nullptr || d_bias != nullptr) { set_error("tiles_wgrad: this kernel takes its rows in expert order and sums no bias"); return YAMOE_E_ARG; }
+    return gemm_f32_wgrad(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
   }
-  if (l_rows != nullptr || d_bias != nullptr) { set_error("tiles_wgrad: this kernel takes its rows in expert order and sums no bias"); return YAMOE_E_ARG; }
-  if constexpr (sizeof(T) == 4) return gemm_f32_wgrad(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
-  else return gemm_wgrad<T>(L, R, dW, counts, offsets, capacity, E, Md, Nd, stream);
 }
 
 __global__ void fill_zero_kernel(uint32_t *p, long long n_words) {
@@ -795,9 +794,9 @@ extern "C" int yamoe_experts_backward_kept(const yamoe_problem *p, const void *g
 }
 
 // ---- gradient of the router step ------------------------------------------------------------------------
-// d_logits from the softmax over the picks (router.hip), then the two products and the column sums on the expert
-// layer's own kernels, with the whole batch as the one "expert": d_hidden = d_logits . W (a [T, E] x [E, H] product of
-// rows), d_weight = d_logits^T . hidden (a weight-gradient product over the T rows), d_bias = column sums.
+// d_logits from the softmax over the picks (router.hip), then d_hidden = d_logits . W, a [T, E] x [E, H] product of rows, on
+// the expert layer's own kernels with the whole batch as the one "expert", and d_weight = d_logits^T . hidden with d_bias,
+// the column sums: for 16-bit data by a kernel of its own (router.hip), for fp32 on the expert layer's.
 struct RouterBackwardBuffers {
   void *d_logits, *schedule;
   int *counts, *offsets;
@@ -829,13 +828,14 @@ static int router_backward_impl(const void *d_scores, const long long *indices, 
   // d_hidden [T, H] = d_logits [T, E] . weight [E, H]: the down-projection launchers compute rows[., Kd] x w[Kd, Nd]
   YAMOE_TRY(down_regular<T>(b.d_logits, weight, nullptr, d_hidden, b.counts, b.offsets, b.schedule, b.schedule_bytes, 1, Tn,
                             /*H=*/H, /*I=*/E, stream));
-  // d_weight [E, H] = d_logits^T . hidden, contraction over the T rows (kernels that read nothing past the end of the
-  // caller's tensors: the register-staged one for 16-bit data)
-  if constexpr (sizeof(T) == 4)
+  // d_weight [E, H] = d_logits^T . hidden, contraction over the T rows, and d_bias (kernels that read nothing past the end
+  // of the caller's tensors)
+  if constexpr (sizeof(T) == 4) {
     YAMOE_TRY(gemm_f32_wgrad(b.d_logits, hidden, d_weight, b.counts, b.offsets, Tn, 1, /*Md=*/E, /*Nd=*/H, stream));
-  else
-    YAMOE_TRY(gemm_wgrad<T>(b.d_logits, hidden, d_weight, b.counts, b.offsets, Tn, 1, /*Md=*/E, /*Nd=*/H, stream));
-  if (d_bias != nullptr) YAMOE_TRY(launch_expert_colsum<T>(b.d_logits, b.counts, b.offsets, Tn, d_bias, 1, E, stream));
+    if (d_bias != nullptr) YAMOE_TRY(launch_expert_colsum<T>(b.d_logits, b.counts, b.offsets, Tn, d_bias, 1, E, stream));
+  } else {
+    YAMOE_TRY(launch_router_weight_grad<T>(b.d_logits, hidden, Tn, H, E, d_weight, d_bias, stream));
+  }
   return 0;
 }
 
