@@ -177,7 +177,7 @@ static int tiles_dgrad(const void *g, const int *g_rows, int g_div, long long g_
 }
 
 // True when the weight-gradient kernel for this dtype and shape can gather the rows of its left operand by token
-// (the register-staged kernel wants them in expert order).
+// (the fp32 kernel wants them in expert order).
 template <typename T> static bool wgrad_gathers(int Md, int Nd) {
   if constexpr (sizeof(T) == 2) return wgrad_async_supported(Md, Nd);
   return false;

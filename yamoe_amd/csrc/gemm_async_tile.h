@@ -779,7 +779,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
 
 #ifdef YAMOE_TILE_STAMPS
   // (after the work-list look-ups and the gathered row numbers: a_off depends on both)
-  asm volatile("s_waitcnt vmcnt(0)" : : "v"(a_off[0]), "v"(a_off[7]) : "memory");
+  asm volatile("s_waitcnt vmcnt(0)" : : "v"(a_off[0]), "v"(a_off[S::kACopies - 1]) : "memory");
   ti.t_lookup = __builtin_amdgcn_s_memtime();
 #endif
   const int n_blocks32 = (ti.rows_valid + 31) >> 5;
