@@ -30,3 +30,34 @@ def test_contractions_that_end_inside_a_slab_pair(gpu, dtype, H, I, T, E):
     for n, a, b in zip(names, (out, *grads), want):
         r = O.rel_l2(a.cpu(), b)
         assert r < REL_L2_TOL[dtype], (n, r)
+
+
+def _with_infinite_up_weights(H, I, dtype):
+    """Infinite weights in the last row of two up columns of every expert: what they reach is clamped, so the result is
+    finite, unless a kernel takes that row once more to fill a slab and multiplies it by zero."""
+    d = make_inputs(300, H, I, 3, 2, dtype, seed=H, w_std=0.05, bias_std=0.1)
+    d["gate_up_proj"][:, H - 1, [1, 2 * I - 1]] = float("inf")
+    return d
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,I", [(8, 24), (56, 72), (104, 40), (152, 264), (168, 40), (264, 72), (456, 520), (1032, 328), (1064, 1032)])
+def test_infinite_weights_at_the_end_of_the_contraction(gpu, dtype, H, I):
+    import yamoe_amd
+    print("ragged inf", dtype, H, I, flush=True)
+    d = _with_infinite_up_weights(H, I, dtype)
+    out = yamoe_amd.experts(*args(to_dev(d, gpu)), 300, 3, 2)
+    torch.cuda.synchronize()
+    want = O.experts_loop(*args(d), compute_dtype=torch.float32)
+    assert torch.isfinite(want).all()
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
+
+
+def test_infinite_gradient_in_an_experts_last_row_fp32(gpu):
+    import yamoe_amd
+    d = make_inputs(301, 96, 64, 3, 3, torch.float32, seed=3, w_std=0.05, bias_std=0.1)  # every expert: rows 0 .. 300
+    gy = torch.randn(301, 96, generator=torch.Generator().manual_seed(5))
+    gy[300, 7] = float("inf")
+    got = yamoe_amd.experts_backward(gy.to(gpu), *args(to_dev(d, gpu)), 301, 3, 3)[4].cpu()
+    assert not torch.isnan(got).any()
+    assert torch.isinf(got[:, :, 7]).all() and torch.isfinite(got[:, :, :7]).all() and torch.isfinite(got[:, :, 8:]).all()

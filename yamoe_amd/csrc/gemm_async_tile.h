@@ -35,8 +35,9 @@
 // (csrc/moe.cpp:164-180) meet in one lane, and the staging stores are 4 or 8 bytes wide.
 //
 // Contraction lengths that are not whole slab pairs (multiples of 64): the copies of the last pair re-read valid data
-// where the contraction has ended, and the wave that copied the activations overwrites what lies past the end with zeros
-// in LDS, between the wait for those copies and the barrier in front of their first use.  Only the last few steps of the
+// where the contraction has ended, and the wave that copied them overwrites what lies past the end with zeros in LDS, between
+// the wait for those copies and the barrier in front of their first use: of both operands, because an infinite weight that
+// is read again would make a NaN with the zero of the activations.  Only the last few steps of the
 // pipeline know about it, in instantiations of their own (RAGGED): the even lengths keep their registers (with
 // the clamps in one kernel for both, prefill at 4096 tokens ran 2 % slower).  A tensor-parallel rank's slice of a layer has
 // such lengths, 720 of 2880: the down product of one, 8012 rows on 32 experts, takes 70 us this way and took 124 us on the
@@ -156,10 +157,12 @@ template <int N> __device__ inline void wait_vmcnt() { asm volatile("s_waitcnt v
 // VM: which wait stands between its k-steps (see the pipeline comment in run_tile)
 enum { VM_NONE, VM_EVEN, VM_ODD, VM_LAST_B, VM_NK, VM_ALL };
 // LAST: where the copies of the two k-steps belong to the last slab pair (bit 0: A, bit 1: B of the first k-step, bit 2: B
-// of the second); ZERO: the last pair's rows have landed, its positions past the end of the contraction are cleared
-template <bool P1A_, bool P1B_, bool P2A_, bool P2B_, bool NEXT_, int VM_, bool BAR_ = true, int LAST_ = 0, bool ZERO_ = false>
+// of the second); ZERO: what is cleared past the end of the contraction after the wait, by which it has landed
+enum { ZERO_NONE, ZERO_PAIR, ZERO_A_AND_FIRST, ZERO_SECOND };  // the last pair; its A and its first B slab; its second B slab
+template <bool P1A_, bool P1B_, bool P2A_, bool P2B_, bool NEXT_, int VM_, bool BAR_ = true, int LAST_ = 0, int ZERO_ = ZERO_NONE>
 struct StepCfg {
-  static constexpr bool P1A = P1A_, P1B = P1B_, P2A = P2A_, P2B = P2B_, NEXT = NEXT_, BAR = BAR_, ZERO = ZERO_;
+  static constexpr bool P1A = P1A_, P1B = P1B_, P2A = P2A_, P2B = P2B_, NEXT = NEXT_, BAR = BAR_;
+  static constexpr int ZERO = ZERO_;
   static constexpr bool LAST_A = LAST_ & 1, LAST_B1 = (LAST_ >> 1) & 1, LAST_B2 = (LAST_ >> 2) & 1;
   static constexpr int VM = VM_;
 };
@@ -271,6 +274,33 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
 #pragma unroll
     for (int c = 0; c < S::kBPairCopies; ++c) copy_bp(pair, c, pair == n_pairs - 1);
   };
+  // the same for what this wave copied of slab `n_slabs - 2 + second` of B, and of the last B pair
+  auto zero_b = [&](int second) {
+    if constexpr (RAGGED) {
+      int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("" : "+v"(l));
+      const int slab = n_slabs - 2 + second, k0 = 8 * wave + l / (kBN / 8);
+      char *at = lds + kBRing + (slab & (kBStages - 1)) * kBStageBytes + 8 * wave * (2 * kBN) + l * 16;
+#pragma unroll
+      for (int i = 0; i < S::kBCopies; ++i)
+        if (slab * kBK + k0 + S::kBRows * i >= args.Kd) *(u32x4 *)(at + S::kBRows * i * (2 * kBN)) = (u32x4){0, 0, 0, 0};
+    }
+  };
+  auto zero_bp = [&]() {
+    if constexpr (RAGGED) {
+      int l = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+      asm volatile("" : "+v"(l));
+      char *at = lds + kBRing + ((n_pairs - 1) % kBPairStages) * kBPairBytes + kBN / 4 * wave * 128 + l * 16;
+#pragma unroll
+      for (int c = 0; c < S::kBPairCopies; ++c)
+        if (((l & 7) ^ ((4 * c + (l >> 4)) & 7)) * 16 >= last_bytes) *(u32x4 *)(at + 8 * c * 128) = (u32x4){0, 0, 0, 0};
+    }
+  };
+  auto zero_last = [&]() {
+    zero_a();
+    if constexpr (BNK) zero_bp();
+    else { zero_b(0); zero_b(1); }
+  };
 
   // ---- MFMA operand reads ----------------------------------------------------------------------------
   // A operand (block mi, slab parity par, k-step ks): row (mi*2+wm)*32 + lane%32, piece par*4 + ks*2 + lane/32
@@ -362,7 +392,7 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
     if (n_slabs >= 8) wait_vmcnt<3 * S::kBCopies + NAB>();  // B1, B2, B3 and A pair 1
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
-  if (RAGGED && n_pairs <= 2) zero_a();
+  if (RAGGED && n_pairs <= 2) zero_last();
   __syncthreads();
   YAMOE_STAMP(2);
   read_frags(0, 0, fa0, fb0);
@@ -402,7 +432,9 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
     else if constexpr (C::VM == VM_LAST_B) wait_vmcnt<kHalfB>();
     else if constexpr (C::VM == VM_NK) wait_vmcnt<S::kBPairCopies>();
     else if constexpr (C::VM == VM_ALL) wait_vmcnt<0>();
-    if constexpr (C::ZERO) zero_a();
+    if constexpr (C::ZERO == ZERO_PAIR) zero_last();
+    else if constexpr (C::ZERO == ZERO_A_AND_FIRST) { zero_a(); zero_b(0); }
+    else if constexpr (C::ZERO == ZERO_SECOND) zero_b(1);
     if constexpr (C::BAR) __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
     {
@@ -430,7 +462,7 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
     read_frags(s, 1, fa1, fb1);
     mma(fa0, fb0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (RAGGED && odd && s + 3 == n_slabs && n_pairs > 2) zero_a();
+    if (RAGGED && odd && s + 3 == n_slabs && n_pairs > 2) zero_last();
     __syncthreads();
     if (odd && s + 3 < n_slabs) issue_a((s + 1) / 2 + 1);
     if constexpr (!BNK) {
@@ -455,7 +487,7 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
     }
     // the last two pairs (s = n_slabs - 4)
     slab_step(s, StepCfg<true, false, false, false, true, VM_NONE, false, 1>());
-    slab_step(s + 1, StepCfg<false, false, false, false, true, VM_ALL, true, 0, true>());
+    slab_step(s + 1, StepCfg<false, false, false, false, true, VM_ALL, true, 0, ZERO_PAIR>());
     slab_step(s + 2, StepCfg<false, false, false, false, true, VM_NONE, false>());
     slab_step(s + 3, StepCfg<false, false, false, false, false, VM_NONE, false>());
   } else if (n_slabs >= 8) {
@@ -471,8 +503,8 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
     slab_step(s, StepCfg<true, true, false, true, true, VM_EVEN, true, 4>());
     slab_step(s + 1, StepCfg<false, true, true, true, true, VM_ODD, true, 1 | 2 | 4>());
     slab_step(s + 2, StepCfg<true, true, false, false, true, VM_EVEN, true, 1 | 2>());
-    slab_step(s + 3, StepCfg<false, false, false, false, true, VM_LAST_B, true, 0, true>());
-    slab_step(s + 4, StepCfg<false, false, false, false, true, VM_ALL>());
+    slab_step(s + 3, StepCfg<false, false, false, false, true, VM_LAST_B, true, 0, ZERO_A_AND_FIRST>());
+    slab_step(s + 4, StepCfg<false, false, false, false, true, VM_ALL, true, 0, ZERO_SECOND>());
     slab_step(s + 5, StepCfg<false, false, false, false, false, VM_NONE>());
   } else {
     for (int s = 0; s < n_slabs; s += 2) {

@@ -29,7 +29,8 @@
 //    interleaved (gate, up) columns of the clamped SwiGLU therefore meet in one lane, and outputs leave as 8-byte stores,
 //    256 contiguous bytes per half wave.
 //  * The contraction may end inside a slab: the last slab's copies re-read valid data past its end, and the waves
-//    overwrite what they copied of the left operand there with zeros before the barrier.
+//    overwrite what they copied of both operands there with zeros before the barrier (an infinity read twice would make a
+//    NaN with a zero).
 //
 // Requirements: leading dimensions and, for row products, the contraction length multiples of 4 elements.
 #include <type_traits>
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
       copy16_to_lds(bb, t.b_off[i] - b_adj, st + kAStage + (uint32_t)(B_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512));
     }
   };
-  // what this wave copied of the last slab's left operand past the end of the contraction
+  // clears what this wave copied of the last slab past the end of the contraction
   auto zero_tail = [&](const Tile &t, int slab, int stage) {
     const int left = t.k_len - slab * kBK;
     char *st = lds + (stage & (kStages - 1)) * kStage + lane * 16;
@@ -206,6 +207,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
     for (int i = 0; i < 4; ++i) {
       const bool past = A_ROWS ? piece * 4 >= left : 8 * wave + 2 * i + (lane >> 5) >= left;
       if (past) *(u32x4 *)(st + (A_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512)) = (u32x4){0, 0, 0, 0};
+      const bool b_past = B_ROWS ? piece * 4 >= left : 8 * wave + 2 * i + (lane >> 5) >= left;
+      if (b_past) *(u32x4 *)(st + kAStage + (B_ROWS ? (32 * i + 8 * wave) * 128 : (8 * wave + 2 * i) * 512)) = (u32x4){0, 0, 0, 0};
     }
   };
 
