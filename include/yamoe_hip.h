@@ -251,6 +251,7 @@ int yamoe_batch_mm(const void *x, const void *weights, void *output, int32_t E, 
  * torch-ext/yamoe/vendored/gpt_oss_mlp.py:128-142) in one kernel:
  *   logits = round(hidden . weight^T + bias)            [T,E]  (optional output)
  *   router_indices = top_k experts by logit, descending; equal logits: lower expert id first   [T,K] int64
+ *                    (a NaN is above every number, whatever its sign, as in torch.topk)
  *   router_scores  = softmax over the K picked logits (fp32, rounded once), scattered into a
  *                    zero [T,E] row; topk_weights (optional) holds the same K values as [T,K].
  * H must be a multiple of 16 (fp32: of 8), E <= 256, top_k <= min(E, 16).  bias may be NULL.  All three dtypes. */

@@ -72,6 +72,25 @@ def test_router_ties_pick_lower_expert(gpu):
     assert torch.all(topw.cpu().float() == 0.25)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E", [16, 40, 100, 200])
+def test_router_nan_logits_are_the_largest(gpu, dtype, E):
+    """As in torch.topk: NaN above everything, +inf among it, whatever the NaN's sign."""
+    from yamoe_amd import _cabi
+    T, H, K = 35, 64, 5
+    x, w, b = draw(T, H, E, dtype, E)
+    bits = b.view(torch.int32 if dtype == torch.float32 else torch.int16)
+    bits[3] = int(torch.tensor(float("inf"), dtype=dtype).view(bits.dtype)) | 64
+    bits[11] = bits[3] - 2 ** (31 if dtype == torch.float32 else 15)   # the same with the sign bit
+    b[7] = float("inf")
+    idx, scores, topw, logits = (t.cpu() for t in _cabi.router_topk(x.to(gpu), w.to(gpu), b.to(gpu), K))
+    assert torch.isnan(logits[:, [3, 11]]).all()
+    assert torch.equal(idx[:, :3], torch.tensor([3, 11, 7]).repeat(T, 1))
+    rest = logits.float().clone()
+    rest[:, [3, 7, 11]] = -float("inf")
+    assert torch.equal(idx[:, 3:], torch.sort(rest, dim=1, descending=True, stable=True).indices[:, :K - 3])
+
+
 def test_router_rejects(gpu):
     import yamoe_amd
     x, w, b = draw(8, 64, 4, torch.bfloat16, 0)

@@ -64,10 +64,11 @@ template <int NB> struct RouterRing {
   static_assert(kRouterTokens * kLd * 4 <= kBytes, "the logits tile fits the ring");
 };
 
-// a logit as an unsigned number in the same order (equal floats give equal numbers: -0 becomes +0 first); 0 is below all
+// a logit as an unsigned number in the same order (equal floats give equal numbers: -0 becomes +0 first); every NaN is the
+// largest, whatever its sign, as in torch.topk; 0 is below all
 __device__ inline uint32_t router_order(float v) {
   const uint32_t b = __builtin_bit_cast(uint32_t, v + 0.0f);
-  return (b & 0x80000000u) ? max(~b, 1u) : (b | 0x80000000u);  // (the lowest is a NaN's: it stays above the 0 of "taken")
+  return v != v ? 0xffffffffu : (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 __device__ inline float router_unorder(uint32_t o) {
   return __builtin_bit_cast(float, (o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
