@@ -91,6 +91,24 @@ def test_router_nan_logits_are_the_largest(gpu, dtype, E):
     assert torch.equal(idx[:, 3:], torch.sort(rest, dim=1, descending=True, stable=True).indices[:, :K - 3])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("first", ["inf", "nan", "-inf"])
+def test_router_scores_of_a_softmax_that_is_not_finite(gpu, dtype, first):
+    """A softmax whose largest logit is not finite is NaN at every pick, also where the exponential is zero; experts that
+    were not picked have a score of zero."""
+    from yamoe_amd import _cabi
+    T, H, E, K = 35, 64, 40, 4
+    x, w, b = draw(T, H, E, dtype, E)
+    if first == "-inf":
+        b[:] = -float("inf")
+    else:
+        b[9] = float(first)
+    idx, scores, topw, logits = (t.cpu() for t in _cabi.router_topk(x.to(gpu), w.to(gpu), b.to(gpu), K))
+    assert torch.isnan(topw).all()
+    picked = torch.zeros(T, E, dtype=torch.bool).scatter_(1, idx, True)
+    assert torch.isnan(scores[picked]).all() and torch.all(scores[~picked] == 0)
+
+
 def test_router_rejects(gpu):
     import yamoe_amd
     x, w, b = draw(8, 64, 4, torch.bfloat16, 0)

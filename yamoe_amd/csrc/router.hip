@@ -221,7 +221,8 @@ __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(co
 #pragma unroll
   for (int j = 0; j < M; ++j) {
     const int e = sub * M + j;
-    if (e < E) scores[t * E + e] = ElemTraits<T>::from_f32(prob[j] == 0.0f ? 0.0f : prob[j] / sum);
+    // (a key of 0 is a pick; the others divide nothing, as the sum may not be finite)
+    if (e < E) scores[t * E + e] = ElemTraits<T>::from_f32(key[j] != 0u ? 0.0f : prob[j] / sum);
   }
   if (topk_weights != nullptr) {
 #pragma unroll
