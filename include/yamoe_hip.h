@@ -5,7 +5,9 @@
  * (passed as void* so that this header needs no HIP include).  Nothing here
  * allocates, frees or synchronises: callers bring the output buffers and one
  * workspace whose size the matching *_workspace_bytes() call returns.  All work
- * is enqueued on `stream` and the call returns at once.
+ * is enqueued on `stream` and the call returns at once.  Tensors begin on a
+ * 4-byte boundary at least, also 16-bit ones (the matrix kernels copy them into
+ * LDS in dwords; the torch operators move those that do not).
  *
  * Return value: 0 on success, a negative YAMOE_E_* code on a rejected argument,
  * a positive hipError_t if a launch failed.  yamoe_last_error() gives the text

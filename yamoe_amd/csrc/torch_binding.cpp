@@ -39,6 +39,13 @@ void check_rc(int rc, const char *what) {
   TORCH_CHECK(rc == 0, what, " failed (", rc, "): ", yamoe_last_error());
 }
 
+// A tensor that the matrix kernels copy into LDS: contiguous, and not beginning in the middle of a dword (16-bit views at
+// an odd offset do), which their asynchronous copies are not specified for and plain loads are.
+at::Tensor operand(const at::Tensor &t) {
+  at::Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(c.data_ptr()) % 4 != 0 ? c.clone() : c;
+}
+
 struct Checked {
   yamoe_problem p;
   at::Tensor hidden, idx, rw, wgu, bgu, wd, bd;
@@ -47,7 +54,8 @@ struct Checked {
 Checked check_inputs(const at::Tensor &hidden_states, const at::Tensor &router_indices,
                      const at::Tensor &routing_weights, const at::Tensor &gate_up_proj,
                      const at::Tensor &gate_up_proj_bias, const at::Tensor &down_proj,
-                     const at::Tensor &down_proj_bias, int64_t expert_capacity, int64_t num_experts, int64_t top_k) {
+                     const at::Tensor &down_proj_bias, int64_t expert_capacity, int64_t num_experts, int64_t top_k,
+                     bool backward) {
   TORCH_CHECK(hidden_states.is_cuda(), "hidden_states must be on the GPU");
   TORCH_CHECK(router_indices.is_cuda(), "router_indices must be on the GPU");
   TORCH_CHECK(routing_weights.is_cuda(), "routing_weights must be on the GPU");
@@ -90,13 +98,16 @@ Checked check_inputs(const at::Tensor &hidden_states, const at::Tensor &router_i
               "all tensors must be on the same device");
   TORCH_CHECK(T * K <= (int64_t)1 << 30, "T*K too large");
 
+  // (a forward with at most 4 assignments per expert runs on the streaming kernels alone, which take any offset: its
+  // weights are not worth a copy)
+  const bool copies = backward || T * K > 4 * E;
   Checked c;
-  c.hidden = hidden_states.contiguous();
+  c.hidden = operand(hidden_states);
   c.idx = router_indices.contiguous();
   c.rw = routing_weights.contiguous();
-  c.wgu = gate_up_proj.contiguous();
+  c.wgu = copies ? operand(gate_up_proj) : gate_up_proj.contiguous();
   c.bgu = gate_up_proj_bias.contiguous();
-  c.wd = down_proj.contiguous();
+  c.wd = copies ? operand(down_proj) : down_proj.contiguous();
   c.bd = down_proj_bias.contiguous();
   c.p.T = (int32_t)T;
   c.p.K = (int32_t)K;
@@ -114,7 +125,7 @@ at::Tensor experts(at::Tensor hidden_states, at::Tensor router_indices, at::Tens
                    at::Tensor gate_up_proj, at::Tensor gate_up_proj_bias, at::Tensor down_proj,
                    at::Tensor down_proj_bias, int64_t expert_capacity, int64_t num_experts, int64_t top_k) {
   Checked c = check_inputs(hidden_states, router_indices, routing_weights, gate_up_proj, gate_up_proj_bias, down_proj,
-                           down_proj_bias, expert_capacity, num_experts, top_k);
+                           down_proj_bias, expert_capacity, num_experts, top_k, false);
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.hidden.device());
   at::Tensor out = at::empty_like(c.hidden);
   if (c.p.T == 0) return out;
@@ -136,13 +147,13 @@ std::vector<at::Tensor> experts_backward(const at::Tensor &grad_out, const at::T
                                          int64_t expert_capacity, int64_t num_experts, int64_t top_k) {
   TORCH_CHECK(grad_out.is_cuda(), "grad_out must be on the GPU");
   Checked c = check_inputs(hidden_states, router_indices, routing_weights, gate_up_proj, gate_up_proj_bias, down_proj,
-                           down_proj_bias, expert_capacity, num_experts, top_k);
+                           down_proj_bias, expert_capacity, num_experts, top_k, true);
   const int64_t T = c.p.T, H = c.p.H, K = c.p.K;
   TORCH_CHECK(grad_out.scalar_type() == c.hidden.scalar_type(), "grad_out must share hidden_states' dtype");
   TORCH_CHECK(grad_out.numel() == T * H || grad_out.numel() == T * K * H, "grad_out numel must be T*H or T*K*H");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.hidden.device());
   // a [T,K,H] gradient is first summed over the slot axis (csrc/experts_backward.cu:224-228)
-  at::Tensor gy = grad_out.numel() == T * H ? grad_out.contiguous().view({T, H})
+  at::Tensor gy = grad_out.numel() == T * H ? operand(grad_out).view({T, H})
                                             : grad_out.contiguous().view({T, K, H}).sum(1).contiguous();
   at::Tensor d_hidden = at::empty_like(c.hidden);
   at::Tensor d_routing = at::empty_like(c.rw);
@@ -170,7 +181,7 @@ std::tuple<at::Tensor, at::Tensor> experts_keep(at::Tensor hidden_states, at::Te
                                                 at::Tensor down_proj_bias, int64_t expert_capacity, int64_t num_experts,
                                                 int64_t top_k) {
   Checked c = check_inputs(hidden_states, router_indices, routing_weights, gate_up_proj, gate_up_proj_bias, down_proj,
-                           down_proj_bias, expert_capacity, num_experts, top_k);
+                           down_proj_bias, expert_capacity, num_experts, top_k, false);
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.hidden.device());
   at::Tensor out = at::empty_like(c.hidden);
   const size_t kept_bytes = yamoe_experts_kept_bytes(&c.p);
@@ -195,7 +206,7 @@ std::vector<at::Tensor> experts_backward_kept(const at::Tensor &grad_out, const 
                                               int64_t top_k) {
   TORCH_CHECK(grad_out.is_cuda(), "grad_out must be on the GPU");
   Checked c = check_inputs(hidden_states, router_indices, routing_weights, gate_up_proj, gate_up_proj_bias, down_proj,
-                           down_proj_bias, expert_capacity, num_experts, top_k);
+                           down_proj_bias, expert_capacity, num_experts, top_k, true);
   const int64_t T = c.p.T, H = c.p.H;
   TORCH_CHECK(grad_out.scalar_type() == c.hidden.scalar_type(), "grad_out must share hidden_states' dtype");
   TORCH_CHECK(grad_out.numel() == T * H, "grad_out must be [T, H]");
@@ -203,7 +214,7 @@ std::vector<at::Tensor> experts_backward_kept(const at::Tensor &grad_out, const 
                   (size_t)kept.numel() >= yamoe_experts_kept_bytes(&c.p),
               "kept must be the byte tensor that experts_keep returned for the same problem");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(c.hidden.device());
-  at::Tensor gy = grad_out.contiguous().view({T, H});
+  at::Tensor gy = operand(grad_out).view({T, H});
   at::Tensor d_hidden = at::empty_like(c.hidden);
   at::Tensor d_routing = at::empty_like(c.rw);
   at::Tensor d_wgu = at::empty_like(c.wgu);
@@ -326,8 +337,8 @@ at::Tensor batch_mm_op(at::Tensor x, at::Tensor weights, at::Tensor batch_sizes,
   TORCH_CHECK(x.size(2) == weights.size(1));
   const int64_t E = x.size(0), C = x.size(1), Kd = x.size(2), Nd = weights.size(2);
   TORCH_CHECK(weights.scalar_type() == x.scalar_type() && output.scalar_type() == x.scalar_type(), "dtypes must match");
-  x = x.contiguous();
-  weights = weights.contiguous();
+  x = operand(x);
+  weights = operand(weights);
   if (output.numel() != E * C * Nd) output.resize_({E, C, Nd});
   TORCH_CHECK(output.is_contiguous(), "output must be contiguous");
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
@@ -347,7 +358,7 @@ std::tuple<at::Tensor, at::Tensor> router_topk_op(const at::Tensor &hidden, cons
               "router_topk: hidden [T, H] and weight [E, H] expected");
   TORCH_CHECK(weight.scalar_type() == hidden.scalar_type(), "router_topk: weight dtype must match hidden");
   const int64_t T = hidden.size(0), H = hidden.size(1), E = weight.size(0);
-  at::Tensor x = hidden.contiguous(), w = weight.contiguous(), b;
+  at::Tensor x = operand(hidden), w = operand(weight), b;
   const void *bp = nullptr;
   if (bias.has_value() && bias->defined()) {
     TORCH_CHECK(bias->is_cuda() && bias->numel() == E && bias->scalar_type() == hidden.scalar_type(),
@@ -380,7 +391,7 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> router_topk_backward_op(const at:
   TORCH_CHECK(weight.scalar_type() == hidden.scalar_type() && scores.scalar_type() == hidden.scalar_type() &&
               d_scores.scalar_type() == hidden.scalar_type(), "router_topk_backward: one dtype for all float tensors");
   const int code = dtype_code(hidden, "hidden");
-  at::Tensor x = hidden.contiguous(), w = weight.contiguous(), g = d_scores.contiguous(), sc = scores.contiguous(),
+  at::Tensor x = hidden.contiguous(), w = operand(weight), g = d_scores.contiguous(), sc = scores.contiguous(),
              ix = indices.contiguous();
   const c10::hip::HIPGuardMasqueradingAsCUDA guard(hidden.device());
   at::Tensor d_hidden = at::empty_like(x), d_weight = at::empty_like(w), d_bias = at::empty({E}, hidden.options());
