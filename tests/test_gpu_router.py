@@ -59,6 +59,21 @@ def test_router_topk_lane_groups(gpu, dtype, T, H, E, K):
     test_router_topk(gpu, dtype, T, H, E, K)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("chunks", [0.5, 1, 2, 3.5, 7, 8, 8.5, 9, 16, 17, 24.5])
+def test_router_stages_of_several_chunks(gpu, dtype, chunks):
+    """Contractions of whole and partial chunks (128 bytes of a row), fewer and more than the 2 and 8 of a ring's stage; up
+    to 256 workgroups and more, which run on rings of different depth: the picks of the oracle, and the same bits in both."""
+    from yamoe_amd import _cabi
+    H, T, K = int(chunks * (128 // (2 if dtype == torch.bfloat16 else 4))), 8192 + 33, 3
+    for E in (6, 40):
+        test_router_topk(gpu, dtype, 70, H, E, K)
+        x, w, b = (t.to(gpu) for t in draw(T, H, E, dtype, H + E))
+        parts = [_cabi.router_topk(x[i:i + 4128], w, b, K) for i in (0, 4128)]
+        for whole, halves in zip(_cabi.router_topk(x, w, b, K), zip(*parts)):
+            assert torch.equal(whole, torch.cat(halves))
+
+
 def test_router_ties_pick_lower_expert(gpu):
     from yamoe_amd import _cabi
     # identical weight rows give identical logits: the pick order must be by expert id

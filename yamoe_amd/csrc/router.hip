@@ -21,6 +21,7 @@ constexpr int kRouterTokens = 32;
 constexpr int kRouterThreads = 256;
 constexpr int kRouterMaxE = 256;
 constexpr int kRouterMaxK = 16;
+constexpr int kRouterCus = 256;
 
 template <typename T> struct RouterMma;
 template <> struct RouterMma<bf16_t> {
@@ -47,21 +48,29 @@ template <> struct RouterMma<float> {
 //
 // What bounds it is getting the operands in: a workgroup reads its 32 token rows and all E weight rows, 32 * (1 + NB) * 128
 // bytes per chunk against a handful of MFMAs.  The chunks come in by asynchronous copies of whole 128-byte pieces, eight
-// rows per instruction, into a ring of S stages (S - 1 chunks on their way while one is used).  Fragments fetched
-// straight from global memory touch 32 cache lines per instruction for 32 bytes of each, which the L1's tag rate holds at
-// 30 us for one token and 58 us for 8192 on a [128, 2880] router (17.7 and 20.1 us this way).
+// rows per instruction, into a ring of S stages of G chunks each (S - 1 stages on their way while one is used).  Fragments
+// fetched straight from global memory touch 32 cache lines per instruction for 32 bytes of each, which the L1's tag rate
+// holds at 30 us for one token and 58 us for 8192 on a [128, 2880] router (17.7 and 20.1 us this way).
+//
+// With few experts that tag rate is no limit (lanes of the same row share their lines), and what counts is the wave's own
+// chain from stage to stage: wait, barrier, copies, LDS read, MFMA, about 500 clocks however little a stage holds.  Hence
+// G: up to 64 experts a stage is several chunks.  [E, 2880] bf16, top-2, us by fragments from global memory / stages of one
+// chunk / now: 1 token, 8 experts 9.8 / 13.9 / 8.3, 32 experts 13.3 / 13.8 / 8.6; fp32, 2048 tokens, 8 experts 26.6 / 33.7 / 21.9.
+// The form of up to 32 experts with most in flight fills a CU's LDS; where there are more workgroups than CUs, small rings of which
+// five share a CU are the better ones (32768 tokens, 8 experts, 1024 wide bf16: 25.3 / 14.2; 2048 tokens: 6.0 / 7.2).  Up
+// to 64 experts two share a CU (40 experts, 32768 tokens, 1024 wide fp32: 58.8 by fragments, 64.6 with one per CU, 52.8 now).
 //
 // The pick is made by the lanes of the token together: L = 8 * NB / WB lanes hold 32 * NB / L consecutive logits each in
 // registers, and every round is a maximum over the lane's own values followed by log2(L) exchanges.  (One thread per
 // token walking its row in LDS, the picks in scratch memory, took 90 of the kernel's 103 us at 1536 tokens of 2048 values,
 // 64 experts, top-8, which takes 13.3 us now.)
-template <int NB> struct RouterRing {
+template <int NB, int G_, int S_> struct RouterRing {
+  static constexpr int G = G_, S = S_;
   static constexpr int kRows = kRouterTokens + 32 * NB;
-  static constexpr int kStage = kRows * 128;
-  static constexpr int S = NB <= 2 ? 8 : NB <= 4 ? 6 : 4;  // 64, 96, 120, 144 KB
+  static constexpr int kChunk = kRows * 128;
+  static constexpr int kStage = G * kChunk, kBytes = S * kStage;
   static constexpr int kLd = 32 * NB + 1;                  // padded row of the logits tile, which takes the ring's place
-  static constexpr int kBytes = S * kStage;
-  static_assert(kRouterTokens * kLd * 4 <= kBytes, "the logits tile fits the ring");
+  static_assert(kRouterTokens * kLd * 4 <= kBytes && kBytes <= 160 * 1024, "the logits tile fits the ring, the ring a CU");
 };
 
 // a logit as an unsigned number in the same order (equal floats give equal numbers: -0 becomes +0 first); every NaN is the
@@ -74,14 +83,13 @@ __device__ inline float router_unorder(uint32_t o) {
   return __builtin_bit_cast(float, (o & 0x80000000u) ? (o & 0x7fffffffu) : ~o);
 }
 
-template <typename T, int NB, int WB>
+template <typename T, int NB, int WB, class R>
 __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(const T *__restrict__ x, const T *__restrict__ w,
                                                                      const T *__restrict__ bias, int Tn, int H, int E, int K,
                                                                      long long *__restrict__ indices, T *__restrict__ scores,
                                                                      T *__restrict__ topk_weights, T *__restrict__ logits_out) {
   constexpr int kThreads = kRouterThreads * NB / WB, kWaves = kThreads / kWave;
-  typedef RouterRing<NB> R;
-  constexpr int kLd = R::kLd, S = R::S;
+  constexpr int kLd = R::kLd, S = R::S, G = R::G;
   extern __shared__ __attribute__((aligned(16))) char ring[];
   float *tile = (float *)ring;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -96,10 +104,10 @@ __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(co
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[nb][v] = 0.0f;
 
-  // Copies: copy q of a chunk brings rows 8 q + lane / 8 of the stage (32 token rows, then the weight rows), 16 bytes per
+  // Copies: copy q of a chunk brings rows 8 q + lane / 8 of it (32 token rows, then the weight rows), 16 bytes per
   // lane; position lane % 8 of row r holds piece pos ^ ((r >> 1) & 7), so that 32 lanes reading one piece of 32 rows touch
-  // every bank.  Wave w issues copies w, w + kWaves, ...  Rows past the end re-read the last valid one, pieces past the
-  // end of a row its first; their products are never used.
+  // every bank.  Wave w issues copies w, w + kWaves, ...  Rows past the end re-read the last valid one, pieces and
+  // chunks past the end of a row its first; their products are never used.
   constexpr int kCopies = R::kRows / 8, kPerWave = (kCopies + kWaves - 1) / kWaves;
   constexpr int kFewer = kPerWave * kWaves - kCopies;  // the last kFewer waves issue one copy less
   const bool fewer = wave >= kWaves - kFewer;
@@ -112,39 +120,49 @@ __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(co
                                  : (const char *)w + (long long)min(row - kRouterTokens, E - 1) * row_bytes;
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)ring);
-  auto issue = [&](int chunk, int stage) {
+  auto issue = [&](int group, int stage) {
 #pragma unroll
-    for (int i = 0; i < kPerWave; ++i) {
-      if (i == kPerWave - 1 && fewer) break;
-      const int row = 8 * (wave + i * kWaves) + (lane >> 3);
-      int at = chunk * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
-      if (at >= row_bytes) at = 0;
-      copy16_to_lds(src[i] + at, lds0 + (uint32_t)(stage * R::kStage + 8 * (wave + i * kWaves) * 128));
-    }
+    for (int j = 0; j < G; ++j)
+#pragma unroll
+      for (int i = 0; i < kPerWave; ++i) {
+        if (i == kPerWave - 1 && fewer) break;
+        const int row = 8 * (wave + i * kWaves) + (lane >> 3);
+        int at = (group * G + j) * 128 + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+        if (at >= row_bytes) at = 0;
+        copy16_to_lds(src[i] + at, lds0 + (uint32_t)(stage * R::kStage + j * R::kChunk + 8 * (wave + i * kWaves) * 128));
+      }
   };
-  // every copy but those of the youngest `chunks` has landed
-  auto wait_but = [&](auto chunks) {
-    constexpr int C = decltype(chunks)::value;
+  // every copy but those of the youngest `groups` has landed
+  auto wait_but = [&](auto groups) {
+    constexpr int C = decltype(groups)::value * G;
     if (kFewer > 0 && fewer) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C * (kPerWave - 1)) : "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C * kPerWave) : "memory");
   };
-  const int n_steps = row_bytes / 32, n_chunks = (n_steps + 3) / 4;
+  const int n_steps = row_bytes / 32, n_groups = (n_steps + 4 * G - 1) / (4 * G);
   const int rd = rl * 128 + (((2 * kq + g) ^ ((rl >> 1) & 7)) << 4);
-  auto use = [&](int chunk, int stage) {
-    if (4 * chunk + kq < n_steps) {
-      const char *st = ring + stage * R::kStage + rd;
-      const u32x4 fa = *(const u32x4 *)st;
+  auto use = [&](int group, int stage) {
+    const char *st = ring + stage * R::kStage + rd;
+    u32x4 fa[G], fb[G][WB];
 #pragma unroll
-      for (int nb = 0; nb < WB; ++nb) RouterMma<T>::run(fa, *(const u32x4 *)(st + (1 + nb0 + nb) * 4096), acc[nb]);
+    for (int j = 0; j < G; ++j) {
+      fa[j] = *(const u32x4 *)(st + j * R::kChunk);
+#pragma unroll
+      for (int nb = 0; nb < WB; ++nb) fb[j][nb] = *(const u32x4 *)(st + j * R::kChunk + (1 + nb0 + nb) * 4096);
     }
+#pragma unroll
+    for (int j = 0; j < G; ++j)
+      if (4 * (group * G + j) + kq < n_steps) {
+#pragma unroll
+        for (int nb = 0; nb < WB; ++nb) RouterMma<T>::run(fa[j], fb[j][nb], acc[nb]);
+      }
   };
 #pragma unroll
   for (int c = 0; c < S - 1; ++c)
-    if (c < n_chunks) issue(c, c);
+    if (c < n_groups) issue(c, c);
   int c = 0, stage = 0;
-  for (; c + S - 1 < n_chunks; ++c) {
+  for (; c + S - 1 < n_groups; ++c) {
     wait_but(std::integral_constant<int, S - 2>());
-    __syncthreads();  // chunk c is there for every wave, and nobody reads the stage of chunk c - 1 any more
+    __syncthreads();  // group c is there for every wave, and nobody reads the stage of group c - 1 any more
     const int free_stage = stage == 0 ? S - 1 : stage - 1;
     issue(c + S - 1, free_stage);
     use(c, stage);
@@ -152,7 +170,7 @@ __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(co
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  for (; c < n_chunks; ++c) {
+  for (; c < n_groups; ++c) {
     use(c, stage);
     stage = stage == S - 1 ? 0 : stage + 1;
   }
@@ -231,13 +249,14 @@ __global__ __launch_bounds__(kRouterThreads *NB / WB) void router_topk_kernel(co
   }
 }
 
-template <typename T, int NB, int WB>
+template <typename T, int NB, int WB, int G, int S>
 static int launch_router(const void *x, const void *w, const void *bias, int Tn, int H, int E, int K, long long *indices,
                          void *scores, void *topk_weights, void *logits, hipStream_t stream) {
-  auto kernel = router_topk_kernel<T, NB, WB>;
+  typedef RouterRing<NB, G, S> R;
+  auto kernel = router_topk_kernel<T, NB, WB, R>;
   static DeviceFlags attr_done;  // one per kernel instantiation
-  if (int rc = ensure_dynamic_lds((const void *)kernel, RouterRing<NB>::kBytes, attr_done, "router_topk_kernel")) return rc;
-  hipLaunchKernelGGL(kernel, dim3(ceil_div(Tn, kRouterTokens)), dim3(kRouterThreads * NB / WB), RouterRing<NB>::kBytes, stream,
+  if (int rc = ensure_dynamic_lds((const void *)kernel, R::kBytes, attr_done, "router_topk_kernel")) return rc;
+  hipLaunchKernelGGL(kernel, dim3(ceil_div(Tn, kRouterTokens)), dim3(kRouterThreads * NB / WB), R::kBytes, stream,
                      (const T *)x, (const T *)w, (const T *)bias, Tn, H, E, K, indices, (T *)scores, (T *)topk_weights,
                      (T *)logits);
   return check_launch("router_topk_kernel");
@@ -246,11 +265,14 @@ static int launch_router(const void *x, const void *w, const void *bias, int Tn,
 template <typename T>
 static int router_dispatch(const void *x, const void *w, const void *bias, int Tn, int H, int E, int K, long long *indices,
                            void *scores, void *topk_weights, void *logits, hipStream_t stream) {
-  int nb = ceil_div(E, 32);
-  if (nb <= 1) return launch_router<T, 1, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  if (nb <= 2) return launch_router<T, 2, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  if (nb <= 4) return launch_router<T, 4, 1>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
-  return launch_router<T, 8, 2>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  const int nb = ceil_div(E, 32);
+  if (nb <= 1) {  // 128 KB of LDS while a CU has one workgroup at most, 32 KB where several should share it
+    if (Tn <= kRouterTokens * kRouterCus) return launch_router<T, 1, 1, 8, 2>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+    return launch_router<T, 1, 1, 2, 2>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);
+  }
+  if (nb <= 2) return launch_router<T, 2, 1, 2, 3>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);  // 72 KB
+  if (nb <= 4) return launch_router<T, 4, 1, 1, 6>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);  // 120 KB
+  return launch_router<T, 8, 2, 1, 4>(x, w, bias, Tn, H, E, K, indices, scores, topk_weights, logits, stream);  // 144 KB
 }
 
 // ---- gradient of the step, first part: from the gradient of the dense scores to the gradient of the logits --------
