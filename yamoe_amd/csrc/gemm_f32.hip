@@ -345,20 +345,23 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
     const int row0 = t.row0, rows_valid = t.rows_valid, expert = t.expert;
     const bool whole = rows_valid == kBM && cols_valid == kBN;
     const int col = t.n0 + (B_ROWS ? wn * 32 + rl : wn * 64 + 2 * rl);  // (GLU: even, the gate column of pair col / 2)
-    L += kWorkgroups;
-    if (L < items) {
-      set_tile(L, t);
-      if (t.k_len > 0) issue(t, 0, stage);
+    float b0 = 0.0f, b1 = 0.0f;
+    if (MODE == ROWS_KN && n_a > 0 && args.bias != nullptr && col < args.Nd) {
+      const float *bp = args.bias + (long long)expert * args.Nd + col;
+      b0 = bp[0];
+      b1 = bp[1];
     }
+    L += kWorkgroups;
+    if (L < items) set_tile(L, t);
+    // The bias is waited for here, with the look-ups and ahead of the next slab's request.  Left to its uses, the compiler's
+    // wait for all vector memory stands in front of every store of a partial tile, one store at a time, and in the
+    // contraction loop, whose registers the load may still be on its way to for all the compiler knows: there it waits for
+    // the next slab right after requesting it.  (16 experts, 3000 x 2 rows, 512 wide, forward: 137 us that way, 130 now.)
+    asm volatile("" : "+v"(b0), "+v"(b1));
+    if (L < items && t.k_len > 0) issue(t, 0, stage);
 
     // epilogue: straight from the accumulators; a half wave covers 256 (128 for act and ROWS_NK) contiguous bytes of a row
     if (n_a > 0) {
-      float b0 = 0.0f, b1 = 0.0f;
-      if (MODE == ROWS_KN && args.bias != nullptr && col < args.Nd) {
-        const float *bp = args.bias + (long long)expert * args.Nd + col;
-        b0 = bp[0];
-        b1 = bp[1];
-      }
       float *C = args.C + (MODE == WGRAD ? (long long)expert * args.Md * args.Nd : 0ll);
       auto store = [&](int a, int v, long long orow) {
         if constexpr (MODE == ROWS_NK) {
