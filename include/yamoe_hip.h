@@ -238,7 +238,7 @@ int yamoe_index_select(const void *input, const int32_t *idx, void *out, int64_t
                        void *stream);
 
 /* counts[e] = rows, offsets[e] = e*rows (offsets has E+1 entries): the regular [E,rows,*] layout
- * described as ragged groups, used by yamoe_batch_mm. */
+ * described as ragged groups, for callers of yamoe_build_schedule (yamoe_batch_mm makes its own). */
 int yamoe_regular_groups(int32_t *counts, int32_t *offsets, int32_t E, int32_t rows, void *stream);
 
 /* batch_mm (csrc/batch_mm.cu:7-31): output[e] = x[e] . weights[e] for x [E,C,Kd], weights

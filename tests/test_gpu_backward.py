@@ -146,7 +146,7 @@ CLAMPED = [
     # dtype, T, H, I, E, K, weight std: pre-activations of std 3 to 8, a good part of them beyond the clamp at 7
     (torch.bfloat16, 700, 256, 128, 4, 2, 0.5),    # asynchronous-copy kernels
     (torch.float16, 700, 256, 128, 4, 2, 0.5),
-    (torch.bfloat16, 64, 200, 72, 4, 2, 0.4),      # register-staged kernels (contraction not a multiple of 64)
+    (torch.bfloat16, 64, 200, 72, 4, 2, 0.4),      # contraction not a multiple of 64
     (torch.bfloat16, 600, 2880, 512, 2, 1, 0.05),  # the GPT-OSS width, where sqrt(2880) * 0.05 does the same
 ]
 

@@ -97,3 +97,13 @@ def test_stages_through_ctypes_compose_to_the_forward(gpu):
     want_y = torch.stack([want_act[p] @ d["down_proj"][ex[p]].float() + d["down_proj_bias"][ex[p]].float()
                           for p in range(T * K)])
     assert O.rel_l2(y.cpu().float(), want_y) < 1e-2
+
+
+@pytest.mark.parametrize("E,rows", [(1, 0), (1, 5), (255, 7), (256, 3), (300, 1)])
+def test_regular_groups(gpu, E, rows):
+    from yamoe_amd import _cabi
+    counts = torch.full((E,), -1, dtype=torch.int32, device=gpu)
+    offsets = torch.full((E + 1,), -1, dtype=torch.int32, device=gpu)
+    _cabi._check(_cabi.lib().yamoe_regular_groups(_cabi._p(counts), _cabi._p(offsets), E, rows, _cabi._stream()), "yamoe_regular_groups")
+    assert torch.equal(counts.cpu(), torch.full((E,), rows, dtype=torch.int32))
+    assert torch.equal(offsets.cpu(), torch.arange(E + 1, dtype=torch.int32) * rows)

@@ -20,7 +20,7 @@ SHAPES = [
     # T, H, I, E, K, capacity (0: tokens), zipf, every expert on the tile kernels in the forward
     (700, 128, 64, 3, 2, 0, 0.0, True),
     (1024, 256, 192, 4, 2, 0, 0.0, True),
-    (513, 320, 136, 5, 3, 0, 0.0, True),       # register-staged kernels
+    (513, 320, 136, 5, 3, 0, 0.0, True),       # contraction not a multiple of 64
     (2000, 64, 64, 64, 2, 0, 0.8, False),      # streamed experts next to tiled ones
     (600, 128, 64, 4, 2, 37, 0.5, True),       # capacity drops assignments
     (40, 64, 64, 16, 1, 0, 0.0, False),        # every expert streams

@@ -61,3 +61,22 @@ def test_infinite_gradient_in_an_experts_last_row_fp32(gpu):
     got = yamoe_amd.experts_backward(gy.to(gpu), *args(to_dev(d, gpu)), 301, 3, 3)[4].cpu()
     assert not torch.isnan(got).any()
     assert torch.isinf(got[:, :, 7]).all() and torch.isfinite(got[:, :, :7]).all() and torch.isfinite(got[:, :, 8:]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,E,I", [(300, 3, 40), (960, 48, 776)])
+@pytest.mark.parametrize("H", [72, 136, 200, 584])
+def test_infinite_weight_where_the_last_slab_of_an_input_gradient_begins(gpu, dtype, H, T, E, I):
+    """The down projection's input gradient contracts over H with its weights stored [n][k].  An infinite weight in what the
+    last slab's copies read once more past the end makes the row's gradient and its routing gradient infinite, and not NaN.
+    (Few and many experts: both tile sizes of the 16-bit kernels.)"""
+    import yamoe_amd
+    print("ragged dgrad inf", dtype, T, H, I, E, flush=True)
+    d = make_inputs(T, H, I, E, 2, dtype, seed=H, w_std=0.05, bias_std=0.1)
+    slab = 32 if dtype == torch.float32 else 64
+    d["down_proj"][:, 3, (H - 1) // slab * slab] = float("inf")
+    gy = torch.randn(T, H, generator=torch.Generator().manual_seed(5)).to(dtype)
+    gy[gy == 0] = 1.0
+    d_routing = yamoe_amd.experts_backward(gy.to(gpu), *args(to_dev(d, gpu)), T, E, 2)[1].cpu()
+    picked = torch.zeros(T, E, dtype=torch.bool).scatter_(1, d["router_indices"], True)
+    assert torch.isinf(d_routing[picked]).all() and torch.all(d_routing[~picked] == 0)

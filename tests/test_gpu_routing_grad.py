@@ -76,7 +76,7 @@ CASES = [
     (torch.bfloat16, 1, 128, 64, 4, 4, 3, 0.0, False),    # one token on every expert
     (torch.float16, 1, 64, 64, 2, 1, 5, 0.0, False),
     (torch.bfloat16, 2, 320, 576, 3, 2, 11, 0.0, False),  # I = 576: three column tiles, the last of 64 columns
-    (torch.bfloat16, 7, 72, 40, 5, 2, 13, 0.0, False),    # H = 72: the register-staged kernel (contraction not a multiple of 64)
+    (torch.bfloat16, 7, 72, 40, 5, 2, 13, 0.0, False),    # H = 72: contraction not a multiple of 64
     (torch.float16, 300, 128, 96, 8, 2, 29, 1.5, True),
     (torch.bfloat16, 700, 192, 320, 3, 2, 17, 0.0, False),  # more than 256 rows per expert: several row tiles
     (torch.float32, 5, 64, 96, 8, 2, 19, 0.0, False),

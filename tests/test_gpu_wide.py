@@ -25,7 +25,7 @@ def permute_always():
 SHAPES = [
     # T, H, I, E, K, capacity (0: tokens), zipf
     (700, 128, 64, 3, 2, 0, 0.0),       # several row tiles per expert
-    (513, 320, 136, 5, 3, 0, 0.0),      # contraction not a multiple of 64: the register-staged kernels
+    (513, 320, 136, 5, 3, 0, 0.0),      # contraction not a multiple of 64
     (2000, 64, 64, 64, 2, 0, 0.8),      # streamed experts next to tiled ones
     (600, 128, 64, 4, 2, 37, 0.5),      # capacity drops assignments
     (40, 64, 64, 16, 1, 0, 0.0),        # every expert streams

@@ -75,6 +75,7 @@ def lib():
         L.yamoe_router_backward_workspace_bytes.restype = sz
         L.yamoe_router_backward_workspace_bytes.argtypes = [i32, i32, i32]
         L.yamoe_router_backward.argtypes = [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp, vp, vp, vp, sz, vp]
+        L.yamoe_regular_groups.argtypes = [vp, vp, i32, i32, vp]
         L.yamoe_probe_mfma_rate.argtypes = [i32, i32, i32, vp, ctypes.POINTER(ctypes.c_double), vp]
         _lib = L
     return _lib

@@ -381,7 +381,7 @@ __global__ void index_select_kernel(const T *in, const int *idx, T *out, long lo
   if (i < n) out[i] = in[idx[i]];
 }
 
-// counts[e] = rows, offsets[e] = e * rows: the regular [E, C, *] layout as a ragged one (for batch_mm)
+// counts[e] = rows, offsets[e] = e * rows: the regular [E, C, *] layout as a ragged one (for callers of the C ABI)
 __global__ void regular_groups_kernel(int *counts, int *offsets, int E, int rows) {
   int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e < E) counts[e] = rows;
