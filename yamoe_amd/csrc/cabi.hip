@@ -119,6 +119,9 @@ static bool takes_small_tiles(int N, int E, int Nd) {
   const long long cols = ceil_div(Nd, 128), rows = ((long long)N + 64ll * E) / 128;
   return rows <= E ? E * cols <= 256 : rows * cols <= 320;
 }
+// How many partial row dots an input-gradient product of Nd columns leaves per row: one per wave column of its tiles, of
+// which a tile has two.  (Whoever reads them adds them up in order, so the tile's width shows in the last bits of the sum.)
+static int row_dot_parts(int N, int E, int Nd) { return 2 * ceil_div(Nd, takes_small_tiles(N, E, Nd) ? 128 : kColTile); }
 
 static int gathered_span_ok(const char *who, long long span_bytes) {
   if (span_bytes < (1ll << 32)) return 0;
@@ -159,7 +162,7 @@ static int tiles_down(const void *act, const void *w, const void *bias, void *y,
 }
 
 // g_rows == nullptr: g holds one row per sorted row; otherwise row p of the product reads g[g_rows[p] / g_div]
-// (g_span_bytes = size of the gathered tensor).  With dot_part the kernels also leave, per row, 2 * ceil(Nd / 256)
+// (g_span_bytes = size of the gathered tensor).  With dot_part the kernels also leave, per row, row_dot_parts
 // partial sums of <fp32 product row, dot_with row> (dot_with has the output's shape).
 template <typename T>
 static int tiles_dgrad(const void *g, const int *g_rows, int g_div, long long g_span_bytes, const void *w, void *out,
@@ -315,9 +318,9 @@ static size_t carve_backward(const yamoe_problem *p, void *ws, BackwardBuffers *
   b->d_x_perm = c.take(N * p->H * es);
   b->w_sorted = (float *)c.take(N * (es == 8 ? sizeof(double) : sizeof(float)));  // (doubles on the double-precision path)
   b->row_dot = (float *)c.take(N * (es == 8 ? sizeof(double) : sizeof(float)));
-  // 16-bit data: partial row dots of the down projection's input gradient with the activations, two per 256-column
-  // tile of I, written by that GEMM from its fp32 accumulators
-  b->n_part = es == 2 ? 2 * ceil_div(p->I, takes_small_tiles(p->T * p->K, p->E, p->I) ? 128 : kColTile) : 0;
+  // 16-bit data: partial row dots of the down projection's input gradient with the activations, written by that GEMM
+  // from its fp32 accumulators
+  b->n_part = es == 2 ? row_dot_parts(p->T * p->K, p->E, p->I) : 0;
   b->dot_part = b->n_part ? (float *)c.take(N * (size_t)b->n_part * sizeof(float)) : nullptr;
   // the weight-gradient kernel's copies of an expert's last, partial slab of rows run up to 32 rows past the
   // end of its operand buffers; every operand is followed by another buffer of this workspace, and this pad

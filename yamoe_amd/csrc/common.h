@@ -143,6 +143,15 @@ __device__ inline void copy16_to_lds(const char *lane_addr, uint32_t lds_base) {
                : "memory", "m0");
 }
 
+// LDS transpose read: lane i of each 16-lane group receives, for j = 0..3, the 16-bit element
+// (i % 4) of the 8 bytes addressed by lane 4*j + i/4 of the group.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+__device__ inline u32x2 lds_read_tr16(const char *p) {
+  s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
+  return __builtin_bit_cast(u32x2, v);
+}
+
 // ---- schedule: device-built work lists shared by the expert GEMM kernels ---------------------
 // Layout of the schedule region (int32 words):
 //   [0] n_row_tiles   number of (expert, row-block) entries for the MFMA kernels

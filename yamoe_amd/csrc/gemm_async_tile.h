@@ -96,7 +96,7 @@ struct Args {
   int Kd, Nd, lda, ldb, ldc, n_col_tiles;
   long long b_expert_stride;
   // EPI_STORE with [n][k] weights, optional: dot_part[row][2 * col_tile + wave column] = the fp32 accumulators of the
-  // row times dot_with[row][same columns] (a [rows, ldc] tensor), summed over the wave's 128 columns
+  // row times dot_with[row][same columns] (a [rows, ldc] tensor), summed over the wave column's half of the tile
   const void *dot_with;
   float *dot_part;
 #ifdef YAMOE_TILE_STAMPS
@@ -139,16 +139,6 @@ template <typename T> __device__ inline void load4_f32(const T *p, float (&out)[
   T4 v = *(const T4 *)p;
 #pragma unroll
   for (int i = 0; i < 4; ++i) out[i] = ElemTraits<T>::to_f32(v[i]);
-}
-
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-
-// LDS transpose read: lane i of each 16-lane group receives, for j = 0..3, the 16-bit element
-// (i % 4) of the 8 bytes addressed by lane 4*j + i/4 of the group.
-__device__ inline u32x2 lds_read_tr16(const char *p) {
-  s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)p);
-  return __builtin_bit_cast(u32x2, v);
 }
 
 template <int N> __device__ inline void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }

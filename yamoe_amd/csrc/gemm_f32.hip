@@ -12,7 +12,7 @@
 //    tiles (160 rows: 128 + 32) a tenth of the matrix work of the README workload went into blocks without rows.
 //    The 32-row blocks of a tile alternate between the two wave rows, so that a remainder keeps both busy.
 //  * Operands go global -> LDS with asynchronous 16-byte copies (no staging registers), two stages of 32 KB, one
-//    workgroup barrier per slab of 32 (16 000 clocks of matrix work): while a workgroup waits at its barrier or
+//    workgroup barrier per slab of 32 (4096 clocks of MFMA issue on each SIMD): while a workgroup waits at its barrier or
 //    runs its epilogue, the other workgroup on the CU keeps the matrix pipe busy.
 //  * The workgroups are resident, two per CU, and go through the tiles that have rows; the next tile is looked up and its
 //    first slab requested before the epilogue of the one before.

@@ -336,7 +336,7 @@ template int launch_router_backward_logits<f16_t>(const void *, const long long 
 // each through a staging area of its own (no workgroup barrier before the end, the next slab's rows on their way while one
 // is multiplied), and their fp32 partial tiles meet in LDS in the order of the waves.  Partial sums that stay inside the
 // workgroup need neither workspace nor a second launch, and 32 columns give 64 to 90 workgroups at widths of 2048 to 2880.
-// Both operands are [token][.] in memory and in LDS and are read with the LDS transpose read (see gemm_async_tile.h); the
+// Both operands are [token][.] in memory and in LDS and are read with the LDS transpose read (see common.h); the
 // bias gradient is summed from the same operand registers by the workgroups of the first columns.  1536 tokens, 64 experts,
 // H = 2048: 8.7 us; on eight 256 x 256 tiles that each walked all tokens 59 us, and 19 to 42 us more in a launch for the bias.
 constexpr int kRwWaves = 16, kRwThreads = kRwWaves * kWave, kRwSlab = 32, kRwExperts = 64, kRwCols = 32;
@@ -347,12 +347,9 @@ constexpr int kRwBias = kRwWaves * kRwPart;                                  // 
 constexpr int kRwLds = kRwBias + kRwWaves * kRwExperts * (int)sizeof(float);
 static_assert(kRwStage <= kRwPart, "the staging areas end where the bias sums start");
 
-typedef short rw_s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) rw_s16x4 rw_lds_s16x4;
 // four k rows `row_bytes` apart, twice: the eight consecutive k of this lane's row of a 32 x 32 x 16 operand
 __device__ inline u32x4 rw_operand(const char *p, int row_bytes) {
-  const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((rw_lds_s16x4 *)p));
-  const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((rw_lds_s16x4 *)(p + 4 * row_bytes)));
+  const u32x2 lo = lds_read_tr16(p), hi = lds_read_tr16(p + 4 * row_bytes);
   return (u32x4){lo[0], lo[1], hi[0], hi[1]};
 }
 

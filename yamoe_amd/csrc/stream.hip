@@ -12,8 +12,9 @@
 // A launch that can hold only a few experts (a handful of tokens: at most kStreamFewBlocks workgroups) has too few
 // workgroups to keep HBM busy that way: 4 experts x 23 slabs with two steps of 8 KB in flight per wave are 6 MB on
 // the way, where 8 TB/s x 2 us of latency want 16 MB.  Such a launch takes 8 waves per workgroup with three steps in
-// flight each instead (a workgroup per CU; 16 waves with two steps each measured 3 % slower), folded into the first
-// four before the same finish.
+// flight each instead (16 waves with two steps each measured 3 % slower), folded into the first four before the same
+// finish.  One token of a 2880-wide layer on four experts is 180 workgroups in the gate_up product and 92 in the down
+// product, on 256 CUs: 22 us for 132 MB of weights and 19 us for 66 MB.
 //
 // The lane that holds accumulator column c of MFMA j owns output column 8c + j, so the 8
 // accumulators of a lane are 8 consecutive output columns: the interleaved (gate, up) pairs of the

@@ -74,7 +74,7 @@ __device__ inline void run_wgrad_tile_small(const WgradArgs &args, const int tid
   const long long lda_bytes = (long long)args.Md * (long long)sizeof(T), ldb_bytes = (long long)args.Nd * (long long)sizeof(T);
 
   // A copies: piece i (0..1) = k rows 4*(2*wave + i) + (lane >> 4) of the slab, 256 bytes each; LDS position lane & 15
-  // holds piece pos ^ ((k & 3) << 2).  B copies as in the large kernel: piece i (0..3) = k rows 8*wave + 2*i + (lane >> 5).
+  // holds piece pos ^ ((k & 3) << 2).  B copies: piece i (0..3) = k rows 8*wave + 2*i + (lane >> 5).
   uint32_t a_off[2], b_off[4];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
