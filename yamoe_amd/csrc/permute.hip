@@ -56,7 +56,8 @@ __device__ inline float slot_weight(const T *rw, const void *idx, int t, int k, 
 // weight) pairs come through scalar loads and the rows of a chunk are requested together before the first of them is
 // added (a dropped slot requests row 0 and adds nothing); with a test in front of each row's load the wave waited for
 // one row after the other: us before -> now, 1536 tokens x 8 x 2048 bf16: 24.4 -> 13.4 (4.2 TB/s); 2003 x 4 x 2880:
-// 15.4 -> 11.9; 4096 x 4 x 2880: 26.2 -> 23.4 (5 TB/s); 1 x 4 x 2880: 5.3 -> 4.5, a launch's own cost.
+// 15.4 -> 11.9; 4096 x 4 x 2880: 26.2 -> 23.4 (5 TB/s); 1 x 4 x 2880: 5.3 -> 4.5, a launch's own cost.  Rounding the slots up
+// costs less than a form that tests each: 8192 x 3, 5, 6, 7 x 2880: 35.0 -> 30.1, 59.6 -> 45.3, 80.6 -> 63.8, 98.6 -> 80.6.
 template <typename T, bool I64, int KS>
 __global__ __launch_bounds__(kRowThreads) void combine_kernel(
     const T *__restrict__ y_perm, const int *__restrict__ inv_pos, const void *__restrict__ idx,
