@@ -1,0 +1,36 @@
+"""Launches of few rounds of tiles whose XCD shares (equal cost, not equal length) hold more tiles than the XCD's CUs take in
+those rounds: the excess goes to workgroups of other XCDs.  Experts of few rows in front, of many behind, so that the
+first XCDs' shares are the long ones; one round exactly filled, one tile more, and fewer; both tile sizes.  Every output row
+against the oracle: a tile that nobody took, or that two workgroups took, shows."""
+import pytest
+import torch
+
+from oracle import yamoe_oracle as O
+from tests.util import REL_L2_TOL, args, to_dev
+from yamoe_amd.workloads import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("light,light_rows,heavy,heavy_rows,I", [(125, 40, 125, 250, 64),   # 250 tiles of 256 x 256, one round
+                                                                 (128, 40, 128, 250, 64),   # 256: exactly one round
+                                                                 (129, 40, 128, 250, 64),   # 257: two rounds
+                                                                 (60, 40, 68, 250, 160),    # two column tiles in the gate_up product
+                                                                 (95, 20, 25, 250, 128)])   # 240 pairs of 128 x 128 tiles
+def test_excess_of_a_share(gpu, light, light_rows, heavy, heavy_rows, I):
+    import yamoe_amd
+    E, H = light + heavy, 64
+    T = light * light_rows + heavy * heavy_rows
+    print("rounds", E, T, I, flush=True)
+    d = make_inputs(T, H, I, E, 1, torch.bfloat16, seed=E, w_std=0.05, bias_std=0.1)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor([light_rows] * light + [heavy_rows] * heavy))
+    d["router_indices"] = ids[torch.randperm(T, generator=torch.Generator().manual_seed(1))].view(T, 1).to(d["router_indices"].dtype)
+    d["routing_weights"] = torch.zeros(T, E).scatter_(1, d["router_indices"].long(), 1.0).to(torch.bfloat16)
+    g = to_dev(d, gpu)
+    out = yamoe_amd.experts(*args(g), T, E, 1)
+    torch.cuda.synchronize()
+    want = O.experts_capacity(*args(d), T, compute_dtype=torch.float32)
+    # row by row: activations rounded once (2^-9) and the output once more, so 1e-2 for the whole holds for most rows; a row
+    # of 64 values that nearly cancel may lie above it by its share of the norm, a missing row at 1
+    err = (out.cpu().float() - want.float()).norm(dim=1) / want.float().norm(dim=1)
+    assert err.max() < 2 * REL_L2_TOL[torch.bfloat16], float(err.max())

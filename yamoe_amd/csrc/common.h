@@ -161,7 +161,7 @@ __device__ inline u32x2 lds_read_tr16(const char *p) {
 //   [4] weight_total  sum of the experts' cost weights (sched_group_weight)
 //   [5] n_half_tiles  number of 128-row tiles when the same experts' rows are cut into full tiles and a remainder
 //   [8 + 4x ...)      x = 0..8: where the tile list is cut so that each of the 8 XCDs gets the same share of
-//                     the cost: {first row tile of the expert the cut falls in, f, 0, row tiles of that
+//                     the cost: {first row tile of the expert the cut falls in, f, n_row_tiles, row tiles of that
 //                     expert}, f = the cut's position inside that expert's tiles in 1/65536ths; in a GEMM
 //                     with n column tiles the cut is at flat tile index
 //                     first * n + ((f * n) >> 16) * row_tiles, i.e. on a column-tile boundary of that expert
@@ -175,6 +175,7 @@ constexpr int kSchedHeader = 48;
 constexpr int kSchedCuts = 8;  // word offset of the XCD cut table
 constexpr int kSchedHalfTiles = 5;
 constexpr int kXcds = 8;
+constexpr int kXcdCus = 32;    // CUs of one XCD
 
 // Relative cost of one row tile in the MFMA kernels: a fixed part (prologue, epilogue, copies of the weight
 // slabs) plus one part per 64 rows (the MFMA blocks of the slower wave row).
@@ -193,6 +194,8 @@ __host__ __device__ inline int sched_cut(const int *sched, int x, int n_col_tile
   const int *c = sched + kSchedCuts + 4 * x;
   return c[0] * n_col_tiles + ((c[1] * n_col_tiles) >> 16) * c[3];
 }
+
+__host__ __device__ inline int sched_cut_row_tiles(const int *sched, int x) { return sched[kSchedCuts + 4 * x + 2]; }  // (x < kXcds)
 
 __host__ __device__ inline int sched_max_row_tiles(int N, int E) {
   // every expert with kept rows adds at most one partly filled tile

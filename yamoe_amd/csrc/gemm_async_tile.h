@@ -56,6 +56,7 @@ namespace async {
 
 constexpr int kBK = 32;
 constexpr int kThreads = 256;
+constexpr int kMostRounds = 8;  // up to this many rounds of tiles, no XCD takes more of them than it must (see gemm_async_kernel)
 constexpr int kBandRows = 8;  // row tiles of one band of an expert with many row tiles (see gemm_async_kernel)
 
 // LDS layout and copy shapes of a tile of BM rows x BN columns
@@ -667,17 +668,26 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
 
   // Workgroup b runs on XCD b % 8 and takes tile b / 8 of that XCD's share of the tile list.  The shares have
   // equal cost, not equal length, and are cut on (expert, column tile) boundaries, so the row tiles that read
-  // the same weight slabs meet in one L2.  A share longer than gridDim.x / 8 hands its excess to the workgroups
-  // of shorter shares (the grid has at least as many workgroups as there are tiles).
+  // the same weight slabs meet in one L2.  A share longer than its slots hands its excess to the workgroups that shorter
+  // shares leave over.  An XCD has as many slots as the rounds that the whole list takes on 256 CUs have places on its
+  // 32: shares of equal cost put 27 to 35 tiles of a 252-tile list on an XCD, and one tile over a round costs a round.
+  // Whole forwards, us, slots for every workgroup / as here: 979 tokens x 2 on 16 experts, 2048 wide: 153 / 123; 3553 x 4 on 32,
+  // 1024: 176 / 134; 3773 x 4 on 128, 2048: 728 / 687; 2003 x 4 on 32, 2880 x 720: 224 / 190.  Beyond kMostRounds a round is
+  // little of a launch, and tiles of very different cost should stay where the cost puts them (29 rounds, Zipf routing: 3250 /
+  // 3276); there only the grid bounds a share (it has at least as many workgroups as there are tiles).
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1;
 #ifdef YAMOE_TILE_STAMPS
   const unsigned long long t_entry = __builtin_amdgcn_s_memtime();
 #endif
   int L;
   {
-    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds / S::kParts, slots = gridDim.x / kXcds / S::kParts;
+    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds / S::kParts;
     const int first = sched_cut(args.sched, xcd, args.n_col_tiles);
     const int count = sched_cut(args.sched, xcd + 1, args.n_col_tiles) - first;
+    const int rounds = ceil_div(sched_cut_row_tiles(args.sched, xcd) * args.n_col_tiles, kXcds * kXcdCus);
+    int slots = gridDim.x / kXcds / S::kParts;
+    if (rounds <= kMostRounds) slots = min(slots, rounds * kXcdCus);
+    if (i >= slots) return;
     if (i < count) {
       L = first + i;
     } else {

@@ -217,7 +217,7 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
           long long t = (long long)x * w_total;  // compare x * W / 8 with the group's weight interval, times 8
           if (t >= 8ll * w_pre && t < 8ll * (w_pre + w)) {
             int *c = sched + kSchedCuts + 4 * x;
-            c[0] = t_pre; c[1] = (int)(((t - 8ll * w_pre) << 16) / (8ll * w)); c[2] = 0; c[3] = tiles;
+            c[0] = t_pre; c[1] = (int)(((t - 8ll * w_pre) << 16) / (8ll * w)); c[2] = n_tiles; c[3] = tiles;
           }
         }
       }
