@@ -34,3 +34,25 @@ def test_excess_of_a_share(gpu, light, light_rows, heavy, heavy_rows, I):
     # of 64 values that nearly cancel may lie above it by its share of the norm, a missing row at 1
     err = (out.cpu().float() - want.float()).norm(dim=1) / want.float().norm(dim=1)
     assert err.max() < 2 * REL_L2_TOL[torch.bfloat16], float(err.max())
+
+
+@pytest.mark.parametrize("rows,capacity", [([1, 15, 16, 17, 0, 2] + [140] * 6, None),   # some stream behind the tiles
+                                           ([300, 1, 300, 1, 9], None),
+                                           ([100] * 8, 24),                             # a capacity that leaves only streamed experts
+                                           ([100] * 4, 32)])
+@pytest.mark.parametrize("H,I", [(64, 64), (200, 328)])
+def test_streamed_experts_in_the_tiles_launch(gpu, rows, capacity, H, I):
+    """More than 32 assignments per expert on average and few tiles: one launch does the tiles and the streamed experts, also
+    where those have up to 32 rows."""
+    import yamoe_amd
+    E, T = len(rows), sum(rows)
+    capacity = T if capacity is None else capacity
+    print("carried", rows, capacity, H, I, flush=True)
+    d = make_inputs(T, H, I, E, 1, torch.bfloat16, seed=T, w_std=0.05, bias_std=0.1)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(rows))
+    d["router_indices"] = ids[torch.randperm(T, generator=torch.Generator().manual_seed(2))].view(T, 1).to(d["router_indices"].dtype)
+    d["routing_weights"] = torch.zeros(T, E).scatter_(1, d["router_indices"].long(), 1.0).to(torch.bfloat16)
+    out = yamoe_amd.experts(*args(to_dev(d, gpu)), capacity, E, 1)
+    torch.cuda.synchronize()
+    want = O.experts_capacity(*args(d), capacity, compute_dtype=torch.float32)
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[torch.bfloat16]

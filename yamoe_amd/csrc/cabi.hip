@@ -69,10 +69,10 @@ int stream_down(const void *, const void *, const void *, void *, const void *, 
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
-                       int, int, int, int, hipStream_t);
+                       int, int, int, int, bool, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, int,
-                    hipStream_t);
+                    bool, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
                      const void *, float *, hipStream_t);
@@ -137,25 +137,26 @@ static int gathered_span_ok(const char *who, long long span_bytes) {
 // more first: the kernels address gathered rows with 32-bit byte offsets from the start of the tensor).
 template <typename T>
 static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
-                         const void *sched, int N, int K, int E, int H, int I, int small_rows, hipStream_t stream) {
+                         const void *sched, int N, int K, int E, int H, int I, int small_rows, bool streams,
+                         hipStream_t stream) {
   // the gathered source rows span the whole hidden_states tensor: N / K tokens of H elements
   const long long span = sorted_idx != nullptr ? (long long)(N / K) * H * (long long)sizeof(T) : 0;
   if (int rc = gathered_span_ok("tiles_gate_up", span)) return rc;
   if constexpr (sizeof(T) == 2) {
     auto run = H % 64 ? gemm_async_gate_up<T, 256, true> : gemm_async_gate_up<T, 256, false>;
     if (takes_small_tiles(N, E, 2 * I)) run = H % 64 ? gemm_async_gate_up<T, 128, true> : gemm_async_gate_up<T, 128, false>;
-    return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, stream);
+    return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, streams, stream);
   } else {
     return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
   }
 }
 template <typename T>
 static int tiles_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E,
-                      int H, int I, int small_rows, hipStream_t stream) {
+                      int H, int I, int small_rows, bool streams, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
     auto run = I % 64 ? gemm_async_down<T, 256, true> : gemm_async_down<T, 256, false>;
     if (takes_small_tiles(N, E, H)) run = I % 64 ? gemm_async_down<T, 128, true> : gemm_async_down<T, 128, false>;
-    return run(act, w, bias, y, sched, N, E, H, I, small_rows, stream);
+    return run(act, w, bias, y, sched, N, E, H, I, small_rows, streams, stream);
   } else {
     return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
   }
@@ -351,6 +352,15 @@ static size_t carve_saved(const yamoe_problem *p, void *base, Saved *s) {
     if (rc_ != 0) return rc_;  \
   } while (0)
 
+// Whether the launches of the tile kernels also work off the streaming list, instead of two launches of their own that
+// usually find it empty.  Where every expert has 32 assignments on average, few if any stream; where they do, the carried
+// form has fewer waves on a CU than the streaming kernel, so it is taken only while the launches are short (an expert's last
+// row tile is half full on average, hence the estimate).
+static bool tiles_carry_streams(int N, int E, int H, int I) {
+  const long long cols = ceil_div(H > 2 * I ? H : 2 * I, kColTile), rows = ((long long)N + 128ll * E) / kRowTile;
+  return N > 32ll * E && rows * cols <= 4 * 256;
+}
+
 template <typename T>
 static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, const void *rw, const void *wgu,
                         const void *bgu, const void *wd, const void *bd, void *out, void *ws, const Saved *keep,
@@ -372,20 +382,21 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
                                b.schedule, b.schedule_bytes, st));
   // with no more assignments than a streamed expert may have rows, every expert is streamed as well
   const bool tiles = !everything && N > stream_rows;
+  const bool carried = HasStreamPath<T>::value && tiles && tiles_carry_streams(N, p->E, p->H, p->I);
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
-                               stream));
+                               carried, stream));
   } else if (tiles) {
     YAMOE_TRY(tiles_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
-                               stream));
+                               carried, stream));
   }
   if constexpr (HasStreamPath<T>::value)
-    YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I,
+    if (!carried) YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I,
                                 stream));
-  if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, stream));
+  if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, carried, stream));
   if constexpr (HasStreamPath<T>::value)
-    YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream));
+    if (!carried) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream));
   YAMOE_TRY(launch_combine<T>(b.y_perm, b.inv_pos, idx, p->idx_i64, rw, p->rw_cols, out, p->T, p->K, p->E, p->H,
                               stream));
   return 0;
@@ -419,9 +430,9 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   if (kept != nullptr) {
     // activations and pre-activations come from the forward
   } else if (permuted) {
-    YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, stream));
+    YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, false, stream));
   } else {
-    YAMOE_TRY(tiles_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, stream));
+    YAMOE_TRY(tiles_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, false, stream));
   }
   // combine backward: g_y_perm = grad_out[tok] * w, and the bias part of the routing gradient
   YAMOE_TRY(launch_combine_backward<T>(gy, bd, b.f.sorted_idx, b.f.inv_pos, idx, p->idx_i64, rw, p->rw_cols, b.g_y_perm,
@@ -551,7 +562,7 @@ static int check_gemm_shape(const char *who, int N, int E, int H, int I, int dty
 template <typename T>
 static int gate_up_both(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
                         const void *sched, int N, int K, int E, int H, int I, hipStream_t stream) {
-  YAMOE_TRY(tiles_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, 0, stream));
+  YAMOE_TRY(tiles_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, 0, false, stream));
   if constexpr (HasStreamPath<T>::value)
     YAMOE_TRY(stream_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream));
   return 0;
@@ -559,7 +570,7 @@ static int gate_up_both(const void *x, const int *sorted_idx, const void *w, con
 template <typename T>
 static int down_both(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
                      int I, hipStream_t stream) {
-  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, stream));
+  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, false, stream));
   if constexpr (HasStreamPath<T>::value) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, stream));
   return 0;
 }
@@ -573,7 +584,7 @@ static int down_regular(const void *act, const void *w, const void *bias, void *
   YAMOE_TRY(regular_schedule(counts, offsets, E, rows, stream_rows, sched, sched_bytes, stream));
   if constexpr (HasStreamPath<T>::value)
     if (rows <= stream_rows) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream);
-  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, stream);
+  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, false, stream);
 }
 
 extern "C" int yamoe_gate_up(const void *x, const int32_t *sorted_idx, const void *gate_up_proj,

@@ -48,7 +48,7 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "stream_slab.h"
 
 namespace yamoe {
 
@@ -100,6 +100,10 @@ struct Args {
   // row times dot_with[row][same columns] (a [rows, ldc] tensor), summed over the wave column's half of the tile
   const void *dot_with;
   float *dot_part;
+  // forward products, optional: the schedule's streaming list is worked off by stream_wgs workgroups of every XCD in this
+  // launch (0: by launches of their own)
+  const int *small;
+  int stream_wgs, n_stream_slabs;
 #ifdef YAMOE_TILE_STAMPS
   unsigned long long *stamps;  // [stamps_cap][8]: see yamoe_debug_tile_stamps
   int stamps_cap;
@@ -662,6 +666,29 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
 #endif
 }
 
+// One workgroup's part of the streaming list: items `first`, first + step, ...  An item is a slab of one expert, and
+// neighbouring items, which different XCDs work on, are neighbouring slabs.  (17 to 32 rows only where a capacity or invalid
+// ids leave no expert more.)  Two launches less per layer: 2048 tokens x 2 on 16 experts, 1024 wide, whole layer 81.6 -> 78.1 us,
+// 426 x 2: 42.4 -> 39.5.  In launches of many rounds these workgroups took the time of the streaming kernel to the
+// microsecond, behind the tiles or between the first of them (Zipf routing, 16 384 tokens: gate_up 1794 + 266 and 2063 us).
+static_assert(kThreads == kStreamWaves * kWave, "a workgroup of the tile kernels is one of the streaming kernel");
+template <typename T, int EPI, bool GATHER, int DEPTH> __device__ __forceinline__ void stream_items(const Args &args, int first, int step) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  StreamArgs a = {};
+  a.A = args.A; a.B = args.B; a.bias = args.bias; a.C = args.C; a.C2 = args.C2; a.a_rows = args.a_rows; a.a_div = args.a_div;
+  a.Kd = args.Kd; a.Nd = args.Nd; a.lda = args.lda; a.ldc = args.ldc;
+  const int items = args.sched[1] * args.n_stream_slabs;
+  for (int it = first; it < items; it += step) {
+    const int s = it / args.n_stream_slabs;
+    const int *e = args.small + 4 * s;
+    const int expert = __builtin_amdgcn_readfirstlane(e[0]), row0 = __builtin_amdgcn_readfirstlane(e[1]);
+    const int rows = __builtin_amdgcn_readfirstlane(e[2]), slab = it - s * args.n_stream_slabs;
+    if (rows > 16) stream_slab<T, EPI == EPI_GLU, GATHER, kStreamWaves, 2, 2>(a, (float *)lds, expert, row0, rows, slab);
+    else stream_slab<T, EPI == EPI_GLU, GATHER, kStreamWaves, DEPTH, 1>(a, (float *)lds, expert, row0, rows, slab);
+    __syncthreads();  // the next item's partial sums take the place of this one's
+  }
+}
+
 template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED>
 __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const Args args) {
   constexpr int kBN = S::BN;
@@ -680,12 +707,24 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
   const unsigned long long t_entry = __builtin_amdgcn_s_memtime();
 #endif
   int L;
+  const int place = blockIdx.x / kXcds;
   {
-    const int xcd = blockIdx.x % kXcds, i = blockIdx.x / kXcds / S::kParts;
+    const int xcd = blockIdx.x % kXcds;
     const int first = sched_cut(args.sched, xcd, args.n_col_tiles);
     const int count = sched_cut(args.sched, xcd + 1, args.n_col_tiles) - first;
     const int rounds = ceil_div(sched_cut_row_tiles(args.sched, xcd) * args.n_col_tiles, kXcds * kXcdCus);
-    int slots = gridDim.x / kXcds / S::kParts;
+    if constexpr (!BNK) {
+      if (args.stream_wgs > 0) {
+        const int places = gridDim.x / kXcds;
+        const int k = place - (places - args.stream_wgs);  // behind the tiles
+        if (k >= 0) {
+          stream_items<T, EPI, GATHER, S::kPerSimd == 1 ? 3 : 2>(args, k * kXcds + xcd, args.stream_wgs * kXcds);
+          return;
+        }
+      }
+    }
+    const int i = place / S::kParts;
+    int slots = (gridDim.x / kXcds - (BNK ? 0 : args.stream_wgs)) / S::kParts;
     if (rounds <= kMostRounds) slots = min(slots, rounds * kXcdCus);
     if (i >= slots) return;
     if (i < count) {
@@ -748,7 +787,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
       // The row tile's two halves are neighbours in the grid, on one XCD.  More than 128 rows are cut into two parts of
       // whole 32-row blocks as equal as they get; up to 128 rows are one part, and the other workgroup has nothing to do.
       const int first_rows = ti.rows_valid > S::BM ? ((ti.rows_valid + 63) >> 6) * 32 : ti.rows_valid;
-      if ((blockIdx.x / kXcds) & 1) {
+      if (place & 1) {
         ti.row0 += first_rows;
         ti.rows_valid -= first_rows;
         if (ti.rows_valid <= 0) return;
@@ -861,7 +900,7 @@ static int launch(const Args &args, int max_row_tiles, hipStream_t stream) {
   if (int rc = ensure_dynamic_lds((const void *)kernel, lds_bytes, attr_done, "gemm_async_kernel")) return rc;
   long long total = (long long)max_row_tiles * args.n_col_tiles;
   if (total <= 0) return 0;
-  total = (total + kXcds - 1) / kXcds * kXcds * S::kParts;
+  total = (total + kXcds - 1) / kXcds * kXcds * S::kParts + args.stream_wgs * kXcds;
 #ifdef YAMOE_TILE_STAMPS
   Args stamped = args;
   stamped.stamps = g_tile_stamps;
