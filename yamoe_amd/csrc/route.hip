@@ -101,49 +101,49 @@ __device__ inline void wave_place(const void *idx, int seg_begin, int seg_end, i
   }
 }
 
-// Exclusive scan over buckets of `total` into `offsets` (both LDS), done by the whole block.
-// offsets[b] for b in [0, buckets]; offsets[buckets] = N.
-__device__ inline void block_exclusive_scan(const int *total, int *offsets, int buckets,
-                                            int *scratch /* kRouteWaves + 1 ints */) {
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+// Inclusive prefix sum over the 64 lanes by DPP moves: six additions whose operand comes from another lane of the row of 16,
+// from the last lane of the row before, and from lane 31, instead of six trips through the LDS crossbar each.  The routing
+// of a small batch is one chain of such scans, barriers and divisions; us before / with these scans, the bucket scan by one
+// wave, and no 64-bit division: 4 keys on 128 experts 8.0 / 4.6, 4096 on 16 12.9 / 9.5, 4004 on 128 15.8 / 10.9; two launches,
+// 12 288 on 64: 12.3 / 10.1 (the second); work lists of one expert's rows alone 8.4 / 5.0.
+template <int CTRL, int ROW_MASK> __device__ inline int dpp_or_zero(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
+}
+__device__ inline int wave_inclusive_scan(int x) {
+  x += dpp_or_zero<0x111, 0xf>(x);  // row_shr:1
+  x += dpp_or_zero<0x112, 0xf>(x);  // row_shr:2
+  x += dpp_or_zero<0x114, 0xf>(x);  // row_shr:4
+  x += dpp_or_zero<0x118, 0xf>(x);  // row_shr:8
+  x += dpp_or_zero<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += dpp_or_zero<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ inline int wave_exclusive_scan(int v, int &total) {
+  const int x = wave_inclusive_scan(v);
+  total = __builtin_amdgcn_readlane(x, kWave - 1);
+  return x - v;
+}
+__device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1); }
+
+// Exclusive scan over buckets of `total` into `offsets` (both LDS), by the first wave of the workgroup; offsets[buckets] = N.
+// The caller puts a barrier on both sides.
+__device__ inline void first_wave_exclusive_scan(const int *total, int *offsets, int buckets) {
+  if (threadIdx.x >= kWave) return;
+  const int lane = threadIdx.x;
   int carry = 0;
-  for (int base = 0; base < buckets; base += blockDim.x) {
-    int b = base + tid;
-    int v = (b < buckets) ? total[b] : 0;
-    // inclusive scan inside the wave
-    int x = v;
-    for (int d = 1; d < kWave; d <<= 1) {
-      int y = __shfl_up(x, d);
-      if (lane >= d) x += y;
-    }
-    if (lane == kWave - 1) scratch[wave] = x;
-    __syncthreads();
-    int wave_off = 0;
-    for (int w = 0; w < wave; ++w) wave_off += scratch[w];
-    int chunk_total = 0;
-    for (int w = 0; w < (int)(blockDim.x / kWave); ++w) chunk_total += scratch[w];
-    if (b < buckets) offsets[b] = carry + wave_off + x - v;
-    carry += chunk_total;
-    __syncthreads();
+  for (int base = 0; base < buckets; base += kWave) {
+    int sum;
+    const int before = wave_exclusive_scan(base + lane < buckets ? total[base + lane] : 0, sum);
+    if (base + lane < buckets) offsets[base + lane] = carry + before;
+    carry += sum;
   }
-  if (tid == 0) offsets[buckets] = carry;
-  __syncthreads();
+  if (lane == 0) offsets[buckets] = carry;
 }
 
 // ---- work lists ------------------------------------------------------------------------------
 // One wave; lane l takes experts l, l+64, ...  Experts with 1..stream_max_rows kept rows go to the
 // streaming list, larger ones are cut into row tiles of kRowTile rows.  Both lists stay in expert
 // order: positions come from wave prefix sums.
-__device__ inline int wave_exclusive_scan(int v, int lane, int &total) {
-  int x = v;
-  for (int d = 1; d < kWave; d <<= 1) {
-    int y = __shfl_up(x, d);
-    if (lane >= d) x += y;
-  }
-  total = __shfl(x, kWave - 1);
-  return x - v;
-}
-
 __device__ inline void build_schedule_wave(const int *counts, const int *offsets, int N, int E, int capacity,
                                            int stream_max_rows, int *sched, const int lane) {
   int *row_tiles = sched + kSchedHeader;
@@ -155,14 +155,9 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   const bool everything = stream_max_rows == kStreamEverything;  // (the host checked sched_may_stream_everything)
   if (everything) stream_max_rows = kStreamMaxRows;
   if (!everything && stream_max_rows > kStreamMixedRows) {
-    int most = 0;
-    for (int base = 0; base < E; base += kWave) {
-      int e = base + lane;
-      int kept = e < E ? min(counts[e], capacity) : 0;
-      most = max(most, kept);
-    }
-    for (int d = kWave / 2; d > 0; d >>= 1) most = max(most, __shfl_xor(most, d));
-    if (most > stream_max_rows) stream_max_rows = kStreamMixedRows;
+    bool beyond = false;
+    for (int base = lane; base < E; base += kWave) beyond |= min(counts[base], capacity) > stream_max_rows;
+    if (__any(beyond)) stream_max_rows = kStreamMixedRows;
   }
   for (int base = 0; base < E; base += kWave) {
     int e = base + lane;
@@ -172,13 +167,12 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     // entries on the streaming list: one, or with `everything` one per chunk of kStreamMaxRows rows
     int is_small = everything ? ceil_div(kept, kStreamMaxRows) : (kept > 0 && kept <= stream_max_rows);
     int tiles = (kept > 0 && !is_small) ? ceil_div(kept, kRowTile) : 0;
-    int tot_small, tot_tiles, tot_active, tot_kept, tot_half;
-    int pos_small = wave_exclusive_scan(is_small, lane, tot_small);
-    int pos_tiles = wave_exclusive_scan(tiles, lane, tot_tiles);
+    int tot_small, tot_tiles, tot_half;
+    int pos_small = wave_exclusive_scan(is_small, tot_small);
+    int pos_tiles = wave_exclusive_scan(tiles, tot_tiles);
     const int halves = tiles > 0 ? ceil_div(kept, kRowTile / 2) : 0;
-    const int pos_half = n_half + wave_exclusive_scan(halves, lane, tot_half);
-    wave_exclusive_scan(kept > 0 ? 1 : 0, lane, tot_active);
-    wave_exclusive_scan(kept, lane, tot_kept);
+    const int pos_half = n_half + wave_exclusive_scan(halves, tot_half);
+    const int tot_active = __popcll(__ballot(kept > 0)), tot_kept = wave_sum(kept);
     for (int c = 0; c < is_small; ++c) {
       int *s = small + 4 * (n_small + pos_small + c);
       s[0] = e; s[1] = first + c * kStreamMaxRows; s[2] = min(kStreamMaxRows, kept - c * kStreamMaxRows); s[3] = 0;
@@ -188,7 +182,8 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     // tiles plus a remainder: tiles of one expert then advance through the contraction at the same pace
     // and the weight slabs one of them fetches are still in L2 when the others ask for them.
     int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(kept, tiles) + 31) & ~31) : 0;
-    const FastDiv by_tiles = make_fast_div(tiles > 0 ? tiles : 1);  // the GEMM kernels divide by the group size
+    FastDiv by_tiles = {1u, 0u};  // the GEMM kernels divide by the group size (a 64-bit division: only where there is a group)
+    if (tiles > 1) by_tiles = make_fast_div(tiles);
     for (int t = 0; t < tiles; ++t) {
       int *w = row_tiles + 8 * (gfirst + t);
       w[0] = e; w[1] = first + t * per_tile; w[2] = min(per_tile, kept - t * per_tile); w[3] = gfirst; w[4] = tiles;
@@ -198,40 +193,47 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   }
   // Second pass: cut the tile list into 8 shares of equal cost.  Groups (experts with row tiles) are weighed
   // by the sum of their tiles' weights; cut x falls into the group that contains x/8 of the total.
-  int w_total = 0;
-  for (int pass = 0; pass < 2; ++pass) {
+  auto group = [&](int e, int &tiles) {
+    int kept = e < E ? min(counts[e], capacity) : 0;
+    tiles = kept > 0 && !everything && kept > stream_max_rows ? ceil_div(kept, kRowTile) : 0;
+    const int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(kept, tiles) + 31) & ~31) : 0;
+    return sched_group_weight(tiles, per_tile, kept);
+  };
+  int w_total = 0, tiles;
+  if (n_tiles > 0)
+    for (int base = 0; base < E; base += kWave) w_total += wave_sum(group(base + lane, tiles));
+  // lane x < 8 gets cut x: its group's first row tile and tiles, how far into the group's 8-fold weight it falls
+  int cut_first = 0, cut_tiles = 0;
+  long long cut_num = 0, cut_w = 1;
+  if (w_total > 0) {
     int w_before = 0, t_before = 0;
     for (int base = 0; base < E; base += kWave) {
-      int e = base + lane;
-      int kept = e < E ? min(counts[e], capacity) : 0;
-      if (kept < 0) kept = 0;
-      int is_small = everything || (kept > 0 && kept <= stream_max_rows);
-      int tiles = (kept > 0 && !is_small) ? ceil_div(kept, kRowTile) : 0;
-      int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(kept, tiles) + 31) & ~31) : 0;
-      int w = sched_group_weight(tiles, per_tile, kept);
       int tot_w, tot_t;
-      int w_pre = w_before + wave_exclusive_scan(w, lane, tot_w);
-      int t_pre = t_before + wave_exclusive_scan(tiles, lane, tot_t);
-      if (pass == 1 && tiles > 0) {
-        for (int x = 0; x < kXcds; ++x) {
-          long long t = (long long)x * w_total;  // compare x * W / 8 with the group's weight interval, times 8
-          if (t >= 8ll * w_pre && t < 8ll * (w_pre + w)) {
-            int *c = sched + kSchedCuts + 4 * x;
-            c[0] = t_pre; c[1] = (int)(((t - 8ll * w_pre) << 16) / (8ll * w)); c[2] = n_tiles; c[3] = tiles;
-          }
-        }
+      const int w = group(base + lane, tiles);
+      const int w_pre = w_before + wave_exclusive_scan(w, tot_w), t_pre = t_before + wave_exclusive_scan(tiles, tot_t);
+      for (int x = 0; x < kXcds; ++x) {
+        const long long t = (long long)x * w_total;  // compare x * W / 8 with the group's weight interval, times 8
+        const uint64_t hit = __ballot(tiles > 0 && t >= 8ll * w_pre && t < 8ll * (w_pre + w));
+        if (hit == 0) continue;
+        const int from = __ffsll((unsigned long long)hit) - 1;
+        const int first = __builtin_amdgcn_readlane(t_pre, from), count = __builtin_amdgcn_readlane(tiles, from);
+        const int pre = __builtin_amdgcn_readlane(w_pre, from), weight = __builtin_amdgcn_readlane(w, from);
+        if (lane == x) { cut_first = first; cut_tiles = count; cut_num = t - 8ll * pre; cut_w = 8ll * weight; }
       }
       w_before += tot_w; t_before += tot_t;
     }
-    if (pass == 0) w_total = w_before;
+  }
+  if (lane < kXcds) {
+    // floor(2^16 * num / w) in double precision: below 2^51 over below 2^35, so a quotient that is no whole number is further
+    // from the next one (2^-35) than it is rounded (2^-37)
+    int *c = sched + kSchedCuts + 4 * lane;
+    c[0] = cut_first; c[1] = (int)((double)(cut_num << 16) / (double)cut_w); c[2] = w_total > 0 ? n_tiles : 0; c[3] = cut_tiles;
   }
   if (lane == 0) {
     sched[0] = n_tiles; sched[1] = n_small; sched[2] = n_active; sched[3] = n_kept;
     sched[4] = w_total; sched[kSchedHalfTiles] = n_half; sched[6] = 0; sched[7] = 0;
     int *c = sched + kSchedCuts + 4 * kXcds;  // the end of the list
     c[0] = n_tiles; c[1] = 0; c[2] = 0; c[3] = 0;
-    if (w_total == 0)
-      for (int x = 0; x < kXcds; ++x) { int *cx = sched + kSchedCuts + 4 * x; cx[0] = 0; cx[1] = 0; cx[2] = 0; cx[3] = 0; }
     for (int i = kSchedCuts + 4 * (kXcds + 1); i < kSchedHeader; ++i) sched[i] = 0;
   }
 }
@@ -250,12 +252,12 @@ __global__ __launch_bounds__(kWave) void regular_schedule_kernel(int *counts, in
 }
 
 // ---- single-block form: everything in one launch -------------------------------------------------
-// Dynamic LDS: hist[kRouteWaves][buckets] + total[buckets] + offsets[buckets+1] + scratch + the N keys as 16-bit
+// Dynamic LDS: hist[kRouteWaves][buckets] + total[buckets] + offsets[buckets+1] + the N keys as 16-bit
 // values.  The kernel runs once per forward on a cold instruction cache, so its loops stay rolled (straight-line
 // code would run at instruction-fetch speed); the keys are read from memory once and kept in LDS for the
 // placement pass.
 __host__ __device__ inline size_t route_single_lds_bytes(int N, int buckets) {
-  size_t ints = (size_t)kRouteWaves * buckets + buckets + buckets + 1 + kRouteWaves + 1;
+  size_t ints = (size_t)kRouteWaves * buckets + buckets + buckets + 1;
   return align_up(ints * sizeof(int), 16) + align_up((size_t)(N > 0 ? N : 1) * sizeof(unsigned short), 16);
 }
 
@@ -268,9 +270,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
   int *hist = lds;                          // [kRouteWaves][buckets]
   int *total = hist + kRouteWaves * buckets;  // [buckets]
   int *offs = total + buckets;              // [buckets + 1]
-  int *scratch = offs + buckets + 1;        // [kRouteWaves + 1]
-  unsigned short *keys = (unsigned short *)((char *)lds + align_up(((size_t)kRouteWaves * buckets + 2 * buckets + 1 +
-                                                                   kRouteWaves + 1) * sizeof(int), 16));
+  unsigned short *keys = (unsigned short *)((char *)lds + align_up(((size_t)kRouteWaves * buckets + 2 * buckets + 1) * sizeof(int), 16));
   const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
 
   for (int i = tid; i < kRouteWaves * buckets; i += blockDim.x) hist[i] = 0;
@@ -297,22 +297,20 @@ __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
   }
   __syncthreads();
 
+  // hist[w][b] <- keys of bucket b in the segments before w; the cursor of a wave is that plus the bucket's offset
   for (int b = tid; b < buckets; b += blockDim.x) {
-    int s = 0;
-    for (int w = 0; w < kRouteWaves; ++w) s += hist[w * buckets + b];
-    total[b] = s;
-  }
-  __syncthreads();
-  block_exclusive_scan(total, offs, buckets, scratch);
-
-  // cursors: hist[w][b] <- offs[b] + sum_{w' < w} hist[w'][b]
-  for (int b = tid; b < buckets; b += blockDim.x) {
-    int run = offs[b];
+    int run = 0;
     for (int w = 0; w < kRouteWaves; ++w) {
-      int c = hist[w * buckets + b];
+      const int c = hist[w * buckets + b];
       hist[w * buckets + b] = run;
       run += c;
     }
+    total[b] = run;
+  }
+  __syncthreads();
+  first_wave_exclusive_scan(total, offs, buckets);
+  __syncthreads();
+  for (int b = tid; b < buckets; b += blockDim.x) {
     if (b < E) {
       counts[b] = total[b];
       offsets_out[b] = offs[b];
@@ -320,7 +318,6 @@ __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
       offsets_out[E] = offs[E];
     }
   }
-  __syncthreads();
 
   // placement, in input order: position = cursor[key] + number of equal keys in lower lanes of the step
   {
@@ -335,14 +332,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
       int rank = __popcll(peers & lt_mask);
       int start = 0;
       if (active) start = cursor[k];
+      const int first = active ? offs[k] : 0;
       __builtin_amdgcn_wave_barrier();
       if (active) {
-        int pos = start + rank;
+        const int in_bucket = start + rank, pos = first + in_bucket;
         // a valid id is its own key; the rare invalid one is fetched again for the sorted_expert output
         sorted_expert[pos] = k < E ? k : load_raw<I64>(idx, i);
         sorted_idx[pos] = i;
-        bool kept = k < E && (pos - offs[k]) < capacity;
-        inv_pos[i] = kept ? pos : -1;
+        inv_pos[i] = k < E && in_bucket < capacity ? pos : -1;
         if (rank == 0) cursor[k] = start + __popcll(peers);
       }
       // the cursor is private to this wave and LDS operations of one wave complete in order: the next step's
@@ -385,23 +382,23 @@ __global__ __launch_bounds__(kRouteThreads) void route_scan_kernel(int *seg_coun
   const int buckets = E + 1;
   int *total = lds;
   int *offs = total + buckets;
-  int *scratch = offs + buckets + 1;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   for (int b = wave; b < buckets; b += kRouteWaves) {
     int s = 0;
     for (int g = lane; g < n_seg; g += kWave) s += seg_counts[(size_t)g * buckets + b];
-    for (int d = kWave / 2; d > 0; d >>= 1) s += __shfl_xor(s, d);
+    s = wave_sum(s);
     if (lane == 0) total[b] = s;
   }
   __syncthreads();
-  block_exclusive_scan(total, offs, buckets, scratch);
+  first_wave_exclusive_scan(total, offs, buckets);
+  __syncthreads();
   for (int b = wave; b < buckets; b += kRouteWaves) {
     int run = offs[b];
     for (int g0 = 0; g0 < n_seg; g0 += kWave) {
       const int g = g0 + lane;
       const int c = g < n_seg ? seg_counts[(size_t)g * buckets + b] : 0;
       int step_total;
-      const int before = wave_exclusive_scan(c, lane, step_total);
+      const int before = wave_exclusive_scan(c, step_total);
       if (g < n_seg) seg_counts[(size_t)g * buckets + b] = run + before;
       run += step_total;
     }
@@ -450,7 +447,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
 // per bucket column, wave prefix sums over the segments).  Workgroup 0 also writes counts and offsets; with sched
 // one workgroup more than there are blocks of segments writes the work lists.
 __host__ __device__ inline size_t route_place_scan_lds_ints(int n_seg, int buckets) {
-  return (size_t)buckets + (buckets + 1) + (kRouteWaves + 1) + (size_t)kRouteWaves * buckets + (size_t)n_seg * buckets;
+  return (size_t)buckets + (buckets + 1) + (size_t)kRouteWaves * buckets + (size_t)n_seg * buckets;
 }
 constexpr size_t kPlaceScanMaxLdsInts = 40000;  // 160 000 bytes
 
@@ -462,8 +459,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
   const int buckets = E + 1;
   int *total = lds;                              // [buckets]
   int *offs = total + buckets;                   // [buckets + 1]
-  int *scratch = offs + buckets + 1;             // [kRouteWaves + 1]
-  int *cursors = scratch + kRouteWaves + 1;      // [kRouteWaves][buckets]
+  int *cursors = offs + buckets + 1;             // [kRouteWaves][buckets]
   int *table = cursors + kRouteWaves * buckets;  // [n_seg][buckets]
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int cells = n_seg * buckets;
@@ -476,14 +472,15 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
       const int g = g0 + lane;
       const int c = g < n_seg ? table[g * buckets + b] : 0;
       int step_total;
-      const int before = wave_exclusive_scan(c, lane, step_total);
+      const int before = wave_exclusive_scan(c, step_total);
       if (g < n_seg && g >= my_first && g < my_first + kRouteWaves) cursors[(g - my_first) * buckets + b] = run + before;
       run += step_total;
     }
     if (lane == 0) total[b] = run;
   }
   __syncthreads();
-  block_exclusive_scan(total, offs, buckets, scratch);
+  first_wave_exclusive_scan(total, offs, buckets);
+  __syncthreads();
   if (blockIdx.x == 0) {
     for (int b = tid; b < buckets; b += blockDim.x) {
       if (b < E) {
@@ -575,7 +572,7 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
   const int n_seg = n_blocks * kRouteWaves;
   int *seg_counts = (int *)workspace;
   size_t lds_a = (size_t)kRouteWaves * buckets * sizeof(int);
-  size_t lds_b = ((size_t)buckets * 2 + 1 + kRouteWaves + 1) * sizeof(int);
+  size_t lds_b = ((size_t)buckets * 2 + 1) * sizeof(int);
   size_t lds_c = ((size_t)kRouteWaves * buckets + buckets) * sizeof(int);
   if (idx_i64)
     hipLaunchKernelGGL(route_hist_kernel<true>, dim3(n_blocks), dim3(kRouteThreads), lds_a, stream,
