@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "../../include/yamoe_hip.h"
 
@@ -116,13 +117,15 @@ __device__ inline void glu_backward(float G, float U, float dh, float &dG, float
 // forward, clamp away (a few elements in ten thousand, but each one wrong by its whole size).  `up`: the up half is
 // clamped on both sides, the gate half from above only.
 template <typename T> __device__ inline T pre_activation_store(float v, bool up) {
-  T r = ElemTraits<T>::from_f32(v);
   if constexpr (sizeof(T) == 2) {
-    const uint16_t lim = __builtin_bit_cast(uint16_t, ElemTraits<T>::from_f32(kGluLimit));  // (exactly representable)
-    uint16_t bits = __builtin_bit_cast(uint16_t, r);
-    if ((bits & 0x7fffu) == lim && (v > kGluLimit || (up && v < -kGluLimit))) r = __builtin_bit_cast(T, (uint16_t)(bits + 1));
+    // The next value of T above the limit (7 is exact, a step there is 2^-5 and 2^-8): what lies between the two becomes it,
+    // what lies beyond it rounds as it would.  (Rounding first and stepping the bits of a value that landed on the limit
+    // gives the same bits for twice the instructions.)
+    constexpr float kNext = std::is_same_v<T, bf16_t> ? 7.03125f : 7.00390625f;
+    if (up) v = fabsf(v) > kGluLimit ? copysignf(fmaxf(fabsf(v), kNext), v) : v;
+    else v = v > kGluLimit ? fmaxf(v, kNext) : v;
   }
-  return r;
+  return ElemTraits<T>::from_f32(v);
 }
 
 // 16 bytes per lane from global memory straight into LDS at lds_base + lane * 16.
