@@ -155,6 +155,28 @@ __device__ inline u32x2 lds_read_tr16(const char *p) {
   return __builtin_bit_cast(u32x2, v);
 }
 
+// ---- wave prefix sums ---------------------------------------------------------------------------------
+// Inclusive prefix sum over the 64 lanes by DPP moves: six additions whose operand comes from another lane of the row of 16,
+// from the last lane of the row before, and from lane 31, instead of six trips through the LDS crossbar each.
+template <int CTRL, int ROW_MASK> __device__ inline int dpp_or_zero(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
+}
+__device__ inline int wave_inclusive_scan(int x) {
+  x += dpp_or_zero<0x111, 0xf>(x);  // row_shr:1
+  x += dpp_or_zero<0x112, 0xf>(x);  // row_shr:2
+  x += dpp_or_zero<0x114, 0xf>(x);  // row_shr:4
+  x += dpp_or_zero<0x118, 0xf>(x);  // row_shr:8
+  x += dpp_or_zero<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
+  x += dpp_or_zero<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ inline int wave_exclusive_scan(int v, int &total) {
+  const int x = wave_inclusive_scan(v);
+  total = __builtin_amdgcn_readlane(x, kWave - 1);
+  return x - v;
+}
+__device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1); }
+
 // ---- schedule: device-built work lists shared by the expert GEMM kernels ---------------------
 // Layout of the schedule region (int32 words):
 //   [0] n_row_tiles   number of (expert, row-block) entries for the MFMA kernels

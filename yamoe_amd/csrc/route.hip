@@ -101,29 +101,10 @@ __device__ inline void wave_place(const void *idx, int seg_begin, int seg_end, i
   }
 }
 
-// Inclusive prefix sum over the 64 lanes by DPP moves: six additions whose operand comes from another lane of the row of 16,
-// from the last lane of the row before, and from lane 31, instead of six trips through the LDS crossbar each.  The routing
+// The routing
 // of a small batch is one chain of such scans, barriers and divisions; us before / with these scans, the bucket scan by one
 // wave, and no 64-bit division: 4 keys on 128 experts 8.0 / 4.6, 4096 on 16 12.9 / 9.5, 4004 on 128 15.8 / 10.9; two launches,
 // 12 288 on 64: 12.3 / 10.1 (the second); work lists of one expert's rows alone 8.4 / 5.0.
-template <int CTRL, int ROW_MASK> __device__ inline int dpp_or_zero(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xf, false);
-}
-__device__ inline int wave_inclusive_scan(int x) {
-  x += dpp_or_zero<0x111, 0xf>(x);  // row_shr:1
-  x += dpp_or_zero<0x112, 0xf>(x);  // row_shr:2
-  x += dpp_or_zero<0x114, 0xf>(x);  // row_shr:4
-  x += dpp_or_zero<0x118, 0xf>(x);  // row_shr:8
-  x += dpp_or_zero<0x142, 0xa>(x);  // row_bcast:15 into rows 1 and 3
-  x += dpp_or_zero<0x143, 0xc>(x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
-__device__ inline int wave_exclusive_scan(int v, int &total) {
-  const int x = wave_inclusive_scan(v);
-  total = __builtin_amdgcn_readlane(x, kWave - 1);
-  return x - v;
-}
-__device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_inclusive_scan(v), kWave - 1); }
 
 // Exclusive scan over buckets of `total` into `offsets` (both LDS), by the first wave of the workgroup; offsets[buckets] = N.
 // The caller puts a barrier on both sides.
