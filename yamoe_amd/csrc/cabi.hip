@@ -72,7 +72,7 @@ int gemm_async_gate_up(const void *, const int *, const void *, const void *, vo
                        int, int, int, int, bool, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, int,
-                    bool, hipStream_t);
+                    bool, int, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
                      const void *, float *, hipStream_t);
@@ -150,13 +150,14 @@ static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, co
     return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
   }
 }
+// regular_rows > 0 (16-bit data only): every expert has that many rows, and there is no schedule.
 template <typename T>
 static int tiles_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E,
-                      int H, int I, int small_rows, bool streams, hipStream_t stream) {
+                      int H, int I, int small_rows, bool streams, int regular_rows, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
     auto run = I % 64 ? gemm_async_down<T, 256, true> : gemm_async_down<T, 256, false>;
     if (takes_small_tiles(N, E, H)) run = I % 64 ? gemm_async_down<T, 128, true> : gemm_async_down<T, 128, false>;
-    return run(act, w, bias, y, sched, N, E, H, I, small_rows, streams, stream);
+    return run(act, w, bias, y, sched, N, E, H, I, small_rows, streams, regular_rows, stream);
   } else {
     return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
   }
@@ -394,7 +395,7 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   if constexpr (HasStreamPath<T>::value)
     if (!carried) YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I,
                                 stream));
-  if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, carried, stream));
+  if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, carried, 0, stream));
   if constexpr (HasStreamPath<T>::value)
     if (!carried) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream));
   YAMOE_TRY(launch_combine<T>(b.y_perm, b.inv_pos, idx, p->idx_i64, rw, p->rw_cols, out, p->T, p->K, p->E, p->H,
@@ -570,21 +571,22 @@ static int gate_up_both(const void *x, const int *sorted_idx, const void *w, con
 template <typename T>
 static int down_both(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
                      int I, hipStream_t stream) {
-  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, false, stream));
+  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, false, 0, stream));
   if constexpr (HasStreamPath<T>::value) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, stream));
   return 0;
 }
-// The same for E groups of `rows` rows each (the work list of yamoe_build_schedule for them is made here, with counts and
-// offsets): whether they stream or are tiles is known on the host, so only one of the two kernels is launched (the other
-// would find an empty list for 4 us).
+// The same for E groups of `rows` rows each: whether they stream or are tiles is known on the host, so only one of the two
+// kernels is launched (the other would find an empty list for 4 us), and 16-bit tiles need no work list (a launch of 3.5 to 5
+// us, which is what the list of yamoe_build_schedule, counts and offsets take where they are made).
 template <typename T>
 static int down_regular(const void *act, const void *w, const void *bias, void *y, int *counts, int *offsets, void *sched,
                         size_t sched_bytes, int E, int rows, int H, int I, hipStream_t stream) {
   const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
+  if (HasStreamPath<T>::value && rows > stream_rows)
+    return tiles_down<T>(act, w, bias, y, nullptr, E * rows, E, H, I, stream_rows, false, rows, stream);
   YAMOE_TRY(regular_schedule(counts, offsets, E, rows, stream_rows, sched, sched_bytes, stream));
-  if constexpr (HasStreamPath<T>::value)
-    if (rows <= stream_rows) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream);
-  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, false, stream);
+  if constexpr (HasStreamPath<T>::value) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream);
+  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, false, 0, stream);
 }
 
 extern "C" int yamoe_gate_up(const void *x, const int32_t *sorted_idx, const void *gate_up_proj,

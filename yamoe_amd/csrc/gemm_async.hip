@@ -43,7 +43,7 @@ int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, cons
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
-                    int I, int small_rows, bool streams, hipStream_t stream) {
+                    int I, int small_rows, bool streams, int regular_rows, hipStream_t stream) {
   async::Args a = {};
   a.A = act; a.B = w; a.bias = bias; a.C = y; a.sched = (const int *)sched;
   a.Kd = I; a.Nd = H; a.lda = I; a.ldb = H; a.ldc = H;
@@ -52,7 +52,17 @@ int gemm_async_down(const void *act, const void *w, const void *bias, void *y, c
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
   if (streams) add_streams(a, N, E);
-  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
+  int row_tiles = sched_grid_row_tiles(N, E, small_rows);
+  if (regular_rows > 0) {  // cut like the schedule's: equal tiles, multiples of 32 rows
+    a.reg_rows = regular_rows;
+    a.reg_tiles = ceil_div(regular_rows, kRowTile);
+    a.reg_per_tile = (ceil_div(regular_rows, a.reg_tiles) + 31) & ~31;
+    a.reg_units = E * a.n_col_tiles;
+    a.reg_div = make_fast_div(a.reg_tiles * a.n_col_tiles);
+    a.reg_tile_div = make_fast_div(a.reg_tiles);
+    row_tiles = E * a.reg_tiles;
+  }
+  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, false, RAGGED>(a, row_tiles, stream);
 }
 
 // C[rows, Nd] = A[rows, Kd] * W[e]^T with W[e] stored [Nd, Kd]: the input gradients of both projections
@@ -78,7 +88,7 @@ int gemm_async_dgrad(const void *g, const int *g_rows, int g_div, const void *w,
   template int gemm_async_gate_up<T, TILE, RAGGED>(const void *, const int *, const void *, const void *, void *,       \
                                                    void *, const void *, int, int, int, int, int, int, bool, hipStream_t);    \
   template int gemm_async_down<T, TILE, RAGGED>(const void *, const void *, const void *, void *, const void *, int,    \
-                                                int, int, int, int, bool, hipStream_t);                                       \
+                                                int, int, int, int, bool, int, hipStream_t);                                  \
   template int gemm_async_dgrad<T, TILE, RAGGED>(const void *, const int *, int, const void *, void *, const void *,    \
                                                  int, int, int, int, const void *, float *, hipStream_t);
 #ifndef YAMOE_INSTANTIATE_ROWS

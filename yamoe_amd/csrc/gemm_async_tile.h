@@ -104,6 +104,10 @@ struct Args {
   // launch (0: by launches of their own)
   const int *small;
   int stream_wgs, n_stream_slabs;
+  // a regular layout (every expert has reg_rows rows, cut into reg_tiles tiles of reg_per_tile) needs no schedule: reg_units =
+  // experts times column tiles, reg_div and reg_tile_div divide by an expert's tiles of all columns and of one
+  int reg_rows, reg_tiles, reg_per_tile, reg_units;
+  FastDiv reg_div, reg_tile_div;
 #ifdef YAMOE_TILE_STAMPS
   unsigned long long *stamps;  // [stamps_cap][8]: see yamoe_debug_tile_stamps
   int stamps_cap;
@@ -708,11 +712,15 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
 #endif
   int L;
   const int place = blockIdx.x / kXcds;
+  const bool regular = args.reg_rows > 0;
+  auto cut_of = [&](int x) {
+    return regular ? (int)((long long)x * args.reg_units / kXcds) * args.reg_tiles : sched_cut(args.sched, x, args.n_col_tiles);
+  };
   {
     const int xcd = blockIdx.x % kXcds;
-    const int first = sched_cut(args.sched, xcd, args.n_col_tiles);
-    const int count = sched_cut(args.sched, xcd + 1, args.n_col_tiles) - first;
-    const int rounds = ceil_div(sched_cut_row_tiles(args.sched, xcd) * args.n_col_tiles, kXcds * kXcdCus);
+    const int first = cut_of(xcd), count = cut_of(xcd + 1) - first;
+    const int total = regular ? args.reg_units * args.reg_tiles : sched_cut_row_tiles(args.sched, xcd) * args.n_col_tiles;
+    const int rounds = ceil_div(total, kXcds * kXcdCus);
     if constexpr (!BNK) {
       if (args.stream_wgs > 0) {
         const int places = gridDim.x / kXcds;
@@ -732,7 +740,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     } else {
       int cut[kXcds + 1];
 #pragma unroll
-      for (int x = 0; x <= kXcds; ++x) cut[x] = sched_cut(args.sched, x, args.n_col_tiles);
+      for (int x = 0; x <= kXcds; ++x) cut[x] = cut_of(x);
       int rank = i - count;  // rank of this workgroup among the idle ones
 #pragma unroll
       for (int x = 0; x < kXcds; ++x)
@@ -752,11 +760,21 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
   TileInfo ti;
   {
     const int *tiles = args.sched + kSchedHeader;
-    int t0 = fast_div(L, args.n_col_div);
-    int gfirst = __builtin_amdgcn_readfirstlane(tiles[8 * t0 + 3]), gcount = __builtin_amdgcn_readfirstlane(tiles[8 * t0 + 4]);
-    FastDiv by_gcount = {(uint32_t)__builtin_amdgcn_readfirstlane(tiles[8 * t0 + 5]),
-                         (uint32_t)__builtin_amdgcn_readfirstlane(tiles[8 * t0 + 6])};
-    int local = L - gfirst * args.n_col_tiles;
+    int gfirst, gcount, local;
+    FastDiv by_gcount;
+    if (regular) {
+      gfirst = fast_div(L, args.reg_div);  // (the expert: it has no tiles in a list)
+      gcount = args.reg_tiles;
+      by_gcount = args.reg_tile_div;
+      local = L - gfirst * gcount * args.n_col_tiles;
+    } else {
+      const int t0 = fast_div(L, args.n_col_div);
+      gfirst = __builtin_amdgcn_readfirstlane(tiles[8 * t0 + 3]);
+      gcount = __builtin_amdgcn_readfirstlane(tiles[8 * t0 + 4]);
+      by_gcount = {(uint32_t)__builtin_amdgcn_readfirstlane(tiles[8 * t0 + 5]),
+                   (uint32_t)__builtin_amdgcn_readfirstlane(tiles[8 * t0 + 6])};
+      local = L - gfirst * args.n_col_tiles;
+    }
     int col_tile, row_tile;
     if (gcount < 2 * kBandRows) {
       // the expert's tiles column by column: its few row tiles follow each other and share the column's weight slabs
@@ -777,12 +795,21 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
       col_tile = (int)((uint32_t)in_band / (uint32_t)band_rows);
       row_tile = band * kBandRows + in_band - col_tile * band_rows;
     }
-    const int *te = tiles + 8 * (gfirst + row_tile);
     // (the same for every lane; said explicitly, so that the operand addresses built from them stay in scalar registers
     // whatever the compiler can prove about the work list's memory)
-    ti.expert = __builtin_amdgcn_readfirstlane(te[0]);
-    ti.row0 = __builtin_amdgcn_readfirstlane(te[1]);
-    ti.rows_valid = __builtin_amdgcn_readfirstlane(te[2]);
+    if (regular) {
+      ti.expert = gfirst;
+      ti.row0 = gfirst * args.reg_rows + row_tile * args.reg_per_tile;
+      ti.rows_valid = min(args.reg_per_tile, args.reg_rows - row_tile * args.reg_per_tile);
+    } else {
+      const int *te = tiles + 8 * (gfirst + row_tile);
+      ti.expert = te[0];
+      ti.row0 = te[1];
+      ti.rows_valid = te[2];
+    }
+    ti.expert = __builtin_amdgcn_readfirstlane(ti.expert);
+    ti.row0 = __builtin_amdgcn_readfirstlane(ti.row0);
+    ti.rows_valid = __builtin_amdgcn_readfirstlane(ti.rows_valid);
     if constexpr (S::kParts == 2) {
       // The row tile's two halves are neighbours in the grid, on one XCD.  More than 128 rows are cut into two parts of
       // whole 32-row blocks as equal as they get; up to 128 rows are one part, and the other workgroup has nothing to do.
