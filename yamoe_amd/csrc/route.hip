@@ -47,14 +47,39 @@ __device__ inline int bits_for(int buckets) {
   return b;
 }
 
-// Histogram of one wave's segment [seg_begin, seg_end) into `hist` (LDS or global, zeroed by caller).
+// Histogram of one wave's segment [seg_begin, seg_end) into `hist_lds` (zeroed by the caller), four loads on their way.
 template <bool I64>
 __device__ inline void wave_histogram(const void *idx, int seg_begin, int seg_end, int E,
                                       int *hist_lds) {
   const int lane = threadIdx.x & (kWave - 1);
-  for (int i = seg_begin + lane; i < seg_end; i += kWave) {
-    int key = load_key<I64>(idx, i, E);
-    atomicAdd(&hist_lds[key], 1);
+  for (int base = seg_begin; base < seg_end; base += 4 * kWave) {
+    int key[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) key[u] = load_key<I64>(idx, min(base + u * kWave + lane, seg_end - 1), E);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (base + u * kWave + lane < seg_end) atomicAdd(&hist_lds[key[u]], 1);
+  }
+}
+
+// The first kAhead steps of a wave's segment (a whole segment of 256 keys), requested before the table that their placement
+// has to wait for: 12 288 keys on 64 experts 10.1 -> 8.8 us, 65 536 on 128 (the first half of each segment) 22 -> 20.3.
+constexpr int kAhead = 4;
+struct KeysAhead {
+  int raw[kAhead];
+  bool bad[kAhead];
+};
+template <bool I64> __device__ inline void load_ahead(const void *idx, int seg_begin, int seg_end, int E, KeysAhead &k) {
+  const int lane = threadIdx.x & (kWave - 1);
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) {
+    const int i = min(seg_begin + u * kWave + lane, seg_end - 1);
+    k.raw[u] = 0;
+    k.bad[u] = false;
+    if (seg_begin < seg_end) {  // (an empty segment may lie behind the last key)
+      k.raw[u] = load_raw<I64>(idx, i);
+      k.bad[u] = load_key<I64>(idx, i, E) == E;
+    }
   }
 }
 
@@ -63,24 +88,15 @@ __device__ inline void wave_histogram(const void *idx, int seg_begin, int seg_en
 template <bool I64>
 __device__ inline void wave_place(const void *idx, int seg_begin, int seg_end, int E, int capacity,
                                   int *cursor, const int *offsets_lds,
-                                  int *sorted_expert, int *sorted_idx, int *inv_pos) {
+                                  int *sorted_expert, int *sorted_idx, int *inv_pos, const KeysAhead &ahead) {
   const int lane = threadIdx.x & (kWave - 1);
   const int key_bits = bits_for(E + 1);
   const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  // the raw id of the next step is fetched one step ahead so that its latency hides behind this step
-  int raw_next = (seg_begin + lane < seg_end) ? load_raw<I64>(idx, seg_begin + lane) : 0;
-  bool bad_next = (seg_begin + lane < seg_end) ? (load_key<I64>(idx, seg_begin + lane, E) == E) : false;
-  for (int base = seg_begin; base < seg_end; base += kWave) {
-    int i = base + lane;
-    bool active = i < seg_end;
-    int raw = raw_next;
-    int key = bad_next ? E : raw;
+  auto place = [&](int base, int raw, bool bad) {
+    const int i = base + lane;
+    const bool active = i < seg_end;
+    int key = bad ? E : raw;
     if (!active) key = 0;
-    int in = i + kWave;
-    if (in < seg_end) {
-      raw_next = load_raw<I64>(idx, in);
-      bad_next = load_key<I64>(idx, in, E) == E;
-    }
     uint64_t peers = match_key(key, active, key_bits);
     int rank = __popcll(peers & lt_mask);
     int start = 0;
@@ -98,6 +114,22 @@ __device__ inline void wave_place(const void *idx, int seg_begin, int seg_end, i
     // read sees this step's write without a fence or a volatile access (both would also wait for the global
     // stores above); lanes address the cursor by key, so the compiler cannot carry its values across steps
     __builtin_amdgcn_wave_barrier();
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+    if (seg_begin + u * kWave < seg_end) place(seg_begin + u * kWave, ahead.raw[u], ahead.bad[u]);
+  // the raw id of the next step is fetched one step ahead so that its latency hides behind this step
+  int base = seg_begin + kAhead * kWave;
+  int raw_next = (base + lane < seg_end) ? load_raw<I64>(idx, base + lane) : 0;
+  bool bad_next = (base + lane < seg_end) ? (load_key<I64>(idx, base + lane, E) == E) : false;
+  for (; base < seg_end; base += kWave) {
+    const int raw = raw_next, in = base + lane + kWave;
+    const bool bad = bad_next;
+    if (in < seg_end) {
+      raw_next = load_raw<I64>(idx, in);
+      bad_next = load_key<I64>(idx, in, E) == E;
+    }
+    place(base, raw, bad);
   }
 }
 
@@ -411,14 +443,16 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
   }
   int *cursor = lds + wave * buckets;
   int *offs = lds + kRouteWaves * buckets;
+  int s = blockIdx.x * kRouteWaves + wave;
+  int seg_begin = min((long long)s * seg, (long long)N), seg_end = min(seg_begin + seg, N);
+  KeysAhead ahead;
+  load_ahead<I64>(idx, seg_begin, seg_end, E, ahead);
   for (int i = tid; i < kRouteWaves * buckets; i += blockDim.x)
     lds[i] = seg_cursors[(size_t)blockIdx.x * kRouteWaves * buckets + i];
   for (int b = tid; b <= E; b += blockDim.x) offs[b] = offsets_in[b];
   __syncthreads();
-  int s = blockIdx.x * kRouteWaves + wave;
-  int seg_begin = min((long long)s * seg, (long long)N), seg_end = min(seg_begin + seg, N);
   wave_place<I64>(idx, seg_begin, seg_end, E, capacity, cursor, offs, sorted_expert, sorted_idx,
-                  inv_pos);
+                  inv_pos, ahead);
 }
 
 // ---- two-kernel form: every workgroup of the placement scans the table for itself -----------------------------
@@ -444,6 +478,10 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
   int *table = cursors + kRouteWaves * buckets;  // [n_seg][buckets]
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   const int cells = n_seg * buckets;
+  const int sgm = blockIdx.x * kRouteWaves + wave;
+  const int seg_begin = (int)min((long long)sgm * seg, (long long)N), seg_end = min(seg_begin + seg, N);
+  KeysAhead ahead;  // (the extra workgroup's segments are empty)
+  load_ahead<I64>(idx, seg_begin, seg_end, E, ahead);
   for (int i = tid; i < cells; i += blockDim.x) table[i] = seg_counts[i];
   __syncthreads();
   const int my_first = blockIdx.x * kRouteWaves;  // this workgroup's segments: my_first + 0..15 (none for the extra one)
@@ -478,9 +516,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
   }
   for (int i = tid; i < kRouteWaves * buckets; i += blockDim.x) cursors[i] += offs[i % buckets];
   __syncthreads();
-  const int sgm = my_first + wave;
-  const int seg_begin = (int)min((long long)sgm * seg, (long long)N), seg_end = min(seg_begin + seg, N);
-  wave_place<I64>(idx, seg_begin, seg_end, E, capacity, cursors + wave * buckets, offs, sorted_expert, sorted_idx, inv_pos);
+  wave_place<I64>(idx, seg_begin, seg_end, E, capacity, cursors + wave * buckets, offs, sorted_expert, sorted_idx, inv_pos, ahead);
 }
 
 }  // namespace yamoe
