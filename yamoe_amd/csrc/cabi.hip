@@ -414,7 +414,6 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   const int N = p->T * p->K, E = p->E, H = p->H, I = p->I, cap = p->capacity < 0 ? 0 : p->capacity;
   const size_t es = sizeof(T);
   void *st = (void *)stream;
-  YAMOE_TRY(fill_zero(d_rw, (size_t)p->T * p->rw_cols * es, stream));
   if (N == 0) {
     YAMOE_TRY(fill_zero(d_wgu, (size_t)E * H * 2 * I * es, stream));
     YAMOE_TRY(fill_zero(d_bgu, (size_t)E * 2 * I * es, stream));
