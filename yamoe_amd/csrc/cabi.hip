@@ -381,8 +381,10 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
                                b.inv_pos, b.route_ws, b.route_ws_bytes, everything ? kStreamEverything : stream_rows,
                                b.schedule, b.schedule_bytes, st));
-  // with no more assignments than a streamed expert may have rows, every expert is streamed as well
-  const bool tiles = !everything && N > stream_rows;
+  // where the assignments or the capacity leave no expert more rows than a streamed one may have, every expert is streamed as
+  // well.  1723 tokens on 8 experts of 2048 x 2048, 32 rows kept: 60 us; with two tile launches that find no tile in front 68,
+  // carried by those 72.
+  const bool tiles = !everything && N > stream_rows && p->capacity > stream_rows;
   const bool carried = HasStreamPath<T>::value && tiles && tiles_carry_streams(N, p->E, p->H, p->I);
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
