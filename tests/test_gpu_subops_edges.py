@@ -38,3 +38,17 @@ def test_scatter_index_forms(gpu, T, K, E):
     torch.cuda.synchronize()
     want = O.padded_scatter(src, pos, bins, w, y0, T, E, C, K)
     assert report("scatter", y.cpu().double(), want, REL_L2_TOL[torch.float32]) < REL_L2_TOL[torch.float32]
+
+
+@pytest.mark.parametrize("n,out_len", [(2**31 - 4096, 3), (2**31 - 4095, 3), (2**31 - 2000, 3), (2**31 - 1, 3), (5, 2**31 - 1)])
+def test_bincount_near_the_largest_size(gpu, n, out_len):
+    """Sizes whose last step of loads or stores ends beyond 2^31 - 1."""
+    import yamoe_amd
+    print("bincount", n, out_len, flush=True)
+    v = torch.zeros(n, dtype=torch.int32, device=gpu)
+    v[-1], v[n // 2] = 1, -1
+    out = torch.full((out_len,), 7, dtype=torch.int32, device=gpu)
+    yamoe_amd.bincount_cumsum(v, out, 3)
+    torch.cuda.synchronize()
+    assert out[:3].tolist() == [n - 2, n - 1, n - 1]
+    assert not out[3:].any()

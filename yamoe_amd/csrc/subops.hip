@@ -240,12 +240,13 @@ __global__ __launch_bounds__(1024) void bincount_cumsum_kernel(const int *in, in
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
   for (int i = tid; i < minlength; i += blockDim.x) hist[i] = 0;
   __syncthreads();
-  for (int i0 = 0; i0 < n; i0 += 4 * blockDim.x) {  // four loads on their way
+  const unsigned count = n;  // (positions are unsigned: the last step's end passes 2^31 - 1 for an n just below it)
+  for (unsigned i0 = 0; i0 < count; i0 += 4 * blockDim.x) {  // four loads on their way
     int bin[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int i = i0 + u * blockDim.x + tid;
-      bin[u] = i < n ? in[i] : -1;
+      const unsigned i = i0 + u * blockDim.x + tid;
+      bin[u] = i < count ? in[i] : -1;
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -273,7 +274,7 @@ __global__ __launch_bounds__(1024) void bincount_cumsum_kernel(const int *in, in
     if (i < minlength) out[i] = before + sum;
     __syncthreads();
   }
-  for (int i = minlength + tid; i < out_len; i += blockDim.x) out[i] = 0;
+  for (unsigned i = minlength + tid; i < (unsigned)out_len; i += blockDim.x) out[i] = 0;
 }
 
 // ---- padded gather (csrc/gather.cu:6-109): out[e,i,:] = x[idx[start_e+i] / top_k,:] or 0 -----------------
