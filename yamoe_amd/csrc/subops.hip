@@ -251,6 +251,7 @@ __global__ __launch_bounds__(1024) void bincount_cumsum_kernel(const int *in, in
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       // sorted input: the 64 values of a wave are usually the same one, which would be 64 additions in a row to one address
+      if (u > 0 && i0 + u * blockDim.x >= count) break;
       const int first = __builtin_amdgcn_readfirstlane(bin[u]);
       const bool one = __all(bin[u] == first);
       if (bin[u] >= 0 && bin[u] < minlength && (!one || lane == 0)) atomicAdd(&hist[bin[u]], one ? kWave : 1);
@@ -258,8 +259,14 @@ __global__ __launch_bounds__(1024) void bincount_cumsum_kernel(const int *in, in
   }
   __syncthreads();
   // inclusive prefix sums, 1024 bins at a time: within the wave, then over the waves
+  if (minlength <= kWave) {  // (one wave has them all)
+    if (wave == 0) {
+      const int sum = wave_inclusive_scan(lane < minlength ? hist[lane] : 0);
+      if (lane < minlength) out[lane] = sum;
+    }
+  }
   int carry = 0;
-  for (int base = 0; base < minlength; base += blockDim.x) {
+  for (int base = minlength <= kWave ? minlength : 0; base < minlength; base += blockDim.x) {
     const int i = base + tid;
     const int sum = wave_inclusive_scan(i < minlength ? hist[i] : 0);
     if (lane == kWave - 1) wave_total[wave] = sum;
