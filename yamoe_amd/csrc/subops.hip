@@ -86,7 +86,7 @@ __device__ inline void sort_place_segment(const K *keys, const K *vals, bool iot
     if constexpr (AHEAD) {
       key = active ? next_key : (K)0;
       val = active ? next_val : (K)0;
-      fetch(i + kWave);
+      if (base + kWave < e) fetch(i + kWave);
     } else {
       key = active ? keys[i] : (K)0;
       val = active ? (iota_vals ? (K)i : vals[i]) : (K)0;
@@ -147,7 +147,8 @@ __global__ __launch_bounds__(kSortThreads) void sort_block_kernel(const K *keys,
   for (int i0 = b; i0 < e; i0 += 4 * kWave) {  // four loads on their way (positions past the end: the last key, not counted)
     std::conditional_t<sizeof(K) == 2, int, K> k[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) k[u] = keys[min(i0 + u * kWave + lane, n - 1)];
+    for (int u = 0; u < 4; ++u)
+      if (u == 0 || i0 + u * kWave < e) k[u] = keys[min(i0 + u * kWave + lane, n - 1)];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
       if (i0 + u * kWave + lane < e) atomicAdd(&cursor[digit_of((K)k[u], shift, bits, flip_sign)], 1);
