@@ -25,6 +25,12 @@ CASES = [
     (32768, 64, 500, torch.int64, False),
     (32769, 64, 500, torch.int32, True),
     (131073, 9, 20000, torch.int64, True),
+    # tables too large for LDS (64 buckets a wave, the segments in 16, 8, 5, 3 and 1 stretches)
+    (1310721, 63, 30000, torch.int32, True),
+    (1310720, 64, 30000, torch.int64, False),
+    (700001, 191, 3000, torch.int32, True),
+    (250000, 320, 900, torch.int64, True),
+    (33000, 767, 50, torch.int32, True),
 ]
 
 
