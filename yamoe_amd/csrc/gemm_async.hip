@@ -37,8 +37,11 @@ int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, cons
   a.n_col_tiles = ceil_div(2 * I, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  if (streams) add_streams(a, N, E);
-  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_GLU, true, false, RAGGED>(a, sched_grid_row_tiles(N, E, small_rows), stream);
+  const int row_tiles = sched_grid_row_tiles(N, E, small_rows);
+  using S = async::Tile<TILE, TILE>;
+  if (!streams) return async::launch<T, S, async::EPI_GLU, true, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
+  add_streams(a, N, E);
+  return async::launch<T, S, async::EPI_GLU, true, false, RAGGED, async::FORM_CARRIER>(a, row_tiles, stream);
 }
 
 template <typename T, int TILE, bool RAGGED>
@@ -51,8 +54,7 @@ int gemm_async_down(const void *act, const void *w, const void *bias, void *y, c
   a.n_col_tiles = ceil_div(H, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  if (streams) add_streams(a, N, E);
-  int row_tiles = sched_grid_row_tiles(N, E, small_rows);
+  using S = async::Tile<TILE, TILE>;
   if (regular_rows > 0) {  // cut like the schedule's: equal tiles, multiples of 32 rows
     a.reg_rows = regular_rows;
     a.reg_tiles = ceil_div(regular_rows, kRowTile);
@@ -60,9 +62,12 @@ int gemm_async_down(const void *act, const void *w, const void *bias, void *y, c
     a.reg_units = E * a.n_col_tiles;
     a.reg_div = make_fast_div(a.reg_tiles * a.n_col_tiles);
     a.reg_tile_div = make_fast_div(a.reg_tiles);
-    row_tiles = E * a.reg_tiles;
+    return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_REGULAR>(a, E * a.reg_tiles, stream);
   }
-  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, false, RAGGED>(a, row_tiles, stream);
+  const int row_tiles = sched_grid_row_tiles(N, E, small_rows);
+  if (!streams) return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
+  add_streams(a, N, E);
+  return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_CARRIER>(a, row_tiles, stream);
 }
 
 // C[rows, Nd] = A[rows, Kd] * W[e]^T with W[e] stored [Nd, Kd]: the input gradients of both projections
@@ -80,8 +85,10 @@ int gemm_async_dgrad(const void *g, const int *g_rows, int g_div, const void *w,
   a.n_col_tiles = ceil_div(Nd, TILE);
   a.n_col_div = make_fast_div(a.n_col_tiles);
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
-  if (g_rows != nullptr) return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, true, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
-  return async::launch<T, async::Tile<TILE, TILE>, async::EPI_STORE, false, true, RAGGED>(a, sched_max_row_tiles(N, E), stream);
+  using S = async::Tile<TILE, TILE>;
+  if (g_rows != nullptr)
+    return async::launch<T, S, async::EPI_STORE, true, true, RAGGED, async::FORM_LIST>(a, sched_max_row_tiles(N, E), stream);
+  return async::launch<T, S, async::EPI_STORE, false, true, RAGGED, async::FORM_LIST>(a, sched_max_row_tiles(N, E), stream);
 }
 
 #define YAMOE_INSTANTIATE_ASYNC(T, TILE, RAGGED)                                                                        \

@@ -100,12 +100,11 @@ struct Args {
   // row times dot_with[row][same columns] (a [rows, ldc] tensor), summed over the wave column's half of the tile
   const void *dot_with;
   float *dot_part;
-  // forward products, optional: the schedule's streaming list is worked off by stream_wgs workgroups of every XCD in this
-  // launch (0: by launches of their own)
+  // FORM_CARRIER: the schedule's streaming list is worked off by stream_wgs workgroups of every XCD in this launch
   const int *small;
   int stream_wgs, n_stream_slabs;
-  // a regular layout (every expert has reg_rows rows, cut into reg_tiles tiles of reg_per_tile) needs no schedule: reg_units =
-  // experts times column tiles, reg_div and reg_tile_div divide by an expert's tiles of all columns and of one
+  // FORM_REGULAR: every expert has reg_rows rows, cut into reg_tiles tiles of reg_per_tile; reg_units = experts times column
+  // tiles, reg_div and reg_tile_div divide by an expert's tiles of all columns and of one
   int reg_rows, reg_tiles, reg_per_tile, reg_units;
   FastDiv reg_div, reg_tile_div;
 #ifdef YAMOE_TILE_STAMPS
@@ -693,7 +692,18 @@ template <typename T, int EPI, bool GATHER, int DEPTH> __device__ __forceinline_
   }
 }
 
-template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED>
+// Where a launch's work comes from.  Instantiations of their own, because all forms in one kernel, told apart at run time, leave
+// it short of scalar registers (19 to 42 spilled, none with the list alone): the gate_up product of 67 600 rows on 128 experts
+// (Zipf routing, 720 x 5760, 29 rounds of tiles with a short contraction) took 744 us instead of 727.  150 drawn calls that carry
+// streamed experts 0.993 in the mean, single ones 0.94 to 1.09: where their workgroups meet tiles on a CU changes with
+// the time at which idle workgroups leave.
+enum {
+  FORM_LIST = 0,     // the schedule's row tiles
+  FORM_CARRIER = 1,  // these and the schedule's streaming list, by stream_wgs workgroups of every XCD
+  FORM_REGULAR = 2,  // every expert has reg_rows rows: no schedule
+};
+
+template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED, int FORM>
 __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const Args args) {
   constexpr int kBN = S::BN;
 
@@ -712,7 +722,8 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
 #endif
   int L;
   const int place = blockIdx.x / kXcds;
-  const bool regular = args.reg_rows > 0;
+  constexpr bool regular = FORM == FORM_REGULAR;
+  const int stream_wgs = FORM == FORM_CARRIER ? args.stream_wgs : 0;
   auto cut_of = [&](int x) {
     return regular ? (int)((long long)x * args.reg_units / kXcds) * args.reg_tiles : sched_cut(args.sched, x, args.n_col_tiles);
   };
@@ -721,18 +732,15 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     const int first = cut_of(xcd), count = cut_of(xcd + 1) - first;
     const int total = regular ? args.reg_units * args.reg_tiles : sched_cut_row_tiles(args.sched, xcd) * args.n_col_tiles;
     const int rounds = ceil_div(total, kXcds * kXcdCus);
-    if constexpr (!BNK) {
-      if (args.stream_wgs > 0) {
-        const int places = gridDim.x / kXcds;
-        const int k = place - (places - args.stream_wgs);  // behind the tiles
-        if (k >= 0) {
-          stream_items<T, EPI, GATHER, S::kPerSimd == 1 ? 3 : 2>(args, k * kXcds + xcd, args.stream_wgs * kXcds);
-          return;
-        }
+    if constexpr (FORM == FORM_CARRIER) {
+      const int k = place - (int)(gridDim.x / kXcds - stream_wgs);  // behind the tiles
+      if (k >= 0) {
+        stream_items<T, EPI, GATHER, S::kPerSimd == 1 ? 3 : 2>(args, k * kXcds + xcd, stream_wgs * kXcds);
+        return;
       }
     }
     const int i = place / S::kParts;
-    int slots = (gridDim.x / kXcds - (BNK ? 0 : args.stream_wgs)) / S::kParts;
+    int slots = (gridDim.x / kXcds - stream_wgs) / S::kParts;
     if (rounds <= kMostRounds) slots = min(slots, rounds * kXcdCus);
     if (i >= slots) return;
     if (i < count) {
@@ -762,7 +770,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     const int *tiles = args.sched + kSchedHeader;
     int gfirst, gcount, local;
     FastDiv by_gcount;
-    if (regular) {
+    if constexpr (regular) {
       gfirst = fast_div(L, args.reg_div);  // (the expert: it has no tiles in a list)
       gcount = args.reg_tiles;
       by_gcount = args.reg_tile_div;
@@ -797,7 +805,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     }
     // (the same for every lane; said explicitly, so that the operand addresses built from them stay in scalar registers
     // whatever the compiler can prove about the work list's memory)
-    if (regular) {
+    if constexpr (regular) {
       ti.expert = gfirst;
       ti.row0 = gfirst * args.reg_rows + row_tile * args.reg_per_tile;
       ti.rows_valid = min(args.reg_per_tile, args.reg_rows - row_tile * args.reg_per_tile);
@@ -919,9 +927,9 @@ static unsigned long long *g_tile_stamps = nullptr;
 static int g_tile_stamps_cap = 0;
 #endif
 
-template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED>
+template <typename T, class S, int EPI, bool GATHER, bool BNK, bool RAGGED, int FORM>
 static int launch(const Args &args, int max_row_tiles, hipStream_t stream) {
-  auto kernel = gemm_async_kernel<T, S, EPI, GATHER, BNK, RAGGED>;
+  auto kernel = gemm_async_kernel<T, S, EPI, GATHER, BNK, RAGGED, FORM>;
   constexpr int lds_bytes = BNK ? S::kLdsNk : S::kLds;
   static DeviceFlags attr_done;  // one per kernel instantiation
   if (int rc = ensure_dynamic_lds((const void *)kernel, lds_bytes, attr_done, "gemm_async_kernel")) return rc;
