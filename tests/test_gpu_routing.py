@@ -176,8 +176,9 @@ def test_schedule_lists(gpu, N, E, C, stream_rows):
     for n_col in (1, 12, 23):
         cuts = []
         for x in range(9):
-            first, frac, _, cnt = sched[8 + 4 * x:12 + 4 * x].tolist()
+            first, frac, all_tiles, cnt = sched[8 + 4 * x:12 + 4 * x].tolist()
             assert 0 <= frac < 65536
+            assert x == 8 or all_tiles == len(want_tiles)  # which places of an XCD have a tile depends on it
             cuts.append(first * n_col + ((frac * n_col) >> 16) * cnt)
         assert cuts[0] == 0 and cuts[8] == len(want_tiles) * n_col
         assert all(a <= b for a, b in zip(cuts, cuts[1:]))
