@@ -23,7 +23,8 @@ def test_bincount_of_sorted_values(gpu, n, bins):
     assert np.array_equal(out.cpu().numpy(), O.bincount_cumsum(v, bins + 3, bins))
 
 
-@pytest.mark.parametrize("T,K,E", [(1536, 4, 8), (1537, 4, 8), (2048, 3, 1024), (700, 2, 1025), (4000, 2, 1100)])
+@pytest.mark.parametrize("T,K,E", [(1536, 4, 8), (1537, 4, 8), (2048, 3, 1024), (700, 2, 1025), (4000, 2, 1100),
+                                   (1280, 4, 32), (1707, 3, 32), (1024, 4, 33), (4097, 1, 1024), (1024, 2, 1025), (683, 3, 1025)])
 def test_scatter_index_forms(gpu, T, K, E):
     import yamoe_amd
     H, C = 8, T * K // E + 2

@@ -17,10 +17,14 @@ constexpr int kSortWaves = kSortThreads / kWave;
 constexpr int kSortSeg = 1024;  // elements per wave segment
 constexpr int kRadix = 256;
 constexpr int kScatterWaves = 16 * 256;    // waves that keep HBM busy in the scatter
-// Slots that one workgroup indexes in one launch; beyond, a clearing launch and a grid.  Whole scatter, 1024 wide, us, one
-// workgroup / grid: 5000 slots of 8 experts 10.0 / 11.3, 6144 of 8 10.5 / 11.1, of 128 12.2 / 11.1, 8000 13.0 / 11.1 and 14.9 / 11.7,
-// 16384 24.3 / 12.8 and 29.8 / 14.0.
-constexpr int kScatterOneBlock = 6144;
+// Slots that one workgroup indexes in one launch; beyond, a clearing launch and a grid.  Whole scatter, 1024 wide, bf16, us, one
+// workgroup / grid, where launches queue up (or are replayed) and where each waits for the host: 4096 slots of 32 experts 9.2 / 7.9
+// and 10.1 / 12.8, 5120 10.6 / 8.4 and 11.3 / 13.1, 6144 11.8 / 8.8 and 12.3 / 13.2; 4096 of 128 9.7 / 8.1 and 10.5 / 13.0, 5120
+// 11.2 / 8.5 and 11.8 / 12.7, 6144 12.7 / 9.1 and 13.1 / 12.8; with the bins in global memory (2000 experts) 2048 9.0 / 8.0 and 9.7 /
+// 12.6, 3072 11.8 / 8.7 and 12.2 / 12.9.  The search for a slot's expert takes longer the more there are, so the lines, where one
+// caller's loss comes up to the other's gain, do too.
+constexpr int kScatterLdsBins = 1024;  // up to this many experts the search for a position's expert runs in LDS
+static int scatter_one_block(int E) { return E <= 32 ? 5120 : E <= kScatterLdsBins ? 4096 : 2048; }
 
 template <typename K>
 __device__ inline unsigned digit_of(K key, int shift, int bits, bool flip_sign) {
@@ -320,7 +324,6 @@ __global__ __launch_bounds__(256) void padded_gather_kernel(const T *x, const in
 // waves own an output row and add that token's rows in slot order.
 // slots[flat] = {padded row, sorted position} of every flat slot, {-1, -1} for slots without a row.  With few slots one
 // workgroup clears and fills them in one launch; `clear` is false where scatter_clear_kernel has run before.
-constexpr int kScatterLdsBins = 1024;  // up to this many experts the search for a position's expert runs in LDS
 __global__ __launch_bounds__(1024) void scatter_index_kernel(const int *idx, const int *bins_in, int2 *slots, int S, int E, int C,
                                                              bool clear) {
   __shared__ int lds_bins[kScatterLdsBins];
@@ -516,7 +519,7 @@ extern "C" int yamoe_padded_scatter(const void *src, const int32_t *indices, con
   }
   hipStream_t st = (hipStream_t)stream;
   int2 *slots = (int2 *)workspace;
-  const bool one = S <= kScatterOneBlock;
+  const bool one = S <= scatter_one_block(E);
   if (!one) hipLaunchKernelGGL(scatter_clear_kernel, dim3(ceil_div(S, 256)), dim3(256), 0, st, slots, S);
   hipLaunchKernelGGL(scatter_index_kernel, dim3(one ? 1 : ceil_div(S, 256)), dim3(one ? 1024 : 256), 0, st, indices, bins, slots,
                      S, E, C, one);
