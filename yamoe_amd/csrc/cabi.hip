@@ -356,7 +356,10 @@ static size_t carve_saved(const yamoe_problem *p, void *base, Saved *s) {
 // Whether the launches of the tile kernels also work off the streaming list, instead of two launches of their own that
 // usually find it empty.  Where every expert has 32 assignments on average, few if any stream; where they do, the carried
 // form has fewer waves on a CU than the streaming kernel, so it is taken only while the launches are short (an expert's last
-// row tile is half full on average, hence the estimate).
+// row tile is half full on average, hence the estimate).  150 drawn forwards, carried over launches of their own, where no
+// expert streams and where some do: up to 2 estimated rounds 0.97 and 0.88, up to 4 0.98 and 0.93 (single ones 0.78 to 1.02), up to 8
+// 0.996 and 0.94 (0.80 to 1.035), up to 16 0.998 and 0.98, beyond 1.00: above 4 what is left of the two launches' time no longer
+// covers what some calls lose.
 static bool tiles_carry_streams(int N, int E, int H, int I) {
   const long long cols = ceil_div(H > 2 * I ? H : 2 * I, kColTile), rows = ((long long)N + 128ll * E) / kRowTile;
   return N > 32ll * E && rows * cols <= 4 * 256;

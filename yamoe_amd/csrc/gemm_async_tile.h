@@ -671,9 +671,11 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
 
 // One workgroup's part of the streaming list: items `first`, first + step, ...  An item is a slab of one expert, and
 // neighbouring items, which different XCDs work on, are neighbouring slabs.  (17 to 32 rows only where invalid ids leave
-// no expert more: a capacity that does keeps the tiles' launches away.)  Two launches less per layer: 2048 tokens x 2 on 16 experts, 1024 wide, whole layer 81.6 -> 78.1 us,
-// 426 x 2: 42.4 -> 39.5.  In launches of many rounds these workgroups took the time of the streaming kernel to the
-// microsecond, behind the tiles or between the first of them (Zipf routing, 16 384 tokens: gate_up 1794 + 266 and 2063 us).
+// no expert more: a capacity that does keeps the tiles' launches away.)  Two launches less per layer: 2048 tokens x 2 on 16
+// experts, 1024 wide, whole layer 81.6 -> 78.1 us, 426 x 2: 42.4 -> 39.5.  In launches of many rounds these workgroups took the
+// time of the streaming kernel to the microsecond, behind the tiles or between the first of them (Zipf routing, 16 384
+// tokens: gate_up 1794 + 266 and 2063 us); in short ones they are best behind the tiles (in front of them: 150 drawn calls 0.996 in the
+// mean, single ones up to 1.24).
 static_assert(kThreads == kStreamWaves * kWave, "a workgroup of the tile kernels is one of the streaming kernel");
 template <typename T, int EPI, bool GATHER, int DEPTH> __device__ __forceinline__ void stream_items(const Args &args, int first, int step) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -713,9 +715,11 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
   // shares leave over.  An XCD has as many slots as the rounds that the whole list takes on 256 CUs have places on its
   // 32: shares of equal cost put 27 to 35 tiles of a 252-tile list on an XCD, and one tile over a round costs a round.
   // Whole forwards, us, slots for every workgroup / as here: 979 tokens x 2 on 16 experts, 2048 wide: 153 / 123; 3553 x 4 on 32,
-  // 1024: 176 / 134; 3773 x 4 on 128, 2048: 728 / 687; 2003 x 4 on 32, 2880 x 720: 224 / 190.  Beyond kMostRounds a round is
-  // little of a launch, and tiles of very different cost should stay where the cost puts them (29 rounds, Zipf routing: 3250 /
-  // 3276); there only the grid bounds a share (it has at least as many workgroups as there are tiles).
+  // 1024: 176 / 134; 3773 x 4 on 128, 2048: 728 / 687; 2003 x 4 on 32, 2880 x 720: 224 / 168 where the routing makes up to 256 gate_up
+  // tiles, 225 / 225 where it makes 258 to 270.  130 drawn forwards, here over slots for everybody in the mean: 2 rounds 0.90,
+  // 3 0.96, 4 0.97, 5 0.99, 6 0.99, 7 0.985, 8 0.985 (single ones 0.76 to 1.009), 9 to 21 1.000 (0.98 to 1.014).  Beyond kMostRounds a
+  // round is little of a launch, and tiles of very different cost should stay where the cost puts them (29 rounds, Zipf
+  // routing: 3250 / 3276); there only the grid bounds a share (it has at least as many workgroups as there are tiles).
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave >> 1;
 #ifdef YAMOE_TILE_STAMPS
   const unsigned long long t_entry = __builtin_amdgcn_s_memtime();

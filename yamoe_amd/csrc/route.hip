@@ -17,7 +17,11 @@ constexpr int kRouteThreads = 1024;
 constexpr int kRouteWaves = kRouteThreads / kWave;
 constexpr int kRouteMaxBuckets = 769;    // E + 1 must not exceed this (keeps dynamic LDS under 64 KB)
 constexpr int kSingleBlockMaxN = 32768;  // the single-workgroup kernel's limit (its keys sit in LDS as 16-bit values)
-constexpr int kSingleBlockN = 4096;      // up to this many assignments the single-workgroup kernel is used
+// Up to this many assignments the single-workgroup kernel is used.  A whole forward of 64-wide experts, which is mostly this, us,
+// two or three launches / one: 4096 assignments on 8 experts 22.3 / 22.9, on 32 22.4 / 22.3, on 128 27.2 / 26.3, on 512 40.5 / 32.3; 6144
+// on 8 23.3 / 25.6, on 128 26.4 / 26.8, on 256 37.6 / 37.5, on 512 48.1 / 40.7.  The line lies where it is right for few experts;
+// from 64 on it could lie higher (5000 on 64: 24.5 / 23.7; 12 288 on 512: 65.2 / 64.6).
+constexpr int kSingleBlockN = 4096;
 
 template <bool I64>
 __device__ inline int load_key(const void *idx, int i, int E) {
@@ -133,11 +137,10 @@ __device__ inline void wave_place(const void *idx, int seg_begin, int seg_end, i
   }
 }
 
-// The routing
-// of a small batch is one chain of such scans, barriers and divisions; us before / with these scans, the bucket scan by one
-// wave, and no 64-bit division: 4 keys on 128 experts 8.0 / 4.6, 4096 on 16 12.9 / 9.5, 4004 on 128 15.8 / 10.9; two launches,
-// 12 288 on 64: 12.3 / 10.1 (the second); work lists of one expert's rows alone 8.4 / 5.0.
-
+// The routing of a small batch is one chain of wave scans (common.h), barriers and divisions.  Kernel times, us, with six trips
+// through the LDS crossbar a scan, the bucket scan by the whole workgroup and 64-bit divisions / with DPP moves, by one wave
+// and without: 4 keys on 128 experts 8.0 / 4.6, 4096 on 16 12.9 / 9.5, 4004 on 128 15.8 / 10.9; work lists of one expert's rows
+// alone 8.4 / 5.0.
 // Exclusive scan over buckets of `total` into `offsets` (both LDS), by the first wave of the workgroup; offsets[buckets] = N.
 // The caller puts a barrier on both sides.
 __device__ inline void first_wave_exclusive_scan(const int *total, int *offsets, int buckets) {
@@ -544,10 +547,11 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
 using namespace yamoe;
 
 // Keys per wave in the forms with more than one launch: short segments spread the counting and the placement over
-// more workgroups, long ones keep the segments x buckets table small.  65 536 keys, 128 experts, three launches:
-// 46 / 40 / 48 us with segments of 1024 / 512 / 256 keys (85 us with 2048 and the work lists in a launch of their own),
-// two launches with 512: 33 us.  16 384 keys, 32 experts, two launches: 20.5 / 16.3 / 18 us with 512 / 256 / 128 against
-// 26 us for the single-workgroup kernel.
+// more workgroups, long ones keep the segments x buckets table small.  Whole routing without work lists, us, with segments of 128 /
+// 256 / 512 / 1024 / 2048 keys: 16 384 keys on 32 experts 9.2 / 9.5 / 13.8 / 22.6 / 33.5, 32 768 on 128 22.6 / 18.2 / 20.8 / 31.3 / 53.8,
+// 65 536 on 128 28.1 / 24.3 / 23.9 / 32.2 / 55.0, 131 072 on 256 68.4 / 43.0 / 35.3 / 45.9 / 64.8.  Beyond that only a large table
+// wants 2048 (1 048 576 on 256: 248 / 138 / 94 / 91 with 256 and up); 262 144 on 32 experts take 44.0, and 22.9 / 20.9 / 27.1
+// with 256 / 512 / 1024.
 static int route_segment(int N) { return N <= 32768 ? 256 : N <= 131072 ? 512 : 2048; }
 static_assert(kSingleBlockN <= kSingleBlockMaxN, "the single-workgroup kernel keeps its keys in LDS");
 

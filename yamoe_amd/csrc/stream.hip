@@ -6,8 +6,8 @@
 // of the slab round-robin; in a step every lane fetches an 8(k) x 8(column) block as eight 16-byte
 // loads (a wave reads 32 rows x 256 contiguous bytes), transposes it in registers and feeds it to
 // eight v_mfma_f32_16x16x32 instructions whose 16-row A operand is the expert's (zero-padded)
-// activations (an expert with 17 to 32 rows has two such operands and runs every column operand through both).  No LDS is touched until the final cross-wave reduction.  Two steps of loads are
-// kept in flight per wave, at least 8 waves per CU.
+// activations (an expert with 17 to 32 rows has two such operands and runs every column operand through both).  No LDS is
+// touched until the final cross-wave reduction.  Two steps of loads are kept in flight per wave, at least 8 waves per CU.
 //
 // A launch that can hold only a few experts (a handful of tokens: at most kStreamFewBlocks workgroups) has too few
 // workgroups to keep HBM busy that way: 4 experts x 23 slabs with two steps of 8 KB in flight per wave are 6 MB on
@@ -15,6 +15,11 @@
 // flight each instead (16 waves with two steps each measured 3 % slower), folded into the first four before the same
 // finish.  One token of a 2880-wide layer on four experts is 180 workgroups in the gate_up product and 92 in the down
 // product, on 256 CUs: 22 us for 132 MB of weights and 19 us for 66 MB.
+//
+// These are the launches of calls in which every expert streams, and of calls whose tile launches are long.  Where those
+// are short and there are tiles, streamed experts ride in them (stream_items in gemm_async_tile.h): the slab code is the
+// same, with four waves whatever the number of experts, two steps in flight beside 128 x 128 tiles and three beside
+// 256 x 256 ones (two for 17 to 32 rows).
 //
 // The lane that holds accumulator column c of MFMA j owns output column 8c + j, so the 8
 // accumulators of a lane are 8 consecutive output columns: the interleaved (gate, up) pairs of the
