@@ -79,7 +79,6 @@ int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const
 template <typename T>
 int gemm_async_wgrad(const void *, const int *, int, int, const void *, void *, void *, const int *, const int *, int, int,
                      int, int, hipStream_t);
-bool wgrad_writes_bias(int Md, int Nd);
 int gemm_f32_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
                      int, int, hipStream_t);
 int gemm_f32_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
@@ -190,10 +189,7 @@ template <typename T> static bool wgrad_gathers(int Md, int Nd) {
 
 // True when the weight-gradient kernel for this dtype and shape also leaves the bias gradient (the per-expert column
 // sums of its right operand), so that no launch of expert_colsum_kernel is needed for it.
-template <typename T> static bool wgrad_sums_bias(int Md, int Nd) {
-  if constexpr (sizeof(T) == 2) return wgrad_writes_bias(Md, Nd);
-  return false;
-}
+template <typename T> static constexpr bool wgrad_sums_bias() { return sizeof(T) == 2; }
 
 // l_rows (with wgrad_gathers only): sorted row p of the left operand is row l_rows[p] / l_div of L; the list holds
 // n_rows values below n_rows and is followed by at least 32 readable ints.  d_bias (with wgrad_sums_bias only): [E, Nd].
@@ -446,8 +442,8 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   // rows of grad_out, gathered by token (its dot with the activations is the rest of the routing gradient)
   // (the bias gradients are the column sums of the weight gradients' right operands: taken by those kernels where
   // they can, by a launch of their own otherwise)
-  const bool bd_fused = wgrad_sums_bias<T>(I, H), bgu_fused = wgrad_sums_bias<T>(H, 2 * I);
-  if (!bd_fused) YAMOE_TRY(launch_expert_colsum<T>(b.g_y_perm, b.f.counts, b.f.offsets, cap, d_bd, E, H, stream));
+  constexpr bool sums = wgrad_sums_bias<T>();
+  if constexpr (!sums) YAMOE_TRY(launch_expert_colsum<T>(b.g_y_perm, b.f.counts, b.f.offsets, cap, d_bd, E, H, stream));
   if (permuted) {
     YAMOE_TRY(launch_permute<T>(gy, b.f.sorted_idx, b.gy_perm, N, p->K, H, stream));
     YAMOE_TRY(tiles_dgrad<T>(b.gy_perm, nullptr, 1, 0, wd, b.d_act, b.f.schedule, N, E, /*Kd=*/H, /*Nd=*/I, b.f.act,
@@ -456,23 +452,23 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
     YAMOE_TRY(tiles_dgrad<T>(gy, b.f.sorted_idx, p->K, (long long)p->T * H * (long long)es, wd, b.d_act, b.f.schedule, N, E,
                              /*Kd=*/H, /*Nd=*/I, b.f.act, b.dot_part, stream));
   }
-  YAMOE_TRY(tiles_wgrad<T>(b.f.act, nullptr, 1, 0, b.g_y_perm, d_wd, bd_fused ? d_bd : nullptr, b.f.counts, b.f.offsets, cap, E,
+  YAMOE_TRY(tiles_wgrad<T>(b.f.act, nullptr, 1, N, b.g_y_perm, d_wd, sums ? d_bd : nullptr, b.f.counts, b.f.offsets, cap, E,
                            /*Md=*/I, /*Nd=*/H, stream));
   // GLU backward (scaled by the routing weight) and the routing gradient
   YAMOE_TRY(glu_backward_rows<T>(b.d_act, b.pre, b.w_sorted, b.dot_part, b.n_part, b.f.sorted_idx, b.f.inv_pos, b.d_pre,
                                  b.row_dot, N, I, stream));
   YAMOE_TRY(launch_routing_grad<T>(b.row_dot, b.f.inv_pos, idx, p->idx_i64, p->rw_cols, d_rw, N, p->K, E, stream));
   // gate_up projection
-  if (!bgu_fused) YAMOE_TRY(launch_expert_colsum<T>(b.d_pre, b.f.counts, b.f.offsets, cap, d_bgu, E, 2 * I, stream));
+  if constexpr (!sums) YAMOE_TRY(launch_expert_colsum<T>(b.d_pre, b.f.counts, b.f.offsets, cap, d_bgu, E, 2 * I, stream));
   YAMOE_TRY(tiles_dgrad<T>(b.d_pre, nullptr, 1, 0, wgu, b.d_x_perm, b.f.schedule, N, E, /*Kd=*/2 * I, /*Nd=*/H, nullptr,
                            nullptr, stream));
   // (the hidden rows gathered by token where the kernel can do that and hidden_states is below 4 GiB; sorted_idx is
   // followed in the workspace by inv_pos and the rest: readable well past its end)
   if (gathers)
-    YAMOE_TRY(tiles_wgrad<T>(x, b.f.sorted_idx, p->K, N, b.d_pre, d_wgu, bgu_fused ? d_bgu : nullptr, b.f.counts, b.f.offsets,
+    YAMOE_TRY(tiles_wgrad<T>(x, b.f.sorted_idx, p->K, N, b.d_pre, d_wgu, sums ? d_bgu : nullptr, b.f.counts, b.f.offsets,
                              cap, E, /*Md=*/H, /*Nd=*/2 * I, stream));
   else
-    YAMOE_TRY(tiles_wgrad<T>(b.x_perm, nullptr, 1, 0, b.d_pre, d_wgu, bgu_fused ? d_bgu : nullptr, b.f.counts, b.f.offsets,
+    YAMOE_TRY(tiles_wgrad<T>(b.x_perm, nullptr, 1, N, b.d_pre, d_wgu, sums ? d_bgu : nullptr, b.f.counts, b.f.offsets,
                              cap, E, /*Md=*/H, /*Nd=*/2 * I, stream));
   // permute backward: d_hidden[t] = sum_k d_x_perm[inv_pos[t,k]]
   YAMOE_TRY(launch_combine<T>(b.d_x_perm, b.f.inv_pos, idx, p->idx_i64, nullptr, p->K, d_x, p->T, p->K, E, H, stream));

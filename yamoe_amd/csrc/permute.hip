@@ -458,12 +458,12 @@ int launch_expert_colsum(const void *src, const int *counts, const int *offsets,
   template int glu_backward_rows<T>(const void *, const void *, const float *, const float *, int, const int *, \
                                     const int *, void *, float *, int, int, hipStream_t);                        \
   template int launch_routing_grad<T>(const float *, const int *, const void *, int, int, void *, int, int, int, \
-                                      hipStream_t);                                                              \
-  template int launch_expert_colsum<T>(const void *, const int *, const int *, int, void *, int, int,  \
-                                       hipStream_t);
+                                      hipStream_t);
 YAMOE_INSTANTIATE_ROWS(float)
 YAMOE_INSTANTIATE_ROWS(bf16_t)
 YAMOE_INSTANTIATE_ROWS(f16_t)
+// (16-bit data: the weight-gradient kernels leave these sums)
+template int launch_expert_colsum<float>(const void *, const int *, const int *, int, void *, int, int, hipStream_t);
 
 }  // namespace yamoe
 
