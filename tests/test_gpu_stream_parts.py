@@ -1,0 +1,70 @@
+"""The streaming kernels where a call has few (expert, column slab) pairs and several workgroups share one: contractions of a
+few steps and of many, whole and cut slabs, one and two blocks of 16 rows, experts in chunks of 32 rows; fp32 on the same path.
+The parts are added up in their order, so a call gives the same bits every time, also when it is replayed from a graph."""
+import pytest
+import torch
+
+from oracle import yamoe_oracle as O
+from tests.util import REL_L2_TOL, args, to_dev
+from yamoe_amd.workloads import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # T, H, I, E, K, one expert for all
+    (1, 64, 72, 8, 1, False), (1, 128, 256, 8, 2, False), (2, 520, 1032, 16, 2, False), (1, 2880, 360, 32, 4, False),
+    (3, 1000, 40, 4, 1, False), (16, 1024, 200, 8, 2, False), (17, 264, 128, 16, 1, True), (31, 1536, 64, 8, 1, True),
+    (32, 256, 264, 8, 1, True), (33, 2048, 128, 16, 1, True), (64, 512, 264, 16, 1, True), (40, 136, 520, 64, 4, False),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("T,H,I,E,K,one", SHAPES)
+def test_shared_slabs(gpu, T, H, I, E, K, one, dtype):
+    import yamoe_amd
+    print("stream parts", T, H, I, E, K, one, dtype, flush=True)
+    d = make_inputs(T, H, I, E, K, dtype, seed=T + H, w_std=0.05, bias_std=0.1)
+    if one:
+        d["router_indices"] = torch.full_like(d["router_indices"], E - 2)
+        d["routing_weights"] = (0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))).to(dtype)
+    g = args(to_dev(d, gpu))
+    out = yamoe_amd.experts(*g, T, E, K)
+    want = O.experts_capacity(*args(d), T, compute_dtype=torch.float64 if dtype == torch.float32 else torch.float32)
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        again = yamoe_amd.experts(*g, T, E, K)
+    for _ in range(3):
+        again.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, again)
+        assert torch.equal(out, yamoe_amd.experts(*g, T, E, K))
+
+
+@pytest.mark.parametrize("capacity", [0, 1, 16, 17, 32, 40])
+def test_fp32_streams_up_to_a_capacity(gpu, capacity):
+    """48 tokens of one expert among 16: chunks of 32 rows, cut by the capacity; gradients of a kept forward as of a recomputed one."""
+    import yamoe_amd
+    T, H, I, E, K = 48, 264, 520, 16, 1
+    d = make_inputs(T, H, I, E, K, torch.float32, seed=capacity, w_std=0.05, bias_std=0.1)
+    d["router_indices"] = torch.full_like(d["router_indices"], 3)
+    d["routing_weights"] = 0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(1))
+    g = args(to_dev(d, gpu))
+    out, kept = yamoe_amd.experts_keep(*g, capacity, E, K)
+    assert torch.equal(out, yamoe_amd.experts(*g, capacity, E, K))
+    want = O.experts_capacity(*args(d), capacity, compute_dtype=torch.float64)
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[torch.float32] or (capacity == 0 and not out.any())
+    gy = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(gpu)
+    for a, b in zip(yamoe_amd.experts_backward_kept(gy, *g, kept, capacity, E, K), yamoe_amd.experts_backward(gy, *g, capacity, E, K)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("C", [1, 15, 16, 17, 32, 33])
+def test_fp32_batch_mm_of_few_rows(gpu, C):
+    import yamoe_amd
+    E, Kd, Nd = 3, 148, 260
+    gen = torch.Generator().manual_seed(C)
+    x, w = torch.randn(E, C, Kd, generator=gen), torch.randn(E, Kd, Nd, generator=gen)
+    y = torch.empty(E, C, Nd, device=gpu)
+    yamoe_amd.batch_mm(x.to(gpu), w.to(gpu), torch.full((E,), C, dtype=torch.int32, device=gpu), y)
+    assert O.rel_l2(y.cpu(), torch.bmm(x.double(), w.double())) < REL_L2_TOL[torch.float32]

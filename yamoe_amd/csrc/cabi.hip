@@ -63,9 +63,10 @@ template <typename T>
 int launch_routing_grad(const float *, const int *, const void *, int, int, void *, int, int, int, hipStream_t);
 template <typename T>
 int stream_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
-                   int, int, hipStream_t);
+                   int, int, float *, hipStream_t);
 template <typename T>
-int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, hipStream_t);
+int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, float *, hipStream_t);
+size_t stream_partial_bytes(int N, int E, int Kd, int Nd, int elem_bytes);
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
@@ -103,7 +104,12 @@ int plain_backward(const void *, const void *, const void *, int, const void *, 
                    int, int, int, int, int, int, hipStream_t);
 template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
-template <typename T> struct HasStreamPath { static constexpr bool value = sizeof(T) == 2; };
+// Experts of at most this many kept rows stream their weights instead of going through the tile kernels (0: none does).  fp32 data
+// streams where every expert does: beside tiles, whose launch takes as long for one of them as for a round, a second pair of
+// launches costs more than it takes off them (64 tokens x 2 on 16 skewed experts, 2048 x 744: 122 us as tiles, 173 so).
+static int stream_rows_of(int dtype, int N, int E) {
+  return dtype != YAMOE_F32 || sched_may_stream_everything(N, E) ? kStreamMaxRows : 0;
+}
 
 // Whether a product of N rows over E experts with Nd columns runs on 128 x 128 tiles (two workgroups per CU) instead of
 // 256 x 256 (one).  The small tiles read twice the operand bytes per flop, so they pay only where the large ones leave CUs
@@ -253,6 +259,14 @@ static bool gathers_need_permute(const yamoe_problem *p) {
   return (long long)p->T * p->H * (long long)dtype_size(p->dtype) >= limit;
 }
 
+// Double precision, and hidden or intermediate sizes that are not whole 16-byte chunks (the unit the MFMA kernels
+// copy): the same lists, then the kernels of plain.hip.
+static bool takes_plain_path(const yamoe_problem *p) {
+  if (p->dtype == YAMOE_F64) return true;
+  const int vec = 16 / (int)dtype_size(p->dtype);
+  return p->H % vec != 0 || p->I % vec != 0;
+}
+
 // Carves 256-byte aligned regions out of the workspace.
 struct Carver {
   char *base;
@@ -269,6 +283,7 @@ struct ForwardBuffers {
   int *sorted_expert, *sorted_idx, *inv_pos, *counts, *offsets;
   void *schedule, *route_ws, *act, *y_perm;
   void *x_perm;  // hidden rows in expert order: only with gathers_need_permute
+  float *partial;  // sums of the workgroups that share a slab of a streaming product: where that happens at all
   size_t schedule_bytes, route_ws_bytes;
 };
 
@@ -288,6 +303,12 @@ static size_t carve_forward(const yamoe_problem *p, void *ws, ForwardBuffers *b)
   // sized for the larger of H and I: the backward reuses this region for d_act [N, I]
   b->y_perm = c.take(N * (size_t)(p->H > p->I ? p->H : p->I) * es);
   b->x_perm = gathers_need_permute(p) ? c.take(N * p->H * es) : nullptr;
+  size_t partial = 0;
+  if (!takes_plain_path(p) && sched_may_stream_everything((int)N, p->E)) {
+    const size_t gate_up = stream_partial_bytes((int)N, p->E, p->H, 2 * p->I, (int)es), down = stream_partial_bytes((int)N, p->E, p->I, p->H, (int)es);
+    partial = gate_up > down ? gate_up : down;
+  }
+  b->partial = partial > 0 ? (float *)c.take(partial) : nullptr;
   return c.used;
 }
 
@@ -372,11 +393,11 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   const int N = p->T * p->K;
   void *st = (void *)stream;
   if (N == 0 || p->T == 0) return 0;
-  const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
+  const int stream_rows = stream_rows_of(p->dtype, N, p->E);
   // At most 4 assignments per expert on average (decode): every expert goes to the streaming kernel, in chunks of
   // stream_rows rows where one has more, and the tile kernels, whose lists are then empty, are not launched (two
   // launches of 4.5 us each that found nothing to do at 64 tokens on 128 experts).
-  const bool everything = HasStreamPath<T>::value && sched_may_stream_everything(N, p->E);
+  const bool everything = sched_may_stream_everything(N, p->E);
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
                                b.inv_pos, b.route_ws, b.route_ws_bytes, everything ? kStreamEverything : stream_rows,
                                b.schedule, b.schedule_bytes, st));
@@ -384,7 +405,7 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   // well.  1723 tokens on 8 experts of 2048 x 2048, 32 rows kept: 60 us; with two tile launches that find no tile in front 68,
   // carried by those 72.
   const bool tiles = !everything && N > stream_rows && p->capacity > stream_rows;
-  const bool carried = HasStreamPath<T>::value && tiles && tiles_carry_streams(N, p->E, p->H, p->I);
+  const bool carried = sizeof(T) == 2 && tiles && tiles_carry_streams(N, p->E, p->H, p->I);
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
@@ -393,12 +414,11 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
     YAMOE_TRY(tiles_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
                                carried, stream));
   }
-  if constexpr (HasStreamPath<T>::value)
-    if (!carried) YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I,
-                                stream));
+  const bool streams = stream_rows > 0 && !carried;
+  if (streams)
+    YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, b.partial, stream));
   if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, carried, 0, stream));
-  if constexpr (HasStreamPath<T>::value)
-    if (!carried) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream));
+  if (streams) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, b.partial, stream));
   YAMOE_TRY(launch_combine<T>(b.y_perm, b.inv_pos, idx, p->idx_i64, rw, p->rw_cols, out, p->T, p->K, p->E, p->H,
                               stream));
   return 0;
@@ -422,14 +442,21 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
     YAMOE_TRY(fill_zero(d_bd, (size_t)E * H * es, stream));
     return 0;
   }
+  // fp32: the recomputation streams where the forward did, so that its gradients are those of a kept forward to the bit; the
+  // other products run on the tile kernels and get their lists afterwards.
+  const bool streamed = sizeof(T) == 4 && kept == nullptr && stream_rows_of(p->dtype, N, E) > 0;
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, E, cap, b.f.sorted_expert, b.f.sorted_idx, b.f.counts, b.f.offsets,
-                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, 0, b.f.schedule, b.f.schedule_bytes, st));
+                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, streamed ? kStreamEverything : 0, b.f.schedule,
+                               b.f.schedule_bytes, st));
   // forward recompute of the first product only: activations and pre-activations
   const bool permuted = b.gy_perm != nullptr;  // hidden_states and grad_out too large to gather from
   const bool gathers = !permuted && wgrad_gathers<T>(H, 2 * I);
   if (!gathers) YAMOE_TRY(launch_permute<T>(x, b.f.sorted_idx, b.x_perm, N, p->K, H, stream));
   if (kept != nullptr) {
     // activations and pre-activations come from the forward
+  } else if (streamed) {
+    YAMOE_TRY(stream_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, b.f.partial, stream));
+    YAMOE_TRY(yamoe_build_schedule(b.f.counts, b.f.offsets, N, E, cap, 0, b.f.schedule, b.f.schedule_bytes, st));
   } else if (permuted) {
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, false, stream));
   } else {
@@ -473,14 +500,6 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   // permute backward: d_hidden[t] = sum_k d_x_perm[inv_pos[t,k]]
   YAMOE_TRY(launch_combine<T>(b.d_x_perm, b.f.inv_pos, idx, p->idx_i64, nullptr, p->K, d_x, p->T, p->K, E, H, stream));
   return 0;
-}
-
-// Double precision, and hidden or intermediate sizes that are not whole 16-byte chunks (the unit the MFMA kernels
-// copy): the same lists, then the kernels of plain.hip.
-static bool takes_plain_path(const yamoe_problem *p) {
-  if (p->dtype == YAMOE_F64) return true;
-  const int vec = 16 / (int)dtype_size(p->dtype);
-  return p->H % vec != 0 || p->I % vec != 0;
 }
 
 template <typename T>
@@ -564,15 +583,15 @@ template <typename T>
 static int gate_up_both(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
                         const void *sched, int N, int K, int E, int H, int I, hipStream_t stream) {
   YAMOE_TRY(tiles_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, 0, false, stream));
-  if constexpr (HasStreamPath<T>::value)
-    YAMOE_TRY(stream_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream));
+  if constexpr (sizeof(T) == 2)
+    YAMOE_TRY(stream_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, nullptr, stream));
   return 0;
 }
 template <typename T>
 static int down_both(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
                      int I, hipStream_t stream) {
   YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, false, 0, stream));
-  if constexpr (HasStreamPath<T>::value) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, stream));
+  if constexpr (sizeof(T) == 2) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, nullptr, stream));
   return 0;
 }
 // The same for E groups of `rows` rows each: whether they stream or are tiles is known on the host, so only one of the two
@@ -581,12 +600,12 @@ static int down_both(const void *act, const void *w, const void *bias, void *y, 
 template <typename T>
 static int down_regular(const void *act, const void *w, const void *bias, void *y, int *counts, int *offsets, void *sched,
                         size_t sched_bytes, int E, int rows, int H, int I, hipStream_t stream) {
-  const int stream_rows = HasStreamPath<T>::value ? kStreamMaxRows : 0;
-  if (HasStreamPath<T>::value && rows > stream_rows)
-    return tiles_down<T>(act, w, bias, y, nullptr, E * rows, E, H, I, stream_rows, false, rows, stream);
-  YAMOE_TRY(regular_schedule(counts, offsets, E, rows, stream_rows, sched, sched_bytes, stream));
-  if constexpr (HasStreamPath<T>::value) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream);
-  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, stream_rows, false, 0, stream);
+  const bool streams = rows <= kStreamMaxRows;
+  if (sizeof(T) == 2 && !streams)
+    return tiles_down<T>(act, w, bias, y, nullptr, E * rows, E, H, I, kStreamMaxRows, false, rows, stream);
+  YAMOE_TRY(regular_schedule(counts, offsets, E, rows, streams ? kStreamMaxRows : 0, sched, sched_bytes, stream));
+  if (streams) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, nullptr, stream);
+  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, 0, false, 0, stream);
 }
 
 extern "C" int yamoe_gate_up(const void *x, const int32_t *sorted_idx, const void *gate_up_proj,

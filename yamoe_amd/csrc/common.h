@@ -194,11 +194,14 @@ __device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_in
 //                       index of the expert's first row tile, number of row tiles of the expert,
 //                       multiplier and shift that divide by that number, 128-row tiles of the experts before this one}
 //   then              small experts: 4 words each {expert, first sorted row, valid rows, 0}
+//   then              kSchedArrivals counters, zero between launches: how many of the workgroups that share a piece of
+//                     work have left their part of it
 constexpr int kRowTile = 256;  // rows of one MFMA row tile
 constexpr int kColTile = 256;  // columns of one MFMA tile
 constexpr int kSchedHeader = 48;
 constexpr int kSchedCuts = 8;  // word offset of the XCD cut table
 constexpr int kSchedHalfTiles = 5;
+constexpr int kSchedArrivals = 512;
 constexpr int kXcds = 8;
 constexpr int kXcdCus = 32;    // CUs of one XCD
 
@@ -248,6 +251,7 @@ struct ScheduleView {
   const int *hdr;
   const int *row_tiles;
   const int *small;
+  const int *arrivals;
 };
 __host__ __device__ inline ScheduleView schedule_view(const void *p, int N, int E) {
   const int *w = (const int *)p;
@@ -255,6 +259,7 @@ __host__ __device__ inline ScheduleView schedule_view(const void *p, int N, int 
   v.hdr = w;
   v.row_tiles = w + kSchedHeader;
   v.small = w + kSchedHeader + 8 * sched_max_row_tiles(N, E);
+  v.arrivals = v.small + 4 * sched_max_small(N, E);
   return v;
 }
 

@@ -164,6 +164,8 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
                                            int stream_max_rows, int *sched, const int lane) {
   int *row_tiles = sched + kSchedHeader;
   int *small = row_tiles + 8 * sched_max_row_tiles(N, E);
+  int *arrivals = small + 4 * sched_max_small(N, E);
+  for (int i = lane; i < kSchedArrivals; i += kWave) arrivals[i] = 0;
   int n_tiles = 0, n_small = 0, n_active = 0, n_kept = 0, n_half = 0;
   // Experts of 17 to 32 rows stream only when every expert streams: next to experts that need the tile kernels anyway
   // they are better off as tiles (two half-filled launches one after the other are slower than one: 0.35 against
@@ -676,7 +678,7 @@ int yamoe::regular_schedule(int *counts, int *offsets, int E, int rows, int stre
 }
 
 extern "C" size_t yamoe_schedule_bytes(int32_t N, int32_t E) {
-  size_t words = kSchedHeader + 8 * (size_t)sched_max_row_tiles(N, E) + 4 * (size_t)sched_max_small(N, E);
+  size_t words = kSchedHeader + 8 * (size_t)sched_max_row_tiles(N, E) + 4 * (size_t)sched_max_small(N, E) + kSchedArrivals;
   return align_up(words * sizeof(int), 256);
 }
 

@@ -9,17 +9,28 @@
 // activations (an expert with 17 to 32 rows has two such operands and runs every column operand through both).  No LDS is
 // touched until the final cross-wave reduction.  Two steps of loads are kept in flight per wave, at least 8 waves per CU.
 //
-// A launch that can hold only a few experts (a handful of tokens: at most kStreamFewBlocks workgroups) has too few
-// workgroups to keep HBM busy that way: 4 experts x 23 slabs with two steps of 8 KB in flight per wave are 6 MB on
-// the way, where 8 TB/s x 2 us of latency want 16 MB.  Such a launch takes 8 waves per workgroup with three steps in
-// flight each instead (16 waves with two steps each measured 3 % slower), folded into the first four before the same
-// finish.  One token of a 2880-wide layer on four experts is 180 workgroups in the gate_up product and 92 in the down
-// product, on 256 CUs: 22 us for 132 MB of weights and 19 us for 66 MB.
+// A launch of a few experts (a handful of tokens) has too few workgroups to keep HBM busy that way: one token of a 2880-wide
+// layer on two experts is 90 slabs in the gate_up product and 46 in the down product, on 256 CUs, and a CU alone moves 43 GB/s.
+// There the contraction of a slab is shared by several workgroups (stream_parts), which costs about 2 us: the parts go
+// through memory, and whoever comes last adds them up.  What counts is how evenly the workgroups fill the CUs, which is known
+// on the device: us for 1 / 2 / 3 / 4 / 6 / 8 parts, 46 slabs of 90 steps 20.1 / 14.3 / 11.6 / 10.6 / 11.9 / 11.0, 92: 21.1 / 15.6 / 17.8 /
+// 15.9 / 16.7 / 15.6, 161: 22.6 / 25.3 / 21.6 / 23.4 / 25.7 / 25.4, 180: 23.4 / 25.4 / 26.1 / 24.7 / 26.7 / 27.5, 64 of 32 steps: 11.7 /
+// 10.2 / 8.5 / 8.0 / 9.0 / 9.4 (workgroups of four waves).  Where the list has at most a slab per CU, a workgroup takes
+// eight waves with three steps in flight each, as much as a CU holds, folded into the first four before the same finish: one
+// token on four experts 44.9 us, with four waves 47.5 (four tokens x 4 on 32 experts, 1024 wide: 28.6 and 30.5).
+//
+// An XCD's workgroups take neighbouring slabs.  Where a weight row is not a whole number of cache lines, a slab's piece of it
+// shares a line with the next slab's, and both come from memory unless they meet in one L2: 64 experts, 2048 x 1544, 16 tokens
+// x 8, gate_up 143.6 us with neighbours on different XCDs and 128.3 so.  Whole lines gain 0 to 2 % (64 tokens of the 128-expert
+// layer: 843 and 829 us); not so fp32, where the slabs of an expert with 17 to 32 rows are bound by the matrix units and
+// should not all be on one XCD (32 x 8 rows, 2880 wide: 324 and 355 us).
+//
+// fp32 takes the same path with v_mfma_f32_16x16x4_f32.  One token on two experts of 2880 x 2880: 229 us on the tile kernel, 53
+// so; 32 x 2 on 16 of them 489 / 267; 16 x 4 on 32, 1024 wide, 123 / 74.
 //
 // These are the launches of calls in which every expert streams, and of calls whose tile launches are long.  Where those
 // are short and there are tiles, streamed experts ride in them (stream_items in gemm_async_tile.h): the slab code is the
-// same, with four waves whatever the number of experts, two steps in flight beside 128 x 128 tiles and three beside
-// 256 x 256 ones (two for 17 to 32 rows).
+// same, two steps in flight beside 128 x 128 tiles and three beside 256 x 256 ones (two for 17 to 32 rows).
 //
 // The lane that holds accumulator column c of MFMA j owns output column 8c + j, so the 8
 // accumulators of a lane are 8 consecutive output columns: the interleaved (gate, up) pairs of the
@@ -28,60 +39,110 @@
 
 namespace yamoe {
 
-constexpr int kStreamManyWaves = 8;
-constexpr int kStreamFewBlocks = 1024;  // launches with fewer (expert, slab) workgroups than this take 8 waves each
-template <typename T, bool GLU, bool GATHER, int WAVES, int DEPTH>
-__global__ __launch_bounds__(64 * WAVES, WAVES == kStreamWaves ? 2 : 1) void stream_gemm_kernel(const StreamArgs args) {
+constexpr int kStreamManyWaves = 8, kStreamMaxParts = 8, kStreamMostShared = 1024;
+constexpr int kChipCus = kXcds * kXcdCus;
+
+// How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
+// fewest steps on the CU that gets most of them, where sharing costs about as much as ten (the parts' way through memory).
+__host__ __device__ inline int stream_parts(int slabs, int steps, int waves) {
+  int best = 1, cost = ceil_div(slabs, kChipCus) * steps;
+  if (slabs > kSchedArrivals) return 1;
+  const int most = waves == kStreamManyWaves ? kChipCus : kStreamMostShared;
+  for (int p = 2; p <= kStreamMaxParts && slabs * p <= most && steps >= waves * p; ++p) {
+    const int c = ceil_div(slabs * p, kChipCus) * ceil_div(steps, p) + 10;
+    if (c < cost) { best = p; cost = c; }
+  }
+  return best;
+}
+// Whether a launch takes eight waves per workgroup, one of which fills a CU (a list holds one entry per expert here, or
+// per assignment where these are fewer, unless an expert has more than a chunk of rows).
+static bool stream_many_waves(int N, int E, int n_slabs) { return (long long)(N < E ? N : E) * n_slabs <= kChipCus; }
+
+template <typename T, bool GLU, bool GATHER, int WAVES>
+__global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void stream_gemm_kernel(const StreamArgs args) {
   __shared__ float red[kStreamWaves * 8 * 4 * kWave];  // [wave][j][v][lane]
   const ScheduleView sv = schedule_view(args.sched, args.N, args.E);
-  const int n_small = sv.hdr[1];
-  const int s = blockIdx.x / args.n_slabs;
-  if (s >= n_small) return;
-  const int slab = blockIdx.x - s * args.n_slabs;
+  const int slabs = sv.hdr[1] * args.n_slabs;
+  const int parts = args.partial != nullptr ? stream_parts(slabs, ceil_div(args.Kd, StreamStep<T>::kRows), WAVES) : 1;
+  const int total = slabs * parts;
+  int b = blockIdx.x;
+  if (args.per_xcd) {  // workgroup b runs on XCD b % 8: that XCD's share of the work is contiguous
+    const int share = ceil_div(total, kXcds), place = b / kXcds;
+    if (place >= share) return;
+    b = b % kXcds * share + place;
+  }
+  if (b >= total) return;
+  const int item = b / parts, part = b - item * parts;
+  const int s = item / args.n_slabs, slab = item - s * args.n_slabs;
   const int expert = sv.small[4 * s], first = sv.small[4 * s + 1], rows = sv.small[4 * s + 2];
-  if (rows > 16) stream_slab<T, GLU, GATHER, WAVES, DEPTH, 2>(args, red, expert, first, rows, slab);
-  else stream_slab<T, GLU, GATHER, WAVES, DEPTH, 1>(args, red, expert, first, rows, slab);
+  constexpr int DEPTH = WAVES == kStreamWaves ? 2 : 3;
+  if (rows > 16) stream_slab<T, GLU, GATHER, WAVES, 2, 2>(args, red, expert, first, rows, slab, item, part, parts);
+  else stream_slab<T, GLU, GATHER, WAVES, DEPTH, 1>(args, red, expert, first, rows, slab, item, part, parts);
+}
+
+// The most workgroups that a launch may need, whatever is on its list, and (`shared`) the most of them that leave parts.
+static long long stream_max_blocks(int N, int E, int Kd, int Nd, int step_rows, long long *shared) {
+  const int entries = sched_max_small(N, E), n_slabs = ceil_div(Nd, kSlabCols), steps = ceil_div(Kd, step_rows);
+  const int waves = stream_many_waves(N, E, n_slabs) ? kStreamManyWaves : kStreamWaves;
+  long long most = (long long)entries * n_slabs;
+  *shared = 0;
+  for (int n = 1; n <= entries && (long long)n * n_slabs <= kSchedArrivals; ++n) {
+    const int parts = stream_parts(n * n_slabs, steps, waves);
+    const long long blocks = (long long)n * n_slabs * parts;
+    if (parts > 1 && blocks > *shared) *shared = blocks;
+  }
+  return most > *shared ? most : *shared;
+}
+// Bytes of the parts of a product, 0 where its slabs are certain not to be shared.
+size_t stream_partial_bytes(int N, int E, int Kd, int Nd, int elem_bytes) {
+  long long shared;
+  stream_max_blocks(N, E, Kd, Nd, elem_bytes == 4 ? StreamStep<float>::kRows : StreamStep<bf16_t>::kRows, &shared);
+  return (size_t)shared * stream_part_floats(N) * sizeof(float);
 }
 
 template <typename T, bool GLU, bool GATHER>
-static int launch_stream(const StreamArgs &a, hipStream_t stream) {
-  long long blocks = (long long)sched_max_small(a.N, a.E) * a.n_slabs;
+static int launch_stream(StreamArgs a, float *partial, hipStream_t stream) {
+  a.n_slabs = ceil_div(a.Nd, kSlabCols);
+  a.partial = partial;
+  a.part_floats = stream_part_floats(a.N);
+  a.arrivals = const_cast<int *>(schedule_view(a.sched, a.N, a.E).arrivals);
+  a.per_xcd = sizeof(T) == 2 || (a.Nd * (int)sizeof(T)) % 128 != 0;
+  long long shared, blocks = stream_max_blocks(a.N, a.E, a.Kd, a.Nd, StreamStep<T>::kRows, &shared);
+  if (partial == nullptr) blocks = (long long)sched_max_small(a.N, a.E) * a.n_slabs;
   if (blocks <= 0) return 0;
-  if (blocks < kStreamFewBlocks) {
-    hipLaunchKernelGGL((stream_gemm_kernel<T, GLU, GATHER, kStreamManyWaves, 3>), dim3((unsigned)blocks),
-                       dim3(64 * kStreamManyWaves), 0, stream, a);
-  } else {
-    hipLaunchKernelGGL((stream_gemm_kernel<T, GLU, GATHER, kStreamWaves, 2>), dim3((unsigned)blocks), dim3(64 * kStreamWaves),
-                       0, stream, a);
-  }
+  blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+  if (stream_many_waves(a.N, a.E, a.n_slabs))
+    hipLaunchKernelGGL((stream_gemm_kernel<T, GLU, GATHER, kStreamManyWaves>), dim3((unsigned)blocks), dim3(kWave * kStreamManyWaves), 0, stream, a);
+  else
+    hipLaunchKernelGGL((stream_gemm_kernel<T, GLU, GATHER, kStreamWaves>), dim3((unsigned)blocks), dim3(kStreamThreads), 0, stream, a);
   return check_launch("stream_gemm_kernel");
 }
 
+// partial: room for stream_partial_bytes of this product, or null (the slabs are not shared then)
 template <typename T>
 int stream_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
-                   const void *sched, int N, int K, int E, int H, int I, hipStream_t stream) {
+                   const void *sched, int N, int K, int E, int H, int I, float *partial, hipStream_t stream) {
   StreamArgs a = {};
   a.A = x; a.B = w; a.bias = bias; a.C = act; a.C2 = pre; a.a_rows = sorted_idx; a.a_div = make_fast_div(K);
-  a.sched = (const int *)sched; a.Kd = H; a.Nd = 2 * I; a.lda = H; a.ldc = I;
-  a.n_slabs = ceil_div(2 * I, kSlabCols); a.N = N; a.E = E;
-  return launch_stream<T, true, true>(a, stream);
+  a.sched = (const int *)sched; a.Kd = H; a.Nd = 2 * I; a.lda = H; a.ldc = I; a.N = N; a.E = E;
+  return launch_stream<T, true, true>(a, partial, stream);
 }
 
 template <typename T>
 int stream_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
-                int I, hipStream_t stream) {
+                int I, float *partial, hipStream_t stream) {
   StreamArgs a = {};
   a.A = act; a.B = w; a.bias = bias; a.C = y; a.a_div = make_fast_div(1); a.sched = (const int *)sched;
-  a.Kd = I; a.Nd = H; a.lda = I; a.ldc = H;
-  a.n_slabs = ceil_div(H, kSlabCols); a.N = N; a.E = E;
-  return launch_stream<T, false, false>(a, stream);
+  a.Kd = I; a.Nd = H; a.lda = I; a.ldc = H; a.N = N; a.E = E;
+  return launch_stream<T, false, false>(a, partial, stream);
 }
 
 #define YAMOE_INSTANTIATE_STREAM(T)                                                                                  \
   template int stream_gate_up<T>(const void *, const int *, const void *, const void *, void *, void *, const void *, \
-                                 int, int, int, int, int, hipStream_t);                                              \
-  template int stream_down<T>(const void *, const void *, const void *, void *, const void *, int, int, int, int,    \
-                              hipStream_t);
+                                 int, int, int, int, int, float *, hipStream_t);                                     \
+  template int stream_down<T>(const void *, const void *, const void *, void *, const void *, int, int, int, int, \
+                              float *, hipStream_t);
+YAMOE_INSTANTIATE_STREAM(float)
 YAMOE_INSTANTIATE_STREAM(bf16_t)
 YAMOE_INSTANTIATE_STREAM(f16_t)
 
