@@ -1,0 +1,35 @@
+"""Who works off the streaming list where a call has at most 32 assignments per expert on average: the tile launches, where the
+routing makes tiles, and launches of its own, where it makes none.  Routings made for either, and for both kinds of expert in
+one call; contractions of whole and of cut slab pairs, 128 x 128 and 256 x 256 tiles."""
+import pytest
+import torch
+
+from oracle import yamoe_oracle as O
+from tests.util import REL_L2_TOL, args, to_dev
+from yamoe_amd.workloads import make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def routed(rows):
+    """Expert ids that give expert e rows[e] assignments, in a scrambled order."""
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(rows)])
+    return ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(len(ids)))].view(-1, 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,I", [(256, 192), (136, 520), (1024, 1032)])
+@pytest.mark.parametrize("rows", [[16] * 8, [32, 1, 17, 0, 31, 5, 30, 16], [33, 1, 17, 0, 31, 5, 30, 16], [200, 0, 0, 3, 16, 17, 0, 1],
+                                  [40] * 3 + [0] * 5, [0] * 7 + [255], [1] * 7 + [120]])
+def test_streamed_beside_tiles_or_alone(gpu, dtype, H, I, rows):
+    import yamoe_amd
+    print("carried", dtype, H, I, rows, flush=True)
+    T, E = sum(rows), len(rows)
+    d = make_inputs(T, H, I, E, 1, dtype, seed=T, w_std=0.05, bias_std=0.1)
+    d["router_indices"] = routed(rows)
+    d["routing_weights"] = (0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))).to(dtype)
+    g = args(to_dev(d, gpu))
+    out = yamoe_amd.experts(*g, T, E, 1)
+    want = O.experts_capacity(*args(d), T, compute_dtype=torch.float32)
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
+    assert torch.equal(out, yamoe_amd.experts(*g, T, E, 1))

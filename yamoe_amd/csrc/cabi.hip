@@ -63,17 +63,17 @@ template <typename T>
 int launch_routing_grad(const float *, const int *, const void *, int, int, void *, int, int, int, hipStream_t);
 template <typename T>
 int stream_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int, int,
-                   int, int, float *, hipStream_t);
+                   int, int, float *, bool, hipStream_t);
 template <typename T>
-int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, float *, hipStream_t);
+int stream_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, float *, bool, hipStream_t);
 size_t stream_partial_bytes(int N, int E, int Kd, int Nd, int elem_bytes);
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *, const int *, const void *, const void *, void *, void *, const void *, int, int,
-                       int, int, int, int, bool, hipStream_t);
+                       int, int, int, int, int, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *, const void *, const void *, void *, const void *, int, int, int, int, int,
-                    bool, int, hipStream_t);
+                    int, int, hipStream_t);
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_dgrad(const void *, const int *, int, const void *, void *, const void *, int, int, int, int,
                      const void *, float *, hipStream_t);
@@ -142,7 +142,7 @@ static int gathered_span_ok(const char *who, long long span_bytes) {
 // more first: the kernels address gathered rows with 32-bit byte offsets from the start of the tensor).
 template <typename T>
 static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
-                         const void *sched, int N, int K, int E, int H, int I, int small_rows, bool streams,
+                         const void *sched, int N, int K, int E, int H, int I, int small_rows, int carries,
                          hipStream_t stream) {
   // the gathered source rows span the whole hidden_states tensor: N / K tokens of H elements
   const long long span = sorted_idx != nullptr ? (long long)(N / K) * H * (long long)sizeof(T) : 0;
@@ -150,7 +150,7 @@ static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, co
   if constexpr (sizeof(T) == 2) {
     auto run = H % 64 ? gemm_async_gate_up<T, 256, true> : gemm_async_gate_up<T, 256, false>;
     if (takes_small_tiles(N, E, 2 * I)) run = H % 64 ? gemm_async_gate_up<T, 128, true> : gemm_async_gate_up<T, 128, false>;
-    return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, streams, stream);
+    return run(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, small_rows, carries, stream);
   } else {
     return gemm_f32_gate_up(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, stream);
   }
@@ -158,11 +158,11 @@ static int tiles_gate_up(const void *x, const int *sorted_idx, const void *w, co
 // regular_rows > 0 (16-bit data only): every expert has that many rows, and there is no schedule.
 template <typename T>
 static int tiles_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E,
-                      int H, int I, int small_rows, bool streams, int regular_rows, hipStream_t stream) {
+                      int H, int I, int small_rows, int carries, int regular_rows, hipStream_t stream) {
   if constexpr (sizeof(T) == 2) {
     auto run = I % 64 ? gemm_async_down<T, 256, true> : gemm_async_down<T, 256, false>;
     if (takes_small_tiles(N, E, H)) run = I % 64 ? gemm_async_down<T, 128, true> : gemm_async_down<T, 128, false>;
-    return run(act, w, bias, y, sched, N, E, H, I, small_rows, streams, regular_rows, stream);
+    return run(act, w, bias, y, sched, N, E, H, I, small_rows, carries, regular_rows, stream);
   } else {
     return gemm_f32_down(act, w, bias, y, sched, N, E, H, I, stream);
   }
@@ -370,16 +370,22 @@ static size_t carve_saved(const yamoe_problem *p, void *base, Saved *s) {
     if (rc_ != 0) return rc_;  \
   } while (0)
 
-// Whether the launches of the tile kernels also work off the streaming list, instead of two launches of their own that
-// usually find it empty.  Where every expert has 32 assignments on average, few if any stream; where they do, the carried
-// form has fewer waves on a CU than the streaming kernel, so it is taken only while the launches are short (an expert's last
-// row tile is half full on average, hence the estimate).  150 drawn forwards, carried over launches of their own, where no
-// expert streams and where some do: up to 2 estimated rounds 0.97 and 0.88, up to 4 0.98 and 0.93 (single ones 0.78 to 1.02), up to 8
-// 0.996 and 0.94 (0.80 to 1.035), up to 16 0.998 and 0.98, beyond 1.00: above 4 what is left of the two launches' time no longer
-// covers what some calls lose.
-static bool tiles_carry_streams(int N, int E, int H, int I) {
+// Whether the launches of the tile kernels also work off the streaming list, instead of two launches of their own.
+// CARRY_ALWAYS: where every expert has 32 assignments on average, few if any stream, and those two launches usually find
+// nothing; where experts do stream, the carried form has fewer waves on a CU than the streaming kernel, so it is taken only
+// while the launches are short (an expert's last row tile is half full on average, hence the estimate).  150 drawn forwards,
+// carried over launches of their own, where no expert streams and where some do: up to 2 estimated rounds 0.97 and 0.88, up to 4
+// 0.98 and 0.93 (single ones 0.78 to 1.02), up to 8 0.996 and 0.94 (0.80 to 1.035), up to 16 0.998 and 0.98, beyond 1.00: above 4 what
+// is left of the two launches' time no longer covers what some calls lose.
+// CARRY_WITH_TILES: with fewer assignments it depends on the routing, which the device knows: where there are tiles, their
+// launches carry the list and the streaming launches find it taken, so that short products run side by side rather than one
+// after the other; where there are none, every expert streams in those, and the tiles' launches do nothing.  56 drawn forwards
+// of 4 to 32 assignments per expert, us with launches of their own / always carried / so: Zipf routing 113 x 4 on 32 experts, 1024
+// wide, 72 / 51 / 55, 64 x 4 on 32, 2880 x 1336, 153 / 113 / 117; even routing 323 x 4 on 128, 2048 x 1432, 417 / 459 / 419; in
+// between, 171 x 8 on 64, 2880 wide, 619 / 568 / 571.
+static int tiles_carry_streams(int N, int E, int H, int I) {
   const long long cols = ceil_div(H > 2 * I ? H : 2 * I, kColTile), rows = ((long long)N + 128ll * E) / kRowTile;
-  return N > 32ll * E && rows * cols <= 4 * 256;
+  return rows * cols > 4 * 256 ? CARRY_NOT : N > 32ll * E ? CARRY_ALWAYS : CARRY_WITH_TILES;
 }
 
 template <typename T>
@@ -405,7 +411,7 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   // well.  1723 tokens on 8 experts of 2048 x 2048, 32 rows kept: 60 us; with two tile launches that find no tile in front 68,
   // carried by those 72.
   const bool tiles = !everything && N > stream_rows && p->capacity > stream_rows;
-  const bool carried = sizeof(T) == 2 && tiles && tiles_carry_streams(N, p->E, p->H, p->I);
+  const int carried = sizeof(T) == 2 && tiles ? tiles_carry_streams(N, p->E, p->H, p->I) : CARRY_NOT;
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
@@ -414,11 +420,11 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
     YAMOE_TRY(tiles_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
                                carried, stream));
   }
-  const bool streams = stream_rows > 0 && !carried;
+  const bool streams = stream_rows > 0 && carried != CARRY_ALWAYS, yields = carried == CARRY_WITH_TILES;
   if (streams)
-    YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, b.partial, stream));
+    YAMOE_TRY(stream_gate_up<T>(x, b.sorted_idx, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, b.partial, yields, stream));
   if (tiles) YAMOE_TRY(tiles_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, stream_rows, carried, 0, stream));
-  if (streams) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, b.partial, stream));
+  if (streams) YAMOE_TRY(stream_down<T>(b.act, wd, bd, b.y_perm, b.schedule, N, p->E, p->H, p->I, b.partial, yields, stream));
   YAMOE_TRY(launch_combine<T>(b.y_perm, b.inv_pos, idx, p->idx_i64, rw, p->rw_cols, out, p->T, p->K, p->E, p->H,
                               stream));
   return 0;
@@ -455,12 +461,12 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   if (kept != nullptr) {
     // activations and pre-activations come from the forward
   } else if (streamed) {
-    YAMOE_TRY(stream_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, b.f.partial, stream));
+    YAMOE_TRY(stream_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, b.f.partial, false, stream));
     YAMOE_TRY(yamoe_build_schedule(b.f.counts, b.f.offsets, N, E, cap, 0, b.f.schedule, b.f.schedule_bytes, st));
   } else if (permuted) {
-    YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, false, stream));
+    YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, CARRY_NOT, stream));
   } else {
-    YAMOE_TRY(tiles_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, false, stream));
+    YAMOE_TRY(tiles_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, CARRY_NOT, stream));
   }
   // combine backward: g_y_perm = grad_out[tok] * w, and the bias part of the routing gradient
   YAMOE_TRY(launch_combine_backward<T>(gy, bd, b.f.sorted_idx, b.f.inv_pos, idx, p->idx_i64, rw, p->rw_cols, b.g_y_perm,
@@ -582,16 +588,16 @@ static int check_gemm_shape(const char *who, int N, int E, int H, int I, int dty
 template <typename T>
 static int gate_up_both(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
                         const void *sched, int N, int K, int E, int H, int I, hipStream_t stream) {
-  YAMOE_TRY(tiles_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, 0, false, stream));
+  YAMOE_TRY(tiles_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, 0, CARRY_NOT, stream));
   if constexpr (sizeof(T) == 2)
-    YAMOE_TRY(stream_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, nullptr, stream));
+    YAMOE_TRY(stream_gate_up<T>(x, sorted_idx, w, bias, act, pre, sched, N, K, E, H, I, nullptr, false, stream));
   return 0;
 }
 template <typename T>
 static int down_both(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
                      int I, hipStream_t stream) {
-  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, false, 0, stream));
-  if constexpr (sizeof(T) == 2) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, nullptr, stream));
+  YAMOE_TRY(tiles_down<T>(act, w, bias, y, sched, N, E, H, I, 0, CARRY_NOT, 0, stream));
+  if constexpr (sizeof(T) == 2) YAMOE_TRY(stream_down<T>(act, w, bias, y, sched, N, E, H, I, nullptr, false, stream));
   return 0;
 }
 // The same for E groups of `rows` rows each: whether they stream or are tiles is known on the host, so only one of the two
@@ -602,10 +608,10 @@ static int down_regular(const void *act, const void *w, const void *bias, void *
                         size_t sched_bytes, int E, int rows, int H, int I, hipStream_t stream) {
   const bool streams = rows <= kStreamMaxRows;
   if (sizeof(T) == 2 && !streams)
-    return tiles_down<T>(act, w, bias, y, nullptr, E * rows, E, H, I, kStreamMaxRows, false, rows, stream);
+    return tiles_down<T>(act, w, bias, y, nullptr, E * rows, E, H, I, kStreamMaxRows, CARRY_NOT, rows, stream);
   YAMOE_TRY(regular_schedule(counts, offsets, E, rows, streams ? kStreamMaxRows : 0, sched, sched_bytes, stream));
-  if (streams) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, nullptr, stream);
-  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, 0, false, 0, stream);
+  if (streams) return stream_down<T>(act, w, bias, y, sched, E * rows, E, H, I, nullptr, false, stream);
+  return tiles_down<T>(act, w, bias, y, sched, E * rows, E, H, I, 0, CARRY_NOT, 0, stream);
 }
 
 extern "C" int yamoe_gate_up(const void *x, const int32_t *sorted_idx, const void *gate_up_proj,

@@ -194,8 +194,8 @@ __device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_in
 //                       index of the expert's first row tile, number of row tiles of the expert,
 //                       multiplier and shift that divide by that number, 128-row tiles of the experts before this one}
 //   then              small experts: 4 words each {expert, first sorted row, valid rows, 0}
-//   then              kSchedArrivals counters, zero between launches: how many of the workgroups that share a piece of
-//                     work have left their part of it
+//   then              kSchedArrivals counters, where every expert streams, zero between launches: how many of the workgroups
+//                     that share a slab have left their part of it
 constexpr int kRowTile = 256;  // rows of one MFMA row tile
 constexpr int kColTile = 256;  // columns of one MFMA tile
 constexpr int kSchedHeader = 48;
@@ -246,6 +246,9 @@ __host__ __device__ inline bool sched_may_stream_everything(int N, int E) { retu
 __host__ __device__ inline int sched_max_small(int N, int E) {
   return (N < E ? N : E) + (sched_may_stream_everything(N, E) ? N / kStreamMaxRows : 0) + 1;
 }
+
+// Whether the launches of the tile kernels work off the streaming list as well (see tiles_carry_streams in cabi.hip).
+enum { CARRY_NOT, CARRY_ALWAYS, CARRY_WITH_TILES };
 
 struct ScheduleView {
   const int *hdr;

@@ -19,16 +19,17 @@ extern "C" void yamoe_debug_tile_stamps(void *buffer, int32_t tiles) {
 #endif
 
 // the streaming list of the schedule goes with the tiles
-static void add_streams(async::Args &a, int N, int E) {
+static void add_streams(async::Args &a, int N, int E, int carries) {
   a.n_stream_slabs = ceil_div(a.Nd, kSlabCols);
   const long long items = (long long)(N < E ? N : E) * a.n_stream_slabs;
   a.stream_wgs = items < kXcds * kXcdCus ? ceil_div((int)items, kXcds) : kXcdCus;
   a.small = schedule_view(a.sched, N, E).small;
+  a.carries_alone = carries == CARRY_ALWAYS;
 }
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
-                       const void *sched, int N, int K, int E, int H, int I, int small_rows, bool streams, hipStream_t stream) {
+                       const void *sched, int N, int K, int E, int H, int I, int small_rows, int carries, hipStream_t stream) {
   async::Args a = {};
   a.A = x; a.B = w; a.bias = bias; a.C = act; a.C2 = pre;
   a.a_rows = sorted_idx; a.a_div = make_fast_div(K); a.sched = (const int *)sched;
@@ -39,14 +40,14 @@ int gemm_async_gate_up(const void *x, const int *sorted_idx, const void *w, cons
   a.band_div = make_fast_div(async::kBandRows * a.n_col_tiles);
   const int row_tiles = sched_grid_row_tiles(N, E, small_rows);
   using S = async::Tile<TILE, TILE>;
-  if (!streams) return async::launch<T, S, async::EPI_GLU, true, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
-  add_streams(a, N, E);
+  if (carries == CARRY_NOT) return async::launch<T, S, async::EPI_GLU, true, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
+  add_streams(a, N, E, carries);
   return async::launch<T, S, async::EPI_GLU, true, false, RAGGED, async::FORM_CARRIER>(a, row_tiles, stream);
 }
 
 template <typename T, int TILE, bool RAGGED>
 int gemm_async_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
-                    int I, int small_rows, bool streams, int regular_rows, hipStream_t stream) {
+                    int I, int small_rows, int carries, int regular_rows, hipStream_t stream) {
   async::Args a = {};
   a.A = act; a.B = w; a.bias = bias; a.C = y; a.sched = (const int *)sched;
   a.Kd = I; a.Nd = H; a.lda = I; a.ldb = H; a.ldc = H;
@@ -65,8 +66,8 @@ int gemm_async_down(const void *act, const void *w, const void *bias, void *y, c
     return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_REGULAR>(a, E * a.reg_tiles, stream);
   }
   const int row_tiles = sched_grid_row_tiles(N, E, small_rows);
-  if (!streams) return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
-  add_streams(a, N, E);
+  if (carries == CARRY_NOT) return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_LIST>(a, row_tiles, stream);
+  add_streams(a, N, E, carries);
   return async::launch<T, S, async::EPI_STORE, false, false, RAGGED, async::FORM_CARRIER>(a, row_tiles, stream);
 }
 
@@ -93,9 +94,9 @@ int gemm_async_dgrad(const void *g, const int *g_rows, int g_div, const void *w,
 
 #define YAMOE_INSTANTIATE_ASYNC(T, TILE, RAGGED)                                                                        \
   template int gemm_async_gate_up<T, TILE, RAGGED>(const void *, const int *, const void *, const void *, void *,       \
-                                                   void *, const void *, int, int, int, int, int, int, bool, hipStream_t);    \
+                                                   void *, const void *, int, int, int, int, int, int, int, hipStream_t);     \
   template int gemm_async_down<T, TILE, RAGGED>(const void *, const void *, const void *, void *, const void *, int,    \
-                                                int, int, int, int, bool, int, hipStream_t);                                  \
+                                                int, int, int, int, int, int, hipStream_t);                                   \
   template int gemm_async_dgrad<T, TILE, RAGGED>(const void *, const int *, int, const void *, void *, const void *,    \
                                                  int, int, int, int, const void *, float *, hipStream_t);
 #ifndef YAMOE_INSTANTIATE_ROWS

@@ -103,6 +103,7 @@ struct Args {
   // FORM_CARRIER: the schedule's streaming list is worked off by stream_wgs workgroups of every XCD in this launch
   const int *small;
   int stream_wgs, n_stream_slabs;
+  bool carries_alone;  // also where there is no tile (otherwise streaming launches of their own do it then)
   // FORM_REGULAR: every expert has reg_rows rows, cut into reg_tiles tiles of reg_per_tile; reg_units = experts times column
   // tiles, reg_div and reg_tile_div divide by an expert's tiles of all columns and of one
   int reg_rows, reg_tiles, reg_per_tile, reg_units;
@@ -739,6 +740,7 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     if constexpr (FORM == FORM_CARRIER) {
       const int k = place - (int)(gridDim.x / kXcds - stream_wgs);  // behind the tiles
       if (k >= 0) {
+        if (total == 0 && !args.carries_alone) return;
         stream_items<T, EPI, GATHER, S::kPerSimd == 1 ? 3 : 2>(args, k * kXcds + xcd, stream_wgs * kXcds);
         return;
       }

@@ -164,14 +164,16 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
                                            int stream_max_rows, int *sched, const int lane) {
   int *row_tiles = sched + kSchedHeader;
   int *small = row_tiles + 8 * sched_max_row_tiles(N, E);
-  int *arrivals = small + 4 * sched_max_small(N, E);
-  for (int i = lane; i < kSchedArrivals; i += kWave) arrivals[i] = 0;
   int n_tiles = 0, n_small = 0, n_active = 0, n_kept = 0, n_half = 0;
   // Experts of 17 to 32 rows stream only when every expert streams: next to experts that need the tile kernels anyway
   // they are better off as tiles (two half-filled launches one after the other are slower than one: 0.35 against
   // 0.31 ms for 32 experts of about 32 rows, where 0.27 against 0.31 ms is gained when all of them have at most 32).
   const bool everything = stream_max_rows == kStreamEverything;  // (the host checked sched_may_stream_everything)
-  if (everything) stream_max_rows = kStreamMaxRows;
+  if (everything) {  // (only then do workgroups share slabs: see stream.hip)
+    stream_max_rows = kStreamMaxRows;
+    int *arrivals = small + 4 * sched_max_small(N, E);
+    for (int i = lane; i < kSchedArrivals; i += kWave) arrivals[i] = 0;
+  }
   if (!everything && stream_max_rows > kStreamMixedRows) {
     bool beyond = false;
     for (int base = lane; base < E; base += kWave) beyond |= min(counts[base], capacity) > stream_max_rows;

@@ -62,6 +62,7 @@ template <typename T, bool GLU, bool GATHER, int WAVES>
 __global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void stream_gemm_kernel(const StreamArgs args) {
   __shared__ float red[kStreamWaves * 8 * 4 * kWave];  // [wave][j][v][lane]
   const ScheduleView sv = schedule_view(args.sched, args.N, args.E);
+  if (args.yields && sv.hdr[0] > 0) return;
   const int slabs = sv.hdr[1] * args.n_slabs;
   const int parts = args.partial != nullptr ? stream_parts(slabs, ceil_div(args.Kd, StreamStep<T>::kRows), WAVES) : 1;
   const int total = slabs * parts;
@@ -121,8 +122,9 @@ static int launch_stream(StreamArgs a, float *partial, hipStream_t stream) {
 // partial: room for stream_partial_bytes of this product, or null (the slabs are not shared then)
 template <typename T>
 int stream_gate_up(const void *x, const int *sorted_idx, const void *w, const void *bias, void *act, void *pre,
-                   const void *sched, int N, int K, int E, int H, int I, float *partial, hipStream_t stream) {
+                   const void *sched, int N, int K, int E, int H, int I, float *partial, bool yields, hipStream_t stream) {
   StreamArgs a = {};
+  a.yields = yields;
   a.A = x; a.B = w; a.bias = bias; a.C = act; a.C2 = pre; a.a_rows = sorted_idx; a.a_div = make_fast_div(K);
   a.sched = (const int *)sched; a.Kd = H; a.Nd = 2 * I; a.lda = H; a.ldc = I; a.N = N; a.E = E;
   return launch_stream<T, true, true>(a, partial, stream);
@@ -130,8 +132,9 @@ int stream_gate_up(const void *x, const int *sorted_idx, const void *w, const vo
 
 template <typename T>
 int stream_down(const void *act, const void *w, const void *bias, void *y, const void *sched, int N, int E, int H,
-                int I, float *partial, hipStream_t stream) {
+                int I, float *partial, bool yields, hipStream_t stream) {
   StreamArgs a = {};
+  a.yields = yields;
   a.A = act; a.B = w; a.bias = bias; a.C = y; a.a_div = make_fast_div(1); a.sched = (const int *)sched;
   a.Kd = I; a.Nd = H; a.lda = I; a.ldc = H; a.N = N; a.E = E;
   return launch_stream<T, false, false>(a, partial, stream);
@@ -139,9 +142,9 @@ int stream_down(const void *act, const void *w, const void *bias, void *y, const
 
 #define YAMOE_INSTANTIATE_STREAM(T)                                                                                  \
   template int stream_gate_up<T>(const void *, const int *, const void *, const void *, void *, void *, const void *, \
-                                 int, int, int, int, int, float *, hipStream_t);                                     \
+                                 int, int, int, int, int, float *, bool, hipStream_t);                                     \
   template int stream_down<T>(const void *, const void *, const void *, void *, const void *, int, int, int, int, \
-                              float *, hipStream_t);
+                              float *, bool, hipStream_t);
 YAMOE_INSTANTIATE_STREAM(float)
 YAMOE_INSTANTIATE_STREAM(bf16_t)
 YAMOE_INSTANTIATE_STREAM(f16_t)

@@ -76,6 +76,7 @@ struct StreamArgs {
   // finishes the slab.
   int part_floats;
   bool per_xcd;  // neighbouring slabs go to one XCD
+  bool yields;   // where there are tiles, their launches carry the list
   float *partial;
   int *arrivals;
 };
