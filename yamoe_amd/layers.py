@@ -81,6 +81,19 @@ def router_kernel_takes(x_flat, weight, top_k, with_grad=False):
     return ok
 
 
+def _option(module, name, default):
+    """getattr(module, name, default).  A torch module answers for a name that it does not have with an exception, 2 us of host
+    time each; whether it has it is looked up first."""
+    kind = type(module)
+    if getattr(kind, "__getattr__", None) is torch.nn.Module.__getattr__ and not hasattr(kind, name):
+        own = module.__dict__
+        if name in own:
+            return own[name]
+        if name not in own["_parameters"] and name not in own["_buffers"] and name not in own["_modules"]:
+            return default
+    return getattr(module, name, default)
+
+
 class Yamoe(torch.nn.Module):
     """Drop-in `forward` for a GPT-OSS MLP block (router + experts), the role of `Yamoe.forward` in
     drbh/yamoe (torch-ext/yamoe/layers.py:106-218).  The host module provides `self.router`
@@ -102,11 +115,15 @@ class Yamoe(torch.nn.Module):
 
     def forward(self, hidden_states):
         batch, seq, hidden = hidden_states.shape
-        num_experts = getattr(self, "num_experts", 32)
-        top_k = getattr(self, "top_k", 4)
-        timing = getattr(self, "_timing_enabled", False)
+        num_experts = _option(self, "num_experts", 32)
+        top_k = _option(self, "top_k", 4)
+        timing = _option(self, "_timing_enabled", False)
         stats = {}
         self._timing_stats = stats   # reset on every call, like the reference's (layers.py:119-122)
+        # (every look-up of a submodule or parameter is a Python call; one token on 128 experts, 1024 wide, is 35 us of GPU time
+        # and was 39 us of host time, of which these and the slices below were half)
+        router, experts = self.router, self.experts
+        router_weight, router_bias = router.weight, router.bias
 
         def lap(name, since):
             torch.cuda.synchronize()
@@ -118,21 +135,21 @@ class Yamoe(torch.nn.Module):
             torch.cuda.synchronize()
             t0 = time.perf_counter()
         x_flat = hidden_states.reshape(-1, hidden)
-        want_router_grads = torch.is_grad_enabled() and getattr(self, "enable_router_grads", False)
-        if router_kernel_takes(x_flat, self.router.weight, top_k, with_grad=want_router_grads):
+        want_router_grads = torch.is_grad_enabled() and _option(self, "enable_router_grads", False)
+        if router_kernel_takes(x_flat, router_weight, top_k, with_grad=want_router_grads):
             # linear + top-k + softmax + dense scatter in one kernel (and, for a router that is being trained, the
             # gradient of the four steps on the HIP kernels as well)
             if want_router_grads:
-                router_indices, router_scores = _RouterFn.apply(x_flat, self.router.weight, self.router.bias, top_k)
+                router_indices, router_scores = _RouterFn.apply(x_flat, router_weight, router_bias, top_k)
             else:
-                router_indices, router_scores = ops.router_topk(x_flat, self.router.weight, self.router.bias, top_k)
+                router_indices, router_scores = ops.router_topk(x_flat, router_weight, router_bias, top_k)
             if timing:
                 t1 = lap("router", t0)
                 stats["topk_softmax"] = 0.0
         else:
             # the same four steps as torch ops on the GPU, for shapes the kernels do not take (more than 256 experts,
             # hidden sizes or, with gradients, expert counts that are not multiples of 16 bytes)
-            logits = torch.nn.functional.linear(x_flat, self.router.weight, self.router.bias)
+            logits = torch.nn.functional.linear(x_flat, router_weight, router_bias)
             if timing:
                 t1 = lap("router", t0)
             top_vals, router_indices = torch.topk(logits, top_k, dim=-1)
@@ -140,11 +157,15 @@ class Yamoe(torch.nn.Module):
             router_scores = torch.zeros_like(logits).scatter_(1, router_indices, top_w)
             if timing:
                 t1 = lap("topk_softmax", t1)
-        I = self.experts.down_proj.shape[1]
-        gate_up = self.experts.gate_up_proj[:, :, : 2 * I].contiguous()
-        gate_up_bias = self.experts.gate_up_proj_bias[:, : 2 * I].contiguous()
+        down, down_bias = experts.down_proj, experts.down_proj_bias
+        gate_up, gate_up_bias = experts.gate_up_proj, experts.gate_up_proj_bias
+        I = down.shape[1]
+        if gate_up.shape[2] != 2 * I or not gate_up.is_contiguous():
+            gate_up = gate_up[:, :, : 2 * I].contiguous()
+        if gate_up_bias.shape[1] != 2 * I or not gate_up_bias.is_contiguous():
+            gate_up_bias = gate_up_bias[:, : 2 * I].contiguous()
         tokens = x_flat.shape[0]
-        capacity = getattr(self, "expert_capacity", None)
+        capacity = _option(self, "expert_capacity", None)
         if capacity is None:
             capacity = tokens
         elif capacity == "reference":
@@ -155,12 +176,15 @@ class Yamoe(torch.nn.Module):
             del stats["setup"]
         if want_router_grads:
             out = experts_autograd(x_flat, router_indices, router_scores, gate_up, gate_up_bias,
-                                   self.experts.down_proj, self.experts.down_proj_bias, capacity, num_experts, top_k,
-                                   True, bool(getattr(self, "save_activations", False)))
-        else:
+                                   down, down_bias, capacity, num_experts, top_k,
+                                   True, bool(_option(self, "save_activations", False)))
+        elif torch.is_grad_enabled():
             with torch.no_grad():
-                out = ops.experts(x_flat, router_indices, router_scores, gate_up, gate_up_bias,
-                                  self.experts.down_proj, self.experts.down_proj_bias, capacity, num_experts, top_k)
+                out = ops.experts(x_flat, router_indices, router_scores, gate_up, gate_up_bias, down, down_bias, capacity,
+                                  num_experts, top_k)
+        else:
+            out = ops.experts(x_flat, router_indices, router_scores, gate_up, gate_up_bias, down, down_bias, capacity, num_experts,
+                              top_k)
         if timing:
             lap("experts_kernel", t1)
             lap("total", t0)
