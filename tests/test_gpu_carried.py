@@ -33,3 +33,26 @@ def test_streamed_beside_tiles_or_alone(gpu, dtype, H, I, rows):
     want = O.experts_capacity(*args(d), T, compute_dtype=torch.float32)
     assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
     assert torch.equal(out, yamoe_amd.experts(*g, T, E, 1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,I", [(64, 2304), (136, 2312)])
+@pytest.mark.parametrize("rows,capacity", [([270] * 8, 0), ([257, 288, 256, 289, 512, 513, 544, 545], 0), ([288] * 7 + [20], 0),
+                                           ([300] * 8, 272), ([400] * 8, 256), ([1, 16, 33, 0] + [272] * 8, 0)])
+def test_last_rows_beside_whole_tiles(gpu, dtype, H, I, rows, capacity):
+    """Experts of a few rows more than whole tiles, in numbers that make the wider product a round longer: those rows stream."""
+    import yamoe_amd
+    print("remainders", dtype, H, I, rows, capacity, flush=True)
+    T, E = sum(rows), len(rows)
+    d = make_inputs(T, H, I, E, 1, dtype, seed=T, w_std=0.05, bias_std=0.1)
+    d["router_indices"] = routed(rows)
+    d["routing_weights"] = (0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))).to(dtype)
+    g = args(to_dev(d, gpu))
+    capacity = capacity or T
+    out, kept = yamoe_amd.experts_keep(*g, capacity, E, 1)
+    assert torch.equal(out, yamoe_amd.experts(*g, capacity, E, 1))
+    want = O.experts_capacity(*args(d), capacity, compute_dtype=torch.float32)
+    assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
+    gy = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(dtype).to(gpu)
+    for a, b in zip(yamoe_amd.experts_backward_kept(gy, *g, kept, capacity, E, 1), yamoe_amd.experts_backward(gy, *g, capacity, E, 1)):
+        assert O.rel_l2(a.cpu(), b.cpu()) < REL_L2_TOL[dtype]

@@ -68,3 +68,21 @@ def test_fp32_batch_mm_of_few_rows(gpu, C):
     y = torch.empty(E, C, Nd, device=gpu)
     yamoe_amd.batch_mm(x.to(gpu), w.to(gpu), torch.full((E,), C, dtype=torch.int32, device=gpu), y)
     assert O.rel_l2(y.cpu(), torch.bmm(x.double(), w.double())) < REL_L2_TOL[torch.float32]
+
+
+@pytest.mark.parametrize("T,H,I,E,K,one", [(60, 264, 200, 8, 2, False), (128, 136, 264, 8, 1, True), (129, 136, 264, 8, 1, True),
+                                           (64, 512, 1000, 16, 4, False), (65, 512, 72, 16, 4, False)])
+def test_fp32_up_to_sixteen_assignments_per_expert(gpu, T, H, I, E, K, one):
+    """Streamed up to there, tiles beyond; a whole batch on one expert in chunks of 32 rows."""
+    import yamoe_amd
+    d = make_inputs(T, H, I, E, K, torch.float32, seed=T, w_std=0.05, bias_std=0.1, zipf=1.2)
+    if one:
+        d["router_indices"] = torch.full_like(d["router_indices"], 5)
+        d["routing_weights"] = 0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))
+    g = args(to_dev(d, gpu))
+    out = yamoe_amd.experts(*g, T, E, K)
+    assert O.rel_l2(out.cpu(), O.experts_capacity(*args(d), T, compute_dtype=torch.float64)) < REL_L2_TOL[torch.float32]
+    gy = torch.randn(T, H, generator=torch.Generator().manual_seed(3))
+    want = O.experts_backward(gy, *args(d), T, compute_dtype=torch.float64)
+    for a, b in zip(yamoe_amd.experts_backward(gy.to(gpu), *g, T, E, K), want):
+        assert O.rel_l2(a.cpu(), b) < REL_L2_TOL[torch.float32]

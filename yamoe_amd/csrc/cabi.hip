@@ -106,9 +106,10 @@ template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
 // Experts of at most this many kept rows stream their weights instead of going through the tile kernels (0: none does).  fp32 data
 // streams where every expert does: beside tiles, whose launch takes as long for one of them as for a round, a second pair of
-// launches costs more than it takes off them (64 tokens x 2 on 16 skewed experts, 2048 x 744: 122 us as tiles, 173 so).
+// launches costs more than it takes off them (64 tokens x 2 on 16 skewed experts, 2048 x 744: 122 us as tiles, 173 with some
+// streamed, 94 with all).
 static int stream_rows_of(int dtype, int N, int E) {
-  return dtype != YAMOE_F32 || sched_may_stream_everything(N, E) ? kStreamMaxRows : 0;
+  return dtype != YAMOE_F32 || sched_may_stream_everything(N, E, 4) ? kStreamMaxRows : 0;
 }
 
 // Whether a product of N rows over E experts with Nd columns runs on 128 x 128 tiles (two workgroups per CU) instead of
@@ -304,7 +305,7 @@ static size_t carve_forward(const yamoe_problem *p, void *ws, ForwardBuffers *b)
   b->y_perm = c.take(N * (size_t)(p->H > p->I ? p->H : p->I) * es);
   b->x_perm = gathers_need_permute(p) ? c.take(N * p->H * es) : nullptr;
   size_t partial = 0;
-  if (!takes_plain_path(p) && sched_may_stream_everything((int)N, p->E)) {
+  if (!takes_plain_path(p) && sched_may_stream_everything((int)N, p->E, (int)es)) {
     const size_t gate_up = stream_partial_bytes((int)N, p->E, p->H, 2 * p->I, (int)es), down = stream_partial_bytes((int)N, p->E, p->I, p->H, (int)es);
     partial = gate_up > down ? gate_up : down;
   }
@@ -382,10 +383,13 @@ static size_t carve_saved(const yamoe_problem *p, void *base, Saved *s) {
 // after the other; where there are none, every expert streams in those, and the tiles' launches do nothing.  56 drawn forwards
 // of 4 to 32 assignments per expert, us with launches of their own / always carried / so: Zipf routing 113 x 4 on 32 experts, 1024
 // wide, 72 / 51 / 55, 64 x 4 on 32, 2880 x 1336, 153 / 113 / 117; even routing 323 x 4 on 128, 2048 x 1432, 417 / 459 / 419; in
-// between, 171 x 8 on 64, 2880 wide, 619 / 568 / 571.
+// between, 171 x 8 on 64, 2880 wide, 619 / 568 / 571.  In launches of 4 to 16 estimated rounds, apart / so: 155 x 4 on 128, Zipf, 2880 x
+// 2080, 249 / 218, 744 x 4 on 128, even, 2048 wide, 612 / 584, 815 x 4, Zipf, 2880 wide, 571 / 569, but 916 x 4 578 / 593: there up to 24
+// assignments per expert.
 static int tiles_carry_streams(int N, int E, int H, int I) {
   const long long cols = ceil_div(H > 2 * I ? H : 2 * I, kColTile), rows = ((long long)N + 128ll * E) / kRowTile;
-  return rows * cols > 4 * 256 ? CARRY_NOT : N > 32ll * E ? CARRY_ALWAYS : CARRY_WITH_TILES;
+  if (rows * cols <= 4 * 256) return N > 32ll * E ? CARRY_ALWAYS : CARRY_WITH_TILES;
+  return rows * cols <= 16 * 256 && N <= 24ll * E ? CARRY_WITH_TILES : CARRY_NOT;
 }
 
 template <typename T>
@@ -403,15 +407,16 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   // At most 4 assignments per expert on average (decode): every expert goes to the streaming kernel, in chunks of
   // stream_rows rows where one has more, and the tile kernels, whose lists are then empty, are not launched (two
   // launches of 4.5 us each that found nothing to do at 64 tokens on 128 experts).
-  const bool everything = sched_may_stream_everything(N, p->E);
-  YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
-                               b.inv_pos, b.route_ws, b.route_ws_bytes, everything ? kStreamEverything : stream_rows,
-                               b.schedule, b.schedule_bytes, st));
+  const bool everything = sched_may_stream_everything(N, p->E, (int)sizeof(T));
   // where the assignments or the capacity leave no expert more rows than a streamed one may have, every expert is streamed as
   // well.  1723 tokens on 8 experts of 2048 x 2048, 32 rows kept: 60 us; with two tile launches that find no tile in front 68,
   // carried by those 72.
   const bool tiles = !everything && N > stream_rows && p->capacity > stream_rows;
   const int carried = sizeof(T) == 2 && tiles ? tiles_carry_streams(N, p->E, p->H, p->I) : CARRY_NOT;
+  const int tile_cols = carried != CARRY_NOT && !takes_small_tiles(N, p->E, 2 * p->I) ? ceil_div(2 * p->I, kColTile) : 0;
+  YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
+                               b.inv_pos, b.route_ws, b.route_ws_bytes, everything ? kStreamEverything : stream_rows, tile_cols,
+                               b.schedule, b.schedule_bytes, st));
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
@@ -452,7 +457,7 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   // other products run on the tile kernels and get their lists afterwards.
   const bool streamed = sizeof(T) == 4 && kept == nullptr && stream_rows_of(p->dtype, N, E) > 0;
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, E, cap, b.f.sorted_expert, b.f.sorted_idx, b.f.counts, b.f.offsets,
-                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, streamed ? kStreamEverything : 0, b.f.schedule,
+                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, streamed ? kStreamEverything : 0, 0, b.f.schedule,
                                b.f.schedule_bytes, st));
   // forward recompute of the first product only: activations and pre-activations
   const bool permuted = b.gy_perm != nullptr;  // hidden_states and grad_out too large to gather from
@@ -517,7 +522,7 @@ static int forward_plain(const yamoe_problem *p, const void *x, const void *idx,
   const int N = p->T * p->K;
   if (N == 0 || p->T == 0) return 0;
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
-                               b.inv_pos, b.route_ws, b.route_ws_bytes, 0, b.schedule, b.schedule_bytes, (void *)stream));
+                               b.inv_pos, b.route_ws, b.route_ws_bytes, 0, 0, b.schedule, b.schedule_bytes, (void *)stream));
   return plain_forward<T>(x, idx, p->idx_i64, rw, p->rw_cols, wgu, bgu, wd, bd, out, b.sorted_idx, b.inv_pos, b.schedule,
                           keep ? keep->act : b.act, keep ? keep->pre : nullptr, b.y_perm, p->T, p->K, p->E, p->H, p->I, stream);
 }
@@ -539,7 +544,7 @@ static int backward_plain(const yamoe_problem *p, const void *gy, const void *x,
     return 0;
   }
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, E, cap, b.f.sorted_expert, b.f.sorted_idx, b.f.counts, b.f.offsets,
-                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, 0, b.f.schedule, b.f.schedule_bytes,
+                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, 0, 0, b.f.schedule, b.f.schedule_bytes,
                                (void *)stream));
   return plain_backward<T>(gy, x, idx, p->idx_i64, rw, p->rw_cols, wgu, bgu, wd, bd, d_x, d_rw, d_wgu, d_bgu, d_wd, d_bd,
                       b.f.sorted_expert, b.f.sorted_idx, b.f.inv_pos, b.f.counts, b.f.offsets, b.f.schedule, b.f.act, b.pre,

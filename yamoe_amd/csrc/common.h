@@ -193,7 +193,7 @@ __device__ inline int wave_sum(int v) { return __builtin_amdgcn_readlane(wave_in
 //   [48 ...)          row tiles: 8 words each  {expert, first sorted row, valid rows,
 //                       index of the expert's first row tile, number of row tiles of the expert,
 //                       multiplier and shift that divide by that number, 128-row tiles of the experts before this one}
-//   then              small experts: 4 words each {expert, first sorted row, valid rows, 0}
+//   then              small experts, or the last rows of others: 4 words each {expert, first sorted row, valid rows, 0}
 //   then              kSchedArrivals counters, where every expert streams, zero between launches: how many of the workgroups
 //                     that share a slab have left their part of it
 constexpr int kRowTile = 256;  // rows of one MFMA row tile
@@ -239,12 +239,16 @@ __host__ __device__ inline int sched_grid_row_tiles(int N, int E, int small_rows
   return N / kRowTile + tiled + 1;
 }
 // Every expert may be put on the streaming list in chunks of at most kStreamMaxRows rows (stream_max_rows =
-// kStreamEverything) when there are at most 4 assignments per expert on average: the weights of an expert with more
-// rows than one chunk are then read once per chunk, which is rare at that load, and the tile kernels are not launched.
+// kStreamEverything) when there are few assignments per expert on average: the weights of an expert with more rows than
+// one chunk are then read once per chunk, which is rare at that load, and the tile kernels are not launched.  16-bit data up
+// to 4; fp32, whose tiles cost as much for a row as for 32, up to 16 (us as tiles / streamed, 64 x 2
+// tokens on 16 experts of 2880 x 2880 490 / 302, 128 x 2 492 / 418, Zipf routing 572 / 405; 24 per expert as tiles 494).  The list has room for either.
 constexpr int kStreamEverything = -1;
-__host__ __device__ inline bool sched_may_stream_everything(int N, int E) { return N <= 4 * E; }
+__host__ __device__ inline bool sched_may_stream_everything(int N, int E, int elem_bytes) {
+  return N <= (elem_bytes == 4 ? 16ll : 4ll) * E;
+}
 __host__ __device__ inline int sched_max_small(int N, int E) {
-  return (N < E ? N : E) + (sched_may_stream_everything(N, E) ? N / kStreamMaxRows : 0) + 1;
+  return (N < E ? N : E) + (sched_may_stream_everything(N, E, 4) ? N / kStreamMaxRows : 0) + 1;
 }
 
 // Whether the launches of the tile kernels work off the streaming list as well (see tiles_carry_streams in cabi.hip).
@@ -268,7 +272,7 @@ __host__ __device__ inline ScheduleView schedule_view(const void *p, int N, int 
 
 int route_and_schedule(const void *router_indices, int32_t idx_i64, int32_t N, int32_t E, int32_t capacity,
                        int32_t *sorted_expert, int32_t *sorted_idx, int32_t *counts, int32_t *offsets, int32_t *inv_pos,
-                       void *workspace, size_t workspace_bytes, int32_t stream_max_rows, void *schedule,
+                       void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t tile_cols, void *schedule,
                        size_t schedule_bytes, void *stream);
 
 int regular_schedule(int *counts, int *offsets, int E, int rows, int stream_max_rows, void *schedule, size_t schedule_bytes,

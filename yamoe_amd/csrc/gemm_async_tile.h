@@ -683,6 +683,7 @@ template <typename T, int EPI, bool GATHER, int DEPTH> __device__ __forceinline_
   StreamArgs a = {};
   a.A = args.A; a.B = args.B; a.bias = args.bias; a.C = args.C; a.C2 = args.C2; a.a_rows = args.a_rows; a.a_div = args.a_div;
   a.Kd = args.Kd; a.Nd = args.Nd; a.lda = args.lda; a.ldc = args.ldc;
+  if (args.sched[0] == 0 && !args.carries_alone) return;
   const int items = args.sched[1] * args.n_stream_slabs;
   for (int it = first; it < items; it += step) {
     const int s = it / args.n_stream_slabs;
@@ -740,7 +741,6 @@ __global__ __launch_bounds__(kThreads, S::kPerSimd) void gemm_async_kernel(const
     if constexpr (FORM == FORM_CARRIER) {
       const int k = place - (int)(gridDim.x / kXcds - stream_wgs);  // behind the tiles
       if (k >= 0) {
-        if (total == 0 && !args.carries_alone) return;
         stream_items<T, EPI, GATHER, S::kPerSimd == 1 ? 3 : 2>(args, k * kXcds + xcd, stream_wgs * kXcds);
         return;
       }

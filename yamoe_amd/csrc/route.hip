@@ -157,17 +157,26 @@ __device__ inline void first_wave_exclusive_scan(const int *total, int *offsets,
 }
 
 // ---- work lists ------------------------------------------------------------------------------
+// Which experts stream: see build_schedule_wave.  cols: the column tiles of the wider product where an expert's last rows may stream, else 0.
+struct StreamRule { int max_rows, cols; };
+// Where an expert has a few rows more than whole tiles, cutting all of them into equal tiles takes one tile more, which costs
+// little in a launch of many rounds and a whole round where it is the first tile of one.  There those rows go to the
+// streaming list, if that saves the wider product a round: its launch then carries them on CUs that have no tile.  2003 tokens x
+// 4 on 32 experts, 2880 x 720, 258 gate_up tiles on 256 CUs: 128 + 72 us, and 89 + 64 with 12 experts' last rows streamed.
+constexpr int kRemainderRounds = 4;  // (beyond, a round is little of a launch)
+
 // One wave; lane l takes experts l, l+64, ...  Experts with 1..stream_max_rows kept rows go to the
 // streaming list, larger ones are cut into row tiles of kRowTile rows.  Both lists stay in expert
 // order: positions come from wave prefix sums.
 __device__ inline void build_schedule_wave(const int *counts, const int *offsets, int N, int E, int capacity,
-                                           int stream_max_rows, int *sched, const int lane) {
+                                           StreamRule streams, int *sched, const int lane) {
   int *row_tiles = sched + kSchedHeader;
   int *small = row_tiles + 8 * sched_max_row_tiles(N, E);
   int n_tiles = 0, n_small = 0, n_active = 0, n_kept = 0, n_half = 0;
   // Experts of 17 to 32 rows stream only when every expert streams: next to experts that need the tile kernels anyway
   // they are better off as tiles (two half-filled launches one after the other are slower than one: 0.35 against
   // 0.31 ms for 32 experts of about 32 rows, where 0.27 against 0.31 ms is gained when all of them have at most 32).
+  int stream_max_rows = streams.max_rows;
   const bool everything = stream_max_rows == kStreamEverything;  // (the host checked sched_may_stream_everything)
   if (everything) {  // (only then do workgroups share slabs: see stream.hip)
     stream_max_rows = kStreamMaxRows;
@@ -179,34 +188,52 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     for (int base = lane; base < E; base += kWave) beyond |= min(counts[base], capacity) > stream_max_rows;
     if (__any(beyond)) stream_max_rows = kStreamMixedRows;
   }
+  // an expert's tiled rows: all of them, or (`remainders`) whole tiles' worth
+  auto tiled_rows = [&](int kept, bool remainders) {
+    if (kept <= stream_max_rows || everything) return 0;
+    const int past = kept % kRowTile;
+    return remainders && kept > kRowTile && past <= kStreamMaxRows ? kept - past : kept;
+  };
+  bool remainders = false;
+  if (streams.cols > 0 && !everything) {
+    int all = 0, fewer = 0;
+    for (int base = 0; base < E; base += kWave) {
+      const int kept = base + lane < E ? max(min(counts[base + lane], capacity), 0) : 0;
+      all += wave_sum(ceil_div(tiled_rows(kept, false), kRowTile));
+      fewer += wave_sum(ceil_div(tiled_rows(kept, true), kRowTile));
+    }
+    const int rounds = ceil_div(all * streams.cols, kXcds * kXcdCus);
+    remainders = rounds <= kRemainderRounds && ceil_div(fewer * streams.cols, kXcds * kXcdCus) < rounds;
+  }
   for (int base = 0; base < E; base += kWave) {
     int e = base + lane;
     int kept = e < E ? min(counts[e], capacity) : 0;
     if (kept < 0) kept = 0;
     int first = e < E ? offsets[e] : 0;
     // entries on the streaming list: one, or with `everything` one per chunk of kStreamMaxRows rows
-    int is_small = everything ? ceil_div(kept, kStreamMaxRows) : (kept > 0 && kept <= stream_max_rows);
-    int tiles = (kept > 0 && !is_small) ? ceil_div(kept, kRowTile) : 0;
+    const int tiled = tiled_rows(kept, remainders);
+    int is_small = everything ? ceil_div(kept, kStreamMaxRows) : kept > tiled;
+    int tiles = ceil_div(tiled, kRowTile);
     int tot_small, tot_tiles, tot_half;
     int pos_small = wave_exclusive_scan(is_small, tot_small);
     int pos_tiles = wave_exclusive_scan(tiles, tot_tiles);
-    const int halves = tiles > 0 ? ceil_div(kept, kRowTile / 2) : 0;
+    const int halves = ceil_div(tiled, kRowTile / 2);
     const int pos_half = n_half + wave_exclusive_scan(halves, tot_half);
     const int tot_active = __popcll(__ballot(kept > 0)), tot_kept = wave_sum(kept);
     for (int c = 0; c < is_small; ++c) {
       int *s = small + 4 * (n_small + pos_small + c);
-      s[0] = e; s[1] = first + c * kStreamMaxRows; s[2] = min(kStreamMaxRows, kept - c * kStreamMaxRows); s[3] = 0;
+      s[0] = e; s[1] = first + tiled + c * kStreamMaxRows; s[2] = min(kStreamMaxRows, kept - tiled - c * kStreamMaxRows); s[3] = 0;
     }
     int gfirst = n_tiles + pos_tiles;
     // An expert's rows are cut into equal tiles (a multiple of 32 rows, the MFMA block), not into full
     // tiles plus a remainder: tiles of one expert then advance through the contraction at the same pace
     // and the weight slabs one of them fetches are still in L2 when the others ask for them.
-    int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(kept, tiles) + 31) & ~31) : 0;
+    int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(tiled, tiles) + 31) & ~31) : 0;
     FastDiv by_tiles = {1u, 0u};  // the GEMM kernels divide by the group size (a 64-bit division: only where there is a group)
     if (tiles > 1) by_tiles = make_fast_div(tiles);
     for (int t = 0; t < tiles; ++t) {
       int *w = row_tiles + 8 * (gfirst + t);
-      w[0] = e; w[1] = first + t * per_tile; w[2] = min(per_tile, kept - t * per_tile); w[3] = gfirst; w[4] = tiles;
+      w[0] = e; w[1] = first + t * per_tile; w[2] = min(per_tile, tiled - t * per_tile); w[3] = gfirst; w[4] = tiles;
       w[5] = (int)by_tiles.mul; w[6] = (int)by_tiles.shift; w[7] = pos_half;
     }
     n_small += tot_small; n_tiles += tot_tiles; n_active += tot_active; n_kept += tot_kept; n_half += tot_half;
@@ -214,10 +241,10 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   // Second pass: cut the tile list into 8 shares of equal cost.  Groups (experts with row tiles) are weighed
   // by the sum of their tiles' weights; cut x falls into the group that contains x/8 of the total.
   auto group = [&](int e, int &tiles) {
-    int kept = e < E ? min(counts[e], capacity) : 0;
-    tiles = kept > 0 && !everything && kept > stream_max_rows ? ceil_div(kept, kRowTile) : 0;
-    const int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(kept, tiles) + 31) & ~31) : 0;
-    return sched_group_weight(tiles, per_tile, kept);
+    const int tiled = tiled_rows(e < E ? max(min(counts[e], capacity), 0) : 0, remainders);
+    tiles = ceil_div(tiled, kRowTile);
+    const int per_tile = tiles > 0 ? min(kRowTile, (ceil_div(tiled, tiles) + 31) & ~31) : 0;
+    return sched_group_weight(tiles, per_tile, tiled);
   };
   int w_total = 0, tiles;
   if (n_tiles > 0)
@@ -259,16 +286,16 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
 }
 
 __global__ __launch_bounds__(kWave) void build_schedule_kernel(const int *counts, const int *offsets, int N, int E,
-                                                               int capacity, int stream_max_rows, int *sched) {
-  build_schedule_wave(counts, offsets, N, E, capacity, stream_max_rows, sched, threadIdx.x);
+                                                               int capacity, StreamRule streams, int *sched) {
+  build_schedule_wave(counts, offsets, N, E, capacity, streams, sched, threadIdx.x);
 }
 
 // counts[e] = rows, offsets[e] = e * rows and their work lists in one launch (a lane reads back only what it wrote itself)
-__global__ __launch_bounds__(kWave) void regular_schedule_kernel(int *counts, int *offsets, int E, int rows, int stream_max_rows,
+__global__ __launch_bounds__(kWave) void regular_schedule_kernel(int *counts, int *offsets, int E, int rows, StreamRule streams,
                                                                  int *sched) {
   for (int e = threadIdx.x; e < E; e += kWave) { counts[e] = rows; offsets[e] = e * rows; }
   if (threadIdx.x == 0) offsets[E] = E * rows;
-  build_schedule_wave(counts, offsets, E * rows, E, rows, stream_max_rows, sched, threadIdx.x);
+  build_schedule_wave(counts, offsets, E * rows, E, rows, streams, sched, threadIdx.x);
 }
 
 // ---- single-block form: everything in one launch -------------------------------------------------
@@ -284,7 +311,7 @@ __host__ __device__ inline size_t route_single_lds_bytes(int N, int buckets) {
 template <bool I64>
 __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
     const void *idx, int N, int E, int capacity, int *sorted_expert, int *sorted_idx, int *counts,
-    int *offsets_out, int *inv_pos, int *sched, int stream_max_rows) {
+    int *offsets_out, int *inv_pos, int *sched, StreamRule streams) {
   extern __shared__ int lds[];
   const int buckets = E + 1;
   int *hist = lds;                          // [kRouteWaves][buckets]
@@ -370,7 +397,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_single_kernel(
   }
   // the work lists of the GEMM kernels, from the counts and offsets still in LDS (the last wave, after its share
   // of the placement): saves the launch of build_schedule_kernel
-  if (sched != nullptr && wave == kRouteWaves - 1) build_schedule_wave(total, offs, N, E, capacity, stream_max_rows, sched, lane);
+  if (sched != nullptr && wave == kRouteWaves - 1) build_schedule_wave(total, offs, N, E, capacity, streams, sched, lane);
 }
 
 // ---- three-kernel form for large N -----------------------------------------------------------
@@ -459,13 +486,13 @@ template <bool I64>
 __global__ __launch_bounds__(kRouteThreads) void route_place_kernel(
     const void *idx, int N, int E, int capacity, int seg, const int *seg_cursors,
     const int *offsets_in, int *sorted_expert, int *sorted_idx, int *inv_pos, int n_blocks, const int *counts,
-    int stream_max_rows, int *sched) {
+    StreamRule streams, int *sched) {
   extern __shared__ int lds[];
   const int buckets = E + 1;
   const int tid = threadIdx.x, wave = tid / kWave;
   if ((int)blockIdx.x >= n_blocks) {  // (uniform for the workgroup: nobody of it reaches the barrier below)
     if (sched != nullptr && wave == 0)
-      build_schedule_wave(counts, offsets_in, N, E, capacity, stream_max_rows, sched, tid);
+      build_schedule_wave(counts, offsets_in, N, E, capacity, streams, sched, tid);
     return;
   }
   int *cursor = lds + wave * buckets;
@@ -496,7 +523,7 @@ constexpr size_t kPlaceScanMaxLdsInts = 40000;  // 160 000 bytes
 template <bool I64>
 __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
     const void *idx, int N, int E, int capacity, int seg, const int *seg_counts, int n_seg, int *sorted_expert,
-    int *sorted_idx, int *inv_pos, int *counts, int *offsets_out, int n_blocks, int stream_max_rows, int *sched) {
+    int *sorted_idx, int *inv_pos, int *counts, int *offsets_out, int n_blocks, StreamRule streams, int *sched) {
   extern __shared__ int lds[];
   const int buckets = E + 1;
   int *total = lds;                              // [buckets]
@@ -538,7 +565,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_place_scan_kernel(
     }
   }
   if ((int)blockIdx.x >= n_blocks) {  // (uniform for the workgroup: nobody of it reaches the barrier below)
-    if (sched != nullptr && wave == 0) build_schedule_wave(total, offs, N, E, capacity, stream_max_rows, sched, lane);
+    if (sched != nullptr && wave == 0) build_schedule_wave(total, offs, N, E, capacity, streams, sched, lane);
     return;
   }
   for (int i = tid; i < kRouteWaves * buckets; i += blockDim.x) cursors[i] += offs[i % buckets];
@@ -571,14 +598,14 @@ extern "C" size_t yamoe_route_workspace_bytes(int32_t N, int32_t E) {
 // with more than one launch the lists come from an extra workgroup of the placement kernel.
 int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32_t N, int32_t E, int32_t capacity,
                               int32_t *sorted_expert, int32_t *sorted_idx, int32_t *counts, int32_t *offsets,
-                              int32_t *inv_pos, void *workspace, size_t workspace_bytes, int32_t stream_max_rows,
+                              int32_t *inv_pos, void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t tile_cols,
                               void *schedule, size_t schedule_bytes, void *stream_) {
   hipStream_t stream = (hipStream_t)stream_;
   if (schedule != nullptr && schedule_bytes < yamoe_schedule_bytes(N, E)) {
     set_error("yamoe_build_schedule: schedule region too small");
     return YAMOE_E_WORKSPACE;
   }
-  if (stream_max_rows == kStreamEverything && !sched_may_stream_everything(N, E)) stream_max_rows = kStreamMaxRows;
+  if (stream_max_rows == kStreamEverything && !sched_may_stream_everything(N, E, 4)) stream_max_rows = kStreamMaxRows;
   if (stream_max_rows < 0 && stream_max_rows != kStreamEverything) stream_max_rows = 0;
   if (stream_max_rows > kStreamMaxRows) stream_max_rows = kStreamMaxRows;
   if (N < 0 || E <= 0 || E + 1 > kRouteMaxBuckets) {
@@ -590,6 +617,7 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
     return YAMOE_E_ARG;
   }
   if (capacity < 0) capacity = 0;
+  const StreamRule streams = {stream_max_rows, tile_cols};
   const int buckets = E + 1;
   if (N <= kSingleBlockN) {
     size_t lds = route_single_lds_bytes(N, buckets);
@@ -601,11 +629,11 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
     if (idx_i64)
       hipLaunchKernelGGL(route_single_kernel<true>, dim3(1), dim3(kRouteThreads), lds, stream,
                          router_indices, N, E, capacity, sorted_expert, sorted_idx, counts, offsets, inv_pos, (int *)schedule,
-                         stream_max_rows);
+                         streams);
     else
       hipLaunchKernelGGL(route_single_kernel<false>, dim3(1), dim3(kRouteThreads), lds, stream,
                          router_indices, N, E, capacity, sorted_expert, sorted_idx, counts, offsets, inv_pos, (int *)schedule,
-                         stream_max_rows);
+                         streams);
     return check_launch("route_single_kernel");
   }
   if (workspace_bytes < yamoe_route_workspace_bytes(N, E) || !workspace) {
@@ -639,11 +667,11 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
     if (idx_i64)
       hipLaunchKernelGGL(route_place_scan_kernel<true>, grid, dim3(kRouteThreads), lds_ps, stream, router_indices, N, E,
                          capacity, seg, seg_counts, n_seg, sorted_expert, sorted_idx, inv_pos, counts, offsets, n_blocks,
-                         stream_max_rows, (int *)schedule);
+                         streams, (int *)schedule);
     else
       hipLaunchKernelGGL(route_place_scan_kernel<false>, grid, dim3(kRouteThreads), lds_ps, stream, router_indices, N, E,
                          capacity, seg, seg_counts, n_seg, sorted_expert, sorted_idx, inv_pos, counts, offsets, n_blocks,
-                         stream_max_rows, (int *)schedule);
+                         streams, (int *)schedule);
     return check_launch("route_place_scan_kernel");
   }
   hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(kRouteThreads), lds_b, stream, seg_counts, n_seg, E, counts, offsets);
@@ -652,11 +680,11 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
   if (idx_i64)
     hipLaunchKernelGGL(route_place_kernel<true>, dim3(n_blocks + (schedule != nullptr ? 1 : 0)), dim3(kRouteThreads), lds_c,
                        stream, router_indices, N, E, capacity, seg, seg_counts, offsets, sorted_expert, sorted_idx, inv_pos,
-                       n_blocks, counts, stream_max_rows, (int *)schedule);
+                       n_blocks, counts, streams, (int *)schedule);
   else
     hipLaunchKernelGGL(route_place_kernel<false>, dim3(n_blocks + (schedule != nullptr ? 1 : 0)), dim3(kRouteThreads), lds_c,
                        stream, router_indices, N, E, capacity, seg, seg_counts, offsets, sorted_expert, sorted_idx, inv_pos,
-                       n_blocks, counts, stream_max_rows, (int *)schedule);
+                       n_blocks, counts, streams, (int *)schedule);
   return check_launch("route_place_kernel");
 }
 
@@ -665,7 +693,7 @@ extern "C" int yamoe_route(const void *router_indices, int32_t idx_i64, int32_t 
                            int32_t *counts, int32_t *offsets, int32_t *inv_pos, void *workspace,
                            size_t workspace_bytes, void *stream_) {
   return route_and_schedule(router_indices, idx_i64, N, E, capacity, sorted_expert, sorted_idx, counts, offsets, inv_pos,
-                            workspace, workspace_bytes, 0, nullptr, 0, stream_);
+                            workspace, workspace_bytes, 0, 0, nullptr, 0, stream_);
 }
 
 int yamoe::regular_schedule(int *counts, int *offsets, int E, int rows, int stream_max_rows, void *schedule,
@@ -674,7 +702,7 @@ int yamoe::regular_schedule(int *counts, int *offsets, int E, int rows, int stre
     set_error("regular_schedule: schedule region too small");
     return YAMOE_E_WORKSPACE;
   }
-  hipLaunchKernelGGL(regular_schedule_kernel, dim3(1), dim3(kWave), 0, stream, counts, offsets, E, rows, stream_max_rows,
+  hipLaunchKernelGGL(regular_schedule_kernel, dim3(1), dim3(kWave), 0, stream, counts, offsets, E, rows, StreamRule{stream_max_rows, 0},
                      (int *)schedule);
   return check_launch("regular_schedule_kernel");
 }
@@ -697,10 +725,10 @@ extern "C" int yamoe_build_schedule(const int32_t *counts, const int32_t *offset
     return YAMOE_E_WORKSPACE;
   }
   if (capacity < 0) capacity = 0;
-  if (stream_max_rows == kStreamEverything && !sched_may_stream_everything(N, E)) stream_max_rows = kStreamMaxRows;
+  if (stream_max_rows == kStreamEverything && !sched_may_stream_everything(N, E, 2)) stream_max_rows = kStreamMaxRows;
   if (stream_max_rows < 0 && stream_max_rows != kStreamEverything) stream_max_rows = 0;
   if (stream_max_rows > kStreamMaxRows) stream_max_rows = kStreamMaxRows;
   hipLaunchKernelGGL(build_schedule_kernel, dim3(1), dim3(kWave), 0, stream, counts, offsets, N, E, capacity,
-                     stream_max_rows, (int *)schedule);
+                     StreamRule{stream_max_rows, 0}, (int *)schedule);
   return check_launch("build_schedule_kernel");
 }

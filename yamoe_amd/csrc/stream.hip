@@ -19,14 +19,15 @@
 // eight waves with three steps in flight each, as much as a CU holds, folded into the first four before the same finish: one
 // token on four experts 44.9 us, with four waves 47.5 (four tokens x 4 on 32 experts, 1024 wide: 28.6 and 30.5).
 //
-// An XCD's workgroups take neighbouring slabs.  Where a weight row is not a whole number of cache lines, a slab's piece of it
-// shares a line with the next slab's, and both come from memory unless they meet in one L2: 64 experts, 2048 x 1544, 16 tokens
-// x 8, gate_up 143.6 us with neighbours on different XCDs and 128.3 so.  Whole lines gain 0 to 2 % (64 tokens of the 128-expert
-// layer: 843 and 829 us); not so fp32, where the slabs of an expert with 17 to 32 rows are bound by the matrix units and
-// should not all be on one XCD (32 x 8 rows, 2880 wide: 324 and 355 us).
+// An XCD's workgroups take neighbouring slabs, eight at a time.  Where a weight row is not a whole number of cache lines, a
+// slab's piece of it shares a line with the next slab's, and both come from memory unless they meet in one L2: 64 experts, 2048 x
+// 1544, 16 tokens x 8, whole layer 206 us with neighbours on different XCDs, 200 / 196 / 194 / 193 in groups of 2 / 4 / 8 / 16.  Whole
+// lines gain up to 2 % (64 tokens of the 128-expert layer 812 / 806 / 806 / 796 / 797).  One stretch for each XCD gains no more,
+// and with a skewed routing the experts of many rows meet on one (24 x 8 on 64, 2880 wide, Zipf: 251 us dealt out one by one, 263 in
+// stretches, 250 in groups of eight).
 //
 // fp32 takes the same path with v_mfma_f32_16x16x4_f32.  One token on two experts of 2880 x 2880: 229 us on the tile kernel, 53
-// so; 32 x 2 on 16 of them 489 / 267; 16 x 4 on 32, 1024 wide, 123 / 74.
+// so; 32 x 2 on 16 of them 489 / 267; 128 x 2 492 / 418; 16 x 4 on 32, 1024 wide, 123 / 74.
 //
 // These are the launches of calls in which every expert streams, and of calls whose tile launches are long.  Where those
 // are short and there are tiles, streamed experts ride in them (stream_items in gemm_async_tile.h): the slab code is the
@@ -40,6 +41,7 @@
 namespace yamoe {
 
 constexpr int kStreamManyWaves = 8, kStreamMaxParts = 8, kStreamMostShared = 1024;
+constexpr int kXcdGroup = 8;
 constexpr int kChipCus = kXcds * kXcdCus;
 
 // How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
@@ -48,9 +50,10 @@ __host__ __device__ inline int stream_parts(int slabs, int steps, int waves) {
   int best = 1, cost = ceil_div(slabs, kChipCus) * steps;
   if (slabs > kSchedArrivals) return 1;
   const int most = waves == kStreamManyWaves ? kChipCus : kStreamMostShared;
-  for (int p = 2; p <= kStreamMaxParts && slabs * p <= most && steps >= waves * p; ++p) {
+#pragma unroll
+  for (int p = 2; p <= kStreamMaxParts; ++p) {  // (unrolled: divisions by constants)
     const int c = ceil_div(slabs * p, kChipCus) * ceil_div(steps, p) + 10;
-    if (c < cost) { best = p; cost = c; }
+    if (slabs * p <= most && steps >= waves * p && c < cost) { best = p; cost = c; }
   }
   return best;
 }
@@ -67,14 +70,13 @@ __global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void 
   const int parts = args.partial != nullptr ? stream_parts(slabs, ceil_div(args.Kd, StreamStep<T>::kRows), WAVES) : 1;
   const int total = slabs * parts;
   int b = blockIdx.x;
-  if (args.per_xcd) {  // workgroup b runs on XCD b % 8: that XCD's share of the work is contiguous
-    const int share = ceil_div(total, kXcds), place = b / kXcds;
-    if (place >= share) return;
-    b = b % kXcds * share + place;
+  {  // workgroup b runs on XCD b % 8: groups of kXcdGroup neighbours there, the groups dealt to the XCDs in turn
+    const int place = b / kXcds, group = place / kXcdGroup;
+    b = (group * kXcds + b % kXcds) * kXcdGroup + place % kXcdGroup;
   }
   if (b >= total) return;
-  const int item = b / parts, part = b - item * parts;
-  const int s = item / args.n_slabs, slab = item - s * args.n_slabs;
+  const int item = parts == 1 ? b : b / parts, part = b - item * parts;
+  const int s = fast_div(item, args.slab_div), slab = item - s * args.n_slabs;
   const int expert = sv.small[4 * s], first = sv.small[4 * s + 1], rows = sv.small[4 * s + 2];
   constexpr int DEPTH = WAVES == kStreamWaves ? 2 : 3;
   if (rows > 16) stream_slab<T, GLU, GATHER, WAVES, 2, 2>(args, red, expert, first, rows, slab, item, part, parts);
@@ -82,8 +84,12 @@ __global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void 
 }
 
 // The most workgroups that a launch may need, whatever is on its list, and (`shared`) the most of them that leave parts.
-static long long stream_max_blocks(int N, int E, int Kd, int Nd, int step_rows, long long *shared) {
-  const int entries = sched_max_small(N, E), n_slabs = ceil_div(Nd, kSlabCols), steps = ceil_div(Kd, step_rows);
+static int stream_max_entries(int N, int E, int elem_bytes) {
+  return (N < E ? N : E) + (sched_may_stream_everything(N, E, elem_bytes) ? N / kStreamMaxRows : 0) + 1;
+}
+static long long stream_max_blocks(int N, int E, int Kd, int Nd, int elem_bytes, long long *shared) {
+  const int step_rows = elem_bytes == 4 ? StreamStep<float>::kRows : StreamStep<bf16_t>::kRows;
+  const int entries = stream_max_entries(N, E, elem_bytes), n_slabs = ceil_div(Nd, kSlabCols), steps = ceil_div(Kd, step_rows);
   const int waves = stream_many_waves(N, E, n_slabs) ? kStreamManyWaves : kStreamWaves;
   long long most = (long long)entries * n_slabs;
   *shared = 0;
@@ -97,21 +103,21 @@ static long long stream_max_blocks(int N, int E, int Kd, int Nd, int step_rows, 
 // Bytes of the parts of a product, 0 where its slabs are certain not to be shared.
 size_t stream_partial_bytes(int N, int E, int Kd, int Nd, int elem_bytes) {
   long long shared;
-  stream_max_blocks(N, E, Kd, Nd, elem_bytes == 4 ? StreamStep<float>::kRows : StreamStep<bf16_t>::kRows, &shared);
+  stream_max_blocks(N, E, Kd, Nd, elem_bytes, &shared);
   return (size_t)shared * stream_part_floats(N) * sizeof(float);
 }
 
 template <typename T, bool GLU, bool GATHER>
 static int launch_stream(StreamArgs a, float *partial, hipStream_t stream) {
   a.n_slabs = ceil_div(a.Nd, kSlabCols);
+  a.slab_div = make_fast_div(a.n_slabs);
   a.partial = partial;
   a.part_floats = stream_part_floats(a.N);
   a.arrivals = const_cast<int *>(schedule_view(a.sched, a.N, a.E).arrivals);
-  a.per_xcd = sizeof(T) == 2 || (a.Nd * (int)sizeof(T)) % 128 != 0;
-  long long shared, blocks = stream_max_blocks(a.N, a.E, a.Kd, a.Nd, StreamStep<T>::kRows, &shared);
-  if (partial == nullptr) blocks = (long long)sched_max_small(a.N, a.E) * a.n_slabs;
+  long long shared, blocks = stream_max_blocks(a.N, a.E, a.Kd, a.Nd, (int)sizeof(T), &shared);
+  if (partial == nullptr) blocks = (long long)stream_max_entries(a.N, a.E, (int)sizeof(T)) * a.n_slabs;
   if (blocks <= 0) return 0;
-  blocks = (blocks + kXcds - 1) / kXcds * kXcds;
+  blocks = (blocks + kXcds * kXcdGroup - 1) / (kXcds * kXcdGroup) * (kXcds * kXcdGroup);
   if (stream_many_waves(a.N, a.E, a.n_slabs))
     hipLaunchKernelGGL((stream_gemm_kernel<T, GLU, GATHER, kStreamManyWaves>), dim3((unsigned)blocks), dim3(kWave * kStreamManyWaves), 0, stream, a);
   else

@@ -68,14 +68,13 @@ struct StreamArgs {
   void *C2;            // GLU: optional pre-activations [rows, Nd]
   const int *a_rows;   // optional gather: source row = a_rows[p] / a_div
   const int *sched;
-  FastDiv a_div;
+  FastDiv a_div, slab_div;  // divisions by the gather divisor and by n_slabs
   int Kd, Nd, lda, ldc, n_slabs, N, E;
   // The contraction of a slab may be shared by several workgroups (stream_parts in stream.hip), which leave their sums in
   // `partial` ([list entry][slab][part][part_floats], null: never shared) and count themselves in arrivals[list entry * n_slabs +
   // slab] (zero before and after the launch); the one that finds all others there adds the parts up, in their order, and
   // finishes the slab.
   int part_floats;
-  bool per_xcd;  // neighbouring slabs go to one XCD
   bool yields;   // where there are tiles, their launches carry the list
   float *partial;
   int *arrivals;

@@ -120,8 +120,8 @@ class Yamoe(torch.nn.Module):
         timing = _option(self, "_timing_enabled", False)
         stats = {}
         self._timing_stats = stats   # reset on every call, like the reference's (layers.py:119-122)
-        # (every look-up of a submodule or parameter is a Python call; one token on 128 experts, 1024 wide, is 35 us of GPU time
-        # and was 39 us of host time, of which these and the slices below were half)
+        # (every look-up of a submodule or parameter is a Python call: one each.  A call of one token, 128 experts, 1024 wide, is 35
+        # us of GPU time; 39 us of host time with a look-up for every use, slices of whole tensors and a second no_grad, 34 so)
         router, experts = self.router, self.experts
         router_weight, router_bias = router.weight, router.bias
 
