@@ -34,3 +34,19 @@ def test_gradients_over_several_rounds_of_tiles(gpu, H, I):
     names = ("out", "d_hidden", "d_routing", "d_gate_up_proj", "d_gate_up_proj_bias", "d_down_proj", "d_down_proj_bias")
     for n, a, b in zip(names, (out, *grads), want):
         assert report(n, a.cpu(), b, REL_L2_TOL[torch.float32]) < REL_L2_TOL[torch.float32], n
+
+
+@pytest.mark.parametrize("H,I", [(64, 72), (132, 260), (516, 36)])
+@pytest.mark.parametrize("rows", [17, 31, 32, 33, 64, 65, 95, 96, 97, 127, 128, 129, 160, 161, 224, 225])
+def test_odd_blocks_of_rows(gpu, H, I, rows):
+    """Tiles of one to four blocks of 32 rows: the last of an odd number is shared by the two wave rows, k-step by k-step."""
+    import yamoe_amd
+    d = make_inputs(rows, H, I, 1, 1, torch.float32, seed=rows, w_std=0.05, bias_std=0.1)
+    d["routing_weights"] = 0.1 + torch.rand(rows, 1, generator=torch.Generator().manual_seed(rows))
+    g = args(to_dev(d, gpu))
+    out = yamoe_amd.experts(*g, rows, 1, 1)
+    assert O.rel_l2(out.cpu(), O.experts_capacity(*args(d), rows, compute_dtype=torch.float64)) < REL_L2_TOL[torch.float32]
+    gy = torch.randn(rows, H, generator=torch.Generator().manual_seed(5))
+    want = O.experts_backward(gy, *args(d), rows, compute_dtype=torch.float64)
+    for a, b in zip(yamoe_amd.experts_backward(gy.to(gpu), *g, rows, 1, 1), want):
+        assert O.rel_l2(a.cpu(), b) < REL_L2_TOL[torch.float32]

@@ -10,7 +10,11 @@
 //  * 128 x 128 output tile, 4 wavefronts 2 x 2, each four 32 x 32 accumulator blocks (64 registers).  An expert's rows are
 //    cut here into full tiles and a remainder, whatever the row tiles of the schedule are: with halves of its equal row
 //    tiles (160 rows: 128 + 32) a tenth of the matrix work of the README workload went into blocks without rows.
-//    The 32-row blocks of a tile alternate between the two wave rows, so that a remainder keeps both busy.
+//    The 32-row blocks of a tile alternate between the two wave rows, so that a remainder keeps both busy; of an odd number the
+//    last one is shared, half of the k-steps each (the sums meet in LDS, 16 KB each way), and a tile takes as long as its blocks
+//    rather than as the wave row with one more of them.  Whole forwards, us, before / so: 140 x 2 tokens on 16 experts of 2880 x 2880
+//    490 / 359, 700 x 2 886 / 793, 1547 x 2 1579 / 1446, 450 x 4 on 32, 1024 wide, 208 / 178, even numbers of blocks the same
+//    (README workload 3331 / 3337); forward + backward of 1500 x 2 on 16, 1024 wide, 796 / 782.
 //  * Operands go global -> LDS with asynchronous 16-byte copies (no staging registers), two stages of 32 KB, one
 //    workgroup barrier per slab of 32 (4096 clocks of MFMA issue on each SIMD): while a workgroup waits at its barrier or
 //    runs its epilogue, the other workgroup on the CU keeps the matrix pipe busy.
@@ -236,12 +240,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
   // copies and the first reads of the next slab are issued under its MFMAs.  (Slab 0's copies are on their way already,
   // into stage `stage`; slab s sits in stage + s.  `stores`: behind them, this wave has exactly
   // kStores stores of the previous tile in flight, which nothing waits for here.)
-  auto contract = [&](const Tile &t, int stage, bool stores, auto na) {
+  // NA blocks are this wave's own; with SHARED there is one more, the tile's last, of which either wave row takes half of the
+  // k-steps (row products only: see where the halves meet).
+  auto contract = [&](const Tile &t, int stage, bool stores, auto na, auto shared) {
     constexpr int NA = decltype(na)::value;
+    constexpr bool SHARED = decltype(shared)::value;
     const int n_slabs = (t.k_len + kBK - 1) / kBK;
     float va[2][4][2], vb[2][4][2];  // [set][q][block]
     auto read = [&](int s, int ks, float (&ra)[4][2], float (&rb)[4][2]) {
-      if constexpr (NA > 0) {
+      if constexpr (NA > 0 || SHARED) {
         const char *sa = lds + ((stage + s) & (kStages - 1)) * kStage;
         const char *sb = sa + kAStage;
         if constexpr (A_ROWS) {
@@ -250,6 +257,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
             const f32x4 v = *(const f32x4 *)(sa + a_rd[ks] + x * 64 * 128);
 #pragma unroll
             for (int q = 0; q < 4; ++q) ra[q][x] = v[q];
+          }
+          if constexpr (SHARED) {
+            if (ks >> 1 == wm) {
+              const f32x4 v = *(const f32x4 *)(sa + a_rd[ks] + (NA * 64 - wm * 32) * 128);
+#pragma unroll
+              for (int q = 0; q < 4; ++q) ra[q][NA] = v[q];
+            }
           }
         } else {
 #pragma unroll
@@ -276,13 +290,21 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
         }
       }
     };
-    auto multiply = [&](const float (&ra)[4][2], const float (&rb)[4][2]) {
+    auto multiply = [&](int ks, const float (&ra)[4][2], const float (&rb)[4][2]) {
 #pragma unroll
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int a = 0; a < NA; ++a)
 #pragma unroll
           for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[q][a], rb[q][b], acc[a][b], 0, 0, 0);
+      if constexpr (SHARED) {
+        if (ks >> 1 == wm) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[NA][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ra[q][NA], rb[q][b], acc[NA][b], 0, 0, 0);
+        }
+      }
     };
     // slab s is there for every wave, and nobody reads the other stage any more (the reads of a wave are complete when it
     // gets here: its next MFMAs need them)
@@ -304,7 +326,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
         __builtin_amdgcn_sched_barrier(0);
         read(s, ks + 1, va[(ks + 1) & 1], vb[(ks + 1) & 1]);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(va[ks & 1], vb[ks & 1]);
+        multiply(ks, va[ks & 1], vb[ks & 1]);
       }
       __builtin_amdgcn_sched_barrier(0);
       if (s + 1 < n_slabs) {
@@ -312,7 +334,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
         read(s + 1, 0, va[0], vb[0]);
       }
       __builtin_amdgcn_sched_barrier(0);
-      multiply(va[1], vb[1]);
+      multiply(3, va[1], vb[1]);
     }
   };
 
@@ -338,10 +360,43 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
     // (every wave of the workgroup goes through the same copies, waits and barriers, whatever it multiplies)
     const int cols_valid = min(kBN, args.Nd - t.n0);
     const bool active_n = B_ROWS ? wn * 32 < cols_valid : wn * 64 < cols_valid;
-    const int n_a = !active_n || t.rows_valid <= 0 ? 0 : A_ROWS ? (((t.rows_valid + 31) >> 5) - wm + 1) >> 1 : (wm * 64 < t.rows_valid ? 2 : 0);
-    if (n_a == 2) contract(t, stage, stores, std::integral_constant<int, 2>());
-    else if (n_a == 1) contract(t, stage, stores, std::integral_constant<int, 1>());
-    else contract(t, stage, stores, std::integral_constant<int, 0>());
+    const int blocks = t.rows_valid <= 0 ? 0 : (t.rows_valid + 31) >> 5;
+    const int n_a = !active_n || t.rows_valid <= 0 ? 0 : A_ROWS ? (blocks - wm + 1) >> 1 : (wm * 64 < t.rows_valid ? 2 : 0);
+    typedef std::integral_constant<int, 0> I0;
+    typedef std::integral_constant<int, 1> I1;
+    typedef std::integral_constant<int, 2> I2;
+    if constexpr (A_ROWS) {
+      // An odd number of blocks, which the two wave rows would be 1 and 0 or 2 and 1 of: the last one's k-steps are shared, and
+      // the halves of its sums meet in the ring stage of the last slab.
+      const bool odd = (blocks & 1) != 0;
+      if (!active_n) contract(t, stage, stores, I0(), std::false_type());
+      else if (blocks == 4) contract(t, stage, stores, I2(), std::false_type());
+      else if (blocks == 3) contract(t, stage, stores, I1(), std::true_type());
+      else if (blocks == 2) contract(t, stage, stores, I1(), std::false_type());
+      else if (blocks == 1) contract(t, stage, stores, I0(), std::true_type());
+      else contract(t, stage, stores, I0(), std::false_type());
+      if (odd) {
+        const int last = stage + (t.k_len + kBK - 1) / kBK - 1;
+        float *meet = (float *)(lds + (last & (kStages - 1)) * kStage) + wn * 32 * kWave + lane;
+        auto add = [&](auto which) {
+          constexpr int A = decltype(which)::value;
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              if (wm == 1) meet[(b * 16 + v) * kWave] = acc[A][b][v];
+              else acc[A][b][v] += meet[(b * 16 + v) * kWave];
+            }
+        };
+        __syncthreads();  // nobody reads the slab any more
+        if (wm == 1 && active_n) { if (blocks == 3) add(I1()); else add(I0()); }
+        __syncthreads();
+        if (wm == 0 && active_n) { if (blocks == 3) add(I1()); else add(I0()); }
+      }
+    } else {
+      if (n_a == 2) contract(t, stage, stores, I2(), std::false_type());
+      else contract(t, stage, stores, I0(), std::false_type());
+    }
 
     // (the stage after the last slab's has been free since the barrier in front of that slab)
     stage += (t.k_len + kBK - 1) / kBK;
