@@ -12,9 +12,10 @@
 //    tiles (160 rows: 128 + 32) a tenth of the matrix work of the README workload went into blocks without rows.
 //    The 32-row blocks of a tile alternate between the two wave rows, so that a remainder keeps both busy; of an odd number the
 //    last one is shared, half of the k-steps each (the sums meet in LDS, 16 KB each way), and a tile takes as long as its blocks
-//    rather than as the wave row with one more of them.  Whole forwards, us, before / so: 140 x 2 tokens on 16 experts of 2880 x 2880
-//    490 / 359, 700 x 2 886 / 793, 1547 x 2 1579 / 1446, 450 x 4 on 32, 1024 wide, 208 / 178, even numbers of blocks the same
-//    (README workload 3331 / 3337); forward + backward of 1500 x 2 on 16, 1024 wide, 796 / 782.
+//    rather than as the wave row with one more of them.  Whole forwards, us, before / so, nothing else changed: 140 x 2 tokens on 16
+//    experts of 2880 x 2880 491 / 361, 300 x 2 505 / 505, 700 x 2 897 / 865, 1547 x 2 1580 / 1447; 450 x 4 on 32, 1024 wide,
+//    185 / 168; 4096 x 2 on 8 of 2880 x 2880, nearly all of it whole tiles, 3288 / 3288 to 3299;
+//    forward + backward of 1500 x 2 on 16, 1024 wide, 800 / 787.
 //  * Operands go global -> LDS with asynchronous 16-byte copies (no staging registers), two stages of 32 KB, one
 //    workgroup barrier per slab of 32 (4096 clocks of MFMA issue on each SIMD): while a workgroup waits at its barrier or
 //    runs its epilogue, the other workgroup on the CU keeps the matrix pipe busy.
@@ -368,14 +369,13 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
     if constexpr (A_ROWS) {
       // An odd number of blocks, which the two wave rows would be 1 and 0 or 2 and 1 of: the last one's k-steps are shared, and
       // the halves of its sums meet in the ring stage of the last slab.
-      const bool odd = (blocks & 1) != 0;
-      if (!active_n) contract(t, stage, stores, I0(), std::false_type());
-      else if (blocks == 4) contract(t, stage, stores, I2(), std::false_type());
-      else if (blocks == 3) contract(t, stage, stores, I1(), std::true_type());
-      else if (blocks == 2) contract(t, stage, stores, I1(), std::false_type());
-      else if (blocks == 1) contract(t, stage, stores, I0(), std::true_type());
+      const int busy = active_n ? blocks : 0;
+      if (busy == 4) contract(t, stage, stores, I2(), std::false_type());
+      else if (busy == 3) contract(t, stage, stores, I1(), std::true_type());
+      else if (busy == 2) contract(t, stage, stores, I1(), std::false_type());
+      else if (busy == 1) contract(t, stage, stores, I0(), std::true_type());
       else contract(t, stage, stores, I0(), std::false_type());
-      if (odd) {
+      if ((blocks & 1) != 0) {
         const int last = stage + (t.k_len + kBK - 1) / kBK - 1;
         float *meet = (float *)(lds + (last & (kStages - 1)) * kStage) + wn * 32 * kWave + lane;
         auto add = [&](auto which) {
@@ -389,9 +389,11 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const Args args) 
             }
         };
         __syncthreads();  // nobody reads the slab any more
-        if (wm == 1 && active_n) { if (blocks == 3) add(I1()); else add(I0()); }
+        if (wm == 1 && busy == 3) add(I1());
+        else if (wm == 1 && busy == 1) add(I0());
         __syncthreads();
-        if (wm == 0 && active_n) { if (blocks == 3) add(I1()); else add(I0()); }
+        if (wm == 0 && busy == 3) add(I1());
+        else if (wm == 0 && busy == 1) add(I0());
       }
     } else {
       if (n_a == 2) contract(t, stage, stores, I2(), std::false_type());
