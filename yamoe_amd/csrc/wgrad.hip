@@ -480,7 +480,7 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_small_kernel(const WgradArg
 }
 
 // ---- short contractions ------------------------------------------------------------------------------------------
-// Up to kShortRows rows per expert on average a launch is bound by the store of the gradient (5.5 TB/s reached) and by what
+// Up to kShortRows rows per expert a launch is bound by the store of the gradient (5.5 TB/s reached) and by what
 // stands between two stores of a CU: a tile's start, its first slab's trip from memory and the staging, which a contraction of
 // one to three slabs does not cover.  So four small workgroups share a CU instead of two: 128 x 128 tiles, 64 accumulators and at
 // most 128 registers per lane, 35 KB of LDS (a ring of two slabs, into which the tile is staged afterwards), no hand-made order:
@@ -489,7 +489,14 @@ __global__ __launch_bounds__(kThreads, 2) void wgrad_small_kernel(const WgradArg
 // 2880 x 2880, 64 rows 379 / 325, 112: 461 / 445, 128: 494 / 481, 192: 573 / 583; 16 of 2048, 64 rows 112 / 91, 112: 117 / 109, 128:
 // 118 / 122.  Beyond, the small tiles' operand traffic decides: a slab costs 29 us instead of 24 (64 experts, 2048 x 2048), 23 of
 // them for its copies from L2, 33 % more bytes.
-constexpr int kShortRows = 112;
+// Those are evenly routed experts.  A skewed routing has most of its rows in a few experts with far more, so the average alone is
+// a sound line only up to kShortRowsAnyRouting; beyond, the capacity has to keep every expert at kShortMostRows or below.  Whole
+// forwards and backwards under Zipf (1.2) routing without a capacity, large tiles / these, 64 experts of 2048 x 2048, 24 rows on
+// average: 1043 / 1030, 40: 1185 / 1193, 72: 1477 / 1569, 112: 1824 / 1933; 32 of 2880 x 2880, 24 rows 1057 / 1021, 40: 1192 / 1204,
+// 72: 1403 / 1486; with 1.25 times the average as the capacity, 64 of 2048 x 2048, 72 rows 1081 / 1018, 104: 1225 / 1175, 32 of
+// 2880 x 2880 1100 / 1019 and 1179 / 1152.  (Both kernels in turn, each for the experts that suit it, lose to either one: a second
+// launch's tail; 72 rows, Zipf, 1663 and 1592 us.)
+constexpr int kShortRows = 112, kShortRowsAnyRouting = 32, kShortMostRows = 128;
 constexpr int kShortBM = 128, kShortBN = 128, kShortStages = 2;
 constexpr int kShortOperand = kBK * kShortBM * 2;      // 8 KB: 32 k rows of 256 bytes
 constexpr int kShortStage = 2 * kShortOperand;
@@ -696,7 +703,8 @@ int gemm_async_wgrad(const void *L, const int *l_rows, int l_div, int n_rows, co
   a.A = L; a.B = R; a.C = dW; a.counts = counts; a.offsets = offsets; a.capacity = capacity; a.bias_grad = d_bias;
   a.a_rows = l_rows; a.a_div = make_fast_div(l_rows != nullptr ? l_div : 1); a.a_rows_max = n_rows > 0 ? n_rows - 1 : 0;
   a.E = E; a.Md = Md; a.Nd = Nd;
-  const bool is_short = min(n_rows / E, capacity) <= async::kShortRows;
+  const int average = min(n_rows / E, capacity), most = min(n_rows, capacity);
+  const bool is_short = average <= async::kShortRowsAnyRouting || (average <= async::kShortRows && most <= async::kShortMostRows);
   if (l_rows != nullptr) return async::launch_wgrad<T, true>(a, is_short, stream);
   return async::launch_wgrad<T, false>(a, is_short, stream);
 }
