@@ -154,9 +154,9 @@ int yamoe_experts_forward(const yamoe_problem *p, const void *hidden_states,
  * image: make that first call before a stream capture begins, not inside it).  Problems whose
  * yamoe_experts_workspace_bytes() exceeds the array are rejected with YAMOE_E_WORKSPACE (at
  * H = I = 2880 in a 16-bit dtype the limit is about 2900 (token, expert) assignments, e.g. 725
- * tokens at top-4).  All calls on one GPU share that GPU's array: two calls whose work overlaps on
+ * tokens at top-4, in fp32 half of that).  All calls on one GPU share that GPU's array: two calls whose work overlaps on
  * the same GPU (different streams, or different threads) race; calls on one stream are ordered. */
-#define YAMOE_STATIC_SCRATCH_BYTES (32u << 20)
+#define YAMOE_STATIC_SCRATCH_BYTES ((32u << 20) + (16u << 10)) /* 32 MiB, and what fp32 work lists are longer by */
 int yamoe_experts_forward_static(const yamoe_problem *p, const void *hidden_states,
                                  const void *router_indices, const void *routing_weights,
                                  const void *gate_up_proj, const void *gate_up_proj_bias,

@@ -69,6 +69,32 @@ def test_size_queries_and_validation_need_no_gpu():
     assert rc == -1
 
 
+def test_shared_slab_sums_push_no_call_out_of_the_built_in_workspace():
+    """The sums of workgroups that share a slab are optional: whatever fits the built-in workspace without them (rows and lists)
+    fits it with what the size query says, and the 16-bit backward, which streams nothing, has no room for them."""
+    from yamoe_amd import _cabi
+    lib = _cabi.lib()
+    up = lambda n: (max(n, 1) + 255) // 256 * 256
+    most = 0
+    for T, K, E, H, I, dt in ((128, 8, 256, 7168, 2048, _cabi.BF16), (250, 4, 128, 2880, 2880, _cabi.F32), (350, 4, 128, 2880, 2880, _cabi.F32),
+                              (200, 4, 128, 2880, 2880, _cabi.F32), (500, 4, 512, 2880, 2880, _cabi.BF16), (725, 4, 181, 2880, 2880, _cabi.F16),
+                              (728, 4, 182, 2880, 2880, _cabi.BF16), (1, 4, 128, 2880, 2880, _cabi.BF16), (64, 4, 128, 2880, 2880, _cabi.BF16),
+                              (32, 2, 16, 2880, 2880, _cabi.F32), (4096, 2, 8, 64, 64, _cabi.F32), (12288, 1, 768, 256, 384, _cabi.F32)):
+        p = ctypes.byref(_cabi.Problem(T=T, K=K, E=E, H=H, I=I, capacity=T, dtype=dt, idx_i64=1, rw_cols=E))
+        n, es = T * K, 4 if dt == _cabi.F32 else 2
+        rows = up(n * I * es) + up(n * max(H, I) * es)
+        lists = 3 * up(4 * n) + up(4 * E) + up(4 * E + 4) + up(lib.yamoe_schedule_bytes(n, E)) + up(lib.yamoe_route_workspace_bytes(n, E))
+        forward, backward = lib.yamoe_experts_workspace_bytes(p), lib.yamoe_experts_backward_workspace_bytes(p)
+        assert rows + lists <= forward <= max(rows + lists, _cabi.STATIC_SCRATCH_BYTES), (T, K, E, H, I, dt)
+        most = max(most, forward - rows - lists)
+        if es == 2:  # pre, d_pre [n, 2I], g_y, d_x [n, H], two fp32 values and the row dots of a row, 32 rows of padding
+            own = 2 * up(n * 2 * I * es) + 2 * up(n * H * es) + 2 * up(4 * n) + up(32 * max(H, 2 * I) * es)
+            assert backward - rows - lists - own <= up(4 * n * (2 * I // 128 + 2)), (T, K, E, H, I, dt)
+    assert 0 < most <= 16 << 20
+    text = open(os.path.join(ROOT, "include", "yamoe_hip.h")).read()
+    assert "YAMOE_STATIC_SCRATCH_BYTES ((32u << 20) + (16u << 10))" in text and _cabi.STATIC_SCRATCH_BYTES == (32 << 20) + (16 << 10)
+
+
 def test_torch_op_schemas_match_reference():
     """The registered schemas are the reference's (torch-ext/torch_binding.cpp:9-56), namespace aside."""
     import yamoe_amd

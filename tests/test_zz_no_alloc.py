@@ -56,6 +56,21 @@ def test_static_workspace_forward_fp32_and_decode_shape(gpu):
     assert torch.equal(got, want)
 
 
+def test_static_workspace_forward_with_rows_beyond_the_room_for_shared_slabs(gpu):
+    """fp32, every expert streams, 20 MiB of rows: with the sums of shared slabs (16 MiB) the workspace would not fit the array."""
+    from yamoe_amd import _cabi
+    T, H, I, E, K = 512, 2048, 512, 128, 4
+    gen = torch.Generator(device=gpu).manual_seed(57)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu) * 0.05
+    for few in (False, True):  # (few: all on eight experts)
+        ids = torch.randint(8 if few else E, (T, K), generator=gen, device=gpu)
+        g = [r(T, H), ids, torch.rand(T, E, generator=gen, device=gpu), r(E, H, 2 * I), r(E, 2 * I), r(E, I, H), r(E, H)]
+        want = _cabi.experts_forward(*g, T)
+        got = _cabi.experts_forward_static(*g, T, torch.full_like(want, float("nan")))
+        torch.cuda.synchronize()
+        assert torch.equal(got, want), few
+
+
 def test_static_workspace_forward_refuses_large_problems(gpu):
     from yamoe_amd import _cabi
     T, H, I, E, K = 4096, 2880, 2880, 2, 4

@@ -255,7 +255,7 @@ def experts_backward(grad_out, hidden, router_indices, routing_weights, gate_up_
     return outs
 
 
-STATIC_SCRATCH_BYTES = 32 << 20  # YAMOE_STATIC_SCRATCH_BYTES of include/yamoe_hip.h
+STATIC_SCRATCH_BYTES = (32 << 20) + (16 << 10)  # YAMOE_STATIC_SCRATCH_BYTES of include/yamoe_hip.h
 
 
 def experts_forward_static(hidden, router_indices, routing_weights, gate_up_proj, gate_up_proj_bias, down_proj,

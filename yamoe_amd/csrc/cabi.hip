@@ -284,11 +284,15 @@ struct ForwardBuffers {
   int *sorted_expert, *sorted_idx, *inv_pos, *counts, *offsets;
   void *schedule, *route_ws, *act, *y_perm;
   void *x_perm;  // hidden rows in expert order: only with gathers_need_permute
-  float *partial;  // sums of the workgroups that share a slab of a streaming product: where that happens at all
+  float *partial;  // sums of the workgroups that share a slab of a streaming product, null where none does: see carve_forward
   size_t schedule_bytes, route_ws_bytes;
 };
 
-static size_t carve_forward(const yamoe_problem *p, void *ws, ForwardBuffers *b) {
+// shares: whether slabs may be shared (`partial`).  That needs up to 16 MiB, and no call has to have it, so it is reserved only
+// where the workspace stays within the built-in array with it: the entry point on that array takes every problem whose rows
+// and lists fit, and both entry points sum alike.  (A call beyond has more than 16 MiB of rows, over 700 assignments at 2880
+// wide: 16 entries of the list and more, which rarely leave CUs idle.)
+static size_t carve_forward(const yamoe_problem *p, void *ws, ForwardBuffers *b, bool shares = true) {
   const size_t N = (size_t)p->T * p->K, es = dtype_size(p->dtype);
   Carver c(ws);
   b->sorted_expert = (int *)c.take(N * 4);
@@ -305,10 +309,11 @@ static size_t carve_forward(const yamoe_problem *p, void *ws, ForwardBuffers *b)
   b->y_perm = c.take(N * (size_t)(p->H > p->I ? p->H : p->I) * es);
   b->x_perm = gathers_need_permute(p) ? c.take(N * p->H * es) : nullptr;
   size_t partial = 0;
-  if (!takes_plain_path(p) && sched_may_stream_everything((int)N, p->E, (int)es)) {
+  if (shares && !takes_plain_path(p) && sched_may_stream_everything((int)N, p->E, (int)es)) {
     const size_t gate_up = stream_partial_bytes((int)N, p->E, p->H, 2 * p->I, (int)es), down = stream_partial_bytes((int)N, p->E, p->I, p->H, (int)es);
     partial = gate_up > down ? gate_up : down;
   }
+  if (c.used + align_up(partial, 256) > (size_t)YAMOE_STATIC_SCRATCH_BYTES) partial = 0;
   b->partial = partial > 0 ? (float *)c.take(partial) : nullptr;
   return c.used;
 }
@@ -322,8 +327,8 @@ struct BackwardBuffers {
 };
 
 static size_t carve_backward(const yamoe_problem *p, void *ws, BackwardBuffers *b) {
-  size_t used = carve_forward(p, ws, &b->f);
   const size_t N = (size_t)p->T * p->K, es = dtype_size(p->dtype);
+  const size_t used = carve_forward(p, ws, &b->f, /*shares=*/es == 4);  // (only an fp32 recomputation streams)
   Carver c(ws ? (char *)ws + used : nullptr);
   // hidden rows in expert order: only where the gate_up weight-gradient kernel cannot gather them itself
   const bool gathers = !gathers_need_permute(p) &&
@@ -755,7 +760,7 @@ extern "C" int yamoe_experts_forward_static(const yamoe_problem *p, const void *
   const size_t need = yamoe_experts_workspace_bytes(p);
   if (need > (size_t)YAMOE_STATIC_SCRATCH_BYTES) {
     set_error("yamoe_experts_forward_static: this problem needs %zu bytes of workspace, the built-in one holds %zu "
-              "(T*K*(I + max(H,I)) elements plus the routing lists); use yamoe_experts_forward with a caller-owned "
+              "(T*K*(I + max(H,I)) elements, the routing lists, and T*K*H elements more for hidden_states of 4 GiB); use yamoe_experts_forward with a caller-owned "
               "workspace", need, (size_t)YAMOE_STATIC_SCRATCH_BYTES);
     return YAMOE_E_WORKSPACE;
   }
