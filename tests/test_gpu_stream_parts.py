@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [  # T, H, I, E, K, one expert for all
     (1, 64, 72, 8, 1, False), (1, 128, 256, 8, 2, False), (2, 520, 1032, 16, 2, False), (1, 2880, 360, 32, 4, False),
     (3, 1000, 40, 4, 1, False), (16, 1024, 200, 8, 2, False), (17, 264, 128, 16, 1, True), (31, 1536, 64, 8, 1, True),
+    (1, 512, 64, 8, 2, False), (1, 520, 136, 32, 1, False), (4, 768, 384, 32, 2, False),  # fewer steps in a part than eight waves
     (32, 256, 264, 8, 1, True), (33, 2048, 128, 16, 1, True), (64, 512, 264, 16, 1, True), (40, 136, 520, 64, 4, False),
 ]
 

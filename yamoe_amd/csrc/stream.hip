@@ -15,7 +15,8 @@
 // through memory, and whoever comes last adds them up.  What counts is how evenly the workgroups fill the CUs, which is known
 // on the device: us for 1 / 2 / 3 / 4 / 6 / 8 parts, 46 slabs of 90 steps 20.1 / 14.3 / 11.6 / 10.6 / 11.9 / 11.0, 92: 21.1 / 15.6 / 17.8 /
 // 15.9 / 16.7 / 15.6, 161: 22.6 / 25.3 / 21.6 / 23.4 / 25.7 / 25.4, 180: 23.4 / 25.4 / 26.1 / 24.7 / 26.7 / 27.5, 64 of 32 steps: 11.7 /
-// 10.2 / 8.5 / 8.0 / 9.0 / 9.4 (workgroups of four waves).  Where the list has at most a slab per CU, a workgroup takes
+// 10.2 / 8.5 / 8.0 / 9.0 / 9.4, 144 of 32: 12.5 / 14.4 / 12.2 / 13.7 / 15.9 / -, 112 of 16: 7.0 / 8.0 / 7.7 / 7.9 / 8.5 / 11.1 (workgroups
+// of four waves, weights from memory): many parts of a short contraction cost more than they spread.  Where the list has at most a slab per CU, a workgroup takes
 // eight waves with three steps in flight each, as much as a CU holds, folded into the first four before the same finish: one
 // token on four experts 44.9 us, with four waves 47.5 (four tokens x 4 on 32 experts, 1024 wide: 28.6 and 30.5).
 //
@@ -45,15 +46,20 @@ constexpr int kXcdGroup = 8;
 constexpr int kChipCus = kXcds * kXcdCus;
 
 // How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
-// fewest steps on the CU that gets most of them, where sharing costs about as much as ten (the parts' way through memory).
+// fewest steps on the CU that gets most of them, where a workgroup's start and finish cost about as much as 14 steps, the
+// parts' way through memory as 6, and another 2 for each part that the last one reads.  (Fitted to 154 lists of 16 to 1440 slabs of
+// 16 to 90 steps: 1 % over the best number of parts on average, 10 % in the worst of them.  With ten steps for the sharing and none
+// for a workgroup's start it was 2.7 and 25 %: 9 x 4 tokens on 64 experts, 1024 wide, Zipf (2) routing, 144 slabs in seven parts,
+// whole layer 29.8 us, 27.0 so, 26.7 unshared with eight waves; 5 x 4 on 128, Zipf, 30.9 / 28.0.)
 __host__ __device__ inline int stream_parts(int slabs, int steps, int waves) {
-  int best = 1, cost = ceil_div(slabs, kChipCus) * steps;
+  int best = 1, cost = ceil_div(slabs, kChipCus) * (steps + 14);
   if (slabs > kSchedArrivals) return 1;
   const int most = waves == kStreamManyWaves ? kChipCus : kStreamMostShared;
 #pragma unroll
   for (int p = 2; p <= kStreamMaxParts; ++p) {  // (unrolled: divisions by constants)
-    const int c = ceil_div(slabs * p, kChipCus) * ceil_div(steps, p) + 10;
-    if (slabs * p <= most && steps >= waves * p && c < cost) { best = p; cost = c; }
+    if (p == 5 || p == 7) continue;  // (never better than a neighbour by more than the runs differ)
+    const int c = ceil_div(slabs * p, kChipCus) * (ceil_div(steps, p) + 14) + 6 + 2 * p;
+    if (slabs * p <= most && steps >= 4 * p && c < cost) { best = p; cost = c; }
   }
   return best;
 }
