@@ -1,6 +1,8 @@
 """The streaming kernels where a call has few (expert, column slab) pairs and several workgroups share one: contractions of a
 few steps and of many, whole and cut slabs, one and two blocks of 16 rows, experts in chunks of 32 rows; fp32 on the same path.
 The parts are added up in their order, so a call gives the same bits every time, also when it is replayed from a graph."""
+import ctypes
+
 import pytest
 import torch
 
@@ -87,3 +89,39 @@ def test_fp32_up_to_sixteen_assignments_per_expert(gpu, T, H, I, E, K, one):
     want = O.experts_backward(gy, *args(d), T, compute_dtype=torch.float64)
     for a, b in zip(yamoe_amd.experts_backward(gy.to(gpu), *g, T, E, K), want):
         assert O.rel_l2(a.cpu(), b) < REL_L2_TOL[torch.float32]
+
+
+@pytest.mark.parametrize("rows,streams", [([16] * 128, True), ([2048] + [0] * 127, False), ([600] * 3 + [8] * 25 + [0] * 100, False),
+                                          ([500] + [12] * 127, True), ([33] * 30 + [8] * 98, True), ([400] * 5 + [0] * 123, False),
+                                          ([129] * 8 + [8] * 120, True)])
+def test_fp32_streams_everything_or_nothing_by_the_routing(gpu, rows, streams):
+    """At most 16 assignments per expert on average, and more of them than streaming can take from a single expert at no loss: the
+    device decides between the two kernels.  The work lists (behind the five lists of the routing) tell which; both give the
+    oracle's result, and a recomputation takes the way of the forward."""
+    import yamoe_amd
+    from yamoe_amd import _cabi
+    T, H, I, E = sum(rows), 1024, 512, 128
+    print("fp32 either", rows[:8], flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu) * 0.05
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(rows)])
+    ids = ids[torch.randperm(T, generator=torch.Generator().manual_seed(1))].view(T, 1).to(gpu)
+    g = [r(T, H), ids, 0.1 + torch.rand(T, E, generator=gen, device=gpu), r(E, H, 2 * I), r(E, 2 * I), r(E, I, H), r(E, H)]
+    p = _cabi.problem(*g[:4], T)
+    ws = torch.zeros(_cabi.lib().yamoe_experts_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=gpu)
+    out = _cabi.experts_forward(*g, T, workspace=ws, out=torch.full_like(g[0], float("nan")))
+    up = lambda n: (n + 255) // 256 * 256
+    at = 3 * up(4 * T) + up(4 * E) + up(4 * E + 4)
+    tiles, listed, active, kept = ws[at:at + 16].view(torch.int32).tolist()
+    assert (active, kept) == (sum(n > 0 for n in rows), T)
+    assert (tiles == 0, listed > 0) == (streams, streams)
+    used = [e for e, n in enumerate(rows) if n][:6]     # (the oracle on a few experts' tokens: 800 MB of weights)
+    some = torch.isin(ids.view(-1).cpu(), torch.tensor(used)).nonzero().view(-1)[:200]
+    x, e, w = (t.cpu()[some] for t in g[:3])
+    sub = [x, torch.searchsorted(torch.tensor(used), e.view(-1)).view(-1, 1), w[:, used].contiguous()] + [t[used].cpu() for t in g[3:]]
+    assert O.rel_l2(out[some.to(gpu)].cpu(), O.experts_capacity(*sub, T, compute_dtype=torch.float64)) < REL_L2_TOL[torch.float32]
+    again, k = yamoe_amd.experts_keep(*g, T, E, 1)
+    assert torch.equal(again, out)
+    gy = r(T, H)
+    for a, b in zip(yamoe_amd.experts_backward_kept(gy, *g, k, T, E, 1), yamoe_amd.experts_backward(gy, *g, T, E, 1)):
+        assert torch.equal(a, b)

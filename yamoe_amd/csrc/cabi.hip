@@ -104,12 +104,18 @@ int plain_backward(const void *, const void *, const void *, int, const void *, 
                    int, int, int, int, int, int, hipStream_t);
 template <typename T> int plain_fill_zero(void *, long long, hipStream_t);
 
-// Experts of at most this many kept rows stream their weights instead of going through the tile kernels (0: none does).  fp32 data
-// streams where every expert does: beside tiles, whose launch takes as long for one of them as for a round, a second pair of
-// launches costs more than it takes off them (64 tokens x 2 on 16 skewed experts, 2048 x 744: 122 us as tiles, 173 with some
-// streamed, 94 with all).
-static int stream_rows_of(int dtype, int N, int E) {
-  return dtype != YAMOE_F32 || sched_may_stream_everything(N, E, 4) ? kStreamMaxRows : 0;
+// The 128-wide column tiles of both products.
+static int f32_columns(const yamoe_problem *p) { return ceil_div(2 * p->I, 128) + ceil_div(p->H, 128); }
+// Who streams in a forward: experts of at most so many kept rows (0: none does), kStreamEverything or kStreamEither.  fp32 data streams
+// all or nothing: beside tiles, whose launch takes as long for one of them as for a round, a second pair of launches costs
+// more than it takes off them (64 tokens x 2 on 16 skewed experts, 2048 x 744: 122 us as tiles, 173 with some streamed, 94
+// with all).
+static int streams_of(const yamoe_problem *p) {
+  const int N = p->T * p->K;
+  const bool f32 = p->dtype == YAMOE_F32;
+  if (!sched_may_stream_everything(N, p->E, (int)dtype_size(p->dtype))) return f32 ? 0 : kStreamMaxRows;
+  const bool any_routing = !f32 || p->capacity <= kStreamMaxRows || f32_streams_any_routing(N, f32_columns(p));
+  return any_routing ? kStreamEverything : kStreamEither;
 }
 
 // Whether a product of N rows over E experts with Nd columns runs on 128 x 128 tiles (two workgroups per CU) instead of
@@ -408,20 +414,19 @@ static int forward_impl(const yamoe_problem *p, const void *x, const void *idx, 
   const int N = p->T * p->K;
   void *st = (void *)stream;
   if (N == 0 || p->T == 0) return 0;
-  const int stream_rows = stream_rows_of(p->dtype, N, p->E);
-  // At most 4 assignments per expert on average (decode): every expert goes to the streaming kernel, in chunks of
-  // stream_rows rows where one has more, and the tile kernels, whose lists are then empty, are not launched (two
+  const int mode = streams_of(p), stream_rows = mode == 0 ? 0 : kStreamMaxRows;
+  // kStreamEverything (decode, at most 4 assignments per expert on average): every expert goes to the streaming kernel, in
+  // chunks of stream_rows rows where one has more, and the tile kernels, whose lists are then empty, are not launched (two
   // launches of 4.5 us each that found nothing to do at 64 tokens on 128 experts).
-  const bool everything = sched_may_stream_everything(N, p->E, (int)sizeof(T));
-  // where the assignments or the capacity leave no expert more rows than a streamed one may have, every expert is streamed as
+  // Where the assignments or the capacity leave no expert more rows than a streamed one may have, every expert is streamed as
   // well.  1723 tokens on 8 experts of 2048 x 2048, 32 rows kept: 60 us; with two tile launches that find no tile in front 68,
   // carried by those 72.
-  const bool tiles = !everything && N > stream_rows && p->capacity > stream_rows;
+  const bool tiles = mode != kStreamEverything && N > stream_rows && p->capacity > stream_rows;
   const int carried = sizeof(T) == 2 && tiles ? tiles_carry_streams(N, p->E, p->H, p->I) : CARRY_NOT;
-  const int tile_cols = carried != CARRY_NOT && !takes_small_tiles(N, p->E, 2 * p->I) ? ceil_div(2 * p->I, kColTile) : 0;
+  int cols = carried != CARRY_NOT && !takes_small_tiles(N, p->E, 2 * p->I) ? ceil_div(2 * p->I, kColTile) : 0;
+  if (mode == kStreamEither) cols = f32_columns(p);
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, p->E, p->capacity, b.sorted_expert, b.sorted_idx, b.counts, b.offsets,
-                               b.inv_pos, b.route_ws, b.route_ws_bytes, everything ? kStreamEverything : stream_rows, tile_cols,
-                               b.schedule, b.schedule_bytes, st));
+                               b.inv_pos, b.route_ws, b.route_ws_bytes, mode, cols, b.schedule, b.schedule_bytes, st));
   if (tiles && b.x_perm != nullptr) {  // (a hidden_states tensor too large to gather from: see gathers_need_permute)
     YAMOE_TRY(launch_permute<T>(x, b.sorted_idx, b.x_perm, N, p->K, p->H, stream));
     YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.act, pre, b.schedule, N, p->K, p->E, p->H, p->I, stream_rows,
@@ -460,23 +465,23 @@ static int backward_impl(const yamoe_problem *p, const void *gy, const void *x, 
   }
   // fp32: the recomputation streams where the forward did, so that its gradients are those of a kept forward to the bit; the
   // other products run on the tile kernels and get their lists afterwards.
-  const bool streamed = sizeof(T) == 4 && kept == nullptr && stream_rows_of(p->dtype, N, E) > 0;
+  const int mode = sizeof(T) == 4 && kept == nullptr ? streams_of(p) : 0;
   YAMOE_TRY(route_and_schedule(idx, p->idx_i64, N, E, cap, b.f.sorted_expert, b.f.sorted_idx, b.f.counts, b.f.offsets,
-                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, streamed ? kStreamEverything : 0, 0, b.f.schedule,
-                               b.f.schedule_bytes, st));
+                               b.f.inv_pos, b.f.route_ws, b.f.route_ws_bytes, mode, mode == kStreamEither ? f32_columns(p) : 0,
+                               b.f.schedule, b.f.schedule_bytes, st));
   // forward recompute of the first product only: activations and pre-activations
   const bool permuted = b.gy_perm != nullptr;  // hidden_states and grad_out too large to gather from
   const bool gathers = !permuted && wgrad_gathers<T>(H, 2 * I);
   if (!gathers) YAMOE_TRY(launch_permute<T>(x, b.f.sorted_idx, b.x_perm, N, p->K, H, stream));
   if (kept != nullptr) {
     // activations and pre-activations come from the forward
-  } else if (streamed) {
-    YAMOE_TRY(stream_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, b.f.partial, false, stream));
-    YAMOE_TRY(yamoe_build_schedule(b.f.counts, b.f.offsets, N, E, cap, 0, b.f.schedule, b.f.schedule_bytes, st));
-  } else if (permuted) {
-    YAMOE_TRY(tiles_gate_up<T>(b.x_perm, nullptr, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, CARRY_NOT, stream));
   } else {
-    YAMOE_TRY(tiles_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, 0, CARRY_NOT, stream));
+    if (mode != 0)
+      YAMOE_TRY(stream_gate_up<T>(x, b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N, p->K, E, H, I, b.f.partial, false, stream));
+    if (mode != kStreamEverything)
+      YAMOE_TRY(tiles_gate_up<T>(permuted ? b.x_perm : x, permuted ? nullptr : b.f.sorted_idx, wgu, bgu, b.f.act, b.pre, b.f.schedule, N,
+                                 p->K, E, H, I, 0, CARRY_NOT, stream));
+    if (mode != 0) YAMOE_TRY(yamoe_build_schedule(b.f.counts, b.f.offsets, N, E, cap, 0, b.f.schedule, b.f.schedule_bytes, st));
   }
   // combine backward: g_y_perm = grad_out[tok] * w, and the bias part of the routing gradient
   YAMOE_TRY(launch_combine_backward<T>(gy, bd, b.f.sorted_idx, b.f.inv_pos, idx, p->idx_i64, rw, p->rw_cols, b.g_y_perm,

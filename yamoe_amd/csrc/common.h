@@ -241,12 +241,25 @@ __host__ __device__ inline int sched_grid_row_tiles(int N, int E, int small_rows
 // Every expert may be put on the streaming list in chunks of at most kStreamMaxRows rows (stream_max_rows =
 // kStreamEverything) when there are few assignments per expert on average: the weights of an expert with more rows than
 // one chunk are then read once per chunk, which is rare at that load, and the tile kernels are not launched.  16-bit data up
-// to 4; fp32, whose tiles cost as much for a row as for 32, up to 16 (us as tiles / streamed, 64 x 2
-// tokens on 16 experts of 2880 x 2880 490 / 302, 128 x 2 492 / 418, Zipf routing 572 / 405; 24 per expert as tiles 494).  The list has room for either.
+// to 4; fp32, whose tiles cost as much for a row as for 32, up to 16 (us as tiles / streamed, even routing, 64 x 2 tokens on 16
+// experts of 2880 x 2880 490 / 302, 128 x 2 491 / 387; 128 of 1024 x 1024, 384 x 4 428 / 299, 512 x 4 430 / 349).
 constexpr int kStreamEverything = -1;
 __host__ __device__ inline bool sched_may_stream_everything(int N, int E, int elem_bytes) {
   return N <= (elem_bytes == 4 ? 16ll : 4ll) * E;
 }
+// kStreamEither (fp32): everything or nothing, whichever the routing makes cheaper, and both kernels are launched.  An expert of many
+// rows costs more in chunks than in tiles: 512 x 4 tokens on 128 experts of 2880 x 2880, Zipf (2) routing, as tiles / streamed 1248 / 1771
+// us, all on one expert 900 / 1493; 96 x 4 on 32, the same, 568 / 485 and 311 / 388.  In sixths of a streamed entry of up to 16 rows, an
+// entry of more costs 9, a 128-row tile 10 for its first block of 32 rows and 4 for another (14.7 us per entry and 25 per tile
+// of one block at 2880 wide, 2.1 and 3.4 at 1024), and however few tiles there are, their launches take as long as
+// kF32FewTiles over the number of 128-wide column tiles of both products (230 us at 2880 wide, 95 at 1024).  Of 60 routings this
+// takes the slower way in one, by 3 %.
+constexpr int kStreamEither = -2, kF32FewTiles = 7000;
+__host__ __device__ inline int f32_stream_cost(int rows) { return rows / 32 * 9 + (rows % 32 == 0 ? 0 : rows % 32 <= 16 ? 6 : 9); }
+__host__ __device__ inline int f32_tile_cost(int rows) { return rows / 128 * 22 + (rows % 128 == 0 ? 0 : 6 + 4 * ((rows % 128 + 31) / 32)); }
+// Where streaming does not lose whatever the routing, since all N rows on one expert cost no more (a tenth allowed for): only
+// the streaming kernels are launched.  All on one of 2880 x 2880, as tiles / streamed: 256 rows 231 / 234 us, 384 rows 311 / 388.
+inline bool f32_streams_any_routing(int N, int cols) { return (N + 31) / 32 * 10 <= kF32FewTiles / cols; }
 __host__ __device__ inline int sched_max_small(int N, int E) {
   return (N < E ? N : E) + (sched_may_stream_everything(N, E, 4) ? N / kStreamMaxRows : 0) + 1;
 }
@@ -272,7 +285,7 @@ __host__ __device__ inline ScheduleView schedule_view(const void *p, int N, int 
 
 int route_and_schedule(const void *router_indices, int32_t idx_i64, int32_t N, int32_t E, int32_t capacity,
                        int32_t *sorted_expert, int32_t *sorted_idx, int32_t *counts, int32_t *offsets, int32_t *inv_pos,
-                       void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t tile_cols, void *schedule,
+                       void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t cols, void *schedule,
                        size_t schedule_bytes, void *stream);
 
 int regular_schedule(int *counts, int *offsets, int E, int rows, int stream_max_rows, void *schedule, size_t schedule_bytes,

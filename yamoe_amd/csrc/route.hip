@@ -157,7 +157,8 @@ __device__ inline void first_wave_exclusive_scan(const int *total, int *offsets,
 }
 
 // ---- work lists ------------------------------------------------------------------------------
-// Which experts stream: see build_schedule_wave.  cols: the column tiles of the wider product where an expert's last rows may stream, else 0.
+// Which experts stream: see build_schedule_wave.  cols: the column tiles of the wider product where an expert's last rows may stream,
+// else 0; with kStreamEither, the 128-wide column tiles of both products.
 struct StreamRule { int max_rows, cols; };
 // Where an expert has a few rows more than whole tiles, cutting all of them into equal tiles takes one tile more, which costs
 // little in a launch of many rounds and a whole round where it is the first tile of one.  There those rows go to the
@@ -177,7 +178,17 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   // they are better off as tiles (two half-filled launches one after the other are slower than one: 0.35 against
   // 0.31 ms for 32 experts of about 32 rows, where 0.27 against 0.31 ms is gained when all of them have at most 32).
   int stream_max_rows = streams.max_rows;
-  const bool everything = stream_max_rows == kStreamEverything;  // (the host checked sched_may_stream_everything)
+  bool everything = stream_max_rows == kStreamEverything;  // (the host checked sched_may_stream_everything)
+  if (stream_max_rows == kStreamEither) {
+    int as_streams = 0, as_tiles = 0;
+    for (int base = 0; base < E; base += kWave) {
+      const int kept = base + lane < E ? max(min(counts[base + lane], capacity), 0) : 0;
+      as_streams += wave_sum(f32_stream_cost(kept));
+      as_tiles += wave_sum(f32_tile_cost(kept));
+    }
+    everything = as_streams <= max(as_tiles, kF32FewTiles / streams.cols);
+    stream_max_rows = 0;
+  }
   if (everything) {  // (only then do workgroups share slabs: see stream.hip)
     stream_max_rows = kStreamMaxRows;
     int *arrivals = small + 4 * sched_max_small(N, E);
@@ -195,7 +206,7 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
     return remainders && kept > kRowTile && past <= kStreamMaxRows ? kept - past : kept;
   };
   bool remainders = false;
-  if (streams.cols > 0 && !everything) {
+  if (streams.max_rows != kStreamEither && streams.cols > 0 && !everything) {
     int all = 0, fewer = 0;
     for (int base = 0; base < E; base += kWave) {
       const int kept = base + lane < E ? max(min(counts[base + lane], capacity), 0) : 0;
@@ -598,7 +609,7 @@ extern "C" size_t yamoe_route_workspace_bytes(int32_t N, int32_t E) {
 // with more than one launch the lists come from an extra workgroup of the placement kernel.
 int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32_t N, int32_t E, int32_t capacity,
                               int32_t *sorted_expert, int32_t *sorted_idx, int32_t *counts, int32_t *offsets,
-                              int32_t *inv_pos, void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t tile_cols,
+                              int32_t *inv_pos, void *workspace, size_t workspace_bytes, int32_t stream_max_rows, int32_t cols,
                               void *schedule, size_t schedule_bytes, void *stream_) {
   hipStream_t stream = (hipStream_t)stream_;
   if (schedule != nullptr && schedule_bytes < yamoe_schedule_bytes(N, E)) {
@@ -606,7 +617,7 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
     return YAMOE_E_WORKSPACE;
   }
   if (stream_max_rows == kStreamEverything && !sched_may_stream_everything(N, E, 4)) stream_max_rows = kStreamMaxRows;
-  if (stream_max_rows < 0 && stream_max_rows != kStreamEverything) stream_max_rows = 0;
+  if (stream_max_rows < 0 && stream_max_rows != kStreamEverything && stream_max_rows != kStreamEither) stream_max_rows = 0;
   if (stream_max_rows > kStreamMaxRows) stream_max_rows = kStreamMaxRows;
   if (N < 0 || E <= 0 || E + 1 > kRouteMaxBuckets) {
     set_error("yamoe_route: need N >= 0 and 1 <= E < %d (got N=%d E=%d)", kRouteMaxBuckets, N, E);
@@ -617,7 +628,7 @@ int yamoe::route_and_schedule(const void *router_indices, int32_t idx_i64, int32
     return YAMOE_E_ARG;
   }
   if (capacity < 0) capacity = 0;
-  const StreamRule streams = {stream_max_rows, tile_cols};
+  const StreamRule streams = {stream_max_rows, cols};
   const int buckets = E + 1;
   if (N <= kSingleBlockN) {
     size_t lds = route_single_lds_bytes(N, buckets);
