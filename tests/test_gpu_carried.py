@@ -1,6 +1,8 @@
 """Who works off the streaming list where a call has at most 32 assignments per expert on average: the tile launches, where the
 routing makes tiles, and launches of its own, where it makes none.  Routings made for either, and for both kinds of expert in
 one call; contractions of whole and of cut slab pairs, 128 x 128 and 256 x 256 tiles."""
+import ctypes
+
 import pytest
 import torch
 
@@ -40,7 +42,8 @@ def test_streamed_beside_tiles_or_alone(gpu, dtype, H, I, rows):
 @pytest.mark.parametrize("rows,capacity", [([270] * 8, 0), ([257, 288, 256, 289, 512, 513, 544, 545], 0), ([288] * 7 + [20], 0),
                                            ([300] * 8, 272), ([400] * 8, 256), ([1, 16, 33, 0] + [272] * 8, 0)])
 def test_last_rows_beside_whole_tiles(gpu, dtype, H, I, rows, capacity):
-    """Experts of a few rows more than whole tiles, in numbers that make the wider product a round longer: those rows stream."""
+    """Experts of a few rows more than whole tiles, in numbers that make the gate_up product a round longer, up to
+    more of them than stream."""
     import yamoe_amd
     print("remainders", dtype, H, I, rows, capacity, flush=True)
     T, E = sum(rows), len(rows)
@@ -56,3 +59,28 @@ def test_last_rows_beside_whole_tiles(gpu, dtype, H, I, rows, capacity):
     gy = torch.randn(T, H, generator=torch.Generator().manual_seed(3)).to(dtype).to(gpu)
     for a, b in zip(yamoe_amd.experts_backward_kept(gy, *g, kept, capacity, E, 1), yamoe_amd.experts_backward(gy, *g, capacity, E, 1)):
         assert O.rel_l2(a.cpu(), b.cpu()) < REL_L2_TOL[dtype]
+
+
+@pytest.mark.parametrize("H,I", [(64, 2304), (136, 2296)])
+@pytest.mark.parametrize("rows,tiles,listed", [
+    ([270] * 3 + [512] * 4 + [256], 12, 3), ([257, 288, 273] + [512] * 4 + [256], 12, 3),  # a round less, few enough rows
+    ([270] * 8, 8, 8), ([270] * 14, 28, 0), ([270] * 11 + [512] * 2 + [256], 27, 0),       # up to four slabs for five CUs
+    ([512] * 5 + [270, 0, 0], 12, 0),                                                      # no round less
+    ([768] * 13 + [522, 256, 0], 42, 1),                                                   # the fourth round
+    ([38 * 256 + 10] + [256] * 4 + [0] * 11, 43, 0)])                                      # the same, most rows on one expert
+def test_which_last_rows_stream(gpu, H, I, rows, tiles, listed):
+    """The work lists themselves, read from the workspace, behind the five lists of the routing."""
+    from yamoe_amd import _cabi
+    print("last rows", H, I, rows[:8], flush=True)
+    T, E = sum(rows), len(rows)
+    d = make_inputs(T, H, I, E, 1, torch.bfloat16, seed=T, w_std=0.05, bias_std=0.1)
+    d["router_indices"] = routed(rows)
+    d["routing_weights"] = (0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))).to(torch.bfloat16)
+    g = args(to_dev(d, gpu))
+    p = _cabi.problem(*g[:4], T)
+    ws = torch.zeros(_cabi.lib().yamoe_experts_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device=gpu)
+    out = _cabi.experts_forward(*g, T, workspace=ws, out=torch.full_like(g[0], float("nan")))
+    up = lambda n: (n + 255) // 256 * 256
+    at = 3 * up(4 * T) + up(4 * E) + up(4 * E + 4)
+    assert ws[at:at + 16].view(torch.int32).tolist() == [tiles, listed, sum(n > 0 for n in rows), T]
+    assert O.rel_l2(out.cpu(), O.experts_capacity(*args(d), T, compute_dtype=torch.float32)) < REL_L2_TOL[torch.bfloat16]

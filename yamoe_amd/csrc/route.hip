@@ -157,14 +157,23 @@ __device__ inline void first_wave_exclusive_scan(const int *total, int *offsets,
 }
 
 // ---- work lists ------------------------------------------------------------------------------
-// Which experts stream: see build_schedule_wave.  cols: the column tiles of the wider product where an expert's last rows may stream,
-// else 0; with kStreamEither, the 128-wide column tiles of both products.
+// Which experts stream: see build_schedule_wave.  cols: the column tiles of the gate_up product where an expert's last rows may
+// stream, else 0; with kStreamEither, the 128-wide column tiles of both products.
 struct StreamRule { int max_rows, cols; };
 // Where an expert has a few rows more than whole tiles, cutting all of them into equal tiles takes one tile more, which costs
 // little in a launch of many rounds and a whole round where it is the first tile of one.  There those rows go to the
-// streaming list, if that saves the wider product a round: its launch then carries them on CUs that have no tile.  2003 tokens x
+// streaming list, if that saves the gate_up product a round (a round of it takes at least as long as one of the down product in
+// layers and slices of them, whose I is at most H): its launch then carries them on CUs that have no tile.  2003 tokens x
 // 4 on 32 experts, 2880 x 720, 258 gate_up tiles on 256 CUs: 128 + 72 us, and 89 + 64 with 12 experts' last rows streamed.
-constexpr int kRemainderRounds = 4;  // (beyond, a round is little of a launch)
+// They read the expert's weights once more, behind the tiles on CUs that are not idle, so there may be at most four slabs of them (two
+// per column tile) for five CUs, those that the tiles leave idle in their last round counted twice.  Whole forwards, us, tiled /
+// streamed: 2032 x 4 on 32, 2880 x 720, 192 slabs, 64 CUs idle 226 / 187, 264 slabs, 52 idle 205 / 210; 2007 x 4 on 32, 2880 x 1440, 264,
+// 116 idle 312 / 285, about 2150 x 4, 504, 80 idle 328 / 359; about 2000 x 4 on 32 of 1024 x 1024, none idle, 160: 102 / 96, 208: 102 /
+// 102, 224: 99 / 106; about 2000 x 8 on 64 of 2048 x 1024, none idle, 80: 324 / 303, 288: 304 / 335.
+// A round is little of a launch beyond four of them, and beyond three where an expert has more than six times the average rows:
+// 115 drawn calls that the rest of the rule takes, streamed over tiled, 0.90 in the mean for 2 rounds (0.78 to 1.045), 0.92 for 3 (0.81 to
+// 1.02), 0.96 for 4 (0.87 to 1.026), but 1.00 (0.946 to 1.044) for 4 with such an expert.
+constexpr int kRemainderRounds = 4;
 
 // One wave; lane l takes experts l, l+64, ...  Experts with 1..stream_max_rows kept rows go to the
 // streaming list, larger ones are cut into row tiles of kRowTile rows.  Both lists stay in expert
@@ -208,13 +217,17 @@ __device__ inline void build_schedule_wave(const int *counts, const int *offsets
   bool remainders = false;
   if (streams.max_rows != kStreamEither && streams.cols > 0 && !everything) {
     int all = 0, fewer = 0;
+    bool skewed = false;
     for (int base = 0; base < E; base += kWave) {
       const int kept = base + lane < E ? max(min(counts[base + lane], capacity), 0) : 0;
       all += wave_sum(ceil_div(tiled_rows(kept, false), kRowTile));
       fewer += wave_sum(ceil_div(tiled_rows(kept, true), kRowTile));
+      skewed |= __any((long long)kept * E > 6ll * N);
     }
     const int rounds = ceil_div(all * streams.cols, kXcds * kXcdCus);
-    remainders = rounds <= kRemainderRounds && ceil_div(fewer * streams.cols, kXcds * kXcdCus) < rounds;
+    const int left = ceil_div(fewer * streams.cols, kXcds * kXcdCus), idle = left * kXcds * kXcdCus - fewer * streams.cols;
+    remainders = rounds <= kRemainderRounds - skewed && left < rounds &&
+                 (all - fewer) * 2 * streams.cols * 5 <= (kXcds * kXcdCus + idle) * 4;
   }
   for (int base = 0; base < E; base += kWave) {
     int e = base + lane;
