@@ -16,16 +16,20 @@
 // on the device: us for 1 / 2 / 3 / 4 / 6 / 8 parts, 46 slabs of 90 steps 20.1 / 14.3 / 11.6 / 10.6 / 11.9 / 11.0, 92: 21.1 / 15.6 / 17.8 /
 // 15.9 / 16.7 / 15.6, 161: 22.6 / 25.3 / 21.6 / 23.4 / 25.7 / 25.4, 180: 23.4 / 25.4 / 26.1 / 24.7 / 26.7 / 27.5, 64 of 32 steps: 11.7 /
 // 10.2 / 8.5 / 8.0 / 9.0 / 9.4, 144 of 32: 12.5 / 14.4 / 12.2 / 13.7 / 15.9 / -, 112 of 16: 7.0 / 8.0 / 7.7 / 7.9 / 8.5 / 11.1 (workgroups
-// of four waves, weights from memory): many parts of a short contraction cost more than they spread.  Where the list has at most a slab per CU, a workgroup takes
-// eight waves with three steps in flight each, as much as a CU holds, folded into the first four before the same finish: one
-// token on four experts 44.9 us, with four waves 47.5 (four tokens x 4 on 32 experts, 1024 wide: 28.6 and 30.5).
+// of four waves, weights from memory): many parts of a short contraction cost more than they spread.  Where no list of the call
+// can have more than a slab per CU, a workgroup takes eight waves with three steps in flight each, as much as a CU holds,
+// folded into the first four before the same finish: one token on four experts 44.9 us, with four waves 47.5 (four tokens x 4 on
+// 32 experts, 1024 wide: 28.6 and 30.5).
 //
 // An XCD's workgroups take neighbouring slabs, eight at a time.  Where a weight row is not a whole number of cache lines, a
 // slab's piece of it shares a line with the next slab's, and both come from memory unless they meet in one L2: 64 experts, 2048 x
 // 1544, 16 tokens x 8, whole layer 206 us with neighbours on different XCDs, 200 / 196 / 194 / 193 in groups of 2 / 4 / 8 / 16.  Whole
-// lines gain up to 2 % (64 tokens of the 128-expert layer 812 / 806 / 806 / 796 / 797).  One stretch for each XCD gains no more,
-// and with a skewed routing the experts of many rows meet on one (24 x 8 on 64, 2880 wide, Zipf: 251 us dealt out one by one, 263 in
-// stretches, 250 in groups of eight).
+// lines gain up to 2 % (64 tokens of the 128-expert layer 812 / 806 / 806 / 796 / 797), but lose where the list is short, since groups
+// of eight put 32 slabs on one XCD and 24 on another where 28 each would do: up to kXcdGroupFrom workgroups they are dealt out one
+// by one.  168 products of up to 1024 workgroups in groups over one by one: whole lines 1.013 in the mean (0.89 to 1.22; 224 slabs of 64
+// steps 24.8 / 23.4 us, 225 of 90 30.0 / 27.4), cut lines 0.94 (0.91 to 0.99; 192 of 90, 28.8 / 31.0).  One stretch for each XCD
+// gains no more, and with a skewed routing the experts of many rows meet on one (24 x 8 on 64, 2880 wide, Zipf: 251 us dealt out one by
+// one, 263 in stretches, 250 in groups of eight).
 //
 // fp32 takes the same path with v_mfma_f32_16x16x4_f32.  One token on two experts of 2880 x 2880: 229 us on the tile kernel, 53
 // so; 32 x 2 on 16 of them 489 / 267; 128 x 2 492 / 418; 16 x 4 on 32, 1024 wide, 123 / 74.
@@ -42,7 +46,7 @@
 namespace yamoe {
 
 constexpr int kStreamManyWaves = 8, kStreamMaxParts = 8, kStreamMostShared = 1024;
-constexpr int kXcdGroup = 8;
+constexpr int kXcdGroup = 8, kXcdGroupFrom = 1024;
 constexpr int kChipCus = kXcds * kXcdCus;
 
 // How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
@@ -76,7 +80,7 @@ __global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void 
   const int parts = args.partial != nullptr ? stream_parts(slabs, ceil_div(args.Kd, StreamStep<T>::kRows), WAVES) : 1;
   const int total = slabs * parts;
   int b = blockIdx.x;
-  {  // workgroup b runs on XCD b % 8: groups of kXcdGroup neighbours there, the groups dealt to the XCDs in turn
+  if (args.cut_lines || total > kXcdGroupFrom) {  // workgroup b runs on XCD b % 8: groups of neighbours there, dealt to the XCDs in turn
     const int place = b / kXcds, group = place / kXcdGroup;
     b = (group * kXcds + b % kXcds) * kXcdGroup + place % kXcdGroup;
   }
@@ -117,6 +121,7 @@ template <typename T, bool GLU, bool GATHER>
 static int launch_stream(StreamArgs a, float *partial, hipStream_t stream) {
   a.n_slabs = ceil_div(a.Nd, kSlabCols);
   a.slab_div = make_fast_div(a.n_slabs);
+  a.cut_lines = a.Nd * (int)sizeof(T) % 128 != 0;
   a.partial = partial;
   a.part_floats = stream_part_floats(a.N);
   a.arrivals = const_cast<int *>(schedule_view(a.sched, a.N, a.E).arrivals);

@@ -76,6 +76,7 @@ struct StreamArgs {
   // finishes the slab.
   int part_floats;
   bool yields;   // where there are tiles, their launches carry the list
+  bool cut_lines;  // a weight row is not a whole number of cache lines
   float *partial;
   int *arrivals;
 };
