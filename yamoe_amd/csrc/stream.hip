@@ -50,20 +50,20 @@ constexpr int kXcdGroup = 8, kXcdGroupFrom = 1024;
 constexpr int kChipCus = kXcds * kXcdCus;
 
 // How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
-// fewest steps on the CU that gets most of them, where a workgroup's start and finish cost about as much as 14 steps, the
-// parts' way through memory as 6, and another 2 for each part that the last one reads.  (Fitted to 154 lists of 16 to 1440 slabs of
-// 16 to 90 steps: 1 % over the best number of parts on average, 10 % in the worst of them.  With ten steps for the sharing and none
-// for a workgroup's start it was 2.7 and 25 %: 9 x 4 tokens on 64 experts, 1024 wide, Zipf (2) routing, 144 slabs in seven parts,
-// whole layer 29.8 us, 27.0 so, 26.7 unshared with eight waves; 5 x 4 on 128, Zipf, 30.9 / 28.0.)
+// fewest steps on the CU that gets most of them, where every wave of a workgroup takes as long as the one with most steps, a
+// workgroup's start and finish cost about as much as 16 steps, the parts' way through memory as 6, and each part one more.  (Fitted
+// to 154 lists of 16 to 1440 slabs of 16 to 90 steps: 0.6 % over the best number of parts on average, 10 % in the worst of them.  With
+// ten steps for the sharing and none for a workgroup's start it was 1.9 and 25 %: 9 x 4 tokens on 64 experts, 1024 wide, Zipf (2)
+// routing, 144 slabs in seven parts, whole layer 29.8 us, 27.0 so, 26.7 unshared with eight waves; 5 x 4 on 128, Zipf, 30.9 / 28.0.)
 __host__ __device__ inline int stream_parts(int slabs, int steps, int waves) {
-  int best = 1, cost = ceil_div(slabs, kChipCus) * (steps + 14);
+  auto steps_of = [&](int parts) { return ceil_div(ceil_div(steps, parts), waves) * waves + 16; };
+  int best = 1, cost = ceil_div(slabs, kChipCus) * steps_of(1);
   if (slabs > kSchedArrivals) return 1;
   const int most = waves == kStreamManyWaves ? kChipCus : kStreamMostShared;
 #pragma unroll
-  for (int p = 2; p <= kStreamMaxParts; ++p) {  // (unrolled: divisions by constants)
-    if (p == 5 || p == 7) continue;  // (never better than a neighbour by more than the runs differ)
-    const int c = ceil_div(slabs * p, kChipCus) * (ceil_div(steps, p) + 14) + 6 + 2 * p;
-    if (slabs * p <= most && steps >= 4 * p && c < cost) { best = p; cost = c; }
+  for (int p = 2; p <= kStreamMaxParts; ++p) {  // (unrolled: divisions by constants; seven parts: never better than six or eight)
+    const int c = ceil_div(slabs * p, kChipCus) * steps_of(p) + 6 + p;
+    if (p != 7 && slabs * p <= most && steps >= 4 * p && c < cost) { best = p; cost = c; }
   }
   return best;
 }
