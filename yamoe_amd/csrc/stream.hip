@@ -62,8 +62,9 @@ __host__ __device__ inline int stream_parts(int slabs, int steps, int waves) {
   const int most = waves == kStreamManyWaves ? kChipCus : kStreamMostShared;
 #pragma unroll
   for (int p = 2; p <= kStreamMaxParts; ++p) {  // (unrolled: divisions by constants; seven parts: never better than six or eight)
+    if (slabs * p > most || steps < 4 * p) break;
     const int c = ceil_div(slabs * p, kChipCus) * steps_of(p) + 6 + p;
-    if (p != 7 && slabs * p <= most && steps >= 4 * p && c < cost) { best = p; cost = c; }
+    if (p != 7 && c < cost) { best = p; cost = c; }
   }
   return best;
 }
