@@ -1,6 +1,6 @@
 """Who works off the streaming list where a call has at most 32 assignments per expert on average: the tile launches, where the
 routing makes tiles, and launches of its own, where it makes none.  Routings made for either, and for both kinds of expert in
-one call; contractions of whole and of cut slab pairs, 128 x 128 and 256 x 256 tiles."""
+one call; contractions of whole and of cut slab pairs, 128 x 128 tiles and (further down) 256 x 256 ones."""
 import ctypes
 
 import pytest
@@ -35,6 +35,28 @@ def test_streamed_beside_tiles_or_alone(gpu, dtype, H, I, rows):
     want = O.experts_capacity(*args(d), T, compute_dtype=torch.float32)
     assert O.rel_l2(out.cpu(), want) < REL_L2_TOL[dtype]
     assert torch.equal(out, yamoe_amd.experts(*g, T, E, 1))
+
+
+@pytest.mark.parametrize("E,H,I", [(32, 1032, 520), (32, 1088, 576),  # both products on 256 x 256 tiles, in up to four estimated rounds
+                                   (64, 264, 4088)])                  # gate_up on such tiles, in more than four
+@pytest.mark.parametrize("tiled,streamed,few", [(0, 8, 8), (0, 31, 3), (1, 8, 8), (1, 16, 1), (3, 5, 0), (8, 2, 3)])
+def test_large_tiles_carry_the_list_or_leave_it(gpu, E, H, I, tiled, streamed, few):
+    """`tiled` experts of 33 to 160 rows, the others of up to `streamed`; expert by expert, so that one that nobody serves shows."""
+    import yamoe_amd
+    print("large tiles", E, H, I, tiled, streamed, few, flush=True)
+    rows = [33 + 127 * e // max(tiled - 1, 1) for e in range(tiled)] + [(streamed, few)[e % 2] for e in range(E - tiled)]
+    T, cols = sum(rows), lambda n, width: (n + width - 1) // width
+    rounds = (T + 128 * E) // 256 * cols(max(H, 2 * I), 256) / 256
+    assert 4 * E < T <= 32 * E and E * cols(2 * I, 128) > 256          # not everything streams, gate_up on large tiles
+    assert rounds <= 4 and E * cols(H, 128) > 256 if E == 32 else 4 < rounds <= 16 and T <= 24 * E
+    d = make_inputs(T, H, I, E, 1, torch.bfloat16, seed=T, w_std=0.05, bias_std=0.1)
+    d["router_indices"] = routed(rows)
+    d["routing_weights"] = (0.1 + torch.rand(T, E, generator=torch.Generator().manual_seed(T))).to(torch.bfloat16)
+    out = yamoe_amd.experts(*args(to_dev(d, gpu)), T, E, 1).cpu()
+    want = O.experts_capacity(*args(d), T, compute_dtype=torch.float32)
+    for e in range(E):
+        mine = d["router_indices"][:, 0] == e
+        assert not mine.any() or O.rel_l2(out[mine], want[mine]) < REL_L2_TOL[torch.bfloat16], e
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

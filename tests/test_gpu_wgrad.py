@@ -35,8 +35,9 @@ def test_weight_gradients_by_rows(gpu, dtype, H, I, rows):
 @pytest.mark.parametrize("H,I", [(24, 72), (128, 136), (264, 500 // 8 * 8), (1024, 128)])
 @pytest.mark.parametrize("rows", [1, 31, 32, 33, 64, 65, 80, 97, 111, 112, 113, 128, 129, 160, 193])
 def test_weight_and_bias_gradients_of_one_expert(gpu, dtype, H, I, rows):
-    """Either kernel (the line between them is at the average rows of an expert), rows around whole slabs; gradients of fewer
-    than 32 rows, of whole and of cut tiles, of whole and of cut cache lines; the bias gradients, which they sum beside."""
+    """Either kernel (small tiles up to 32 rows per expert on average, and up to 112 where no routing gives an expert more than 128:
+    with a single expert, up to 112), rows around whole slabs; gradients of fewer than 32 rows, of whole and of cut tiles, of
+    whole and of cut cache lines; the bias gradients, which they sum beside."""
     import yamoe_amd
     print("wgrad one", dtype, H, I, rows, flush=True)
     d = make_inputs(rows, H, I, 1, 1, dtype, seed=rows, w_std=0.05, bias_std=0.1)
