@@ -24,10 +24,11 @@
 // An XCD's workgroups take neighbouring slabs, eight at a time.  Where a weight row is not a whole number of cache lines, a
 // slab's piece of it shares a line with the next slab's, and both come from memory unless they meet in one L2: 64 experts, 2048 x
 // 1544, 16 tokens x 8, whole layer 206 us with neighbours on different XCDs, 200 / 196 / 194 / 193 in groups of 2 / 4 / 8 / 16.  Whole
-// lines gain up to 2 % (64 tokens of the 128-expert layer 812 / 806 / 806 / 796 / 797), but lose where the list is short, since groups
-// of eight put 32 slabs on one XCD and 24 on another where 28 each would do: up to kXcdGroupFrom workgroups they are dealt out one
-// by one.  168 products of up to 1024 workgroups in groups over one by one: whole lines 1.013 in the mean (0.89 to 1.22; 224 slabs of 64
-// steps 24.8 / 23.4 us, 225 of 90 30.0 / 27.4), cut lines 0.94 (0.91 to 0.99; 192 of 90, 28.8 / 31.0).  One stretch for each XCD
+// lines gain up to 2 % (64 tokens of the 128-expert layer 812 / 806 / 806 / 796 / 797), and more where experts have rows that their
+// slabs share (16 experts of 1024 x 1024, whole layer one by one / in groups: 12 rows each 38.1 / 36.3 us, 5 rows 35.0 / 34.0).  But
+// groups of eight put 32 slabs of a short list on one XCD and 24 on another where 28 each would do, so with up to kXcdGroupRows
+// rows per expert and kXcdGroupFrom workgroups whole lines are dealt out one by one: 168 such products of one row per expert
+// 1.013 in groups (0.89 to 1.22; 224 slabs of 64 steps 24.8 / 23.4 us, 225 of 90 30.0 / 27.4), cut lines 0.94.  One stretch for each XCD
 // gains no more, and with a skewed routing the experts of many rows meet on one (24 x 8 on 64, 2880 wide, Zipf: 251 us dealt out one by
 // one, 263 in stretches, 250 in groups of eight).
 //
@@ -46,7 +47,7 @@
 namespace yamoe {
 
 constexpr int kStreamManyWaves = 8, kStreamMaxParts = 8, kStreamMostShared = 1024;
-constexpr int kXcdGroup = 8, kXcdGroupFrom = 1024;
+constexpr int kXcdGroup = 8, kXcdGroupFrom = 1024, kXcdGroupRows = 4;
 constexpr int kChipCus = kXcds * kXcdCus;
 
 // How many workgroups of `waves` waves share the contraction of a slab, for `slabs` of them of `steps` steps each: what takes the
@@ -81,7 +82,8 @@ __global__ __launch_bounds__(kWave * WAVES, WAVES == kStreamWaves ? 2 : 1) void 
   const int parts = args.partial != nullptr ? stream_parts(slabs, ceil_div(args.Kd, StreamStep<T>::kRows), WAVES) : 1;
   const int total = slabs * parts;
   int b = blockIdx.x;
-  if (args.cut_lines || total > kXcdGroupFrom) {  // workgroup b runs on XCD b % 8: groups of neighbours there, dealt to the XCDs in turn
+  // workgroup b runs on XCD b % 8: groups of neighbours there, dealt to the XCDs in turn (hdr[3]: the rows of all experts)
+  if (args.cut_lines || total > kXcdGroupFrom || sv.hdr[3] > kXcdGroupRows * sv.hdr[1]) {
     const int place = b / kXcds, group = place / kXcdGroup;
     b = (group * kXcds + b % kXcds) * kXcdGroup + place % kXcdGroup;
   }
