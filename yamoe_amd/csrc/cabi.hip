@@ -397,6 +397,11 @@ static size_t carve_saved(const yamoe_problem *p, void *base, Saved *s) {
 // between, 171 x 8 on 64, 2880 wide, 619 / 568 / 571.  In launches of 4 to 16 estimated rounds, apart / so: 155 x 4 on 128, Zipf, 2880 x
 // 2080, 249 / 218, 744 x 4 on 128, even, 2048 wide, 612 / 584, 815 x 4, Zipf, 2880 wide, 571 / 569, but 916 x 4 578 / 593: there up to 24
 // assignments per expert.
+// One tile is enough for that, however many experts stream.  1 to 16 experts of 40 or 120 rows beside 31 to 127 streamed ones, 270 calls,
+// over the same launches apart: 0.69 to 1.00 in nearly all; up to 1.02 where no expert streams (17 rows or more each and one of
+// more than 32: what 256 more workgroups of a launch cost, 2 to 3 us) and 1.03 in launches of 4 to 16 rounds (4 experts of 120 rows and
+// 124 streamed, 2880 wide, 967 / 995 us; 16 and 112, of 40 rows, 975 / 984).  Where weight rows cut cache lines a list in launches of
+// its own is up to 9 % faster still (128 experts of 2048 x 1432, 8 of 120 rows, 436 / 476): its slabs go to the XCDs in groups there.
 static int tiles_carry_streams(int N, int E, int H, int I) {
   const long long cols = ceil_div(H > 2 * I ? H : 2 * I, kColTile), rows = ((long long)N + 128ll * E) / kRowTile;
   if (rows * cols <= 4 * 256) return N > 32ll * E ? CARRY_ALWAYS : CARRY_WITH_TILES;
@@ -617,7 +622,10 @@ static int down_both(const void *act, const void *w, const void *bias, void *y, 
 }
 // The same for E groups of `rows` rows each: whether they stream or are tiles is known on the host, so only one of the two
 // kernels is launched (the other would find an empty list for 4 us), and 16-bit tiles need no work list (a launch of 3.5 to 5
-// us, which is what the list of yamoe_build_schedule, counts and offsets take where they are made).
+// us, which is what the list of yamoe_build_schedule, counts and offsets take where they are made).  Groups of up to 32 rows stream
+// in fp32 as well, us as tiles / streamed, 17, 24 and 32 rows: 16 groups of 2880 x 2880 190 / 133, 190 / 143, 190 / 151; 32 of 2048 x 5760
+// 400 / 360, 401 / 371, 401 / 382; 64 of 1024 x 1024 73 / 56, 74 / 58, 74 / 61; a router's input gradient, 128 experts, 2880 wide, 24
+// tokens 25.3 / 22.6, 32 24.8 / 22.2.
 template <typename T>
 static int down_regular(const void *act, const void *w, const void *bias, void *y, int *counts, int *offsets, void *sched,
                         size_t sched_bytes, int E, int rows, int H, int I, hipStream_t stream) {

@@ -672,11 +672,11 @@ __device__ __forceinline__ void run_tile(const Args &args, const TileInfo &ti, c
 
 // One workgroup's part of the streaming list: items `first`, first + step, ...  An item is a slab of one expert, and
 // neighbouring items, which different XCDs work on, are neighbouring slabs.  (17 to 32 rows as the last rows of an
-// expert beside its tiles, or where invalid ids leave no expert more: a capacity that does keeps the tiles' launches away.)  Two launches less per layer: 2048 tokens x 2 on 16
-// experts, 1024 wide, whole layer 81.6 -> 78.1 us, 426 x 2: 42.4 -> 39.5.  In launches of many rounds these workgroups took the
-// time of the streaming kernel to the microsecond, behind the tiles or between the first of them (Zipf routing, 16 384
-// tokens: gate_up 1794 + 266 and 2063 us); in short ones they are best behind the tiles (in front of them: 150 drawn calls 0.996 in the
-// mean, single ones up to 1.24).
+// expert beside its tiles, or where invalid ids leave no expert more: a capacity that does keeps the tiles' launches away.)  Two
+// launches less per layer: 2048 tokens x 2 on 16 experts, 1024 wide, whole layer 81.6 -> 78.1 us, 426 x 2: 42.4 -> 39.5.  In
+// launches of many rounds these workgroups took the time of the streaming kernel to the microsecond, behind the tiles or
+// between the first of them (Zipf routing, 16 384 tokens: gate_up 1794 + 266 and 2063 us); in short ones they are best behind
+// the tiles (in front of them: 150 drawn calls 0.996 in the mean, single ones up to 1.24).
 static_assert(kThreads == kStreamWaves * kWave, "a workgroup of the tile kernels is one of the streaming kernel");
 template <typename T, int EPI, bool GATHER, int DEPTH> __device__ __forceinline__ void stream_items(const Args &args, int first, int step) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
