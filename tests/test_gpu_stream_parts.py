@@ -125,3 +125,24 @@ def test_fp32_streams_everything_or_nothing_by_the_routing(gpu, rows, streams):
     gy = r(T, H)
     for a, b in zip(yamoe_amd.experts_backward_kept(gy, *g, k, T, E, 1), yamoe_amd.experts_backward(gy, *g, T, E, 1)):
         assert torch.equal(a, b)
+
+
+def test_fp32_choice_is_made_anew_at_every_replay(gpu):
+    """Captured once; the routing in the captured buffer changes between replays from one that streams to one that is tiled."""
+    import yamoe_amd
+    T, H, I, E = 2048, 1024, 512, 128
+    gen = torch.Generator(device=gpu).manual_seed(9)
+    r = lambda *s: torch.randn(*s, generator=gen, device=gpu) * 0.05
+    g = [r(T, H), torch.zeros(T, 1, dtype=torch.int64, device=gpu), 0.1 + torch.rand(T, E, generator=gen, device=gpu), r(E, H, 2 * I), r(E, 2 * I),
+         r(E, I, H), r(E, H)]
+    even, one = (torch.arange(T, device=gpu) % E).view(T, 1), torch.full((T, 1), 7, device=gpu)
+    yamoe_amd.experts(*g, T, E, 1)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = yamoe_amd.experts(*g, T, E, 1)
+    for ids in (even, one, even, one):
+        g[1].copy_(ids)
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, yamoe_amd.experts(*g, T, E, 1))
